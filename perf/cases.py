@@ -52,29 +52,29 @@ _LOGITS_VOCABS = [151936, 131072, 32768, 32000]
 def listed():
     return [
         # one sequence decoding: the smallest call, a weight read once for one token
-        {"name": "qkv, 1 token", "kind": "projection", "tokens": 1, "in": 4096, "out": 6144},
+        {"name": "qkv_1_token", "kind": "projection", "tokens": 1, "in": 4096, "out": 6144},
         # a chunk of a prompt next to decoding sequences
-        {"name": "down, 333 tokens", "kind": "projection", "tokens": 333, "in": 12288, "out": 4096},
+        {"name": "down_333_tokens", "kind": "projection", "tokens": 333, "in": 12288, "out": 4096},
         # a full packed batch of ragged sequences
-        {"name": "qkv, 16384 tokens", "kind": "projection", "tokens": 16384, "in": 4096, "out": 6144},
+        {"name": "qkv_16384_tokens", "kind": "projection", "tokens": 16384, "in": 4096, "out": 6144},
         # a decode step of 64 rollouts
-        {"name": "ffn, 64 tokens", "kind": "ffn", "tokens": 64, "hidden": 4096, "inter": 12288},
+        {"name": "ffn_64_tokens", "kind": "ffn", "tokens": 64, "hidden": 4096, "inter": 12288},
         # attention output projection in a training micro-batch of ragged sequences
-        {"name": "o_proj train, 2047 tokens", "kind": "projection_train", "tokens": 2047, "in": 4096, "out": 4096},
+        {"name": "o_proj_train_2047_tokens", "kind": "projection_train", "tokens": 2047, "in": 4096, "out": 4096},
         # the FFN of one layer in training
-        {"name": "ffn train, 4096 tokens", "kind": "ffn_train", "tokens": 4096, "hidden": 4096, "inter": 12288},
+        {"name": "ffn_train_4096_tokens", "kind": "ffn_train", "tokens": 4096, "hidden": 4096, "inter": 12288},
         # log-probs of the ids a sampler just drew, at its temperature
-        {"name": "logp, 16 tokens", "kind": "logp", "tokens": 16, "vocab": 151936, "hidden": 4096, "temperature": True},
+        {"name": "logp_16_tokens", "kind": "logp", "tokens": 16, "vocab": 151936, "hidden": 4096, "temperature": True},
         # scoring of packed rollouts
-        {"name": "logp, 8192 tokens", "kind": "logp", "tokens": 8192, "vocab": 151936, "hidden": 4096, "temperature": False},
+        {"name": "logp_8192_tokens", "kind": "logp", "tokens": 8192, "vocab": 151936, "hidden": 4096, "temperature": False},
         # one GRPO micro-batch of 8 rollouts through the lm_head, both ways
-        {"name": "logp train, 8 x 515", "kind": "logp_train", "rollouts": 8, "length": 515, "vocab": 151936, "hidden": 4096},
+        {"name": "logp_train_8x515", "kind": "logp_train", "rollouts": 8, "length": 515, "vocab": 151936, "hidden": 4096},
         # log-probs from logits the model has written already, and their gradient
-        {"name": "logits, 2048 rows", "kind": "logits", "rows": 2048, "vocab": 151936, "dtype": "bf16", "backward": True},
+        {"name": "logits_2048_rows", "kind": "logits", "rows": 2048, "vocab": 151936, "dtype": "bf16", "backward": True},
         # the loss of a whole rollout batch: many small launches in a framework that is not careful
-        {"name": "grpo, 64 x 1024", "kind": "grpo", "rollouts": 64, "length": 1024, "mask": True},
+        {"name": "grpo_64x1024", "kind": "grpo", "rollouts": 64, "length": 1024, "mask": True},
         # a prefill chunk under the contract that tensor parallelism leaves unchanged
-        {"name": "k-tree qkv, 509 tokens", "kind": "tree", "tokens": 509, "in": 4096, "out": 6144},
+        {"name": "k_tree_qkv_509_tokens", "kind": "tree", "tokens": 509, "in": 4096, "out": 6144},
     ]  # fmt: skip
 
 
