@@ -472,6 +472,19 @@ int rlk_grpo_ratio_kl_loss(const float* logp, const float* old_logp, const float
                            float clip_eps, float beta, float* ratio, float* k3, float* out3, void* workspace,
                            size_t workspace_bytes, void* stream);
 
+/*
+ * Gradient of the three scalars of rlk_grpo_ratio_kl_loss with respect to logp:
+ *   grad = ((g_loss + g_policy) * d policy_i + (beta * g_loss + g_kl) * (1 - exp(d_i))) * mask_i / max(active, 1e-8)
+ * with d policy_i = -A ratio_i where the unclipped branch is the minimum or ties it (ratio in [clip_lo, clip_hi], above
+ * it with A < 0, below it with A > 0), else 0. g_loss, g_policy and g_kl are device scalars or NULL (zero); `workspace`
+ * is the one the forward wrote for the same inputs (it holds the active tokens of every sequence); clip_lo / clip_hi are
+ * 1 -+ clip_eps.
+ */
+int rlk_grpo_ratio_kl_loss_bwd(const float* logp, const float* old_logp, const float* ref_logp, const float* advantages,
+                               const uint8_t* mask, void* workspace, size_t workspace_bytes, const float* g_loss,
+                               const float* g_policy, const float* g_kl, int rollouts, int tokens_per_rollout,
+                               float clip_lo, float clip_hi, float beta, float* grad_logp, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -592,4 +592,28 @@ int rlk_grpo_ratio_kl_loss(const float* logp, const float* old_logp, const float
   return err == hipSuccess ? RLK_OK : device_error("rlk_grpo_ratio_kl_loss", err);
 }
 
+int rlk_grpo_ratio_kl_loss_bwd(const float* logp, const float* old_logp, const float* ref_logp, const float* advantages,
+                               const uint8_t* mask, void* workspace, size_t workspace_bytes, const float* g_loss,
+                               const float* g_policy, const float* g_kl, int rollouts, int tokens_per_rollout,
+                               float clip_lo, float clip_hi, float beta, float* grad_logp, void* stream) {
+  if (rollouts < 0 || tokens_per_rollout < 0) {
+    set_last_error("rlk_grpo_ratio_kl_loss_bwd: negative sizes");
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  if (rollouts == 0 || tokens_per_rollout == 0) return RLK_OK;
+  if (logp == nullptr || old_logp == nullptr || ref_logp == nullptr || advantages == nullptr || grad_logp == nullptr) {
+    set_last_error("rlk_grpo_ratio_kl_loss_bwd: null argument");
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  if (workspace == nullptr || workspace_bytes < rlk_grpo_workspace_bytes(rollouts)) {
+    set_last_error("rlk_grpo_ratio_kl_loss_bwd: the forward's workspace of %zu bytes needed, %zu given",
+                   rlk_grpo_workspace_bytes(rollouts), workspace_bytes);
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  hipError_t err = grpo_backward_launch(logp, old_logp, ref_logp, advantages, mask, reinterpret_cast<float*>(workspace),
+                                        g_loss, g_policy, g_kl, rollouts, tokens_per_rollout, clip_lo, clip_hi, beta,
+                                        grad_logp, reinterpret_cast<hipStream_t>(stream));
+  return err == hipSuccess ? RLK_OK : device_error("rlk_grpo_ratio_kl_loss_bwd", err);
+}
+
 }  // extern "C"

@@ -157,6 +157,11 @@ hipError_t det_gemm_swiglu_launch(const MatView& W, const MatView& X, void* Y, i
 hipError_t grpo_launch(const float* logp, const float* old_logp, const float* ref_logp, const float* advantages,
                        const uint8_t* mask, int rollouts, int tokens, float clip_eps, float beta, float* ratio,
                        float* k3, float* out3, float* workspace, hipStream_t stream);
+// Gradient of the loss triple with respect to logp; `workspace` is the one grpo_launch wrote, g_* device scalars or null.
+hipError_t grpo_backward_launch(const float* logp, const float* old_logp, const float* ref_logp, const float* advantages,
+                                const uint8_t* mask, float* workspace, const float* g_loss, const float* g_policy,
+                                const float* g_kl, int rollouts, int tokens, float clip_lo, float clip_hi, float beta,
+                                float* grad, hipStream_t stream);
 
 void set_last_error(const char* fmt, ...);
 

@@ -916,6 +916,13 @@ def det_gemm_swiglu(a: torch.Tensor, weight: torch.Tensor, out: Optional[torch.T
     return out
 
 
+def _grpo_mask(mask: torch.Tensor, device: torch.device) -> torch.Tensor:
+    """The mask as bytes: any non-zero value keeps the token (mask.bool(), rl_engine/reference/definitions.py:50-70)."""
+    if mask.dtype != torch.bool or mask.device != device:
+        mask = mask.to(device=device).bool()
+    return mask.contiguous().view(torch.uint8)  # a bool is a byte of 0 or 1: no conversion
+
+
 def grpo_ratio_kl_loss(
     logp: torch.Tensor,
     old_logp: torch.Tensor,
@@ -930,6 +937,20 @@ def grpo_ratio_kl_loss(
     ``logp`` / ``old_logp`` / ``ref_logp`` are fp32 ``[rollouts, tokens]``,
     ``advantages`` fp32 ``[rollouts]``, ``mask`` bool/uint8 ``[rollouts, tokens]`` or None.
     """
+    return grpo_ratio_kl_loss_saved(logp, old_logp, ref_logp, advantages, mask, clip_eps, beta)[:3]
+
+
+def grpo_ratio_kl_loss_saved(
+    logp: torch.Tensor,
+    old_logp: torch.Tensor,
+    ref_logp: torch.Tensor,
+    advantages: torch.Tensor,
+    mask: Optional[torch.Tensor],
+    clip_eps: float,
+    beta: float,
+) -> tuple:
+    """:func:`grpo_ratio_kl_loss` plus what its backward reads: ``(loss3, ratio, k3, inputs, workspace)`` with the
+    contiguous ``inputs = (logp, old_logp, ref_logp, advantages, mask bytes or None)``."""
     for name, t in (("logp", logp), ("old_logp", old_logp), ("ref_logp", ref_logp), ("advantages", advantages)):
         if not t.is_cuda:
             raise RuntimeError(f"grpo_ratio_kl_loss: {name} must be a CUDA tensor")
@@ -946,8 +967,7 @@ def grpo_ratio_kl_loss(
     if mask is not None:
         if tuple(mask.shape) != (rollouts, tokens):
             raise RuntimeError("grpo_ratio_kl_loss: mask shape must match logp")
-        # any non-zero mask value keeps the token (mask.bool(), rl_engine/reference/definitions.py:50-70)
-        mask_u8 = mask.to(device=logp.device).bool().to(torch.uint8).contiguous()
+        mask_u8 = _grpo_mask(mask, logp.device)
     lib = _lib.load()
     ratio = torch.empty_like(logp_c)
     k3 = torch.empty_like(logp_c)
@@ -973,4 +993,29 @@ def grpo_ratio_kl_loss(
             _stream_handle(logp.device),
         )
     _lib.check(status, "rlk_grpo_ratio_kl_loss failed")
-    return [out3, ratio, k3]
+    return [out3, ratio, k3, (logp_c, old_c, ref_c, adv_c, mask_u8), workspace]
+
+
+def grpo_ratio_kl_loss_bwd(
+    inputs: tuple,
+    workspace: torch.Tensor,
+    g_loss: Optional[torch.Tensor],
+    g_policy: Optional[torch.Tensor],
+    g_kl: Optional[torch.Tensor],
+    clip_eps: float,
+    beta: float,
+) -> torch.Tensor:
+    """d(loss3 . (g_loss, g_policy, g_kl)) / d(logp), fp32 ``[rollouts, tokens]``; ``inputs`` and ``workspace`` as
+    :func:`grpo_ratio_kl_loss_saved` returned them, ``g_*`` fp32 scalars or None (zero)."""
+    logp, old, ref, adv, mask = inputs
+    rollouts, tokens = logp.shape
+    grad = torch.empty_like(logp)
+    with _on(logp.device):
+        status = _lib.load().rlk_grpo_ratio_kl_loss_bwd(
+            logp.data_ptr(), old.data_ptr(), ref.data_ptr(), adv.data_ptr(), mask.data_ptr() if mask is not None else None,
+            workspace.data_ptr(), workspace.numel() * 4,
+            *(g.data_ptr() if g is not None else None for g in (g_loss, g_policy, g_kl)),
+            rollouts, tokens, 1.0 - clip_eps, 1.0 + clip_eps, beta, grad.data_ptr(), _stream_handle(logp.device),
+        )  # fmt: skip
+    _lib.check(status, "rlk_grpo_ratio_kl_loss_bwd failed")
+    return grad

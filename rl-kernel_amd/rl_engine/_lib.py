@@ -83,6 +83,7 @@ EXPORTED_SYMBOLS = (
     "rlk_det_gemm_swiglu_bf16",
     "rlk_grpo_workspace_bytes",
     "rlk_grpo_ratio_kl_loss",
+    "rlk_grpo_ratio_kl_loss_bwd",
 )
 
 
@@ -185,6 +186,8 @@ def load() -> ctypes.CDLL:
     lib.rlk_grpo_workspace_bytes.argtypes = [i32]
     lib.rlk_grpo_ratio_kl_loss.restype = i32
     lib.rlk_grpo_ratio_kl_loss.argtypes = [vp, vp, vp, vp, vp, i32, i32, f32, f32, vp, vp, vp, vp, sz, vp]
+    lib.rlk_grpo_ratio_kl_loss_bwd.restype = i32
+    lib.rlk_grpo_ratio_kl_loss_bwd.argtypes = [vp, vp, vp, vp, vp, vp, sz, vp, vp, vp, i32, i32, f32, f32, f32, vp, vp]
     _lib = lib
     return lib
 

@@ -37,8 +37,25 @@ def _bool_mask(mask: torch.Tensor, device: torch.device) -> torch.Tensor:
     return _as_2d(mask).to(device=device).bool()
 
 
+def _elementwise_gradient(cur, old, ref, adv, mask, g_loss, g_policy, g_kl, clip_eps: float, beta: float) -> torch.Tensor:
+    """The gradient of the backward kernel in differentiable tensor operations (the same values)."""
+    keep = torch.ones_like(cur) if mask is None else mask.to(torch.float32)
+    count = torch.clamp(keep.sum(), min=1e-8)
+    a = adv.reshape(-1, 1)
+    r = torch.exp(cur - old)
+    lo, hi = 1.0 - clip_eps, 1.0 + clip_eps
+    flows = ((r >= lo) & (r <= hi)) | ((r > hi) & (a < 0)) | ((r < lo) & (a > 0))
+    d_policy = -(a * r) * flows.to(torch.float32)
+    d_kl = 1.0 - torch.exp(ref - cur)
+    zero = torch.zeros((), dtype=torch.float32, device=cur.device)
+    g_loss = zero if g_loss is None else g_loss
+    w_policy = g_loss + (zero if g_policy is None else g_policy)
+    w_kl = beta * g_loss + (zero if g_kl is None else g_kl)
+    return (w_policy * d_policy + w_kl * d_kl) * keep / count
+
+
 class _GrpoLossAutograd(torch.autograd.Function):
-    """Forward on the HIP kernel; backward elementwise on the saved per-token outputs.
+    """Forward and backward on the HIP kernels.
 
     With ``r = exp(logp - old)``, ``d = ref - logp``, ``n = max(active, 1e-8)``:
     ``d policy_i / d logp_i = -A r_i`` where the unclipped branch is the minimum or ties it
@@ -48,30 +65,26 @@ class _GrpoLossAutograd(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, cur, old, ref, adv, mask, clip_eps, beta):
-        # `mask` is already the boolean mask (see _bool_mask): the kernel and the backward weigh with the same tensor
-        out3, ratio, k3 = _C.grpo_ratio_kl_loss(cur, old, ref, adv, mask, clip_eps, beta)
-        ctx.save_for_backward(cur, old, ref, adv, mask if mask is not None else torch.empty(0, device=cur.device))
+        out3, ratio, k3, inputs, workspace = _C.grpo_ratio_kl_loss_saved(cur, old, ref, adv, mask, clip_eps, beta)
         ctx.has_mask = mask is not None
+        ctx.save_for_backward(*(inputs if ctx.has_mask else inputs[:4]), workspace)
         ctx.clip_eps, ctx.beta = float(clip_eps), float(beta)
         ctx.mark_non_differentiable(ratio, k3)
-        return out3[0], out3[1], out3[2], ratio, k3
+        ctx.set_materialize_grads(False)  # an unused output costs no zero tensor
+        loss, policy, kl = out3.unbind(0)
+        return loss, policy, kl, ratio, k3
 
     @staticmethod
     def backward(ctx, g_loss, g_policy, g_kl, _g_ratio, _g_k3):
-        cur, old, ref, adv, mask = ctx.saved_tensors
-        keep = mask.to(torch.float32) if ctx.has_mask else torch.ones_like(cur)
-        count = torch.clamp(keep.sum(), min=1e-8)
-        a = adv.reshape(-1, 1)
-        r = torch.exp(cur - old)
-        lo, hi = 1.0 - ctx.clip_eps, 1.0 + ctx.clip_eps
-        flows = ((r >= lo) & (r <= hi)) | ((r > hi) & (a < 0)) | ((r < lo) & (a > 0))
-        d_policy = -(a * r) * flows.to(torch.float32)
-        d_kl = 1.0 - torch.exp(ref - cur)
-        zero = torch.zeros((), dtype=torch.float32, device=cur.device)
-        g_loss = zero if g_loss is None else g_loss
-        w_policy = g_loss + (zero if g_policy is None else g_policy)
-        w_kl = ctx.beta * g_loss + (zero if g_kl is None else g_kl)
-        grad = (w_policy * d_policy + w_kl * d_kl) * keep / count
+        if g_loss is None and g_policy is None and g_kl is None:
+            return (None,) * 7
+        *inputs, workspace = ctx.saved_tensors
+        if not ctx.has_mask:
+            inputs.append(None)
+        if torch.is_grad_enabled():  # create_graph: the gradient itself is to be differentiated
+            grad = _elementwise_gradient(*inputs, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
+            return grad, None, None, None, None, None, None
+        grad = _C.grpo_ratio_kl_loss_bwd(inputs, workspace, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
         return grad, None, None, None, None, None, None
 
 
