@@ -405,6 +405,13 @@ int rlk_logits_logp_backward(const void* logits, int dtype, int64_t row_stride, 
                              int64_t vocab_start, int64_t real_vocab, void* stream);
 
 /*
+ * Value checks without a copy back: flags[0] is set to 1 when one of the n ids lies outside [lo, hi), flags[1] when a
+ * temperature (may be NULL) is <= 0. `flags` points to two words the device can write, normally pinned host memory that
+ * the caller has zeroed and reads after an event behind this call.
+ */
+int rlk_check_rows(const int64_t* ids, const float* temperature, int n, int64_t lo, int64_t hi, int32_t* flags, void* stream);
+
+/*
  * SwiGLU on rows of element type `dtype` (rlk_dtype: bf16, fp16 or fp32; every tensor of a
  * call has it; strides in elements): y[m, c] = round((g * sigmoid(g)) * u) with
  * g = gate[m * ld_gate + c], u = up[m * ld_up + c] widened to fp32 and

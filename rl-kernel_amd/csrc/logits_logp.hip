@@ -424,9 +424,39 @@ __global__ __launch_bounds__(256) void logits_backward_kernel(LogitsBackwardArgs
   }
 }
 
+// The value checks of the from-logits entry: flags[0] becomes 1 for an id outside [lo, hi), flags[1] for a temperature that
+// is not above zero (two words of pinned host memory, zero before the launch). One launch in front of the forward: the
+// host waits for this kernel alone, while the forward behind it already runs. (As tensor operations the checks were
+// five launches and a copy, and the device stood idle from their end until the host had launched the forward.)
+constexpr int kCheckThreads = 256;
+
+__global__ __launch_bounds__(kCheckThreads) void check_rows_kernel(const int64_t* __restrict__ ids,
+                                                                   const float* __restrict__ temperature, int n, int64_t lo,
+                                                                   int64_t hi, int* flags) {
+  int bad = 0;
+  for (int i = blockIdx.x * kCheckThreads + threadIdx.x; i < n; i += gridDim.x * kCheckThreads) {
+    if (ids[i] < lo || ids[i] >= hi) bad |= 1;
+    if (temperature != nullptr && temperature[i] <= 0.f) bad |= 2;
+  }
+  const bool any_id = __ballot(bad & 1) != 0, any_temperature = __ballot(bad & 2) != 0;
+  if ((threadIdx.x & 63) == 0) {  // whoever finds one stores the same 1
+    if (any_id) __hip_atomic_store(&flags[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (any_temperature) __hip_atomic_store(&flags[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
+
+hipError_t check_rows_launch(const int64_t* ids, const float* temperature, int n, int64_t lo, int64_t hi, int* flags,
+                             hipStream_t stream) {
+  if (n <= 0) return hipSuccess;
+  const int blocks = (n + kCheckThreads - 1) / kCheckThreads;
+  hipLaunchKernelGGL(check_rows_kernel, dim3(blocks < 64 ? blocks : 64), dim3(kCheckThreads), 0, stream, ids, temperature, n,
+                     lo, hi, flags);
+  return hipGetLastError();
+}
 
 static int tiles_per_group_for(int T, int num_tiles) {
   // Enough workgroups to fill 256 CUs several times over when T is small; one workgroup

@@ -477,6 +477,15 @@ int rlk_logits_logp_backward(const void* logits, int dtype, int64_t row_stride, 
   return err == hipSuccess ? RLK_OK : device_error("rlk_logits_logp_backward", err);
 }
 
+int rlk_check_rows(const int64_t* ids, const float* temperature, int n, int64_t lo, int64_t hi, int32_t* flags, void* stream) {
+  if (n < 0 || (n > 0 && ids == nullptr) || flags == nullptr) {
+    set_last_error("rlk_check_rows: negative count or null ids / flags");
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  hipError_t err = check_rows_launch(ids, temperature, n, lo, hi, flags, reinterpret_cast<hipStream_t>(stream));
+  return err == hipSuccess ? RLK_OK : device_error("rlk_check_rows", err);
+}
+
 static bool activation_dtype_ok(int dtype) {
   return dtype == RLK_DTYPE_BF16 || dtype == RLK_DTYPE_FP16 || dtype == RLK_DTYPE_FP32;
 }

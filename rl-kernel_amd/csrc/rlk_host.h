@@ -118,6 +118,8 @@ hipError_t linear_logp_merge_launch(const float* part, float* logp, float* lse, 
 // Per-row, per-tile (max, sum of exp relative to it[, target logit]) of materialised logits
 // of element type `dtype` (rlk_dtype); element (row, tile) of each output sits at
 // out[row * out_row_stride + tile * out_tile_stride]. V % num_tiles == 0.
+hipError_t check_rows_launch(const int64_t* ids, const float* temperature, int n, int64_t lo, int64_t hi, int* flags,
+                             hipStream_t stream);
 hipError_t logits_tile_stats_launch(const void* logits, int dtype, int64_t row_stride, const int64_t* target,
                                     const float* temperature, int T, int64_t V, int64_t vocab_start,
                                     int64_t real_vocab, int num_tiles, float* out_max, float* out_sum,

@@ -763,6 +763,31 @@ def hip_deterministic_logp_backward(
     return grad
 
 
+class RowChecks:
+    """Value checks of ids and temperatures that run on the device in front of the work that uses them.
+
+    The constructor launches one kernel and records an event behind it; :meth:`results` waits for that event only - not
+    for what the caller launched meanwhile - and returns ``(an id is outside [lo, hi), a temperature is <= 0)``."""
+
+    __slots__ = ("_flags", "_event")
+
+    def __init__(self, ids: torch.Tensor, lo: int, hi: int, temperature: Optional[torch.Tensor] = None) -> None:
+        self._flags = torch.zeros((2,), dtype=torch.int32, pin_memory=True)
+        self._event = torch.cuda.Event()
+        with _on(ids.device):
+            status = _lib.load().rlk_check_rows(
+                ids.data_ptr(), temperature.data_ptr() if temperature is not None else None, ids.numel(), int(lo), int(hi),
+                self._flags.data_ptr(), _stream_handle(ids.device),
+            )  # fmt: skip
+            self._event.record()
+        _lib.check(status, "rlk_check_rows failed")
+
+    def results(self) -> tuple:
+        self._event.synchronize()
+        bad_id, bad_temperature = self._flags.tolist()
+        return bool(bad_id), bool(bad_temperature)
+
+
 def _check_act(t: torch.Tensor, name: str) -> None:
     """Checks of check_cuda_contig (csrc/cuda/activation/activation.cu:145-156)."""
     if not t.is_cuda:

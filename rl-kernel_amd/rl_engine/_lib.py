@@ -77,6 +77,7 @@ EXPORTED_SYMBOLS = (
     "rlk_logp_from_logits_workspace_bytes",
     "rlk_logp_from_logits",
     "rlk_logits_logp_backward",
+    "rlk_check_rows",
     "rlk_swiglu_fwd",
     "rlk_swiglu_bwd",
     "rlk_det_gemm_swiglu_workspace_bytes",
@@ -172,6 +173,9 @@ def load() -> ctypes.CDLL:
     lib.rlk_logp_from_logits.argtypes = [vp, i32, i64, vp, vp, i32, i64, i64, i64, i32, vp, vp, vp, sz, vp]
     lib.rlk_logits_logp_backward.restype = i32
     lib.rlk_logits_logp_backward.argtypes = [vp, i32, i64, vp, vp, vp, vp, vp, vp, i64, i32, i64, i64, i64, vp]
+
+    lib.rlk_check_rows.restype = i32
+    lib.rlk_check_rows.argtypes = [vp, vp, i32, i64, i64, vp, vp]
 
     lib.rlk_swiglu_fwd.restype = i32
     lib.rlk_swiglu_fwd.argtypes = [vp, i64, vp, i64, vp, i64, i32, i32, i32, vp]

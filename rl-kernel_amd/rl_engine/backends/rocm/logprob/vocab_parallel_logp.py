@@ -50,8 +50,6 @@ def _temperature_rows(temperature, rows: int, device) -> Optional[torch.Tensor]:
     temp = temperature.to(device=device, dtype=torch.float32).reshape(-1)
     if temp.numel() == 1:
         temp = temp.expand(rows)
-    if temp.numel() != rows or bool((temp <= 0).any().item()):
-        raise ValueError("temperature must be positive and scalar or per-token")
     return temp.contiguous()
 
 
@@ -75,17 +73,17 @@ class _HipLogpFromLogits(torch.autograd.Function):
         if not ctx.needs_input_grad[0] or (grad_logp is None and grad_lse is None):
             return None, None, None, None, None, None
         logits, lse, target_1d, temp = ctx.saved_tensors
-        rows, local_vocab = logits.shape
+        rows = logits.size(0)
         start = ctx.vocab_start
         if grad_logp is not None:
             coef_logp = grad_logp.reshape(-1).float().contiguous()
-            owns = (target_1d >= start) & (target_1d < start + local_vocab)
-            target_local = torch.where(owns, target_1d - start, torch.full_like(target_1d, -1)).contiguous()
+            # the kernel compares columns with it: an id of another shard, left of or behind this one, matches none
+            target_local = (target_1d - start if start else target_1d).contiguous()
         else:
             coef_logp = lse.new_zeros((rows,))
             target_local = torch.full((rows,), -1, dtype=torch.long, device=logits.device)
         has_lse_grad = grad_lse is not None
-        coef_lse = grad_lse.reshape(-1).float().contiguous() if has_lse_grad else lse.new_zeros((rows,))
+        coef_lse = grad_lse.reshape(-1).float().contiguous() if has_lse_grad else coef_logp  # not read without a gradient
         grad = _C.hip_deterministic_logp_backward(
             logits, lse.contiguous(), coef_logp, coef_lse, target_local, start, ctx.real_vocab, has_lse_grad,
             temperature=temp if temp.numel() else None,
@@ -126,12 +124,19 @@ def hip_deterministic_logp_from_logits(
     target_1d = target_ids.reshape(-1).to(dtype=torch.long)
     if target_1d.numel() != rows:
         raise ValueError("target_ids must have one id per logits row")
-    if rows and bool(((target_1d < 0) | (target_1d >= real)).any().item()):
-        raise ValueError(f"target_ids must be in the real vocabulary [0, {real})")
+    target_1d = target_1d.contiguous()
     temp = _temperature_rows(temperature, rows, local_logits.device)
-    logp, lse = _HipLogpFromLogits.apply(
-        local_logits, target_1d, temp, int(vocab_start_index), real, int(num_vocab_tiles)
-    )
+    fits = temp is None or temp.numel() == rows
+    checks = _C.RowChecks(target_1d, 0, real, temp if fits else None)
+    if fits:  # runs behind the checks; the wait below is for them alone
+        logp, lse = _HipLogpFromLogits.apply(
+            local_logits, target_1d, temp, int(vocab_start_index), real, int(num_vocab_tiles)
+        )
+    bad_id, bad_temperature = checks.results()
+    if bad_id:
+        raise ValueError(f"target_ids must be in the real vocabulary [0, {real})")
+    if bad_temperature or not fits:
+        raise ValueError("temperature must be positive and scalar or per-token")
     return logp.reshape(target_ids.shape), lse.reshape(target_ids.shape)
 
 
