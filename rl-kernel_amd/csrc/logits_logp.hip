@@ -370,7 +370,8 @@ struct LogitsBackwardArgs {
   int64_t V, vocab_start, real_vocab;
 };
 
-template <int ELEM>
+// STREAM: the gradient is stored non-temporally (see logits_backward_launch).
+template <int ELEM, bool STREAM>
 __global__ __launch_bounds__(256) void logits_backward_kernel(LogitsBackwardArgs a) {
   using L = LogitElem<ELEM>;
   using E = typename L::type;
@@ -415,7 +416,14 @@ __global__ __launch_bounds__(256) void logits_backward_kernel(LogitsBackwardArgs
       u32x4_t raw[kBytes / 16];
       __builtin_memcpy(raw, out, kBytes);
 #pragma unroll
-      for (int i = 0; i < kBytes / 16; ++i) reinterpret_cast<u32x4_t*>(row_out + col)[i] = raw[i];
+      for (int i = 0; i < kBytes / 16; ++i) {
+        u32x4_t* dst = reinterpret_cast<u32x4_t*>(row_out + col) + i;
+        if constexpr (STREAM) {
+          __builtin_nontemporal_store(raw[i], dst);
+        } else {
+          *dst = raw[i];
+        }
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < VEC; ++i)
@@ -459,10 +467,12 @@ hipError_t check_rows_launch(const int64_t* ids, const float* temperature, int n
 }
 
 static int tiles_per_group_for(int T, int num_tiles) {
-  // Enough workgroups to fill 256 CUs several times over when T is small; one workgroup
-  // (4 waves) per row once T alone does that. A group is a multiple of 16 tiles (four per wave).
+  // 256 CUs hold 2048 of these workgroups (4 waves) at a time: enough workgroups for eight rounds, so that the last
+  // one, and the first loads of every workgroup, weigh little; one per row once T alone gives that. A group is a
+  // multiple of 16 tiles (four per wave). (Two rounds -> eight, bf16: 2048 x 151936 125.7 -> 122.5 us,
+  // 4096 x 32000 66.9 -> 61.1; equal below 512 rows, where a group has its 16 tiles either way.)
   int groups = 1;
-  while ((int64_t)T * groups < 4096 && groups * 16 < num_tiles) groups *= 2;
+  while ((int64_t)T * groups < 16384 && groups * 16 < num_tiles) groups *= 2;
   int per = (num_tiles + groups - 1) / groups;
   per = (per + 15) / 16 * 16;
   return per;
@@ -548,19 +558,31 @@ hipError_t logits_backward_launch(const void* logits, int dtype, int64_t row_str
   if (chunks < 1) chunks = 1;
   if (chunks > 65535) chunks = 65535;
   const dim3 grid((unsigned)T, (unsigned)chunks);
+  // A gradient of 128 MB and more does not stay in the 256 MB memory-side cache beside the logits it is made from, so
+  // it goes past it: the logits that the forward left there survive (bf16, forward and backward, ordinary ->
+  // non-temporal: 2048 x 151936 391 -> 370 us, 4096 x 32000 178 -> 159). A smaller one is left for its reader; at 155 MB
+  // (512 x 151936) the two are equal.
+  const bool stream_out = T * V * (dtype == RLK_DTYPE_FP32 ? 4 : 2) >= (int64_t)128 << 20;
+#define RLK_LAUNCH_LOGITS_BACKWARD(ELEM)                                                               \
+  if (stream_out) {                                                                                    \
+    hipLaunchKernelGGL((logits_backward_kernel<ELEM, true>), grid, dim3(256), 0, stream, a);           \
+  } else {                                                                                             \
+    hipLaunchKernelGGL((logits_backward_kernel<ELEM, false>), grid, dim3(256), 0, stream, a);          \
+  }
   switch (dtype) {
     case RLK_DTYPE_BF16:
-      hipLaunchKernelGGL(logits_backward_kernel<RLK_DTYPE_BF16>, grid, dim3(256), 0, stream, a);
+      RLK_LAUNCH_LOGITS_BACKWARD(RLK_DTYPE_BF16)
       break;
     case RLK_DTYPE_FP16:
-      hipLaunchKernelGGL(logits_backward_kernel<RLK_DTYPE_FP16>, grid, dim3(256), 0, stream, a);
+      RLK_LAUNCH_LOGITS_BACKWARD(RLK_DTYPE_FP16)
       break;
     case RLK_DTYPE_FP32:
-      hipLaunchKernelGGL(logits_backward_kernel<RLK_DTYPE_FP32>, grid, dim3(256), 0, stream, a);
+      RLK_LAUNCH_LOGITS_BACKWARD(RLK_DTYPE_FP32)
       break;
     default:
       return hipErrorInvalidValue;
   }
+#undef RLK_LAUNCH_LOGITS_BACKWARD
   return hipGetLastError();
 }
 
