@@ -24,7 +24,8 @@ enum : int {
   kLoopPingPongBothKMajor = 5,
   kLoopSolo = 6,  // four waves, one per SIMD
   kLoopStagedKMajor = 7,     // register-staged, weight K-major (the small tiles), K % 64 == 0
-  kLoopStagedKMajorTail = 8  // the same with a zero-filled last K tile
+  kLoopStagedKMajorTail = 8, // the same with a zero-filled last K tile
+  kLoopPingPongWStream = 9   // kLoopPingPong with the weight read past the caches
 };
 constexpr bool loop_weight_kmajor(int loop) {
   return loop == kLoopPingPongKMajor || loop == kLoopPingPongBothKMajor || loop == kLoopStagedKMajor ||
@@ -57,6 +58,8 @@ __global__ __launch_bounds__(S::kThreads) void det_gemm_kernel(MatView W, MatVie
     tile_mainloop_solo<S>(W, X, n0, m0, K, lds, acc);
   } else if constexpr (LOOP == kLoopStagedKMajor || LOOP == kLoopStagedKMajorTail) {
     tile_mainloop_staged_kmajor<S, KS, LOOP == kLoopStagedKMajorTail>(W, X, n0, m0, K, lds, acc);
+  } else if constexpr (LOOP == kLoopPingPongWStream) {
+    tile_mainloop_pingpong<S, false, false, PlainRowMap<S>, KS, NS, true>(W, X, n0, m0, K, lds, acc);
   } else if constexpr (LOOP >= kLoopPingPongKMajor) {
     // whole K tiles through the ping-pong loop, the rest of a reduction length that 64 does not divide behind it
     const int k_whole = K & ~(kTileK - 1);
@@ -274,6 +277,10 @@ static hipError_t launch_tile(const MatView& W, const MatView& X, void* C, int64
   if (err != hipSuccess) return err;
   const int tiles_m = (M + S::BM - 1) / S::BM;
   const int tiles_n = (N + S::BN - 1) / S::BN;
+  if constexpr (LOOP == kLoopPingPong && S::BM <= 128 && !OUT_F32) {
+    if (streamed_weight(N, K, M, S::BM))
+      return launch_tile<S, kLoopPingPongWStream, OUT_F32, KS, NS>(W, X, C, ldc, M, N, K, stream);
+  }
   int group_m = tiles_m < 8 ? tiles_m : 8;
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(S::kThreads), kLds, stream, W, X, C, ldc, M, N, K,
                      tiles_m, tiles_n, group_m);

@@ -30,7 +30,8 @@ namespace rlk {
 // up of an output element sit 32 lanes apart in one accumulator; the epilogue brings them
 // together, rounds both to bf16 as the unfused projection would, and stores swiglu(gate, up) into
 // C[M, I] (bf16).
-template <int KT, int RING, int MT, bool OUT_F32, bool GATED = false>
+// WSTREAM: the weight is read past the caches (streamed_weight() in rlk_host.h).
+template <int KT, int RING, int MT, bool OUT_F32, bool GATED = false, bool WSTREAM = false>
 __global__ __launch_bounds__(64 * (MT + 4)) void det_gemm_stream_kernel(MatView W, MatView X,
                                                                               void* __restrict__ C, int64_t ldc, int M,
                                                                               int N, int K) {
@@ -39,7 +40,8 @@ __global__ __launch_bounds__(64 * (MT + 4)) void det_gemm_stream_kernel(MatView 
   constexpr int kPairs = KT * (1 + MT);
   constexpr int kStageBytes = kPairs * kSubBytes;
   constexpr int kLoads = kPairs / 2;  // per producer wave per stage
-  static_assert(RING >= 2 && kPairs % 2 == 0 && MT >= 1 && MT <= 4, "ring geometry");
+  static_assert(RING >= 2 && kPairs % 2 == 0 && KT % 2 == 0 && MT >= 1 && MT <= 4, "ring geometry");
+  constexpr int kWLoads = KT / 2;  // the first of a producer's loads of a stage are its weight halves
   extern __shared__ __attribute__((aligned(16))) char lds[];
 
   const int tid = threadIdx.x;
@@ -75,7 +77,7 @@ __global__ __launch_bounds__(64 * (MT + 4)) void det_gemm_stream_kernel(MatView 
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
       const int q = (producer >> 1) + 2 * j;  // pair: [0, KT) weights, then KT per token tile
-      const bool is_w = q < KT;
+      const bool is_w = j < kWLoads;
       const int tile = is_w ? 0 : (q - KT) / KT;
       const int sub = is_w ? q : (q - KT) % KT;
       int ks = s * KT + sub;
@@ -83,8 +85,12 @@ __global__ __launch_bounds__(64 * (MT + 4)) void det_gemm_stream_kernel(MatView 
       const bf16_bits* row = w_base;
 #pragma unroll
       for (int t = 0; t < MT; ++t) row = (!is_w && tile == t) ? x_base[t] : row;
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(row + ks * kTileK), (lds_ptr_t)(base + (2 * q + half) * 1024), 16,
-                                       0, 0);
+      const global_ptr_t src = (global_ptr_t)(row + ks * kTileK);
+      const lds_ptr_t dst = (lds_ptr_t)(base + (2 * q + half) * 1024);
+      if (WSTREAM && j < kWLoads)
+        __builtin_amdgcn_global_load_lds(src, dst, 16, 0, kLoadNonTemporal);
+      else
+        __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
     }
   };
 
@@ -176,10 +182,15 @@ __global__ __launch_bounds__(64 * (MT + 4)) void det_gemm_stream_kernel(MatView 
   }
 }
 
-template <int KT, int RING, int MT, bool OUT_F32>
+template <int KT, int RING, int MT, bool OUT_F32, bool WSTREAM = false>
 static hipError_t launch_stream(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
                                       hipStream_t stream) {
-  auto kernel = det_gemm_stream_kernel<KT, RING, MT, OUT_F32>;
+  // Two to four token tiles gain nothing (down at 32 / 64 tokens 26.0 / 36.6 us either way: the activations, four times
+  // the weight's loads there, set the pace).
+  if constexpr (MT == 1 && !OUT_F32 && !WSTREAM) {
+    if (streamed_weight(N, K, M, 16)) return launch_stream<KT, RING, MT, OUT_F32, true>(W, X, C, ldc, M, N, K, stream);
+  }
+  auto kernel = det_gemm_stream_kernel<KT, RING, MT, OUT_F32, false, WSTREAM>;
   constexpr int kLds = RING * KT * (1 + MT) * 16 * kRowBytes;
   static_assert(kLds <= 160 * 1024, "ring exceeds the LDS");
   static PerDeviceOnce once;
@@ -193,10 +204,11 @@ static hipError_t launch_stream(const MatView& W, const MatView& X, void* C, int
 // the two-workgroups-per-CU geometry, I / 8 workgroups.
 hipError_t det_gemm_stream_gated_launch(const MatView& W, const MatView& X, void* Y, int64_t ldy, int M, int I, int K,
                                         hipStream_t stream) {
-  auto kernel = det_gemm_stream_kernel<2, 8, 1, false, true>;
+  const bool streamed = streamed_weight(2 * (int64_t)I, K, M, 16);
+  auto kernel = streamed ? det_gemm_stream_kernel<2, 8, 1, false, true, true> : det_gemm_stream_kernel<2, 8, 1, false, true>;
   constexpr int kLds = 8 * 2 * 2 * 16 * kRowBytes;
-  static PerDeviceOnce once;
-  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds, once);
+  static PerDeviceOnce once[2];
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds, once[streamed]);
   if (err != hipSuccess) return err;
   hipLaunchKernelGGL(kernel, dim3((I + 7) / 8), dim3(64 * 5), kLds, stream, W, X, Y, ldy, M, 2 * I, K);
   return hipGetLastError();

@@ -467,6 +467,9 @@ __device__ __forceinline__ void tile_mainloop_staged(const MatView& W, const Mat
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* global_ptr_t;
 
+// Cache policy of a direct-to-LDS load (the instruction's nt bit): the line is the first to leave the caches again.
+constexpr int kLoadNonTemporal = 2;
+
 // s_waitcnt immediates (gfx9 encoding: vmcnt [3:0]+[15:14], expcnt [6:4], lgkmcnt [11:8]).
 constexpr int kWaitVm0 = 0x0f70;     // vmcnt(0)
 constexpr int kWaitLgkm0 = 0xc07f;   // lgkmcnt(0)
@@ -570,8 +573,10 @@ struct StridedColumnRowMap {
   }
 };
 
-template <class S, bool WK = false, bool XK = false, class Map = PlainRowMap<S>>
+// WSTREAM: the weight is read past the caches (streamed_weight() in rlk_host.h says when).
+template <class S, bool WK = false, bool XK = false, class Map = PlainRowMap<S>, bool WSTREAM = false>
 struct DmaLoader {
+  static constexpr int kWAux = WSTREAM ? kLoadNonTemporal : 0;
   static_assert(!(WK && Map::kGated), "the gated row map is for the native weight layout");
   static constexpr int kWaveRows = 16 * S::TN;
   static_assert(!WK || S::BN % 64 == 0, "K-major weights are staged in 64-feature columns");
@@ -655,7 +660,7 @@ struct DmaLoader {
   __device__ __forceinline__ void load_w_block(char* stage, int k0, int b) const {
     if constexpr (WK) {
       const bf16_bits* src = kmajor_src(w_base, ldw, w_lane_off[0], kmajor_chunk, n0, n_rows, k0, b);
-      __builtin_amdgcn_global_load_lds((global_ptr_t)src, (lds_ptr_t)(stage + b * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((global_ptr_t)src, (lds_ptr_t)(stage + b * 1024), 16, 0, kWAux);
       return;
     }
     const int row0 = Map::block_offset(b);  // block-uniform feature offset
@@ -669,7 +674,7 @@ struct DmaLoader {
       g = g < n_rows ? g : n_rows - 1;
       src = half_base + (int64_t)(g - n0) * ldw + k0 + chunk_elems;
     }
-    __builtin_amdgcn_global_load_lds((global_ptr_t)src, (lds_ptr_t)(stage + b * 1024), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((global_ptr_t)src, (lds_ptr_t)(stage + b * 1024), 16, 0, kWAux);
   }
 
   __device__ __forceinline__ void load_x_block(char* stage, int k0, int xb) const {
@@ -694,7 +699,7 @@ struct DmaLoader {
   __device__ __forceinline__ void load_w_block_inside(char* stage, int k0, int b) const {
     const bf16_bits* src = w_base + (int64_t)(Map::block_half(b) * n_rows + Map::block_offset(b)) * ldw + k0 +
                            w_lane_off[b & 1];
-    __builtin_amdgcn_global_load_lds((global_ptr_t)src, (lds_ptr_t)(stage + b * 1024), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((global_ptr_t)src, (lds_ptr_t)(stage + b * 1024), 16, 0, kWAux);
   }
   __device__ __forceinline__ void load_x_block_inside(char* stage, int k0, int xb) const {
     const bf16_bits* src = x_base + (int64_t)(xb * 8) * ldx + k0 + x_lane_off;
@@ -737,14 +742,14 @@ constexpr bool pingpong_supported() {
 // tile t + NS start as soon as tile t has been read, so NS - 1 tiles are in flight behind the
 // one being read. Two stages cover the latency of L2 hits; a weight tile that is used by one
 // workgroup only comes through the fabric and wants three. Needs NS * KS * S::kStageBytes of LDS.
-template <class S, bool WK = false, bool XK = false, class Map = PlainRowMap<S>, int KS = 1, int NS = 2>
+template <class S, bool WK = false, bool XK = false, class Map = PlainRowMap<S>, int KS = 1, int NS = 2, bool WSTREAM = false>
 __device__ __forceinline__ void tile_mainloop_pingpong(const MatView& W, const MatView& X, int n0, int m0, int K,
                                                        char* lds, f32x4_t (&acc)[S::TN][S::TM]) {
   static_assert(pingpong_supported<S>(), "two groups of four waves, 4 x 2 wave layout");
   static_assert(KS >= 1 && NS >= 2 && (NS - 1) * KS * (DmaLoader<S, WK, XK, Map>::kLateLoads) <= 63 &&
                     KS * (DmaLoader<S, WK, XK, Map>::kLateLoads) <= 31,
                 "loads in flight must fit vmcnt");
-  using Loader = DmaLoader<S, WK, XK, Map>;
+  using Loader = DmaLoader<S, WK, XK, Map, WSTREAM>;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

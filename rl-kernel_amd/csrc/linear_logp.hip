@@ -165,7 +165,7 @@ __global__ __launch_bounds__(S::kThreads) void linear_logp_partial_kernel(LogpAr
 // columns into the state that column t - 1 left in LDS. Per-(split, stream) states go to
 // linear_logp_stream_merge_kernel, which repeats the in-kernel stream merge above. Same bits
 // as every other configuration.
-template <class S, int NS>
+template <class S, int NS, bool WSTREAM>
 __global__ __launch_bounds__(S::kThreads) void linear_logp_streamgroup_kernel(LogpArgs a, float* __restrict__ spart,
                                                                               int split_first, int split_count) {
   static_assert(S::BN == kLogpTileCols && S::kRun == 16 && S::WN == 4, "wave column = tile of the split");
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(S::kThreads) void linear_logp_streamgroup_kernel(Lo
   const int tok_local = wave_m * 16 * S::TM + l16;
 
   f32x4_t acc[S::TN][S::TM];
-  tile_mainloop_pingpong<S, false, false, StridedColumnRowMap<S, kLogpTileCols>, 1, NS>(a.W, a.H, n0, m0, a.D, lds, acc);
+  tile_mainloop_pingpong<S, false, false, StridedColumnRowMap<S, kLogpTileCols>, 1, NS, WSTREAM>(a.W, a.H, n0, m0, a.D, lds, acc);
 
   const int v0 = split * kLogpSplitCols + tile * kLogpTileCols;
   const int col0 = v0 + (sg * 4 + grp) * 16;  // first column of this lane's run
@@ -400,11 +400,15 @@ static hipError_t launch_logp(LogpArgs a, hipStream_t stream) {
 
 // Up to 128 tokens every weight tile is used by one workgroup only: three stages for the
 // 64- and 128-token tiles (120 / 144 KiB); the 256-token tile has room for two.
-template <class S>
+template <class S, bool WSTREAM = false>
 static hipError_t launch_streamgroup_range(LogpArgs a, float* spart, int split_first, int split_count,
                                            hipStream_t stream) {
+  if constexpr (S::BM <= 128 && !WSTREAM) {
+    if (a.T <= S::BM && streamed_weight(a.V, a.D, a.T, S::BM))
+      return launch_streamgroup_range<S, true>(a, spart, split_first, split_count, stream);
+  }
   constexpr int kStages = S::BM <= 128 ? 3 : 2;
-  auto kernel = linear_logp_streamgroup_kernel<S, kStages>;
+  auto kernel = linear_logp_streamgroup_kernel<S, kStages, WSTREAM>;
   constexpr int kLdsBytes = kStages * S::kStageBytes;
   static PerDeviceOnce once;
   hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLdsBytes, once);

@@ -185,7 +185,7 @@ hipError_t swiglu_launch(const void* gate, int64_t ld_g, const void* up, int64_t
 // W is the packed weight [2 * I, K]; a workgroup owns S::BN / 2 features of both halves.
 // ---------------------------------------------------------------------------
 
-template <class S>
+template <class S, bool WSTREAM>
 __global__ __launch_bounds__(S::kThreads) void det_gemm_swiglu_kernel(MatView W, MatView X, bf16_bits* __restrict__ Y,
                                                                        int64_t ldy, int M, int I, int K, int tiles_m,
                                                                        int tiles_n, int group_m) {
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(S::kThreads) void det_gemm_swiglu_kernel(MatView W,
   const int m0 = tile_m * S::BM;
 
   f32x4_t acc[S::TN][S::TM];
-  tile_mainloop_pingpong<S, false, false, GatedRowMap<S>>(W, X, f0, m0, K, lds, acc);
+  tile_mainloop_pingpong<S, false, false, GatedRowMap<S>, 1, 2, WSTREAM>(W, X, f0, m0, K, lds, acc);
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -233,10 +233,13 @@ using GatedShape256 = TileShape<256, 256, 4, 2>;
 using GatedShape128 = TileShape<256, 128, 4, 2>;
 using GatedShape64 = TileShape<256, 64, 4, 2>;
 
-template <class S>
+template <class S, bool WSTREAM = false>
 static hipError_t launch_gated(const MatView& W, const MatView& X, void* Y, int64_t ldy, int M, int I, int K,
                                hipStream_t stream) {
-  auto kernel = det_gemm_swiglu_kernel<S>;
+  if constexpr (!WSTREAM) {
+    if (streamed_weight(2 * (int64_t)I, K, M, S::BM)) return launch_gated<S, true>(W, X, Y, ldy, M, I, K, stream);
+  }
+  auto kernel = det_gemm_swiglu_kernel<S, WSTREAM>;
   static PerDeviceOnce once;
   hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), S::kLdsBytes, once);
   if (err != hipSuccess) return err;

@@ -1,0 +1,55 @@
+"""Weights of 96 MiB and more are read past the caches where one or two token tiles share them: the same bits."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+N, K = 12290, 4096  # 96.02 MiB, and 2 rows more than whole tiles
+
+
+@pytest.fixture(scope="module")
+def operands():
+    gen = torch.Generator(device=DEV).manual_seed(90)
+    w = torch.randn((N, K), generator=gen, device=DEV).to(torch.bfloat16) * 0.02
+    x = torch.randn((300, K), generator=gen, device=DEV).to(torch.bfloat16)
+    return x, w
+
+
+# one token, the last of the 16-token panel, one and two whole token tiles of every height, the sizes beside them
+@pytest.mark.parametrize("tokens", [1, 16, 17, 64, 65, 127, 128, 129, 255, 256, 257])
+def test_gemm_rows_equal_those_of_a_small_weight(operands, tokens):
+    from rl_engine import _C
+
+    x, w = operands
+    out = _C.det_gemm_fwd_rhs_transposed(x[:tokens], w)
+    for lo, hi in ((0, 130), (6100, 6300), (N - 131, N)):  # 131 rows are 1 MiB: the ordinary loads
+        part = _C.det_gemm_fwd_rhs_transposed(x[:tokens], w[lo:hi])
+        assert torch.equal(out[:, lo:hi].view(torch.int16), part.view(torch.int16))
+
+
+@pytest.mark.parametrize("tokens", [1, 16, 128, 129, 256, 257])
+def test_gated_projection_equals_gemm_and_activation(operands, tokens):
+    from rl_engine import _C
+    from rl_engine.backends.rocm.gemm import swiglu_gemm
+
+    x, w = operands
+    fused = swiglu_gemm.forward(x[:tokens], w)
+    two = _C.swiglu_packed_forward(_C.det_gemm_fwd_rhs_transposed(x[:tokens], w))
+    assert torch.equal(fused.view(torch.int16), two.view(torch.int16))
+
+
+@pytest.mark.parametrize("tokens", [1, 63, 64, 65, 128, 129])
+def test_logp_rows_equal_those_of_a_larger_batch(operands, tokens):
+    from rl_engine.ops.logprob import deterministic_linear_logp
+
+    x, w = operands
+    ids = (torch.arange(300, device=DEV) * 41) % N
+    with torch.no_grad():
+        whole = deterministic_linear_logp(x, w, ids)
+        part = deterministic_linear_logp(x[:tokens], w, ids[:tokens])
+    for a, b in zip(whole, part):
+        assert torch.equal(a[:tokens].view(torch.int32), b.view(torch.int32))
