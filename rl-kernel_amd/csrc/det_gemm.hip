@@ -33,8 +33,15 @@ constexpr bool loop_weight_kmajor(int loop) {
 }
 constexpr bool loop_act_kmajor(int loop) { return loop == kLoopPingPongXKMajor || loop == kLoopPingPongBothKMajor; }
 
+// The small K-major tiles have a wave that prefetches their weight panel when two or more workgroups read it.
+template <int LOOP, int KS>
+constexpr bool has_prefetch_wave() {
+  return LOOP == kLoopPingPongKMajor && KS > 1;
+}
+constexpr int kPrefetchDumpBytes = kWave * 4;
+
 template <class S, int LOOP, bool OUT_F32, int KS = 1, int NS = 2>
-__global__ __launch_bounds__(S::kThreads) void det_gemm_kernel(MatView W, MatView X, void* __restrict__ C,
+__global__ __launch_bounds__(S::kThreads + (has_prefetch_wave<LOOP, KS>() ? kWave : 0)) void det_gemm_kernel(MatView W, MatView X, void* __restrict__ C,
                                                                 int64_t ldc, int M, int N, int K,
                                                                 int tiles_m, int tiles_n, int group_m) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -53,6 +60,16 @@ __global__ __launch_bounds__(S::kThreads) void det_gemm_kernel(MatView W, MatVie
   const int n0 = tile_n * S::BN;
   const int m0 = tile_m * S::BM;
 
+  if constexpr (has_prefetch_wave<LOOP, KS>()) {
+    if (threadIdx.x >= S::kThreads) {
+      // the workgroups of this panel that run on this XCD: their ids are neighbours
+      const int panel = id - within % width;
+      const int lo = max(panel, xcd_compact_id(blockIdx.x % kXcds, total));
+      const int hi = min(panel + width, xcd_compact_id(blockIdx.x % kXcds, total) + xcd_id_count(blockIdx.x, total));
+      prefetch_kmajor_panel<S, KS, NS>(W, n0, K, id - lo, hi - lo, lds + NS * KS * S::kStageBytes);
+      return;
+    }
+  }
   f32x4_t acc[S::TN][S::TM];
   if constexpr (LOOP == kLoopSolo) {
     tile_mainloop_solo<S>(W, X, n0, m0, K, lds, acc);
@@ -270,7 +287,7 @@ template <class S, int LOOP, bool OUT_F32, int KS = 1, int NS = 2>
 static hipError_t launch_tile(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
                               hipStream_t stream) {
   auto kernel = det_gemm_kernel<S, LOOP, OUT_F32, KS, NS>;
-  constexpr int kLds = NS * KS * S::kStageBytes;
+  constexpr int kLds = NS * KS * S::kStageBytes + (has_prefetch_wave<LOOP, KS>() ? kPrefetchDumpBytes : 0);
   static_assert(kLds <= 160 * 1024, "stages exceed the LDS");
   static PerDeviceOnce once;
   hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds, once);
@@ -282,7 +299,11 @@ static hipError_t launch_tile(const MatView& W, const MatView& X, void* C, int64
       return launch_tile<S, kLoopPingPongWStream, OUT_F32, KS, NS>(W, X, C, ldc, M, N, K, stream);
   }
   int group_m = tiles_m < 8 ? tiles_m : 8;
-  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(S::kThreads), kLds, stream, W, X, C, ldc, M, N, K,
+  // Two readers, one of them with a few tokens only (whose loads are mostly repeats of its last row), drift apart, and the
+  // wave then costs up to 10 % (67 tokens on 64-token tiles, K = 24576: 105 -> 116 us) instead of gaining 18 % (128).
+  const bool shared_panel = tiles_m > 2 || M > S::BM + S::BM / 2;
+  const int threads = S::kThreads + (has_prefetch_wave<LOOP, KS>() && shared_panel ? kWave : 0);
+  hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(threads), kLds, stream, W, X, C, ldc, M, N, K,
                      tiles_m, tiles_n, group_m);
   return hipGetLastError();
 }

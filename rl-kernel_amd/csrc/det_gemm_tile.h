@@ -730,6 +730,51 @@ constexpr bool pingpong_supported() {
   return S::WN == 4 && S::WM == 2 && S::BM % 64 == 0;
 }
 
+// A ninth wave that brings a K-major weight panel into the L2 ahead of the ping-pong loop it belongs to (deep stages:
+// KS > 1), for the `count` workgroups of one XCD that read the panel, each touching its own share of it.
+//
+// A CU's vector memory path returns its loads in order, with about 32 KiB outstanding: while every stretch of the load
+// stream holds lines that come from HBM (600 ns), the whole stream runs at 32 KiB per HBM latency (54 GB/s per CU),
+// the operands that wait in the L2 (210 ns) included. Touching every K tile a little ahead changes nothing for that
+// reason. Touches in bursts do: kPrefetchTiles K tiles at once, then loads that all hit the L2 for as many K tiles. A
+// reader's share is 1 / count of the panel, so the more workgroups share it the rarer the slow stretches are.
+// Measured with weights from HBM, without -> with (dX = dY W, 4096 outputs): K = 12288 at 128 / 256 / 512 / 1024 tokens
+// 69.0 / 67.0 / 87.0 / 122 -> 56.3 / 52.7 / 75.5 / 110 us, K = 151936 at 256 / 512 / 1024 tokens 792 / 1032 / 1464 ->
+// 643 / 899 / 1282 us. Bursts of 8 and 16 K tiles: equal to 4 % slower; leads of 1 to 4 K tiles beyond the ring: equal.
+// (The native-layout loops do not gain: their small tiles take as long from the caches.)
+// The wave takes part in the loop's barriers, all 2 K / (64 KS) + 3 of them, and loads into `dump` (256 bytes of LDS).
+constexpr int kPrefetchTiles = 4;
+
+template <class S, int KS, int NS>
+__device__ __forceinline__ void prefetch_kmajor_panel(const MatView& W, int n0, int K, int index, int count, char* dump) {
+  static_assert(S::BN % 64 == 0 && kPrefetchTiles % KS == 0, "whole lines, whole stages");
+  constexpr int kLines = S::BN / 64;  // 128-byte lines of the panel per K row
+  const int lane = threadIdx.x & 63;
+  const int nk = K / (KS * kTileK);
+  const int k_tiles = nk * KS;
+  wg_barrier();
+  for (int t = 0; t < nk; ++t) {
+    const int kt = t * KS + NS * KS + 1;  // the ring's loads are already at K tile t KS + NS KS - 1
+    if ((t * KS) % kPrefetchTiles == 0 && kt < k_tiles) {
+      const int k_rows = (k_tiles - kt < kPrefetchTiles ? k_tiles - kt : kPrefetchTiles) * kTileK;
+      const int per = (k_rows + count - 1) / count;
+      const int first = index * per;
+      const int mine = k_rows - first < per ? k_rows - first : per;
+      for (int i = lane; i < mine * kLines; i += kWave) {
+        int n = n0 + (i % kLines) * 64;
+        n = n < W.rows ? n : W.rows - kChunkElems;
+        const bf16_bits* line = W.ptr + (int64_t)(kt * kTileK + first + i / kLines) * W.k_stride + n;
+        __builtin_amdgcn_global_load_lds((global_ptr_t)line, (lds_ptr_t)dump, 4, 0, 0);
+      }
+    }
+    wg_barrier();
+    wg_barrier();
+  }
+  wg_barrier();
+  __builtin_amdgcn_s_waitcnt(kWaitAll0);
+  wg_barrier();
+}
+
 // With WK the accumulator of MFMA tile jn holds features wave_n*64 + jn*16 + (lane>>4)*4 + q
 // (no run permutation: a K-major chunk is eight consecutive features).
 //

@@ -63,8 +63,8 @@ __device__ __forceinline__ int lds_chunk_offset(int row, int chunk) {
 // Workgroup id -> tile id such that the workgroups one XCD runs together cover
 // a compact range of tiles. The hardware deals consecutive workgroup ids to the
 // eight XCDs round robin; each XCD has its own L2.
+constexpr int kXcds = 8;
 __device__ __forceinline__ int xcd_compact_id(int wg, int total) {
-  constexpr int kXcds = 8;
   const int per = total / kXcds;
   const int rem = total % kXcds;
   const int xcd = wg % kXcds;
@@ -72,6 +72,10 @@ __device__ __forceinline__ int xcd_compact_id(int wg, int total) {
   // XCDs [0, rem) own per+1 ids, the rest own per ids.
   const int base = xcd * per + (xcd < rem ? xcd : rem);
   return base + slot;
+}
+// How many ids the XCD of workgroup `wg` owns.
+__device__ __forceinline__ int xcd_id_count(int wg, int total) {
+  return total / kXcds + (wg % kXcds < total % kXcds ? 1 : 0);
 }
 
 }  // namespace rlk
