@@ -540,7 +540,7 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     const int rest = M % 256;
     const bool natives = view_is_vectorizable(W) && view_is_vectorizable(X) && K % kTileK == 0 && K >= 1024;
     const bool kmajor_w = !view_is_vectorizable(W) && view_is_kmajor_fast(W) && view_is_vectorizable(X) &&
-                          K % kChunkElems == 0;
+                          (K % kChunkElems == 0 || X.k_padded);
     if ((natives || kmajor_w) && remainder_launch_pays(M, N, K, rest, natives, kmajor_w)) {
       MatView head = X, tail = X;
       head.rows = M - rest;
@@ -569,8 +569,8 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
   const bool w_kmajor = !w_native && view_is_kmajor_fast(W), x_kmajor = !x_native && view_is_kmajor_fast(X);
   // A reduction length that 64 does not divide (the token count of a weight gradient) runs its whole K tiles in
   // the same loops and the rest in a register-staged step behind them; a native operand of the pair then
-  // needs whole 16-byte chunks (K % 8 == 0).
-  const bool k_fits = K >= 1 && ((K % kChunkElems) == 0 || (w_kmajor && x_kmajor));
+  // needs whole 16-byte chunks (K % 8 == 0, or rows that go on to the end of the chunk).
+  const bool k_fits = K >= 1 && ((K % kChunkElems) == 0 || (w_kmajor && x_kmajor) || (w_kmajor && X.k_padded));
   if (allow_pingpong && k_fits && (w_kmajor || x_kmajor) && (w_native || w_kmajor) && (x_native || x_kmajor)) {
     const int loop = w_kmajor ? (x_kmajor ? kLoopPingPongBothKMajor : kLoopPingPongKMajor) : kLoopPingPongXKMajor;
     // Only the shapes with 64-feature wave columns have the transposing loop, and a K-major

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256, (NS * KT > 8 ? 1 : 2)) void det_gemm_shortk_ke
   const int64_t ldk = X.k_stride;
   auto issue = [&](int t, char* stage) {
     const int m0 = t * kShortKTokens;
-    const int last = M - kChunkElems - m0;  // tokens past the edge are computed from valid data, never stored
+    const int last = X.rows - kChunkElems - m0;  // tokens past the edge are computed from valid data, never stored
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
       const int b = wave * kLoads + j;

@@ -47,6 +47,9 @@ struct MatView {
   int64_t row_stride;  // elements between consecutive rows
   int64_t k_stride;    // elements between consecutive k
   int rows;
+  // Rows of a reduction-contiguous operand hold finite values up to the next multiple of 8 behind a reduction length
+  // that 8 does not divide: whole 16-byte chunks may be read (the other operand is zero there).
+  bool k_padded = false;
 };
 
 // LDS row r of the weight stage holds feature perm(r) of the tile: lane group
