@@ -320,6 +320,19 @@ int rlk_linear_logp_bwd(const void* hidden, int64_t h_row_stride, const void* we
                         size_t workspace_bytes, int T, int D, int V, int64_t vocab_start, int real_vocab_end,
                         int config, void* stream);
 
+/*
+ * rlk_linear_logp_bwd for a caller that kept the logits rlk_linear_logp_fwd_logits stored for the same inputs
+ * (logits [T, logits_row_stride >= V] fp32): d(logits) is an elementwise pass over them instead of the lm_head GEMM
+ * run again. Same bits in every output. With a bias gradient the logits are not read (it sums the unrounded
+ * d(logits) inside that GEMM). HBM-bound in that pass: 6 bytes per logit.
+ */
+int rlk_linear_logp_bwd_logits(const void* hidden, int64_t h_row_stride, const void* weight, int64_t w_row_stride,
+                               const int64_t* target, const float* bias, const float* temperature, const float* lse,
+                               const float* logits, int64_t logits_row_stride, const float* grad_logp,
+                               const float* grad_lse, void* grad_hidden, int64_t gh_row_stride, void* grad_weight,
+                               int64_t gw_row_stride, float* grad_bias, void* workspace, size_t workspace_bytes,
+                               int T, int D, int V, int64_t vocab_start, int real_vocab_end, int config, void* stream);
+
 /* Element types of materialised logits. */
 typedef enum rlk_dtype { RLK_DTYPE_BF16 = 0, RLK_DTYPE_FP16 = 1, RLK_DTYPE_FP32 = 2 } rlk_dtype;
 

@@ -14,6 +14,8 @@
 //          dz = dz * (1 / temperature)              when a temperature is given
 //      rounded once to bf16 and written to dz[T, ld] (the only [T, V]-sized buffer;
 //      2 bytes per logit).
+//      Where the caller kept the forward's fp32 logits (linear_logp_dlogits_saved_kernel) the GEMM of this step is
+//      not run again: the same expression on the same fp32 values, so the same bits.
 //   2. grad_hidden[T, D] = dz[T, V] @ W[V, D]: det_gemm over the vocabulary, ascending,
 //      with W read as a K-major operand. A row depends on that token's dz row only, so
 //      it is batch invariant like the forward.
@@ -184,6 +186,84 @@ __global__ __launch_bounds__(S::kThreads) void linear_logp_dlogits_kernel(LogpBw
   }
 }
 
+// d(logits) from the fp32 logits that the forward stored (biased, padded lanes -inf, no temperature): the expression of
+// linear_logp_dlogits_kernel on the same values, elementwise. HBM-bound, 6 bytes per logit: a workgroup takes
+// kSavedCols columns of one row, a thread two vectors of eight columns with all four 16-byte loads issued before the
+// first is used. 4120 x 151936 (D = 4096): 731 us, 5.1 TB/s, where the GEMM kernel takes 4063 us.
+struct LogpSavedArgs {
+  const float* z;  // [T, ld_z]
+  int64_t ld_z;
+  const int64_t* target;
+  const float* temperature;  // [T] or null
+  const float* lse;
+  const float* grad_logp;  // [T] or null (= 0)
+  const float* grad_lse;   // [T] or null (= 0)
+  bf16_bits* dz;           // [T, ld_dz]
+  int64_t ld_dz;
+  int V, vocab_limit;
+  int64_t vocab_start;
+};
+
+constexpr int kSavedThreads = 256;
+constexpr int kSavedVectors = 2;  // of 8 columns, per thread
+constexpr int kSavedCols = kSavedThreads * kSavedVectors * 8;
+
+__global__ __launch_bounds__(kSavedThreads) void linear_logp_dlogits_saved_kernel(LogpSavedArgs a) {
+  const int m = blockIdx.x;
+  const float* __restrict__ row = a.z + (int64_t)m * a.ld_z;
+  bf16_bits* __restrict__ out = a.dz + (int64_t)m * a.ld_dz;
+  const bool aligned = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
+  const int first = blockIdx.y * kSavedCols + threadIdx.x * 8;
+
+  f32x4_t z[kSavedVectors][2];
+#pragma unroll
+  for (int i = 0; i < kSavedVectors; ++i) {
+    const int col = first + i * kSavedThreads * 8;
+    if (aligned && col + 8 <= a.V) {
+      z[i][0] = *reinterpret_cast<const f32x4_t*>(row + col);
+      z[i][1] = *reinterpret_cast<const f32x4_t*>(row + col + 4);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) z[i][c >> 2][c & 3] = (col + c < a.V) ? row[col + c] : kNegInf;
+    }
+  }
+
+  const int64_t local = a.target[m] - a.vocab_start;
+  const int target = (local >= 0 && local < a.vocab_limit) ? (int)local : -1;
+  const bool has_temp = a.temperature != nullptr;
+  const float inv_t = has_temp ? 1.0f / a.temperature[m] : 1.0f;
+  const float row_lse = a.lse[m];
+  const float g_logp = a.grad_logp ? a.grad_logp[m] : 0.f;
+  const float g_lse = a.grad_lse ? a.grad_lse[m] : 0.f;
+  const float coeff = g_lse - g_logp;
+#pragma unroll
+  for (int i = 0; i < kSavedVectors; ++i) {
+    const int col = first + i * kSavedThreads * 8;
+    if (col >= a.ld_dz) break;
+    uint32_t packed[4];
+#pragma unroll
+    for (int c = 0; c < 8; c += 2) {
+      float d[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        float y = z[i][(c + e) >> 2][(c + e) & 3];
+        if (has_temp) y = y * inv_t;
+        float v = pinned_exp(y - row_lse) * coeff;
+        if (target == col + c + e) v = v + g_logp;
+        if (has_temp) v = v * inv_t;
+        d[e] = v;
+      }
+      packed[c >> 1] = pack_bf16x2(d[0], d[1]);
+    }
+    if (col + 8 > a.V) {  // zeros behind the vocabulary up to the end of the row
+#pragma unroll
+      for (int c = 0; c < 8; c += 2)
+        packed[c >> 1] &= (col + c < a.V ? 0xffffu : 0u) | (col + c + 1 < a.V ? 0xffff0000u : 0u);
+    }
+    *reinterpret_cast<u32x4_t*>(out + col) = u32x4_t{packed[0], packed[1], packed[2], packed[3]};
+  }
+}
+
 // grad_bias from the per-tile column sums: the `per_block` tiles of a 256-token block are added in the
 // balanced tree that continues the in-kernel one (adjacent pairs first, a tile past the last one is +0),
 // then the block sums ascending.
@@ -300,8 +380,8 @@ __global__ __launch_bounds__(256) void transpose_bf16_kernel(const bf16_bits* __
 }
 
 hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int64_t* target, const float* bias,
-                                  const float* temperature, const float* lse, const float* grad_logp,
-                                  const float* grad_lse, void* grad_hidden, int64_t gh_row_stride, void* grad_weight,
+                                  const float* temperature, const float* lse, const float* logits,
+                                  int64_t logits_ld, const float* grad_logp, const float* grad_lse, void* grad_hidden, int64_t gh_row_stride, void* grad_weight,
                                   int64_t gw_row_stride, float* grad_bias, void* workspace, int T, int D, int V,
                                   int64_t vocab_start, int vocab_limit, int config, hipStream_t stream) {
   LogpBwdArgs a;
@@ -340,8 +420,16 @@ hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int6
   if (grad_bias && config == RLK_LOGP_CFG_16 && T > kBiasSmallTileMaxTokens) config = RLK_LOGP_CFG_64;
   const int tile_tokens = config == RLK_LOGP_CFG_256 ? 256 : config == RLK_LOGP_CFG_128 ? 128 : config == RLK_LOGP_CFG_64 ? 64 : 16;
   const int loop = !vec ? 0 : (D % kTileK == 0 && !force_staged) ? 2 : 1;
+  // The bias gradient sums the unrounded d(logits) inside the GEMM kernels, so it needs them; the last two conditions
+  // are the limits of a launch grid.
+  const int64_t saved_chunks = (a.ld_dz + kSavedCols - 1) / kSavedCols;
+  const bool from_saved = logits != nullptr && grad_bias == nullptr && T < (1 << 23) && saved_chunks <= 65535;
   hipError_t err;
-  switch (config) {
+  if (from_saved) {
+    const LogpSavedArgs s{logits, logits_ld, target, temperature, lse, grad_logp, grad_lse, a.dz, a.ld_dz, V, vocab_limit, vocab_start};
+    hipLaunchKernelGGL(linear_logp_dlogits_saved_kernel, dim3((unsigned)T, (unsigned)saved_chunks), dim3(kSavedThreads), 0, stream, s);
+    err = hipGetLastError();
+  } else switch (config) {
     case RLK_LOGP_CFG_256:
       err = loop == 2 ? launch_dlogits<LogpShape256, 2>(a, stream) : launch_dlogits<LogpShape256, 1>(a, stream);
       break;

@@ -329,36 +329,37 @@ size_t rlk_linear_logp_bwd_workspace_bytes(int T, int V, int with_bias) {
   return linear_logp_bwd_workspace_bytes(T, V, with_bias != 0);
 }
 
-int rlk_linear_logp_bwd(const void* hidden, int64_t h_row_stride, const void* weight, int64_t w_row_stride,
-                        const int64_t* target, const float* bias, const float* temperature, const float* lse,
-                        const float* grad_logp, const float* grad_lse, void* grad_hidden, int64_t gh_row_stride,
-                        void* grad_weight, int64_t gw_row_stride, float* grad_bias, void* workspace,
-                        size_t workspace_bytes, int T, int D, int V, int64_t vocab_start, int real_vocab_end,
-                        int config, void* stream) {
+static int linear_logp_bwd_checked(const char* who, const void* hidden, int64_t h_row_stride, const void* weight, int64_t w_row_stride,
+                                   const int64_t* target, const float* bias, const float* temperature,
+                                   const float* lse, const float* logits, int64_t logits_ld, const float* grad_logp,
+                                   const float* grad_lse, void* grad_hidden, int64_t gh_row_stride, void* grad_weight,
+                                   int64_t gw_row_stride, float* grad_bias, void* workspace, size_t workspace_bytes,
+                                   int T, int D, int V, int64_t vocab_start, int real_vocab_end, int config,
+                                   void* stream) {
   if (T < 0 || D <= 0 || V <= 0) {
-    set_last_error("rlk_linear_logp_bwd: bad sizes T=%d D=%d V=%d", T, D, V);
+    set_last_error("%s: bad sizes T=%d D=%d V=%d", who, T, D, V);
     return RLK_ERR_INVALID_ARGUMENT;
   }
   if (real_vocab_end <= 0 || real_vocab_end > V) {
-    set_last_error("rlk_linear_logp_bwd: real_vocab_end must be in [1, %d], got %d", V, real_vocab_end);
+    set_last_error("%s: real_vocab_end must be in [1, %d], got %d", who, V, real_vocab_end);
     return RLK_ERR_INVALID_ARGUMENT;
   }
   if (config < 0 || (config & ~RLK_LOGP_CFG_FORCE_STAGED) >= RLK_LOGP_CFG_COUNT) {
-    set_last_error("rlk_linear_logp_bwd: unknown config %d", config);
+    set_last_error("%s: unknown config %d", who, config);
     return RLK_ERR_INVALID_ARGUMENT;
   }
   if ((grad_hidden && gh_row_stride < D) || (grad_weight && gw_row_stride < D)) {
-    set_last_error("rlk_linear_logp_bwd: gradient row strides must be >= D");
+    set_last_error("%s: gradient row strides must be >= D", who);
     return RLK_ERR_INVALID_ARGUMENT;
   }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (T > 0) {
     if (hidden == nullptr || weight == nullptr || target == nullptr || lse == nullptr) {
-      set_last_error("rlk_linear_logp_bwd: null hidden / weight / target / lse");
+      set_last_error("%s: null hidden / weight / target / lse", who);
       return RLK_ERR_INVALID_ARGUMENT;
     }
     if (h_row_stride < D || w_row_stride < D) {
-      set_last_error("rlk_linear_logp_bwd: row strides must be >= D");
+      set_last_error("%s: row strides must be >= D", who);
       return RLK_ERR_INVALID_ARGUMENT;
     }
   }
@@ -367,20 +368,47 @@ int rlk_linear_logp_bwd(const void* hidden, int64_t h_row_stride, const void* we
     hipError_t err = hipSuccess;
     if (grad_weight) err = fill_zero_launch(grad_weight, V, D, gw_row_stride, 2, s);
     if (err == hipSuccess && grad_bias) err = fill_zero_launch(grad_bias, 1, V, V, 4, s);
-    return err == hipSuccess ? RLK_OK : device_error("rlk_linear_logp_bwd", err);
+    return err == hipSuccess ? RLK_OK : device_error(who, err);
   }
   const size_t need = linear_logp_bwd_workspace_bytes(T, V, grad_bias != nullptr);
   if (workspace == nullptr || workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255) != 0) {
-    set_last_error("rlk_linear_logp_bwd: 256-byte aligned workspace of %zu bytes needed, %zu given", need,
-                   workspace_bytes);
+    set_last_error("%s: 256-byte aligned workspace of %zu bytes needed, %zu given", who, need, workspace_bytes);
     return RLK_ERR_INVALID_ARGUMENT;
   }
   MatView H{reinterpret_cast<const bf16_bits*>(hidden), h_row_stride, 1, T};
   MatView W{reinterpret_cast<const bf16_bits*>(weight), w_row_stride, 1, V};
-  hipError_t err = linear_logp_bwd_launch(H, W, target, bias, temperature, lse, grad_logp, grad_lse, grad_hidden,
-                                          gh_row_stride, grad_weight, gw_row_stride, grad_bias, workspace, T, D, V,
-                                          vocab_start, real_vocab_end, config, s);
-  return err == hipSuccess ? RLK_OK : device_error("rlk_linear_logp_bwd", err);
+  hipError_t err = linear_logp_bwd_launch(H, W, target, bias, temperature, lse, logits, logits_ld, grad_logp,
+                                          grad_lse, grad_hidden, gh_row_stride, grad_weight, gw_row_stride, grad_bias,
+                                          workspace, T, D, V, vocab_start, real_vocab_end, config, s);
+  return err == hipSuccess ? RLK_OK : device_error(who, err);
+}
+
+int rlk_linear_logp_bwd(const void* hidden, int64_t h_row_stride, const void* weight, int64_t w_row_stride,
+                        const int64_t* target, const float* bias, const float* temperature, const float* lse,
+                        const float* grad_logp, const float* grad_lse, void* grad_hidden, int64_t gh_row_stride,
+                        void* grad_weight, int64_t gw_row_stride, float* grad_bias, void* workspace,
+                        size_t workspace_bytes, int T, int D, int V, int64_t vocab_start, int real_vocab_end,
+                        int config, void* stream) {
+  return linear_logp_bwd_checked("rlk_linear_logp_bwd", hidden, h_row_stride, weight, w_row_stride, target, bias,
+                                 temperature, lse, nullptr, 0, grad_logp, grad_lse, grad_hidden, gh_row_stride,
+                                 grad_weight, gw_row_stride, grad_bias, workspace, workspace_bytes, T, D, V,
+                                 vocab_start, real_vocab_end, config, stream);
+}
+
+int rlk_linear_logp_bwd_logits(const void* hidden, int64_t h_row_stride, const void* weight, int64_t w_row_stride,
+                               const int64_t* target, const float* bias, const float* temperature, const float* lse,
+                               const float* logits, int64_t logits_row_stride, const float* grad_logp,
+                               const float* grad_lse, void* grad_hidden, int64_t gh_row_stride, void* grad_weight,
+                               int64_t gw_row_stride, float* grad_bias, void* workspace, size_t workspace_bytes,
+                               int T, int D, int V, int64_t vocab_start, int real_vocab_end, int config, void* stream) {
+  if (T > 0 && (logits == nullptr || logits_row_stride < V)) {
+    set_last_error("rlk_linear_logp_bwd_logits: null logits or a row stride below V=%d", V);
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  return linear_logp_bwd_checked("rlk_linear_logp_bwd_logits", hidden, h_row_stride, weight, w_row_stride, target,
+                                 bias, temperature, lse, logits, logits_row_stride, grad_logp, grad_lse, grad_hidden,
+                                 gh_row_stride, grad_weight, gw_row_stride, grad_bias, workspace, workspace_bytes, T,
+                                 D, V, vocab_start, real_vocab_end, config, stream);
 }
 
 static int check_logits_args(const char* what, const void* logits, int dtype, int64_t row_stride, int T, int64_t V,

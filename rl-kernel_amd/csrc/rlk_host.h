@@ -146,14 +146,16 @@ hipError_t logits_backward_launch(const void* logits, int dtype, int64_t row_str
 
 // Backward of the fused linear-LogP. workspace holds linear_logp_bwd_workspace_bytes() bytes
 // (the bf16 d(logits) with row stride linear_logp_dz_row_stride(V), then the bias block sums).
-// grad_hidden / grad_weight / grad_bias may each be null.
+// grad_hidden / grad_weight / grad_bias may each be null. logits [T, logits_ld >= V]: what linear_logp_launch stored for
+// the same inputs, or null (the logits are computed again, and always where a bias gradient is wanted).
 int64_t linear_logp_dz_row_stride(int V);
 size_t linear_logp_bwd_workspace_bytes(int T, int V, bool with_bias);
 hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int64_t* target, const float* bias,
-                                  const float* temperature, const float* lse, const float* grad_logp,
-                                  const float* grad_lse, void* grad_hidden, int64_t gh_row_stride, void* grad_weight,
-                                  int64_t gw_row_stride, float* grad_bias, void* workspace, int T, int D, int V,
-                                  int64_t vocab_start, int vocab_limit, int config, hipStream_t stream);
+                                  const float* temperature, const float* lse, const float* logits,
+                                  int64_t logits_ld, const float* grad_logp, const float* grad_lse, void* grad_hidden,
+                                  int64_t gh_row_stride, void* grad_weight, int64_t gw_row_stride,
+                                  float* grad_bias, void* workspace, int T, int D, int V, int64_t vocab_start,
+                                  int vocab_limit, int config, hipStream_t stream);
 
 // SwiGLU on rows of `dtype` (rlk_dtype; strides in elements): forward writes y = out; backward
 // writes d_gate = out, d_up = out2.

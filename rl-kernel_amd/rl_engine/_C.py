@@ -346,11 +346,13 @@ def _linear_logp_forward(
     vocab_start_index: int,
     config: int,
     want_logits: bool = False,
+    logits: Optional[torch.Tensor] = None,
 ):
     """Checks shared by the fused linear-LogP entries, then one call of ``entry`` in the C ABI.
 
     Returns ``(first, lse, logits)``; ``first`` is logp or the target logit, whichever ``entry``
-    writes; ``logits`` is the fp32 ``[N, V]`` tensor the same pass stored when ``want_logits``, else None."""
+    writes; ``logits`` is the fp32 tensor ``[N, >= V]`` the same pass stored: the given one, or a new ``[N, V]`` one when
+    ``want_logits``, else None."""
     if not hidden.is_cuda or not weight.is_cuda or not target.is_cuda:
         raise RuntimeError(f"{who}: hidden, weight and target must be CUDA tensors")
     if hidden.dtype != _BF16 or weight.dtype != _BF16:
@@ -383,7 +385,8 @@ def _linear_logp_forward(
     lib = _lib.load()
     first = torch.empty((n,), dtype=torch.float32, device=hidden.device)
     lse = torch.empty((n,), dtype=torch.float32, device=hidden.device)
-    logits = torch.empty((n, v), dtype=torch.float32, device=hidden.device) if want_logits else None
+    if want_logits and logits is None:
+        logits = torch.empty((n, v), dtype=torch.float32, device=hidden.device)
     ws_bytes = int(lib.rlk_linear_logp_workspace_bytes(n, v))
     workspace = torch.empty((max(ws_bytes, 4) // 4,), dtype=torch.float32, device=hidden.device)
     if n > 0:
@@ -395,7 +398,7 @@ def _linear_logp_forward(
         )  # fmt: skip
         tail = (workspace.data_ptr(), ws_bytes, n, d, v, int(vocab_start_index), real_vocab, config, _stream_handle(hidden.device))
         with _on(hidden.device):
-            if want_logits:  # the logits come out of the same pass: entry + "_logits"
+            if logits is not None:  # the logits come out of the same pass: entry + "_logits"
                 entry = entry + "_logits"
                 status = getattr(lib, entry)(*head, logits.data_ptr(), logits.stride(0), *tail)
             else:
@@ -429,6 +432,31 @@ def fused_linear_logp(
         real_vocab_size, vocab_start_index, config, want_logits=bool(return_logits),
     )  # fmt: skip
     return [logp, lse, logits] if return_logits else [logp, lse]
+
+
+def linear_logp_logits_row_stride(vocab: int) -> int:
+    """Elements per row of the logits that :func:`fused_linear_logp_into` stores: whole 256-byte pieces."""
+    return (vocab + 63) // 64 * 64
+
+
+def fused_linear_logp_into(
+    hidden: torch.Tensor,
+    weight: torch.Tensor,
+    target: torch.Tensor,
+    bias: Optional[torch.Tensor],
+    temperature: Optional[torch.Tensor],
+    real_vocab_size: int,
+    logits: torch.Tensor,
+    *,
+    vocab_start_index: int = 0,
+    config: int = 0,
+) -> List[torch.Tensor]:
+    """:func:`fused_linear_logp` that also stores its fp32 logits in ``logits`` for :func:`fused_linear_logp_bwd`."""
+    logp, lse, _ = _linear_logp_forward(
+        "fused_linear_logp", "rlk_linear_logp_fwd", hidden, weight, target, bias, temperature,
+        real_vocab_size, vocab_start_index, config, logits=logits,
+    )  # fmt: skip
+    return [logp, lse]
 
 
 # The name the reference's CUDA build binds the same function under (csrc/bindings/ops.cpp:514).
@@ -478,12 +506,14 @@ def fused_linear_logp_bwd(
     need_grad_weight: bool = True,
     need_grad_bias: bool = False,
     config: int = 0,
+    logits: Optional[torch.Tensor] = None,
 ) -> List[Optional[torch.Tensor]]:
     """Backward of :func:`fused_linear_logp` -> ``[grad_hidden, grad_weight, grad_bias]``.
 
     ``lse`` is the forward's result; ``grad_logp`` / ``grad_lse`` are fp32 ``[N]`` or
     ``None``. ``grad_hidden`` / ``grad_weight`` are bf16, ``grad_bias`` fp32; an entry
-    that was not asked for is ``None``. Stands in for
+    that was not asked for is ``None``. ``logits``: what :func:`fused_linear_logp_into` stored for the same inputs, fp32
+    ``[N, linear_logp_logits_row_stride(V)]``; without it the logits are computed again. Stands in for
     ``_DetTritonLinearLogpAutograd.backward``
     (rl_engine/backends/shared/triton/logprob/linear_logp.py:600-628) and
     ``chunked_linear_logp_backward`` (rl_engine/reference/logprob/linear_logp.py:642-715).
@@ -505,6 +535,12 @@ def fused_linear_logp_bwd(
     real_vocab = v if int(real_vocab_size) < 0 else int(real_vocab_size)
     if not 0 < real_vocab <= v:
         raise RuntimeError(f"fused_linear_logp_bwd: real_vocab_size must be in [1, {v}]")
+
+    if logits is not None and (
+        logits.dtype != torch.float32 or logits.device != hidden.device or not logits.is_contiguous()
+        or tuple(logits.shape) != (n, linear_logp_logits_row_stride(v))
+    ):  # fmt: skip
+        raise RuntimeError("fused_linear_logp_bwd: logits must be the fp32 tensor the forward stored")
 
     def _per_row(t: Optional[torch.Tensor], name: str) -> Optional[torch.Tensor]:
         if t is None:
@@ -541,33 +577,19 @@ def fused_linear_logp_bwd(
         if grad_bias is not None:
             grad_bias.zero_()
         return [grad_hidden, grad_weight, grad_bias]
+    head = (
+        hidden.data_ptr(), hidden.stride(0), weight.data_ptr(), weight.stride(0), target_i64.data_ptr(),
+        _ptr(bias_f32), _ptr(temp_f32), lse_f32.data_ptr(),
+    )  # fmt: skip
+    tail = (
+        _ptr(g_logp), _ptr(g_lse), _ptr(grad_hidden), d, _ptr(grad_weight), d, _ptr(grad_bias), workspace.data_ptr(), ws_bytes,
+        n, d, v, int(vocab_start_index), real_vocab, int(config), _stream_handle(hidden.device),
+    )  # fmt: skip
     with _on(hidden.device):
-        status = lib.rlk_linear_logp_bwd(
-            hidden.data_ptr(),
-            hidden.stride(0),
-            weight.data_ptr(),
-            weight.stride(0),
-            target_i64.data_ptr(),
-            _ptr(bias_f32),
-            _ptr(temp_f32),
-            lse_f32.data_ptr(),
-            _ptr(g_logp),
-            _ptr(g_lse),
-            _ptr(grad_hidden),
-            d,
-            _ptr(grad_weight),
-            d,
-            _ptr(grad_bias),
-            workspace.data_ptr(),
-            ws_bytes,
-            n,
-            d,
-            v,
-            int(vocab_start_index),
-            real_vocab,
-            int(config),
-            _stream_handle(hidden.device),
-        )
+        if logits is not None:
+            status = lib.rlk_linear_logp_bwd_logits(*head, logits.data_ptr(), logits.stride(0), *tail)
+        else:
+            status = lib.rlk_linear_logp_bwd(*head, *tail)
     _lib.check(status, "rlk_linear_logp_bwd failed")
     return [grad_hidden, grad_weight, grad_bias]
 

@@ -72,6 +72,7 @@ EXPORTED_SYMBOLS = (
     "rlk_linear_logp_fwd_noalloc",
     "rlk_linear_logp_bwd_workspace_bytes",
     "rlk_linear_logp_bwd",
+    "rlk_linear_logp_bwd_logits",
     "rlk_logits_tile_stats",
     "rlk_logits_logp_contract_id",
     "rlk_logp_from_logits_workspace_bytes",
@@ -161,6 +162,10 @@ def load() -> ctypes.CDLL:
     lib.rlk_linear_logp_bwd.restype = i32
     lib.rlk_linear_logp_bwd.argtypes = [
         vp, i64, vp, i64, vp, vp, vp, vp, vp, vp, vp, i64, vp, i64, vp, vp, sz, i32, i32, i32, i64, i32, i32, vp,
+    ]  # fmt: skip
+    lib.rlk_linear_logp_bwd_logits.restype = i32
+    lib.rlk_linear_logp_bwd_logits.argtypes = [
+        vp, i64, vp, i64, vp, vp, vp, vp, vp, i64, vp, vp, vp, i64, vp, i64, vp, vp, sz, i32, i32, i32, i64, i32, i32, vp,
     ]  # fmt: skip
 
     lib.rlk_logits_tile_stats.restype = i32

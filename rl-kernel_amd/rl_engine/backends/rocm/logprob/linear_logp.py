@@ -68,12 +68,55 @@ def _requires_grad(*tensors: Optional[torch.Tensor]) -> bool:
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
 
+# Training keeps the forward's fp32 logits, and the backward reads them instead of running the lm_head GEMM again: 8 bytes
+# written and read per logit against 2 D operations. Forward + backward, kept / computed again, us:
+#   D = 4096, V = 151936:  64 tokens 1330 / 1581, 256: 1450 / 1815, 1000: 3820 / 4570, 4096: 12200 / 14650, 8192: 23930 / 29070
+#   D = 2048, V = 131072:  64 tokens  930 / 1016, 256:  932 / 1045, 1000: 2145 / 2340, 4096:  6380 /  7145, 8192: 11540 / 13170
+#   D = 1536, V = 32768:  192 tokens  229 / 253,  1000:  463 / 502, 4096: 1375 / 1493;  D = 1024: 4096 tokens 1037 / 1065
+# (a forward alone becomes 10 to 27 % longer). A weight that the memory-side cache holds is worth reading early for a few
+# tokens of a short reduction: the input gradient then finds it there (D = 2048, V = 50257: 64 tokens 405 / 314, 128: 366 /
+# 344, 192: 336 / 368; D = 4096, V = 18992: 16 tokens 209 / 252, 128: 232 / 275).
+_SAVED_LOGITS_MIN_HIDDEN = 1536
+_SAVED_LOGITS_ANY_TOKENS_HIDDEN = 4096
+_SAVED_LOGITS_MIN_TOKENS = 192
+_MEMORY_SIDE_CACHE_BYTES = 256 << 20
+_SAVED_LOGITS_MAX_BYTES = 8 << 30
+_SAVED_LOGITS_UNCHECKED_BYTES = 64 << 20
+
+
+def _logits_to_save(hidden_2d: torch.Tensor, vocab: int) -> Optional[torch.Tensor]:
+    """A buffer for the forward's logits, or None where the backward computes them again (the same bits).
+
+    Only memory that the device can spare is taken: at most 8 GiB and a quarter of what is free. Under saved-tensor
+    hooks (activation checkpointing, offloading) and under graph capture nothing more is saved than the inputs."""
+    n, d = hidden_2d.shape
+    shape = (n, _C.linear_logp_logits_row_stride(vocab))
+    size = 4 * shape[0] * shape[1]
+    if n == 0 or d < _SAVED_LOGITS_MIN_HIDDEN or size > _SAVED_LOGITS_MAX_BYTES:
+        return None
+    if torch._C._autograd._top_saved_tensors_default_hooks(True) is not None or torch.cuda.is_current_stream_capturing():
+        return None
+    if n < _SAVED_LOGITS_MIN_TOKENS and d < _SAVED_LOGITS_ANY_TOKENS_HIDDEN and 2 * vocab * d <= _MEMORY_SIDE_CACHE_BYTES:
+        return None
+    device = hidden_2d.device
+    if size > _SAVED_LOGITS_UNCHECKED_BYTES:
+        spare = torch.cuda.mem_get_info(device)[0]
+        if size > spare // 4:
+            spare += torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+            if size > spare // 4:
+                return None
+    try:
+        return torch.empty(shape, dtype=torch.float32, device=device)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
 class _HipLinearLogpAutograd(torch.autograd.Function):
     """Differentiable ``(logp, lse)``: forward and backward both on the HIP library.
 
     Mirrors ``_DetTritonLinearLogpAutograd``
     (rl_engine/backends/shared/triton/logprob/linear_logp.py:573-628): the backward
-    recomputes the logits from the saved ``lse`` and returns gradients in the dtypes
+    takes the logits the forward kept or computes them again, and returns gradients in the dtypes
     of ``hidden``, ``lm_head_weight`` and ``bias``; the clamp ``logp = min(., 0)`` is
     not differentiated.
     """
@@ -81,10 +124,18 @@ class _HipLinearLogpAutograd(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden_2d, weight, bias, target_1d, temp_arg, real_vocab, vocab_start, config):
         bias_c = bias.contiguous() if bias is not None else None
-        logp, lse = _C.fused_linear_logp(
-            hidden_2d, weight, target_1d, bias_c, temp_arg, False, real_vocab,
-            vocab_start_index=vocab_start, config=config,
-        )  # fmt: skip
+        # a bias gradient sums the unrounded d(logits) inside the GEMM, which then runs anyway
+        logits = None if ctx.needs_input_grad[2] else _logits_to_save(hidden_2d, weight.size(0))
+        if logits is None:
+            logp, lse = _C.fused_linear_logp(
+                hidden_2d, weight, target_1d, bias_c, temp_arg, False, real_vocab,
+                vocab_start_index=vocab_start, config=config,
+            )  # fmt: skip
+        else:
+            logp, lse = _C.fused_linear_logp_into(
+                hidden_2d, weight, target_1d, bias_c, temp_arg, real_vocab, logits,
+                vocab_start_index=vocab_start, config=config,
+            )  # fmt: skip
         ctx.save_for_backward(
             hidden_2d,
             weight,
@@ -92,6 +143,7 @@ class _HipLinearLogpAutograd(torch.autograd.Function):
             target_1d,
             lse,
             temp_arg if temp_arg is not None else hidden_2d.new_empty(0),
+            logits,
         )
         ctx.has_bias = bias is not None
         ctx.bias_dtype = bias.dtype if bias is not None else None
@@ -105,7 +157,7 @@ class _HipLinearLogpAutograd(torch.autograd.Function):
     def backward(ctx, grad_logp, grad_lse):
         if grad_logp is None and grad_lse is None:
             return (None,) * 8
-        hidden_2d, weight, bias, target_1d, lse, temp = ctx.saved_tensors
+        hidden_2d, weight, bias, target_1d, lse, temp, logits = ctx.saved_tensors
         need_h, need_w, need_b = ctx.needs_input_grad[0], ctx.needs_input_grad[1], ctx.needs_input_grad[2]
         with torch.no_grad():
             grad_hidden, grad_weight, grad_bias = _C.fused_linear_logp_bwd(
@@ -123,6 +175,7 @@ class _HipLinearLogpAutograd(torch.autograd.Function):
                 need_grad_weight=need_w,
                 need_grad_bias=bool(ctx.has_bias and need_b),
                 config=ctx.config,
+                logits=logits,
             )
         if grad_bias is not None:
             grad_bias = grad_bias.to(ctx.bias_dtype)
