@@ -376,7 +376,10 @@ __global__ __launch_bounds__(256) void logits_backward_kernel(LogitsBackwardArgs
   using L = LogitElem<ELEM>;
   using E = typename L::type;
   constexpr int VEC = L::kVec;
-  const int row = blockIdx.x;
+  // Workgroups run in the order of their ids, so the columns are taken from the last to the first: the forward, which goes
+  // through them in ascending order, has left the last ones in the memory-side cache (2048 x 151936 bf16, forward and
+  // backward 368 -> 355 us).
+  const int row = gridDim.x - 1 - blockIdx.x;
   const E* row_in = reinterpret_cast<const E*>(a.logits) + (int64_t)row * a.row_stride;
   E* row_out = reinterpret_cast<E*>(a.grad) + (int64_t)row * a.grad_row_stride;
   const bool aligned_in = (reinterpret_cast<uintptr_t>(row_in) & 15) == 0;
@@ -392,7 +395,10 @@ __global__ __launch_bounds__(256) void logits_backward_kernel(LogitsBackwardArgs
   const int64_t real_cols = a.real_vocab - a.vocab_start > 0 ? a.real_vocab - a.vocab_start : 0;
   const int64_t real_end = a.V < real_cols ? a.V : real_cols;
   const int64_t vectors = (a.V + VEC - 1) / VEC;
-  for (int64_t g = (int64_t)blockIdx.y * 256 + threadIdx.x; g < vectors; g += (int64_t)gridDim.y * 256) {
+  const int64_t per_block = (vectors + gridDim.y - 1) / gridDim.y;
+  const int64_t first = (int64_t)(gridDim.y - 1 - blockIdx.y) * per_block;
+  const int64_t end = first + per_block < vectors ? first + per_block : vectors;
+  for (int64_t g = first + threadIdx.x; g < end; g += 256) {
     const int64_t col = g * VEC;
     float z[VEC];
     load_logit_vector<ELEM>(row_in, (int)col, (int)a.V, aligned_in, z);
