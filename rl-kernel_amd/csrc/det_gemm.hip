@@ -302,8 +302,14 @@ static hipError_t launch_tile(const MatView& W, const MatView& X, void* C, int64
   int group_m = tiles_m < 8 ? tiles_m : 8;
   // Two readers, one of them with a few tokens only (whose loads are mostly repeats of its last row), drift apart, and the
   // wave then costs up to 10 % (67 tokens on 64-token tiles, K = 24576: 105 -> 116 us) instead of gaining 18 % (128).
+  // A weight that the forward has just left in the memory-side cache costs 3 to 9 % with the wave (dX of 6144 outputs, 4096
+  // inputs at 333 tokens 33.3 -> 35.1 us, of 14336 outputs 71.9 -> 76.7), where it saves 10 to 20 % from HBM (42.6 -> 38.1,
+  // 94.3 -> 79.8): it runs where the weight is too large to still be there, from 128 MiB, or from 96 MiB with many tokens,
+  // whose activations displace it (14336 outputs at 700 / 1000 tokens right behind the forward 117 / 132 -> 103 / 114).
   const bool shared_panel = tiles_m > 2 || M > S::BM + S::BM / 2;
-  const int threads = S::kThreads + (has_prefetch_wave<LOOP, KS>() && shared_panel ? kWave : 0);
+  const int64_t weight_bytes = (int64_t)N * K * 2;
+  const bool from_hbm = weight_bytes >= ((int64_t)128 << 20) || (weight_bytes >= ((int64_t)96 << 20) && M > 512);
+  const int threads = S::kThreads + (has_prefetch_wave<LOOP, KS>() && shared_panel && from_hbm ? kWave : 0);
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(threads), kLds, stream, W, X, C, ldc, M, N, K,
                      tiles_m, tiles_n, group_m);
   return hipGetLastError();
