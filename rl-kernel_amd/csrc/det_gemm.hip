@@ -355,9 +355,9 @@ static hipError_t launch_shape(const MatView& W, const MatView& X, void* C, int6
   return launch_loop<S, kLoopGeneric>(W, X, C, ldc, M, N, K, out_f32, stream);
 }
 
-constexpr int kDeep64 = 4;   // 64x64: 4 K tiles per stage, 2 x 64 KiB of LDS
-constexpr int kDeep128 = 2;  // 128x64 / 128x128: 2 K tiles per stage, 3 x 48 / 2 x 64 KiB (three stages measured
-                             // 8 % faster for 128x64; deeper rings did not pay for the other two)
+constexpr int kDeep64 = 4;   // 64x32 / 64x64: 4 K tiles per stage, 3 x 48 / 2 x 64 KiB of LDS
+constexpr int kDeep128 = 2;  // 64x96 / 128x64 / 128x128: 2 K tiles per stage, 3 x 40 / 3 x 48 / 2 x 64 KiB (three stages
+                             // measured 8 % faster for 128x64; deeper rings did not pay for the square ones)
 
 // Deep-stage variant (KS K tiles per barrier pair) of a small tile; native layout only.
 template <class S, int KS, int NS = 2>
@@ -399,6 +399,8 @@ using Shape256x64 = TileShape<256, 64, 4, 2>;
 using Shape128x128 = TileShape<128, 128, 4, 2>;
 using Shape128x64 = TileShape<128, 64, 4, 2>;
 using Shape64x64 = TileShape<64, 64, 4, 2>;
+using Shape64x96 = TileShape<64, 96, 4, 2>;
+using Shape64x32 = TileShape<64, 32, 4, 2>;
 using Shape64x16 = TileShape<64, 16, 4, 1>;
 using Shape16x16 = TileShape<16, 16, 1, 1>;
 
@@ -499,9 +501,18 @@ int pick_det_gemm_config(int M, int N, int K) {
     return RLK_GEMM_CFG_STREAM64;
   // Problems that give the chip at most one small tile per CU: the deep-stage variants
   // (one workgroup per CU, several K tiles per barrier pair) beat the same tile run several
-  // workgroups per CU. Smallest tile first: it spreads the weight stream over most CUs.
-  if (K % (kTileK * kDeep64) == 0 && tile_count(M, N, 64, 64) <= cus) return RLK_GEMM_CFG_64x64_DEEP;
+  // workgroups per CU. Smallest tile first: it spreads the weight stream over most CUs, and a CU's time goes with the rows
+  // (features + tokens) its workgroup brings in and reads back from LDS per K tile. 64 features x 32 or 96 tokens stand
+  // between the square ones, with weights from HBM: down at 65 / 128 tokens 45.2 / 50.4 (64 x 64, on half the CUs) -> 38.8 /
+  // 43.0 us with 32 tokens, N = K = 4096 at 128 tokens 18.4 -> 16.4, N = 1536 at 200 tokens 16.0 -> 14.5; down at 288 / 384
+  // tokens 76.3 / 78.8 (128 x 64) -> 66.8 / 67.7 with 96 tokens, N = 14336 at 80 tokens 33.0 -> 28.4, N = 6144 at 160 tokens
+  // 28.2 -> 24.0.
+  if (K % (kTileK * kDeep64) == 0) {
+    if (tile_count(M, N, 32, 64) <= cus) return RLK_GEMM_CFG_64x32_DEEP;
+    if (tile_count(M, N, 64, 64) <= cus) return RLK_GEMM_CFG_64x64_DEEP;
+  }
   if (K % (kTileK * kDeep128) == 0) {
+    if (tile_count(M, N, 96, 64) <= cus) return RLK_GEMM_CFG_64x96_DEEP;
     if (tile_count(M, N, 64, 128) <= cus) return RLK_GEMM_CFG_128x64_DEEP;
     if (tile_count(M, N, 128, 128) <= cus) return RLK_GEMM_CFG_128x128_DEEP;
   }
@@ -617,16 +628,19 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
   }
   // Deep-stage variants need the fast layout and whole stages; otherwise the plain shape
   // computes the same bits.
-  if (config == RLK_GEMM_CFG_64x64_DEEP || config == RLK_GEMM_CFG_128x64_DEEP || config == RLK_GEMM_CFG_128x128_DEEP) {
-    const int ks = config == RLK_GEMM_CFG_64x64_DEEP ? kDeep64 : kDeep128;
+  if (config == RLK_GEMM_CFG_64x32_DEEP || config == RLK_GEMM_CFG_64x64_DEEP || config == RLK_GEMM_CFG_64x96_DEEP ||
+      config == RLK_GEMM_CFG_128x64_DEEP || config == RLK_GEMM_CFG_128x128_DEEP) {
+    const int ks = config == RLK_GEMM_CFG_64x32_DEEP || config == RLK_GEMM_CFG_64x64_DEEP ? kDeep64 : kDeep128;
     if (vec && allow_pingpong && K % (kTileK * ks) == 0) {
+      if (config == RLK_GEMM_CFG_64x32_DEEP) return launch_deep<Shape64x32, kDeep64, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
+      if (config == RLK_GEMM_CFG_64x96_DEEP) return launch_deep<Shape64x96, kDeep128, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
       if (config == RLK_GEMM_CFG_64x64_DEEP) return launch_deep<Shape64x64, kDeep64>(W, X, C, ldc, M, N, K, out_f32, stream);
       if (config == RLK_GEMM_CFG_128x64_DEEP) return launch_deep<Shape128x64, kDeep128, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
       return launch_deep<Shape128x128, kDeep128>(W, X, C, ldc, M, N, K, out_f32, stream);
     }
-    config = config == RLK_GEMM_CFG_64x64_DEEP    ? RLK_GEMM_CFG_64x64
-             : config == RLK_GEMM_CFG_128x64_DEEP ? RLK_GEMM_CFG_128x64
-                                                  : RLK_GEMM_CFG_128x128;
+    config = config == RLK_GEMM_CFG_128x128_DEEP                                           ? RLK_GEMM_CFG_128x128
+             : config == RLK_GEMM_CFG_128x64_DEEP || config == RLK_GEMM_CFG_64x96_DEEP ? RLK_GEMM_CFG_128x64
+                                                                                       : RLK_GEMM_CFG_64x64;
   }
   // The element-wise loader of the generic path keeps eight values per chunk in
   // flight; the largest shapes would spill registers with it.

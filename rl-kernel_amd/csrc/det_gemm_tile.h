@@ -602,9 +602,6 @@ struct DmaLoader {
   static_assert(!(kSharedWColumn && kSplitColumn), "a shared stage column is refilled by the late group alone");
   static constexpr int kWBlocksLate = kSplitColumn ? kWBlocksPerWave / 2 : kWBlocksPerWave;
   static constexpr int kWBlocksEarly = kWBlocksPerWave - kWBlocksLate;
-  static constexpr int kXBlocksPerWave = (S::BM / 16) / 4;  // every wave
-  static constexpr int kLateLoads = kWBlocksLate + kXBlocksPerWave;
-  static constexpr int kEarlyLoads = kWBlocksEarly + kXBlocksPerWave;
   static constexpr int kBlocksW = S::BN / 8;
 
   const bf16_bits* w_base;  // W + n0 * ldw   (uniform)
@@ -709,28 +706,53 @@ struct DmaLoader {
     __builtin_amdgcn_global_load_lds((global_ptr_t)src, (lds_ptr_t)(stage + (kBlocksW + xb) * 1024), 16, 0, 0);
   }
 
-  // `wave` is the workgroup wave index 0..7.
+  // A stage is KS K tiles. `wave` is the workgroup wave index 0..7. Four waves bring in the token blocks of one group's
+  // rows: as many of every K tile where four divides them, else (32 and 96 tokens) equal shares of the whole stage.
+  template <int KS>
+  static constexpr int kXLoads = KS * (S::BM / 16) / 4;
+  template <int KS>
+  static constexpr int kLateLoads = KS * kWBlocksLate + kXLoads<KS>;
+  template <int KS>
+  static constexpr int kEarlyLoads = KS * kWBlocksEarly + kXLoads<KS>;
+  template <int KS>
+  __device__ __forceinline__ void load_x_share(char* stage, int k0, int col, int first_block) const {
+    constexpr int kBlocks = S::BM / 16;  // of one group's rows, per K tile
+    static_assert((KS * kBlocks) % 4 == 0, "equal shares for the four waves of a group");
+#pragma unroll
+    for (int i = 0; i < kXLoads<KS>; ++i) {
+      const int at = col * kXLoads<KS> + i;
+      const int s = kBlocks % 4 == 0 ? i / (kBlocks / 4) : at / kBlocks;
+      const int b = kBlocks % 4 == 0 ? col * (kBlocks / 4) + i % (kBlocks / 4) : at % kBlocks;
+      load_x_block(stage + s * S::kStageBytes, k0 + s * kTileK, first_block + b);
+    }
+  }
+  template <int KS>
   __device__ __forceinline__ void issue_early(char* stage, int k0, int wave) const {
 #pragma unroll
-    for (int j = kWBlocksLate; j < kWBlocksPerWave; ++j) load_w_block(stage, k0, wave * kWBlocksPerWave + j);
+    for (int s = 0; s < KS; ++s)
 #pragma unroll
-    for (int j = 0; j < kXBlocksPerWave; ++j) load_x_block(stage, k0, S::BM / 16 + wave * kXBlocksPerWave + j);
+      for (int j = kWBlocksLate; j < kWBlocksPerWave; ++j)
+        load_w_block(stage + s * S::kStageBytes, k0 + s * kTileK, wave * kWBlocksPerWave + j);
+    load_x_share<KS>(stage, k0, wave, S::BM / 16);
   }
+  template <int KS>
   __device__ __forceinline__ void issue_late_x(char* stage, int k0, int wave) const {
-    const int col = wave - 4;
-#pragma unroll
-    for (int j = 0; j < kXBlocksPerWave; ++j) load_x_block(stage, k0, col * kXBlocksPerWave + j);
+    load_x_share<KS>(stage, k0, wave - 4, 0);
   }
+  template <int KS>
   __device__ __forceinline__ void issue_late_w(char* stage, int k0, int wave) const {
     const int col = wave - 4;
 #pragma unroll
-    for (int j = 0; j < kWBlocksLate; ++j) load_w_block(stage, k0, col * kWBlocksPerWave + j);
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int j = 0; j < kWBlocksLate; ++j)
+        load_w_block(stage + s * S::kStageBytes, k0 + s * kTileK, col * kWBlocksPerWave + j);
   }
 };
 
 template <class S>
 constexpr bool pingpong_supported() {
-  return S::WN == 4 && S::WM == 2 && S::BM % 64 == 0;
+  return S::WN == 4 && S::WM == 2 && S::BM % 32 == 0;
 }
 
 // A ninth wave that brings a K-major weight panel into the L2 ahead of the ping-pong loop it belongs to (deep stages:
@@ -794,8 +816,8 @@ template <class S, bool WK = false, bool XK = false, class Map = PlainRowMap<S>,
 __device__ __forceinline__ void tile_mainloop_pingpong(const MatView& W, const MatView& X, int n0, int m0, int K,
                                                        char* lds, f32x4_t (&acc)[S::TN][S::TM]) {
   static_assert(pingpong_supported<S>(), "two groups of four waves, 4 x 2 wave layout");
-  static_assert(KS >= 1 && NS >= 2 && (NS - 1) * KS * (DmaLoader<S, WK, XK, Map>::kLateLoads) <= 63 &&
-                    KS * (DmaLoader<S, WK, XK, Map>::kLateLoads) <= 31,
+  static_assert(KS >= 1 && NS >= 2 && (NS - 1) * DmaLoader<S, WK, XK, Map>::template kLateLoads<KS> <= 63 &&
+                    DmaLoader<S, WK, XK, Map>::template kLateLoads<KS> <= 31,
                 "loads in flight must fit vmcnt");
   using Loader = DmaLoader<S, WK, XK, Map, WSTREAM>;
   const int tid = threadIdx.x;
@@ -827,18 +849,9 @@ __device__ __forceinline__ void tile_mainloop_pingpong(const MatView& W, const M
   // immediate) the same in every iteration.
   auto tile_k = [&](int t) { return (t < nk ? t : nk - 1) * kStageK; };
   auto stage = [&](int t) { return lds + (t % NS) * kStageSpan; };
-  auto issue_early = [&](char* st, int k0) {
-#pragma unroll
-    for (int s = 0; s < KS; ++s) loader.issue_early(st + s * S::kStageBytes, k0 + s * kTileK, wave);
-  };
-  auto issue_late_x = [&](char* st, int k0) {
-#pragma unroll
-    for (int s = 0; s < KS; ++s) loader.issue_late_x(st + s * S::kStageBytes, k0 + s * kTileK, wave);
-  };
-  auto issue_late_w = [&](char* st, int k0) {
-#pragma unroll
-    for (int s = 0; s < KS; ++s) loader.issue_late_w(st + s * S::kStageBytes, k0 + s * kTileK, wave);
-  };
+  auto issue_early = [&](char* st, int k0) { loader.template issue_early<KS>(st, k0, wave); };
+  auto issue_late_x = [&](char* st, int k0) { loader.template issue_late_x<KS>(st, k0, wave); };
+  auto issue_late_w = [&](char* st, int k0) { loader.template issue_late_w<KS>(st, k0, wave); };
 
   // K-major fragments: the transposing read takes, from lane r of a 16-lane group, the address
   // of 4 features (tokens) at K row (r >> 2), positions 4 (r & 3) .. +3 of MFMA tile `j16` of a
@@ -930,7 +943,7 @@ __device__ __forceinline__ void tile_mainloop_pingpong(const MatView& W, const M
   if (!late_group) {
 #pragma unroll
     for (int i = 0; i < NS; ++i) issue_early(stage(i), tile_k(i));
-    __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 1) * KS * Loader::kEarlyLoads));  // my part of tile 0 has landed
+    __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 1) * Loader::template kEarlyLoads<KS>));  // my part of tile 0 has landed
     wg_barrier();
     for (int t = 0; t < nk; ++t) {
       read_tile(t);
@@ -938,7 +951,7 @@ __device__ __forceinline__ void tile_mainloop_pingpong(const MatView& W, const M
       __builtin_amdgcn_s_waitcnt(kWaitLgkm0);  // my fragments are in registers
       wg_barrier();
       compute();
-      __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 2) * KS * Loader::kEarlyLoads));  // my part of tile t+1 has landed
+      __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 2) * Loader::template kEarlyLoads<KS>));  // my part of tile t+1 has landed
       wg_barrier();
     }
     wg_barrier();  // pairs with the late group's leading barrier
@@ -948,7 +961,7 @@ __device__ __forceinline__ void tile_mainloop_pingpong(const MatView& W, const M
       issue_late_x(stage(i), tile_k(i));
       issue_late_w(stage(i), tile_k(i));
     }
-    __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 1) * KS * Loader::kLateLoads));  // my part of tile 0 has landed
+    __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 1) * Loader::template kLateLoads<KS>));  // my part of tile 0 has landed
     wg_barrier();
     wg_barrier();  // half an iteration behind the early group
     // LDS reads return in order, so once at most kXReads of them are outstanding the weight
@@ -980,11 +993,11 @@ __device__ __forceinline__ void tile_mainloop_pingpong(const MatView& W, const M
       if constexpr (Loader::kSharedWColumn) {
         // Behind tile t + 1 this wave has started tiles t + 2 .. t + NS - 1 and the token rows of tile t + NS;
         // the weight blocks of tile t + NS follow the barrier, when every wave has read tile t.
-        __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 2) * KS * Loader::kLateLoads + KS * Loader::kXBlocksPerWave));
+        __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 2) * Loader::template kLateLoads<KS> + Loader::template kXLoads<KS>));
         wg_barrier();
         issue_late_w(stage(t), tile_k(t + NS));
       } else {
-        __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 1) * KS * Loader::kLateLoads));  // my part of tile t+1 has landed
+        __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 1) * Loader::template kLateLoads<KS>));  // my part of tile t+1 has landed
         wg_barrier();
       }
       compute();

@@ -41,6 +41,8 @@ GEMM_CONFIGS = {
     "192x256": 16,
     "shortk": 17,
     "192x128": 18,
+    "64x32_deep": 19,
+    "64x96_deep": 20,
 }
 # OR-ed into a GEMM or LogP configuration: register-staged main loop (bit-neutral).
 FORCE_STAGED = 0x100

@@ -1,0 +1,48 @@
+"""The tiles of 64 features x 32 and 96 tokens: the bits of the other kernels at every edge."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+# tokens: below, at and above the edges of 32- and 96-token tiles; features: less than a tile, whole tiles, a last tile that
+# is not whole; reductions: the fewest stages, fewer stages than the ring holds, more
+@pytest.mark.parametrize("config,stage", [("64x32_deep", 256), ("64x96_deep", 128)])
+@pytest.mark.parametrize("tokens", [1, 31, 32, 33, 65, 95, 96, 97, 193])
+@pytest.mark.parametrize("features", [40, 64, 200])
+def test_same_bits_as_the_one_wave_tile(config, stage, tokens, features):
+    from rl_engine import _C, _lib
+
+    gen = torch.Generator(device=DEV).manual_seed(tokens * 1000 + features)
+    for stages in (1, 2, 3, 7):
+        k = stage * stages
+        x = torch.randn((tokens, k), generator=gen, device=DEV, dtype=torch.bfloat16)
+        w = torch.randn((features, k), generator=gen, device=DEV, dtype=torch.bfloat16)
+        for dtype in (torch.bfloat16, torch.float32):
+            out = torch.full((tokens, features), 7.0, dtype=dtype, device=DEV)
+            want = torch.empty_like(out)
+            _C.gemm_strided(x, w.t(), out, config=_lib.GEMM_CONFIGS[config])
+            _C.gemm_strided(x, w.t(), want, config=_lib.GEMM_CONFIGS["16x16"])
+            bits = torch.int16 if dtype == torch.bfloat16 else torch.int32
+            assert torch.equal(out.view(bits), want.view(bits)), (stages, dtype)
+
+
+# Shapes that the automatic choice gives to them (a padded row pitch among them): a weight of 96 MiB and more is read past
+# the caches there.
+@pytest.mark.parametrize("tokens,features,k", [(65, 4096, 4096), (200, 1536, 4096), (333, 4096, 12288), (90, 12288, 4096)])
+def test_chosen_shapes(tokens, features, k):
+    from rl_engine import _C, _lib
+
+    gen = torch.Generator(device=DEV).manual_seed(tokens)
+    x = torch.randn((tokens, k + 8), generator=gen, device=DEV, dtype=torch.bfloat16)[:, :k]
+    w = torch.randn((features, k), generator=gen, device=DEV, dtype=torch.bfloat16)
+    out = torch.empty((tokens, features), dtype=torch.bfloat16, device=DEV)
+    want = torch.empty_like(out)
+    _C.gemm_strided(x, w.t(), out)
+    _C.gemm_strided(x, w.t(), want, config=_lib.GEMM_CONFIGS["16x16"])
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
