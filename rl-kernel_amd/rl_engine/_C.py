@@ -140,6 +140,60 @@ def linear_plain(a: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor
     return out
 
 
+def _rows_of_chunks(t: torch.Tensor) -> bool:
+    """A 2-D row-major operand that the K-major loader takes as it is (the condition of :func:`_reduction_major`)."""
+    stride = t.stride()
+    return stride[1] == 1 and stride[0] % 8 == 0 and stride[0] >= 0 and t.size(1) % 8 == 0 and t.data_ptr() % 16 == 0
+
+
+def _plain_pair(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Two non-empty 2-D bf16 tensors on one GPU."""
+    return (
+        a.dtype is _BF16 and b.dtype is _BF16 and a.is_cuda and a.device == b.device
+        and a.dim() == 2 and b.dim() == 2 and a.numel() > 0 and b.numel() > 0
+    )  # fmt: skip
+
+
+def linear_input_gradient_plain(grad: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
+    """``grad[M,N] @ weight[N,K]`` for the everyday operands of a backward, or ``None`` for anything else (including
+    everything that has to raise). The same call that :func:`gemm_strided` makes for ``(grad, weight)``, without the
+    rule tables and the views: the backward runs on a thread of its own whose core holds none of this interpreter's
+    data, so there every Python object touched costs several times what it costs the forward (projection of 64 tokens,
+    forward and both gradients 134 -> 83 us of host time)."""
+    if not _plain_pair(grad, weight) or grad.size(1) != weight.size(0) or not _rows_of_chunks(weight):
+        return None
+    sg = grad.stride()
+    if sg[1] != 1 or sg[0] < 0:
+        return None
+    (m, n), k = grad.shape, weight.size(1)
+    out = torch.empty((m, k), dtype=_BF16, device=grad.device)
+    return _launch_plain(grad, sg[0], 1, weight, weight.stride(0), out, m, k, n)
+
+
+def linear_weight_gradient_plain(a: torch.Tensor, grad: torch.Tensor) -> Optional[torch.Tensor]:
+    """``grad[M,N].T @ a[M,K]`` under the conditions of :func:`linear_input_gradient_plain`."""
+    if not _plain_pair(a, grad) or a.size(0) != grad.size(0) or not _rows_of_chunks(a) or not _rows_of_chunks(grad):
+        return None
+    (m, n), k = grad.shape, a.size(1)
+    out = torch.empty((n, k), dtype=_BF16, device=grad.device)
+    return _launch_plain(grad, 1, grad.stride(0), a, a.stride(0), out, n, k, m)
+
+
+def _launch_plain(a, a_row_stride, a_k_stride, b, b_k_stride, out, m, n, k) -> torch.Tensor:
+    global _gemm_entry
+    if _gemm_entry is None:
+        _gemm_entry = _lib.load().rlk_det_gemm_bf16
+    device = out.device
+    with _on(device):
+        status = _gemm_entry(
+            a.data_ptr(), a_row_stride, a_k_stride, b.data_ptr(), b_k_stride, 1, out.data_ptr(), n, m, n, k, 0, 0,
+            torch._C._cuda_getCurrentRawStream(device.index),
+        )  # fmt: skip
+    if status:
+        _lib.check(status, "rlk_det_gemm_bf16 failed")
+    return out
+
+
 def gemm_tree_strided(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor, config: int = 0) -> torch.Tensor:
     """``out[M,N] = a[M,K] @ b[K,N]`` under the k-tree contract, arbitrary non-negative strides.
 

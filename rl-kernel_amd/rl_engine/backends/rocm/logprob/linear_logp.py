@@ -151,6 +151,7 @@ class _HipLinearLogpAutograd(torch.autograd.Function):
         ctx.vocab_start = vocab_start
         ctx.config = config
         ctx.mark_non_differentiable(target_1d)
+        ctx.set_materialize_grads(False)  # an output nobody differentiates costs no zero tensor
         return logp, lse
 
     @staticmethod
