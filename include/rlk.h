@@ -48,16 +48,19 @@ typedef enum rlk_gemm_config {
   RLK_GEMM_CFG_STREAM16 = 9,      /* M <= 16: same with a 64 KiB ring, two workgroups per CU */
   RLK_GEMM_CFG_256x64 = 10,
   RLK_GEMM_CFG_64x64_DEEP = 11,   /* 64x64 tile, 256 K values per barrier pair (few, long tiles) */
-  RLK_GEMM_CFG_128x64_DEEP = 12,  /* 128x64 tile, 128 K values per barrier pair */
+  RLK_GEMM_CFG_128x64_DEEP = 12,  /* 128x64 tile; K % 128 == 0 */
   RLK_GEMM_CFG_128x128_DEEP = 13, /* 128x128 tile, 128 K values per barrier pair */
   RLK_GEMM_CFG_STREAM64 = 14,     /* M <= 64: 16-feature panels streamed through an LDS ring, one consumer wave per 16 tokens */
   RLK_GEMM_CFG_256x256_SOLO = 15, /* 256 x 256 tile on four waves (one per SIMD, 128 x 128 each) */
   RLK_GEMM_CFG_192x256 = 16,      /* 192 features x 256 tokens (N / 192 tiles where N / 256 leaves a round half empty) */
   RLK_GEMM_CFG_SHORTK = 17,       /* K <= 256, K-major token operand: features stationary in registers, tokens streamed */
   RLK_GEMM_CFG_192x128 = 18,      /* 192 features x 128 tokens, three stages (N / 192 x M / 128 tiles that fill one round) */
-  RLK_GEMM_CFG_64x32_DEEP = 19,   /* 64 features x 32 tokens, 256 K values per barrier pair */
-  RLK_GEMM_CFG_64x96_DEEP = 20,   /* 64 features x 96 tokens, 128 K values per barrier pair */
-  RLK_GEMM_CFG_COUNT = 21,
+  RLK_GEMM_CFG_64x32_DEEP = 19,   /* 64 features x 32 tokens, 256 K values per barrier */
+  RLK_GEMM_CFG_64x96_DEEP = 20,   /* 64 features x 96 tokens, 128 K values per barrier */
+  RLK_GEMM_CFG_32x32_DEEP = 21,   /* 32 features x 32 tokens, 128 K values per barrier */
+  RLK_GEMM_CFG_32x64_DEEP = 22,   /* 32 features x 64 tokens, 256 K values per barrier */
+  RLK_GEMM_CFG_64x160_DEEP = 23,  /* 64 features x 160 tokens; K % 128 == 0 */
+  RLK_GEMM_CFG_COUNT = 24,
   /* OR-ed into a configuration: use the register-staged main loop even where the
    * direct-to-LDS ping-pong loop applies. Bit-neutral; exists so tests can
    * compare the two loops. */

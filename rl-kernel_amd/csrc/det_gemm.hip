@@ -25,7 +25,10 @@ enum : int {
   kLoopSolo = 6,  // four waves, one per SIMD
   kLoopStagedKMajor = 7,     // register-staged, weight K-major (the small tiles), K % 64 == 0
   kLoopStagedKMajorTail = 8, // the same with a zero-filled last K tile
-  kLoopPingPongWStream = 9   // kLoopPingPong with the weight read past the caches
+  kLoopPingPongWStream = 9,  // kLoopPingPong with the weight read past the caches
+  kLoopQuad = 10,            // four waves 2 x 2
+  kLoopQuadWStream = 11,     // the same with the weight read past the caches
+  kLoopQuadPrefetch = 12     // the same with a wave that prefetches the weight panel
 };
 constexpr bool loop_weight_kmajor(int loop) {
   return loop == kLoopPingPongKMajor || loop == kLoopPingPongBothKMajor || loop == kLoopStagedKMajor ||
@@ -36,7 +39,7 @@ constexpr bool loop_act_kmajor(int loop) { return loop == kLoopPingPongXKMajor |
 // The small K-major tiles have a wave that prefetches their weight panel when two or more workgroups read it.
 template <int LOOP, int KS>
 constexpr bool has_prefetch_wave() {
-  return LOOP == kLoopPingPongKMajor && KS > 1;
+  return (LOOP == kLoopPingPongKMajor && KS > 1) || LOOP == kLoopQuadPrefetch;
 }
 constexpr int kPrefetchDumpBytes = kWave * 4;
 
@@ -66,12 +69,17 @@ __global__ __launch_bounds__(S::kThreads + (has_prefetch_wave<LOOP, KS>() ? kWav
       const int panel = id - within % width;
       const int lo = max(panel, xcd_compact_id(blockIdx.x % kXcds, total));
       const int hi = min(panel + width, xcd_compact_id(blockIdx.x % kXcds, total) + xcd_id_count(blockIdx.x, total));
-      prefetch_kmajor_panel<S, KS, NS>(W, n0, K - K % (KS * kTileK), id - lo, hi - lo, lds + NS * KS * S::kStageBytes);
+      if constexpr (LOOP == kLoopQuadPrefetch)
+        prefetch_quad_panel<S, KS, NS>(W, n0, K, id - lo, hi - lo, lds + NS * KS * S::kStageBytes);
+      else
+        prefetch_kmajor_panel<S, KS, NS>(W, n0, K - K % (KS * kTileK), id - lo, hi - lo, lds + NS * KS * S::kStageBytes);
       return;
     }
   }
   f32x4_t acc[S::TN][S::TM];
-  if constexpr (LOOP == kLoopSolo) {
+  if constexpr (LOOP == kLoopQuad || LOOP == kLoopQuadWStream || LOOP == kLoopQuadPrefetch) {
+    tile_mainloop_quad<S, KS, NS, LOOP == kLoopQuadWStream>(W, X, n0, m0, K, lds, acc);
+  } else if constexpr (LOOP == kLoopSolo) {
     tile_mainloop_solo<S>(W, X, n0, m0, K, lds, acc);
   } else if constexpr (LOOP == kLoopStagedKMajor || LOOP == kLoopStagedKMajorTail) {
     tile_mainloop_staged_kmajor<S, KS, LOOP == kLoopStagedKMajorTail>(W, X, n0, m0, K, lds, acc);
@@ -309,7 +317,8 @@ static hipError_t launch_tile(const MatView& W, const MatView& X, void* C, int64
   const bool shared_panel = tiles_m > 2 || M > S::BM + S::BM / 2;
   const int64_t weight_bytes = (int64_t)N * K * 2;
   const bool from_hbm = weight_bytes >= ((int64_t)128 << 20) || (weight_bytes >= ((int64_t)96 << 20) && M > 512);
-  const int threads = S::kThreads + (has_prefetch_wave<LOOP, KS>() && shared_panel && from_hbm ? kWave : 0);
+  const bool prefetch = LOOP == kLoopQuadPrefetch || (has_prefetch_wave<LOOP, KS>() && shared_panel && from_hbm);
+  const int threads = S::kThreads + (prefetch ? kWave : 0);
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(threads), kLds, stream, W, X, C, ldc, M, N, K,
                      tiles_m, tiles_n, group_m);
   return hipGetLastError();
@@ -355,16 +364,42 @@ static hipError_t launch_shape(const MatView& W, const MatView& X, void* C, int6
   return launch_loop<S, kLoopGeneric>(W, X, C, ldc, M, N, K, out_f32, stream);
 }
 
-constexpr int kDeep64 = 4;   // 64x32 / 64x64: 4 K tiles per stage, 3 x 48 / 2 x 64 KiB of LDS
-constexpr int kDeep128 = 2;  // 64x96 / 128x64 / 128x128: 2 K tiles per stage, 3 x 40 / 3 x 48 / 2 x 64 KiB (three stages
-                             // measured 8 % faster for 128x64; deeper rings did not pay for the square ones)
-
-// Deep-stage variant (KS K tiles per barrier pair) of a small tile; native layout only.
+// Deep-stage variant (KS K tiles per barrier pair) of a small tile; native layout only. Two stages of 64 KiB, three of 48
+// for 128x64 (8 % faster; deeper rings did not pay for the square ones).
+constexpr int kDeep64 = 4;   // 64x32 / 64x64: K tiles per stage
+constexpr int kDeep128 = 2;  // 64x96 / 128x64 / 128x128
 template <class S, int KS, int NS = 2>
 static hipError_t launch_deep(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
                               bool out_f32, hipStream_t stream) {
   return out_f32 ? launch_tile<S, kLoopPingPong, true, KS, NS>(W, X, C, ldc, M, N, K, stream)
                  : launch_tile<S, kLoopPingPong, false, KS, NS>(W, X, C, ldc, M, N, K, stream);
+}
+
+// The quad loop, with the prefetch wave where several workgroups read a weight panel: from HBM all of them wait for the
+// same lines, and whole token tiles keep them in step (a nearly empty one runs ahead and is the others' prefetch). Weights
+// from HBM / from the memory-side cache, eight waves in two groups -> four -> four and the prefetch wave, 4096 outputs,
+// K = 12288:
+//   64 x 96, 384 tokens:  66.6 / 58.3 -> 68.5 / 51.0 -> 59.2 / 50.9 us      333 tokens:  64.0 / 60.7 -> 60.1 / 52.9 -> 58.0 / 50.5
+//   128 x 64, 512 tokens: 78.1 / 65.6 -> 86.9 / 63.9 -> 69.8 / 62.2 (six stages of one K tile)
+//   32 x 64, 128 tokens:  45.2 / 29.6 -> 42.0 / 32.8 with the wave            80 tokens:  33.4 / 28.7 -> 36.1 / 30.8
+// (64 x 64, 256 tokens: 49.2 / 41.4 -> 59.2 / 39.3 -> 50.2 / 41.2, 128 x 128: 99 / 93 -> 117 / 107: they stay with eight
+// waves.) The 64 x 96, 64 x 160 and 128 x 64 tiles always run with it, the smaller ones where the weight is larger than what the
+// memory-side cache holds beside others (96 MiB) and the last token tile is more than half full, 32 x 32 never (two readers
+// at most: 64 tokens 33.2 -> 35.1).
+template <class S, int KS, int NS, bool PREFETCH = true>
+static hipError_t launch_quad(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K, bool out_f32,
+                              hipStream_t stream) {
+  if constexpr (PREFETCH) {
+    const bool shared_panel = M > S::BM + S::BM / 2;  // (see launch_tile)
+    const bool in_step = (M - 1) % S::BM >= S::BM / 2 && (int64_t)N * K * 2 >= ((int64_t)96 << 20);
+    if (shared_panel && (S::BN + S::BM >= 160 || in_step))
+      return out_f32 ? launch_tile<S, kLoopQuadPrefetch, true, KS, NS>(W, X, C, ldc, M, N, K, stream)
+                     : launch_tile<S, kLoopQuadPrefetch, false, KS, NS>(W, X, C, ldc, M, N, K, stream);
+  }
+  if (out_f32) return launch_tile<S, kLoopQuad, true, KS, NS>(W, X, C, ldc, M, N, K, stream);
+  if (M <= S::BM && streamed_weight(N, K, M, S::BM))
+    return launch_tile<S, kLoopQuadWStream, false, KS, NS>(W, X, C, ldc, M, N, K, stream);
+  return launch_tile<S, kLoopQuad, false, KS, NS>(W, X, C, ldc, M, N, K, stream);
 }
 
 // The register-staged K-major-weight loop of a small tile with as many K tiles per stage as 128 KiB of LDS
@@ -399,9 +434,13 @@ using Shape256x64 = TileShape<256, 64, 4, 2>;
 using Shape128x128 = TileShape<128, 128, 4, 2>;
 using Shape128x64 = TileShape<128, 64, 4, 2>;
 using Shape64x64 = TileShape<64, 64, 4, 2>;
-using Shape64x96 = TileShape<64, 96, 4, 2>;
-using Shape64x32 = TileShape<64, 32, 4, 2>;
 using Shape64x16 = TileShape<64, 16, 4, 1>;
+using Quad128x64 = TileShape<128, 64, 2, 2>;
+using Quad64x160 = TileShape<64, 160, 2, 2>;
+using Quad64x96 = TileShape<64, 96, 2, 2>;
+using Quad64x32 = TileShape<64, 32, 2, 2>;
+using Quad32x64 = TileShape<32, 64, 2, 2>;
+using Quad32x32 = TileShape<32, 32, 2, 2>;
 using Shape16x16 = TileShape<16, 16, 1, 1>;
 
 static bool view_is_vectorizable(const MatView& v) {
@@ -494,26 +533,35 @@ int pick_det_gemm_config(int M, int N, int K) {
   // many layers, not from the 256 MB memory-side cache): up to 16 tokens the streaming kernel with
   // two workgroups per CU is the fastest or equal for every Qwen3-8B projection (gate_up 52 -> 38 us,
   // qkv 14 -> 12 us against the one-wave tile kernel, which wins only when the weight is cache
-  // resident). Up to 32 / 64 tokens it holds while there are at most 1.5 / 1 panels per CU: a
-  // 64-token tile kernel would run on N / 64 CUs only.
+  // resident). Up to 32 tokens it holds while there is at most a panel per CU; for a K that the 32 x 32 tiles below do not
+  // take, up to 32 / 64 tokens with 1.5 / 1 panels per CU.
   if (M <= 16) return (K >= 1024 && K % kTileK == 0) ? RLK_GEMM_CFG_STREAM16 : RLK_GEMM_CFG_16x16;
-  if (K >= 1024 && K % kTileK == 0 && ((M <= 32 && N <= 24 * cus) || (M <= 64 && N <= 16 * cus)))
+  const bool deep = K % (kTileK * kDeep128) == 0;
+  if (K >= 1024 && K % kTileK == 0 &&
+      ((M <= 32 && N <= (deep ? 16 : 24) * cus) || (M <= 64 && !deep && N <= 16 * cus)))
     return RLK_GEMM_CFG_STREAM64;
-  // Problems that give the chip at most one small tile per CU: the deep-stage variants
-  // (one workgroup per CU, several K tiles per barrier pair) beat the same tile run several
-  // workgroups per CU. Smallest tile first: it spreads the weight stream over most CUs, and a CU's time goes with the rows
-  // (features + tokens) its workgroup brings in and reads back from LDS per K tile. 64 features x 32 or 96 tokens stand
-  // between the square ones, with weights from HBM: down at 65 / 128 tokens 45.2 / 50.4 (64 x 64, on half the CUs) -> 38.8 /
-  // 43.0 us with 32 tokens, N = K = 4096 at 128 tokens 18.4 -> 16.4, N = 1536 at 200 tokens 16.0 -> 14.5; down at 288 / 384
-  // tokens 76.3 / 78.8 (128 x 64) -> 66.8 / 67.7 with 96 tokens, N = 14336 at 80 tokens 33.0 -> 28.4, N = 6144 at 160 tokens
-  // 28.2 -> 24.0.
+  // Problems that give the chip at most one small tile per CU: one workgroup per CU with several K tiles in flight beats
+  // the same tile run several workgroups per CU. A CU's time goes with the rows (features + tokens) that its workgroup
+  // brings in and reads back from LDS per K tile, so the tile with the fewest that still fits one round is taken. Weights
+  // from HBM / from the memory-side cache, before each tile was there -> with it:
+  //   32 x 32: down at 33 / 64 tokens 28.0 / 25.0, 36.7 / 28.0 (streaming kernel) -> 24.4 / 20.6, 33.2 / 20.4 us; N = 6144 at
+  //            17 / 32 tokens 15.8 / 13.5, 17.8 / 14.3 -> 12.0 / 10.3, 13.5 / 10.5; N = 1536 at 128 tokens 16.0 / 11.3 -> 11.1 / 8.1
+  //   32 x 64: down at 80 tokens 45.8 / 36.4 (64 x 64, on half the CUs) -> 33.4 / 28.7, at 128 tokens 50.4 / 37.0 -> 42.0 / 32.8
+  //   64 x 32: N = 12288 at 17 tokens 22.1 / 17.0 -> 21.6 / 16.9
+  //   64 x 96: down at 288 / 384 tokens 74.6 / 60.2, 76.7 / 60.5 (128 x 64) -> 59.0 / 49.1, 59.4 / 51.4; N = 6144 at 192 tokens
+  //            29.1 / 23.6 -> 23.3 / 20.2
+  //   128 x 64 with the prefetch: down at 512 tokens 76.6 / 65.0 -> 70.1 / 60.7, N = K = 4096 at 512 tokens 27.6 / 24.8 -> 25.0 / 22.6
+  //   64 x 160: down at 600 tokens 90.6 / 75.1 (128 x 128) -> 80.2 / 74.1, N = K = 4096 at 600 tokens 32.0 / 28.1 -> 29.3 / 27.6
+  if (deep && tile_count(M, N, 32, 32) <= cus) return RLK_GEMM_CFG_32x32_DEEP;
   if (K % (kTileK * kDeep64) == 0) {
+    if (tile_count(M, N, 64, 32) <= cus) return RLK_GEMM_CFG_32x64_DEEP;
     if (tile_count(M, N, 32, 64) <= cus) return RLK_GEMM_CFG_64x32_DEEP;
     if (tile_count(M, N, 64, 64) <= cus) return RLK_GEMM_CFG_64x64_DEEP;
   }
-  if (K % (kTileK * kDeep128) == 0) {
+  if (deep) {
     if (tile_count(M, N, 96, 64) <= cus) return RLK_GEMM_CFG_64x96_DEEP;
     if (tile_count(M, N, 64, 128) <= cus) return RLK_GEMM_CFG_128x64_DEEP;
+    if (tile_count(M, N, 160, 64) <= cus) return RLK_GEMM_CFG_64x160_DEEP;
     if (tile_count(M, N, 128, 128) <= cus) return RLK_GEMM_CFG_128x128_DEEP;
   }
   return pick_tile_candidate(M, N, K, false, false);
@@ -628,17 +676,29 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
   }
   // Deep-stage variants need the fast layout and whole stages; otherwise the plain shape
   // computes the same bits.
-  if (config == RLK_GEMM_CFG_64x32_DEEP || config == RLK_GEMM_CFG_64x64_DEEP || config == RLK_GEMM_CFG_64x96_DEEP ||
+  if (config == RLK_GEMM_CFG_32x32_DEEP || config == RLK_GEMM_CFG_32x64_DEEP || config == RLK_GEMM_CFG_64x32_DEEP ||
+      config == RLK_GEMM_CFG_64x64_DEEP || config == RLK_GEMM_CFG_64x96_DEEP || config == RLK_GEMM_CFG_64x160_DEEP ||
       config == RLK_GEMM_CFG_128x64_DEEP || config == RLK_GEMM_CFG_128x128_DEEP) {
-    const int ks = config == RLK_GEMM_CFG_64x32_DEEP || config == RLK_GEMM_CFG_64x64_DEEP ? kDeep64 : kDeep128;
+    const int ks = config == RLK_GEMM_CFG_32x64_DEEP || config == RLK_GEMM_CFG_64x32_DEEP || config == RLK_GEMM_CFG_64x64_DEEP
+                       ? kDeep64
+                       : kDeep128;
     if (vec && allow_pingpong && K % (kTileK * ks) == 0) {
-      if (config == RLK_GEMM_CFG_64x32_DEEP) return launch_deep<Shape64x32, kDeep64, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
-      if (config == RLK_GEMM_CFG_64x96_DEEP) return launch_deep<Shape64x96, kDeep128, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
+      if (config == RLK_GEMM_CFG_32x32_DEEP)
+        return launch_quad<Quad32x32, kDeep128, 8, false>(W, X, C, ldc, M, N, K, out_f32, stream);
+      if (config == RLK_GEMM_CFG_32x64_DEEP) return launch_quad<Quad32x64, kDeep64, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
+      if (config == RLK_GEMM_CFG_64x32_DEEP) return launch_quad<Quad64x32, kDeep64, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
+      if (config == RLK_GEMM_CFG_64x96_DEEP) return launch_quad<Quad64x96, kDeep128, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
+      if (config == RLK_GEMM_CFG_64x160_DEEP) return launch_quad<Quad64x160, 1, 5>(W, X, C, ldc, M, N, K, out_f32, stream);
+      if (config == RLK_GEMM_CFG_128x64_DEEP) {
+        // Two token tiles only (12288 outputs at 97 ... 128 tokens) gain nothing from HBM and lose from the cache (K = 4096,
+        // 100 tokens: 31.7 / 23.7 us with eight waves, 32.0 / 26.5 with four and the prefetch).
+        return M <= 2 * Shape128x64::BM ? launch_deep<Shape128x64, kDeep128, 3>(W, X, C, ldc, M, N, K, out_f32, stream)
+                                        : launch_quad<Quad128x64, 1, 6>(W, X, C, ldc, M, N, K, out_f32, stream);
+      }
       if (config == RLK_GEMM_CFG_64x64_DEEP) return launch_deep<Shape64x64, kDeep64>(W, X, C, ldc, M, N, K, out_f32, stream);
-      if (config == RLK_GEMM_CFG_128x64_DEEP) return launch_deep<Shape128x64, kDeep128, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
       return launch_deep<Shape128x128, kDeep128>(W, X, C, ldc, M, N, K, out_f32, stream);
     }
-    config = config == RLK_GEMM_CFG_128x128_DEEP                                           ? RLK_GEMM_CFG_128x128
+    config = config == RLK_GEMM_CFG_128x128_DEEP || config == RLK_GEMM_CFG_64x160_DEEP     ? RLK_GEMM_CFG_128x128
              : config == RLK_GEMM_CFG_128x64_DEEP || config == RLK_GEMM_CFG_64x96_DEEP ? RLK_GEMM_CFG_128x64
                                                                                        : RLK_GEMM_CFG_64x64;
   }

@@ -706,25 +706,21 @@ struct DmaLoader {
     __builtin_amdgcn_global_load_lds((global_ptr_t)src, (lds_ptr_t)(stage + (kBlocksW + xb) * 1024), 16, 0, 0);
   }
 
-  // A stage is KS K tiles. `wave` is the workgroup wave index 0..7. Four waves bring in the token blocks of one group's
-  // rows: as many of every K tile where four divides them, else (32 and 96 tokens) equal shares of the whole stage.
+  // A stage is KS K tiles. `wave` is the workgroup wave index 0..7.
+  static constexpr int kXBlocksPerWave = (S::BM / 16) / 4;  // every wave
   template <int KS>
-  static constexpr int kXLoads = KS * (S::BM / 16) / 4;
+  static constexpr int kXLoads = KS * kXBlocksPerWave;
   template <int KS>
   static constexpr int kLateLoads = KS * kWBlocksLate + kXLoads<KS>;
   template <int KS>
   static constexpr int kEarlyLoads = KS * kWBlocksEarly + kXLoads<KS>;
   template <int KS>
   __device__ __forceinline__ void load_x_share(char* stage, int k0, int col, int first_block) const {
-    constexpr int kBlocks = S::BM / 16;  // of one group's rows, per K tile
-    static_assert((KS * kBlocks) % 4 == 0, "equal shares for the four waves of a group");
 #pragma unroll
-    for (int i = 0; i < kXLoads<KS>; ++i) {
-      const int at = col * kXLoads<KS> + i;
-      const int s = kBlocks % 4 == 0 ? i / (kBlocks / 4) : at / kBlocks;
-      const int b = kBlocks % 4 == 0 ? col * (kBlocks / 4) + i % (kBlocks / 4) : at % kBlocks;
-      load_x_block(stage + s * S::kStageBytes, k0 + s * kTileK, first_block + b);
-    }
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int j = 0; j < kXBlocksPerWave; ++j)
+        load_x_block(stage + s * S::kStageBytes, k0 + s * kTileK, first_block + col * kXBlocksPerWave + j);
   }
   template <int KS>
   __device__ __forceinline__ void issue_early(char* stage, int k0, int wave) const {
@@ -752,7 +748,7 @@ struct DmaLoader {
 
 template <class S>
 constexpr bool pingpong_supported() {
-  return S::WN == 4 && S::WM == 2 && S::BM % 32 == 0;
+  return S::WN == 4 && S::WM == 2 && S::BM % 64 == 0;
 }
 
 // A ninth wave that brings a K-major weight panel into the L2 ahead of the ping-pong loop it belongs to (deep stages:
@@ -1259,6 +1255,178 @@ __device__ __forceinline__ void tile_mainloop_solo_impl(const MatView& W, const 
   iteration(t, BoolTag<false>{}, BoolTag<false>{});
   __builtin_amdgcn_s_waitcnt(kWaitAll0);
   wg_barrier();  // callers reuse the LDS after the loop
+}
+
+// ---------------------------------------------------------------------------
+// Four waves in a 2 x 2 layout over a small tile, one per SIMD, each with the fragments of a whole stage (KS K tiles) in
+// registers and the next stage's on their way.
+//
+// What bounds a small tile whose operands are in the L2 is LDS bandwidth: a wave reads its 16 TN weight and 16 TM token
+// rows of every K tile, so eight waves in a 4 x 2 layout read each weight row twice and each token row four times. Four
+// waves in a 2 x 2 layout read every row twice.
+//
+//   iteration t (fragments of stage t in registers, all of them read before the barrier)
+//     wait: my loads of stage t + 1 landed; barrier
+//     start the loads of stage t + NS into the place of stage t; read the fragments of stage t + 1 | MFMAs of stage t
+//
+// Same MFMA chain per output element as every other loop. Needs the native layouts, 16-byte aligned rows and
+// K % (64 KS) == 0.
+// ---------------------------------------------------------------------------
+template <class S>
+constexpr bool quad_supported() {
+  return S::WN == 2 && S::WM == 2 && S::BN % 32 == 0 && S::BM % 32 == 0;
+}
+
+template <class S, int KS, int NS, bool WSTREAM>
+__device__ __forceinline__ void tile_mainloop_quad(const MatView& W, const MatView& X, int n0, int m0, int K, char* lds,
+                                                   f32x4_t (&acc)[S::TN][S::TM]) {
+  static_assert(quad_supported<S>() && NS >= 2, "2 x 2 waves");
+  using Map = PlainRowMap<S>;
+  constexpr int kLoadsW = S::BN / 32, kLoadsX = S::BM / 32;  // blocks of 8 rows per wave and K tile
+  constexpr int kLoads = KS * (kLoadsW + kLoadsX);
+  static_assert((NS - 1) * kLoads <= 63, "loads in flight must fit vmcnt");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_n = wave % S::WN;
+  const int wave_m = wave / S::WN;
+  const int l16 = lane & 15;
+  const int grp = lane >> 4;
+  const int rib = lane >> 3;
+  const int chunk_elems = ((lane & 7) ^ rib) * kChunkElems;
+
+  // The addresses of this lane's chunks at K = 0, rows clamped into the matrix.
+  const bf16_bits* w_src[kLoadsW];
+  const bf16_bits* x_src[kLoadsX];
+  auto block = [&](int j) { return 4 * j + wave; };
+#pragma unroll
+  for (int j = 0; j < kLoadsW; ++j) {
+    int g = n0 + Map::block_offset(block(j)) + Map::lane_offset(wave & 1, rib);
+    g = g < W.rows ? g : W.rows - 1;
+    w_src[j] = W.ptr + (int64_t)g * W.row_stride + chunk_elems;
+  }
+#pragma unroll
+  for (int j = 0; j < kLoadsX; ++j) {
+    int g = m0 + 8 * block(j) + rib;
+    g = g < X.rows ? g : X.rows - 1;
+    x_src[j] = X.ptr + (int64_t)g * X.row_stride + chunk_elems;
+  }
+  constexpr int kStageSpan = KS * S::kStageBytes;
+  const int nk = K / (KS * kTileK);
+  auto after = [](int at) { return at + kStageSpan < NS * kStageSpan ? at + kStageSpan : 0; };  // the next stage's place
+  auto issue = [&](int t, int at) __attribute__((always_inline)) {  // past the last stage: the last one again, never read
+    const int k0 = (t < nk ? t : nk - 1) * (KS * kTileK);
+    char* const st = lds + at;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+#pragma unroll
+      for (int j = 0; j < kLoadsW; ++j)
+        __builtin_amdgcn_global_load_lds((global_ptr_t)(w_src[j] + k0 + s * kTileK),
+                                         (lds_ptr_t)(st + s * S::kStageBytes + block(j) * 1024), 16, 0,
+                                         WSTREAM ? kLoadNonTemporal : 0);
+#pragma unroll
+      for (int j = 0; j < kLoadsX; ++j)
+        __builtin_amdgcn_global_load_lds((global_ptr_t)(x_src[j] + k0 + s * kTileK),
+                                         (lds_ptr_t)(st + s * S::kStageBytes + (S::BN / 8 + block(j)) * 1024), 16, 0, 0);
+    }
+  };
+
+#pragma unroll
+  for (int jn = 0; jn < S::TN; ++jn)
+#pragma unroll
+    for (int jm = 0; jm < S::TM; ++jm) acc[jn][jm] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int frag_lo = (grp ^ (l16 & 7)) << 4;
+  const int w_row_base = (wave_n * 16 * S::TN + l16) * kRowBytes;
+  const int x_row_base = S::BN * kRowBytes + (wave_m * 16 * S::TM + l16) * kRowBytes;
+  struct Frags {
+    u32x4_t w[KS][2][S::TN], x[KS][2][S::TM];
+  };
+  constexpr int kSlices = KS * 2;  // K steps of a stage
+  const char* const read_at[2] = {lds + frag_lo, lds + (frag_lo ^ 64)};
+  // One fragment of a stage: the weight fragments of a K step, then its token fragments.
+  auto read_one = [&](int at, int i, Frags& f) __attribute__((always_inline)) {
+    const int slice = i / (S::TN + S::TM), j = i % (S::TN + S::TM);
+    const char* const st = read_at[slice & 1] + at + (slice >> 1) * S::kStageBytes;
+    if (j < S::TN)
+      f.w[slice >> 1][slice & 1][j] = *reinterpret_cast<const u32x4_t*>(st + w_row_base + j * 16 * kRowBytes);
+    else
+      f.x[slice >> 1][slice & 1][j - S::TN] =
+          *reinterpret_cast<const u32x4_t*>(st + x_row_base + (j - S::TN) * 16 * kRowBytes);
+  };
+  auto mfma_one = [&](int i, const Frags& f) __attribute__((always_inline)) {
+    const int slice = i / (S::TN * S::TM), jn = i % (S::TN * S::TM) / S::TM, jm = i % S::TM;
+    acc[jn][jm] = mfma_16x16x32(f.w[slice >> 1][slice & 1][jn], f.x[slice >> 1][slice & 1][jm], acc[jn][jm]);
+  };
+  constexpr int kReads = kSlices * (S::TN + S::TM), kMfmas = kSlices * S::TN * S::TM;
+  int place = 0;  // of stage t
+  auto iteration = [&](int t, const Frags& now, Frags& next) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 2) * kLoads));  // my part of stage t + 1 has landed
+    wg_barrier();
+    const int free_place = place;
+    place = after(place);
+    issue(t + NS, free_place);
+    __builtin_amdgcn_sched_barrier(0);
+    // reads and MFMAs in turn, so that the MFMAs never wait behind a full queue of reads
+#pragma unroll
+    for (int i = 0; i < kReads; ++i) {
+      read_one(place, i, next);
+#pragma unroll
+      for (int m = i * kMfmas / kReads; m < (i + 1) * kMfmas / kReads; ++m) mfma_one(m, now);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+    asm volatile("" ::: "memory");
+  };
+  Frags a, b;
+#pragma unroll
+  for (int i = 0; i < NS; ++i) issue(i, i * kStageSpan);
+  __builtin_amdgcn_s_waitcnt(wait_vmcnt((NS - 1) * kLoads));
+  wg_barrier();
+#pragma unroll
+  for (int i = 0; i < kReads; ++i) read_one(0, i, a);
+  __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+  // Two exits instead of pairs and a rest: the accumulators then stay in their registers (as pairs, the compiler copied
+  // them once per turn).
+  for (int t = 0;;) {
+    iteration(t, a, b);
+    if (++t == nk) break;
+    iteration(t, b, a);
+    if (++t == nk) break;
+  }
+  __builtin_amdgcn_s_waitcnt(kWaitAll0);
+  wg_barrier();
+}
+
+// The wave that brings the weight panel of a quad loop into the L2 ahead of it: prefetch_kmajor_panel() for the native
+// layout, where a burst is kPrefetchTiles lines of each of the panel's rows. The barriers are the loop's.
+template <class S, int KS, int NS>
+__device__ __forceinline__ void prefetch_quad_panel(const MatView& W, int n0, int K, int index, int count, char* dump) {
+  static_assert(kPrefetchTiles % KS == 0, "whole stages");
+  const int lane = threadIdx.x & 63;
+  const int nk = K / (KS * kTileK);
+  const int k_tiles = nk * KS;
+  wg_barrier();
+  for (int t = 0; t < nk; ++t) {
+    const int kt = t * KS + NS * KS + 1;  // the ring's loads are already at K tile t KS + NS KS - 1
+    if ((t * KS) % kPrefetchTiles == 0 && kt < k_tiles) {
+      const int lines = k_tiles - kt < kPrefetchTiles ? k_tiles - kt : kPrefetchTiles;
+      constexpr int kRowsOf = S::BN;
+      const int per = (kRowsOf + count - 1) / count;
+      const int first = index * per;
+      const int mine = kRowsOf - first < per ? kRowsOf - first : per;
+      for (int i = lane; i < mine * kPrefetchTiles; i += kWave) {
+        int line = i % kPrefetchTiles;
+        line = line < lines ? line : lines - 1;
+        int n = n0 + first + i / kPrefetchTiles;
+        n = n < W.rows ? n : W.rows - 1;
+        const bf16_bits* at = W.ptr + (int64_t)n * W.row_stride + (int64_t)(kt + line) * kTileK;
+        __builtin_amdgcn_global_load_lds((global_ptr_t)at, (lds_ptr_t)dump, 4, 0, 0);
+      }
+    }
+    wg_barrier();
+  }
+  __builtin_amdgcn_s_waitcnt(kWaitAll0);
+  wg_barrier();
 }
 
 template <class S>

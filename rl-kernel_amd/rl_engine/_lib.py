@@ -43,6 +43,9 @@ GEMM_CONFIGS = {
     "192x128": 18,
     "64x32_deep": 19,
     "64x96_deep": 20,
+    "32x32_deep": 21,
+    "32x64_deep": 22,
+    "64x160_deep": 23,
 }
 # OR-ed into a GEMM or LogP configuration: register-staged main loop (bit-neutral).
 FORCE_STAGED = 0x100

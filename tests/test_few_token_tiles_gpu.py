@@ -1,4 +1,4 @@
-"""The tiles of 64 features x 32 and 96 tokens: the bits of the other kernels at every edge."""
+"""The tiles of four waves (32 x 32 to 64 x 160): the bits of the other kernels at every edge."""
 
 from __future__ import annotations
 
@@ -10,10 +10,11 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-# tokens: below, at and above the edges of 32- and 96-token tiles; features: less than a tile, whole tiles, a last tile that
+# tokens: below, at and above the edges of the tiles, and of the one and a half tiles that bring in the prefetching wave; features: less than a tile, whole tiles, a last tile that
 # is not whole; reductions: the fewest stages, fewer stages than the ring holds, more
-@pytest.mark.parametrize("config,stage", [("64x32_deep", 256), ("64x96_deep", 128)])
-@pytest.mark.parametrize("tokens", [1, 31, 32, 33, 65, 95, 96, 97, 193])
+@pytest.mark.parametrize("config,stage", [("32x32_deep", 128), ("32x64_deep", 256), ("64x32_deep", 256), ("64x96_deep", 128), ("64x160_deep", 128),
+                                          ("128x64_deep", 128)])
+@pytest.mark.parametrize("tokens", [1, 31, 32, 33, 65, 95, 96, 97, 129, 144, 145, 160, 161, 193, 241])
 @pytest.mark.parametrize("features", [40, 64, 200])
 def test_same_bits_as_the_one_wave_tile(config, stage, tokens, features):
     from rl_engine import _C, _lib
@@ -32,9 +33,14 @@ def test_same_bits_as_the_one_wave_tile(config, stage, tokens, features):
             assert torch.equal(out.view(bits), want.view(bits)), (stages, dtype)
 
 
-# Shapes that the automatic choice gives to them (a padded row pitch among them): a weight of 96 MiB and more is read past
-# the caches there.
-@pytest.mark.parametrize("tokens,features,k", [(65, 4096, 4096), (200, 1536, 4096), (333, 4096, 12288), (90, 12288, 4096)])
+# Shapes that the automatic choice gives to them, with a padded row pitch: 32 x 32, with the weight read past the caches
+# too; 32 x 64 without and (from 96 MiB of weight, an odd number of stages among them) with the prefetching wave; 64 x 32;
+# 64 x 96 with the wave and with the weight read past the caches; 128 x 64 and 64 x 160 with the wave.
+@pytest.mark.parametrize(
+    "tokens,features,k",
+    [(20, 6144, 4096), (30, 6144, 8320), (50, 4096, 4096), (65, 4096, 4096), (200, 1536, 4096), (80, 4096, 12288),
+     (128, 4096, 12544), (20, 12288, 4096), (333, 4096, 12288), (90, 12288, 4096), (500, 4096, 4096), (600, 4096, 4096)],
+)  # fmt: skip
 def test_chosen_shapes(tokens, features, k):
     from rl_engine import _C, _lib
 
