@@ -50,15 +50,18 @@ inline double rounds_of_workgroups(int64_t tiles, int cus) {
 }
 
 // Whether a kernel loads the weight past the caches (non-temporal): its M tokens are one token tile of `bm`, or two whole
-// ones, whose workgroups read a weight line at the same time. A weight of 96 MiB or more does not wait in the 256 MB memory-side cache for its next use once the
-// other layers have passed through, and reads that leave nothing there are faster: pure reads of 1.2 GB, 5.2 -> 5.9 TB/s
-// in the kernels' pattern. Measured with weights from HBM: gate_up (201 MB) at 1 / 32 / 64 / 128 tokens
-// 37.1 / 45.6 / 46.8 / 52.2 -> 35.4 / 42.3 / 44.3 / 48.4 us, gated at 256 tokens 67.8 -> 62.9, down (101 MB) at 1 token
-// 20.1 -> 18.3, LogP (1.2 GB) at 16 tokens 258 -> 243. Below 96 MiB it gains nothing (qkv, 50 MB: 12.3 / 11.9 at one token,
-// equal at 16) and takes the cache from a weight that would have stayed (11.9 -> 13.3 us). Readers that drift apart miss a
-// line that the first of them has had: gate_up at 160 tokens (128 + 32) 60 -> 66 us, at 256 (128 + 128) 63 -> 60.
+// ones, whose workgroups read a weight line at the same time. A weight of 96 MiB or more does not wait in the 256 MB
+// memory-side cache for its next use once the other layers have passed through, and reads that leave nothing there are
+// faster: pure reads of 1.2 GB, 5.2 -> 5.9 TB/s in the kernels' pattern. Measured with weights from HBM: gate_up (201 MB) at
+// 1 / 32 / 64 / 128 tokens 37.1 / 45.6 / 46.8 / 52.2 -> 35.4 / 42.3 / 44.3 / 48.4 us, gated at 256 tokens 67.8 -> 62.9, down
+// (101 MB) at 1 token 20.1 -> 18.3, LogP (1.2 GB) at 16 tokens 258 -> 243. Below 96 MiB it gains nothing (qkv, 50 MB:
+// 12.3 / 11.9 at one token, equal at 16) and takes the cache from a weight that would have stayed (11.9 -> 13.3 us). Readers
+// that drift apart miss a line that the first of them has had: gate_up at 160 tokens (128 + 32) 60 -> 66 us, at 256
+// (128 + 128) 63 -> 60. Two readers of a weight between the two (12288 outputs, K = 4096, 256 tokens, three weights in turn:
+// 36.6 -> 38.6 us) are better served by what the cache still holds: they want 128 MiB.
 inline bool streamed_weight(int64_t rows, int64_t k, int M, int bm) {
-  return (M <= bm || M == 2 * bm) && rows * k * 2 >= ((int64_t)96 << 20);
+  const int64_t bytes = rows * k * 2;
+  return (M <= bm && bytes >= ((int64_t)96 << 20)) || (M == 2 * bm && bytes >= ((int64_t)128 << 20));
 }
 
 int pick_det_gemm_config(int M, int N, int K);

@@ -1,4 +1,4 @@
-"""Weights of 96 MiB and more are read past the caches where one or two token tiles share them: the same bits."""
+"""Weights of 96 MiB and more are read past the caches where one token tile reads them, of 128 MiB where two do: the same bits."""
 
 from __future__ import annotations
 
@@ -8,7 +8,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda"
-N, K = 12290, 4096  # 96.02 MiB, and 2 rows more than whole tiles
+N, K = 16386, 4096  # 128.02 MiB, and 2 rows more than whole tiles
 
 
 @pytest.fixture(scope="module")
