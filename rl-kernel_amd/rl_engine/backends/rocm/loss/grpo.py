@@ -67,7 +67,8 @@ class _GrpoLossAutograd(torch.autograd.Function):
     def forward(ctx, cur, old, ref, adv, mask, clip_eps, beta):
         out3, ratio, k3, inputs, workspace = _C.grpo_ratio_kl_loss_saved(cur, old, ref, adv, mask, clip_eps, beta)
         ctx.has_mask = mask is not None
-        ctx.save_for_backward(*(inputs if ctx.has_mask else inputs[:4]), workspace)
+        # `cur` itself, not the contiguous copy that the kernel read: a gradient of the gradient flows to it
+        ctx.save_for_backward(cur, *(inputs[1:] if ctx.has_mask else inputs[1:4]), workspace)
         ctx.clip_eps, ctx.beta = float(clip_eps), float(beta)
         ctx.mark_non_differentiable(ratio, k3)
         ctx.set_materialize_grads(False)  # an unused output costs no zero tensor
@@ -84,6 +85,7 @@ class _GrpoLossAutograd(torch.autograd.Function):
         if torch.is_grad_enabled():  # create_graph: the gradient itself is to be differentiated
             grad = _elementwise_gradient(*inputs, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
             return grad, None, None, None, None, None, None
+        inputs[0] = inputs[0].contiguous()
         grad = _C.grpo_ratio_kl_loss_bwd(inputs, workspace, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
         return grad, None, None, None, None, None, None
 

@@ -72,3 +72,28 @@ def test_backward_kernel_equals_the_differentiable_form():
     assert torch.equal(grads[0].view(torch.int32), grads[1].detach().view(torch.int32))
     (second,) = torch.autograd.grad(grads[1].sum(), x)
     assert bool(torch.isfinite(second).all()) and float(second.abs().max()) > 0
+
+
+@pytest.mark.parametrize("layout", ["column_slice", "transposed"])
+def test_strided_log_probs_can_be_differentiated_twice(layout):
+    """Log-probs that are not contiguous (a slice without the last token, a transpose): both orders of gradient are
+    those of the contiguous copy, bit for bit."""
+    from rl_engine.ops.loss import grpo_ratio_kl_loss
+
+    cur, old, ref, adv, mask = (t.to(DEV) for t in _case(5, 301, 78, True))
+    results = []
+    for strided in (False, True):
+        x = cur.clone()
+        if strided and layout == "column_slice":
+            x = torch.cat([x, x[:, :1]], dim=1)[:, :-1]
+        elif strided:
+            x = x.t().contiguous().t()
+        assert x.is_contiguous() != strided
+        x = x.detach().requires_grad_(True)
+        out = grpo_ratio_kl_loss(x, old, ref, adv, mask, clip_eps=0.2, beta=0.1)
+        (plain,) = torch.autograd.grad(out.loss, x, retain_graph=True)
+        (grad,) = torch.autograd.grad(out.loss, x, create_graph=True)
+        (second,) = torch.autograd.grad(grad.square().sum(), x)
+        results.append([t.detach().contiguous().view(torch.int32) for t in (plain, grad, second)])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
