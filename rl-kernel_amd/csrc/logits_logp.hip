@@ -65,7 +65,17 @@ struct LogitElem<RLK_DTYPE_FP32> {
 
 // Columns [g * VEC, g * VEC + VEC) of a row as floats; `aligned` says the row base is 16-byte
 // aligned, `cols` bounds the row (a vector that would run past it is read element by element).
-template <int ELEM>
+// NT: the load leaves nothing in the caches.
+template <bool NT, class V>
+__device__ __forceinline__ V load_vector(const V* p) {
+  if constexpr (NT) {
+    return __builtin_nontemporal_load(p);
+  } else {
+    return *p;
+  }
+}
+
+template <int ELEM, bool NT>
 __device__ __forceinline__ void load_logit_vector(const typename LogitElem<ELEM>::type* row, int col, int cols,
                                                   bool aligned, float (&out)[LogitElem<ELEM>::kVec]) {
   using L = LogitElem<ELEM>;
@@ -76,7 +86,7 @@ __device__ __forceinline__ void load_logit_vector(const typename LogitElem<ELEM>
     const u32x4_t* src = reinterpret_cast<const u32x4_t*>(row + col);
     u32x4_t raw[kBytes / 16];
 #pragma unroll
-    for (int i = 0; i < kBytes / 16; ++i) raw[i] = src[i];
+    for (int i = 0; i < kBytes / 16; ++i) raw[i] = load_vector<NT>(src + i);
     __builtin_memcpy(vals, raw, kBytes);
 #pragma unroll
     for (int i = 0; i < L::kVec; ++i) out[i] = L::to_float(vals[i]);
@@ -98,6 +108,7 @@ struct TileStatsArgs {
   int T;
   int64_t V, vocab_start, real_vocab;
   int num_tiles, tiles_per_group;
+  int64_t streamed;  // workgroups, in the order of their ids
 };
 
 // The eight values of vector g of a row, widened to fp32. ALIGNED: every row is made of whole,
@@ -109,9 +120,10 @@ struct RawVector;
 template <bool ALIGNED>
 struct RawVector<RLK_DTYPE_BF16, ALIGNED> {
   u32x4_t w;
+  template <bool NT>
   __device__ __forceinline__ void load(const uint16_t* row, int g, int cols) {
     if constexpr (ALIGNED) {
-      w = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const char*>(row) + (uint32_t)g * 16u);
+      w = load_vector<NT>(reinterpret_cast<const u32x4_t*>(reinterpret_cast<const char*>(row) + (uint32_t)g * 16u));
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -133,9 +145,10 @@ struct RawVector<RLK_DTYPE_BF16, ALIGNED> {
 template <bool ALIGNED>
 struct RawVector<RLK_DTYPE_FP16, ALIGNED> {
   _Float16 h[8];
+  template <bool NT>
   __device__ __forceinline__ void load(const _Float16* row, int g, int cols) {
     if constexpr (ALIGNED) {
-      const u32x4_t w = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const char*>(row) + (uint32_t)g * 16u);
+      const u32x4_t w = load_vector<NT>(reinterpret_cast<const u32x4_t*>(reinterpret_cast<const char*>(row) + (uint32_t)g * 16u));
       __builtin_memcpy(h, &w, 16);
     } else {
 #pragma unroll
@@ -151,11 +164,12 @@ struct RawVector<RLK_DTYPE_FP16, ALIGNED> {
 template <bool ALIGNED>
 struct RawVector<RLK_DTYPE_FP32, ALIGNED> {
   f32x4_t lo, hi;
+  template <bool NT>
   __device__ __forceinline__ void load(const float* row, int g, int cols) {
     if constexpr (ALIGNED) {
       const char* p = reinterpret_cast<const char*>(row) + (uint32_t)g * 32u;
-      lo = reinterpret_cast<const f32x4_t*>(p)[0];
-      hi = reinterpret_cast<const f32x4_t*>(p)[1];
+      lo = load_vector<NT>(reinterpret_cast<const f32x4_t*>(p));
+      hi = load_vector<NT>(reinterpret_cast<const f32x4_t*>(p) + 1);
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -230,8 +244,8 @@ struct BoolConstant {
 constexpr int kTileLanes = 16;                    // lanes that share a tile
 constexpr int kTilesPerWave = kWave / kTileLanes;  // 4
 
-template <int ELEM, bool HAS_TEMP, bool ALIGNED>
-__global__ __launch_bounds__(256) void logits_tile_stats_kernel(TileStatsArgs a) {
+template <int ELEM, bool HAS_TEMP, bool ALIGNED, bool NT>
+__device__ __forceinline__ void logits_tile_stats(const TileStatsArgs& a) {
   using L = LogitElem<ELEM>;
   using E = typename L::type;
   constexpr int VEC = 8, kBatch = 4;
@@ -284,14 +298,14 @@ __global__ __launch_bounds__(256) void logits_tile_stats_kernel(TileStatsArgs a)
     RawVector<ELEM, ALIGNED> raw[kBatch];
     if (clean > 0) {
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) raw[u].load(row_ptr, g + u * kTileLanes, cols);
+      for (int u = 0; u < kBatch; ++u) raw[u].template load<NT>(row_ptr, g + u * kTileLanes, cols);
     }
     auto clean_batch = [&](auto more, bool first) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
         float y[VEC];
         raw[u].unpack(y);
-        if constexpr (decltype(more)::value) raw[u].load(row_ptr, g + kStep + u * kTileLanes, cols);
+        if constexpr (decltype(more)::value) raw[u].template load<NT>(row_ptr, g + kStep + u * kTileLanes, cols);
         if (u == 0 && first) {  // the tile may start inside its first vector (lane 0 of the 16)
           const int lo = lo_col - g * VEC;
 #pragma unroll
@@ -313,7 +327,7 @@ __global__ __launch_bounds__(256) void logits_tile_stats_kernel(TileStatsArgs a)
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
         const int gu = g + u * kTileLanes;
-        raw[u].load(row_ptr, gu < g1 ? gu : g_last, cols);
+        raw[u].template load<NT>(row_ptr, gu < g1 ? gu : g_last, cols);
       }
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
@@ -353,6 +367,18 @@ __global__ __launch_bounds__(256) void logits_tile_stats_kernel(TileStatsArgs a)
   }
 }
 
+// The first `streamed` workgroups read past the caches (kCachedLogitsBytes). HBM-bound: 2048 x 151936 bf16 4.9 TB/s.
+template <int ELEM, bool HAS_TEMP, bool ALIGNED>
+__global__ __launch_bounds__(256) void logits_tile_stats_kernel(TileStatsArgs a) {
+  if constexpr (ALIGNED) {
+    if ((int64_t)blockIdx.y * gridDim.x + blockIdx.x < a.streamed) {
+      logits_tile_stats<ELEM, HAS_TEMP, ALIGNED, true>(a);
+      return;
+    }
+  }
+  logits_tile_stats<ELEM, HAS_TEMP, ALIGNED, false>(a);
+}
+
 // grad = coef_logp * (onehot - p) + coef_lse * p with p = e(y - lse) (0 when lse is not
 // finite), 0 on padded columns, multiplied by 1 / temperature once more when one is given.
 // Elementwise; written in the dtype of the logits.
@@ -370,7 +396,7 @@ struct LogitsBackwardArgs {
   int64_t V, vocab_start, real_vocab;
 };
 
-// STREAM: the gradient is stored non-temporally (see logits_backward_launch).
+// STREAM: the logits are read and the gradient is stored past the caches (see logits_backward_launch).
 template <int ELEM, bool STREAM>
 __global__ __launch_bounds__(256) void logits_backward_kernel(LogitsBackwardArgs a) {
   using L = LogitElem<ELEM>;
@@ -401,7 +427,7 @@ __global__ __launch_bounds__(256) void logits_backward_kernel(LogitsBackwardArgs
   for (int64_t g = first + threadIdx.x; g < end; g += 256) {
     const int64_t col = g * VEC;
     float z[VEC];
-    load_logit_vector<ELEM>(row_in, (int)col, (int)a.V, aligned_in, z);
+    load_logit_vector<ELEM, STREAM>(row_in, (int)col, (int)a.V, aligned_in, z);
     E out[VEC];
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
@@ -472,6 +498,15 @@ hipError_t check_rows_launch(const int64_t* ids, const float* temperature, int n
   return hipGetLastError();
 }
 
+// What the forward leaves of the logits in the 256 MB memory-side cache, for a backward that starts at the columns the
+// forward ended with: of larger logits the first workgroups read past the caches, or their lines would push out one another
+// and those that are still to be used (the backward, whose reads are the last ones, does the same, see
+// logits_backward_launch). Forward + backward, bf16, everything cached / 128 / 192 / 232 MiB: 2048 x 151936 356.5 / 364.2 /
+// 349.6 / 347.0 us, 1000 x 151936 168.2 / 179.6 / 170.7 / 166.2, 4096 x 32000 149.8 / 159.7 / 154.9 / 149.6, 20000 x 32000
+// 798.6 / 765.5 / 759.8 / 757.9, fp32 2048 x 65536 322.4 / 322.6 / 313.4 / 309.7; the forward alone 129.5 -> 126.4 us at
+// 2048 x 151936, 305 -> 294 at 20000 x 32000, equal below.
+constexpr int64_t kCachedLogitsBytes = (int64_t)232 << 20;
+
 static int tiles_per_group_for(int T, int num_tiles) {
   // 256 CUs hold 2048 of these workgroups (4 waves) at a time: enough workgroups for eight rounds, so that the last
   // one, and the first loads of every workgroup, weigh little; one per row once T alone gives that. A group is a
@@ -511,6 +546,8 @@ hipError_t logits_tile_stats_launch(const void* logits, int dtype, int64_t row_s
   // every row made of whole, 16-byte aligned vectors: vector loads (the same arithmetic either way)
   const int64_t elem_bytes = dtype == RLK_DTYPE_FP32 ? 4 : 2;
   const bool aligned = (reinterpret_cast<uintptr_t>(logits) & 15) == 0 && (row_stride * elem_bytes) % 16 == 0 && V % 8 == 0;
+  const int64_t bytes = T * V * elem_bytes;
+  a.streamed = bytes > kCachedLogitsBytes ? (int64_t)((double)T * groups * (1.0 - (double)kCachedLogitsBytes / bytes)) : 0;
 #define RLK_LAUNCH_TILE_STATS(ELEM)                                                                          \
   if (aligned && has_temp) {                                                                                 \
     hipLaunchKernelGGL((logits_tile_stats_kernel<ELEM, true, true>), grid, dim3(256), 0, stream, a);         \
@@ -567,7 +604,8 @@ hipError_t logits_backward_launch(const void* logits, int dtype, int64_t row_str
   // A gradient of 128 MB and more does not stay in the 256 MB memory-side cache beside the logits it is made from, so
   // it goes past it: the logits that the forward left there survive (bf16, forward and backward, ordinary ->
   // non-temporal: 2048 x 151936 391 -> 370 us, 4096 x 32000 178 -> 159). A smaller one is left for its reader; at 155 MB
-  // (512 x 151936) the two are equal.
+  // (512 x 151936) the two are equal. The logits are read for the last time, and past the caches too: what a read brings in
+  // would take the place of what is still to be read (2048 x 151936 355 -> 349.6 us, 20000 x 32000 792 -> 760).
   const bool stream_out = T * V * (dtype == RLK_DTYPE_FP32 ? 4 : 2) >= (int64_t)128 << 20;
 #define RLK_LAUNCH_LOGITS_BACKWARD(ELEM)                                                               \
   if (stream_out) {                                                                                    \

@@ -65,3 +65,23 @@ def test_a_rejected_call_leaves_nothing_behind():
             deterministic_logp_from_logits(z, bad, temperature=temperature)
         again = deterministic_logp_from_logits(z, ids)
         assert all(torch.equal(a, b) for a, b in zip(want, again))
+
+
+# logits of more than 232 MiB: their first workgroups read past the caches, the split lying inside a row, at a row and
+# (several column groups) inside a group
+@pytest.mark.parametrize("dtype,rows,vocab", [
+    (torch.bfloat16, 812, 151936), (torch.bfloat16, 1700, 151936), (torch.float16, 20000, 6400), (torch.float32, 950, 65536),
+])  # fmt: skip
+@pytest.mark.parametrize("temperature", [None, 0.7])
+def test_streamed_forward_equals_the_same_rows_alone(dtype, rows, vocab, temperature):
+    from rl_engine.ops.logprob import deterministic_logp_from_logits
+
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    z = torch.randn((rows, vocab), generator=gen, device=DEV).to(dtype)
+    assert z.numel() * z.element_size() > 232 << 20
+    ids = torch.randint(0, vocab, (rows,), generator=gen, device=DEV)
+    whole = deterministic_logp_from_logits(z, ids, temperature=temperature)
+    for lo in range(0, rows, 256):
+        part = deterministic_logp_from_logits(z[lo : lo + 256], ids[lo : lo + 256], temperature=temperature)
+        for a, b in zip(whole, part):
+            assert torch.equal(a[lo : lo + 256].view(torch.int32), b.view(torch.int32))
