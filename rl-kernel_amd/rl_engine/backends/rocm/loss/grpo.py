@@ -15,6 +15,7 @@ from __future__ import annotations
 from typing import NamedTuple, Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from rl_engine import _C
 
@@ -54,6 +55,20 @@ def _elementwise_gradient(cur, old, ref, adv, mask, g_loss, g_policy, g_kl, clip
     return (w_policy * d_policy + w_kl * d_kl) * keep / count
 
 
+def _plain_values(tensors) -> bool:
+    """Whether the tensors are their values and nothing else, so that a kernel may read their memory: no batch of
+    gradients (``is_grads_batched``, a vectorised Jacobian), no forward-mode tangent, no subclass, nothing that records
+    the operations on them."""
+    if forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack():
+        return False
+    for t in tensors:
+        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
+            return False
+        if torch._C._functorch.is_legacy_batchedtensor(t) or torch._C._functorch.is_functorch_wrapped_tensor(t):
+            return False
+    return True
+
+
 class _GrpoLossAutograd(torch.autograd.Function):
     """Forward and backward on the HIP kernels.
 
@@ -82,7 +97,9 @@ class _GrpoLossAutograd(torch.autograd.Function):
         *inputs, workspace = ctx.saved_tensors
         if not ctx.has_mask:
             inputs.append(None)
-        if torch.is_grad_enabled():  # create_graph: the gradient itself is to be differentiated
+        given = [g for g in (g_loss, g_policy, g_kl) if g is not None]
+        # create_graph (the gradient itself is to be differentiated), or more than the values is asked for
+        if torch.is_grad_enabled() or not _plain_values(given):
             grad = _elementwise_gradient(*inputs, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
             return grad, None, None, None, None, None, None
         inputs[0] = inputs[0].contiguous()
