@@ -69,6 +69,20 @@ def _plain_values(tensors) -> bool:
     return True
 
 
+def _as_saved(inputs, shape, device) -> bool:
+    """Whether the saved tensors still are what the forward saved, in kind, type, shape and layout: a caller's
+    saved-tensor hooks may hand back anything that has the values."""
+    cur, old, ref, adv, mask = inputs
+    for t, dtype, size in ((cur, torch.float32, shape), (old, torch.float32, shape), (ref, torch.float32, shape),
+                           (adv, torch.float32, shape[:1]), (mask, torch.uint8, shape)):  # fmt: skip
+        if t is not None and not (
+            t.dtype is dtype and t.shape == size and t.is_contiguous() and t.device == device
+            and (type(t) is torch.Tensor or type(t) is torch.nn.Parameter)
+        ):  # fmt: skip
+            return False
+    return True
+
+
 class _GrpoLossAutograd(torch.autograd.Function):
     """Forward and backward on the HIP kernels.
 
@@ -83,7 +97,9 @@ class _GrpoLossAutograd(torch.autograd.Function):
         out3, ratio, k3, inputs, workspace = _C.grpo_ratio_kl_loss_saved(cur, old, ref, adv, mask, clip_eps, beta)
         ctx.has_mask = mask is not None
         # `cur` itself, not the contiguous copy that the kernel read: a gradient of the gradient flows to it
-        ctx.save_for_backward(cur, *(inputs[1:] if ctx.has_mask else inputs[1:4]), workspace)
+        ctx.save_for_backward(cur, *(inputs[1:] if ctx.has_mask else inputs[1:4]))
+        ctx.shape, ctx.device = inputs[0].shape, inputs[0].device
+        ctx.workspace = workspace  # the kernel's own numbers, no values of the caller's: not for saved-tensor hooks
         ctx.clip_eps, ctx.beta = float(clip_eps), float(beta)
         ctx.mark_non_differentiable(ratio, k3)
         ctx.set_materialize_grads(False)  # an unused output costs no zero tensor
@@ -94,16 +110,15 @@ class _GrpoLossAutograd(torch.autograd.Function):
     def backward(ctx, g_loss, g_policy, g_kl, _g_ratio, _g_k3):
         if g_loss is None and g_policy is None and g_kl is None:
             return (None,) * 7
-        *inputs, workspace = ctx.saved_tensors
-        if not ctx.has_mask:
-            inputs.append(None)
+        inputs = ctx.saved_tensors if ctx.has_mask else (*ctx.saved_tensors, None)
         given = [g for g in (g_loss, g_policy, g_kl) if g is not None]
-        # create_graph (the gradient itself is to be differentiated), or more than the values is asked for
-        if torch.is_grad_enabled() or not _plain_values(given):
-            grad = _elementwise_gradient(*inputs, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
-            return grad, None, None, None, None, None, None
-        inputs[0] = inputs[0].contiguous()
-        grad = _C.grpo_ratio_kl_loss_bwd(inputs, workspace, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
+        if not torch.is_grad_enabled() and _plain_values(given):
+            memory = (inputs[0].contiguous(), *inputs[1:])
+            if _as_saved(memory, ctx.shape, ctx.device):
+                grad = _C.grpo_ratio_kl_loss_bwd(memory, ctx.workspace, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
+                return grad, None, None, None, None, None, None
+        # the gradient itself is to be differentiated (create_graph), or more than values came in
+        grad = _elementwise_gradient(*inputs, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
         return grad, None, None, None, None, None, None
 
 

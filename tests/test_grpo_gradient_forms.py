@@ -33,12 +33,22 @@ def kernel_calls(monkeypatch):
             out3, ratio, k3 = _scalars(cur, old, ref, adv, mask)
         inputs = tuple(t.contiguous() for t in (cur, old, ref, adv))
         keep = mask.contiguous().view(torch.uint8) if mask is not None else None
-        return [out3, ratio, k3, (*inputs, keep), torch.empty(3 * cur.size(0))]
+        counts = (mask if mask is not None else torch.ones_like(cur)).sum(1, dtype=torch.float32)
+        return [out3, ratio, k3, (*inputs, keep), torch.cat([torch.zeros(2 * cur.size(0)), counts])]
 
     def backward(inputs, workspace, g_loss, g_policy, g_kl, clip_eps, beta):
         calls.append((g_loss, g_policy, g_kl))
-        memory = [t if t is None else torch.from_numpy(t.detach().numpy()) for t in (*inputs, g_loss, g_policy, g_kl)]
-        return grpo._elementwise_gradient(*memory, clip_eps, beta)
+        shape = inputs[0].shape
+        memory = []
+        for t, dtype in zip((*inputs, g_loss, g_policy, g_kl), [torch.float32] * 4 + [torch.uint8] + [torch.float32] * 3):
+            if t is not None:  # the kernel reads rows of values, whatever the tensor's own type and strides say
+                assert t.dtype is dtype, "the kernel would read past the tensor"
+                t = torch.from_numpy(t.detach().numpy())
+                t = t.as_strided(shape, (shape[1], 1)) if t.dim() == 2 else t
+            memory.append(t)
+        grad = grpo._elementwise_gradient(*memory, clip_eps, beta)
+        active = inputs[4].sum() if inputs[4] is not None else torch.tensor(shape.numel())
+        return grad * active / workspace[2 * shape[0] :].sum()
 
     monkeypatch.setattr(grpo._C, "grpo_ratio_kl_loss_saved", forward)
     monkeypatch.setattr(grpo._C, "grpo_ratio_kl_loss_bwd", backward)
@@ -90,3 +100,34 @@ def test_the_tangent_of_an_incoming_gradient(kernel_calls):
         tangent = fwd.unpack_dual(grad).tangent
     assert tangent is not None
     torch.testing.assert_close(tangent, want, rtol=2.0**-22, atol=1e-9)
+
+
+def _hooks(pack, unpack):
+    return torch.autograd.graph.saved_tensors_hooks(pack, unpack)
+
+
+def test_saved_tensors_that_hooks_hand_back(kernel_calls):
+    """Hooks that keep the values but not the layout or the type, and hooks that round them."""
+    cur, *rest = _case(rollouts=3, tokens=301)
+    x = cur.clone().requires_grad_(True)
+    (want,) = torch.autograd.grad(_loss(x, rest).loss, x)
+
+    def gradient(pack, unpack):
+        with _hooks(pack, unpack):
+            loss = _loss(x, rest).loss
+        return torch.autograd.grad(loss, x)[0]
+
+    def turned(t):
+        return t.t().contiguous().t() if t.dim() == 2 else t
+
+    torch.testing.assert_close(gradient(lambda t: t, turned), want, rtol=2.0**-22, atol=1e-9)
+    torch.testing.assert_close(gradient(lambda t: t, torch.Tensor.double), want, rtol=2.0**-19, atol=1e-9)
+
+    # values rounded to bf16: the gradient of the rounded values, over the tokens that are really there
+    def rounded(t):
+        return t.to(torch.bfloat16).to(t.dtype) if t.is_floating_point() else t
+
+    y = rounded(cur).requires_grad_(True)
+    near = [rounded(t) for t in rest[:3]] + rest[3:]
+    (want,) = torch.autograd.grad(_loss(y, near).loss, y)
+    torch.testing.assert_close(gradient(rounded, lambda t: t), want, rtol=2.0**-22, atol=1e-9)
