@@ -40,7 +40,7 @@ def _bool_mask(mask: torch.Tensor, device: torch.device) -> torch.Tensor:
 
 def _elementwise_gradient(cur, old, ref, adv, mask, g_loss, g_policy, g_kl, clip_eps: float, beta: float) -> torch.Tensor:
     """The gradient of the backward kernel in differentiable tensor operations (the same values)."""
-    keep = torch.ones_like(cur) if mask is None else mask.to(torch.float32)
+    keep = torch.ones_like(cur) if mask is None else mask.ne(0).to(torch.float32)
     count = torch.clamp(keep.sum(), min=1e-8)
     a = adv.reshape(-1, 1)
     r = torch.exp(cur - old)

@@ -131,3 +131,12 @@ def test_saved_tensors_that_hooks_hand_back(kernel_calls):
     near = [rounded(t) for t in rest[:3]] + rest[3:]
     (want,) = torch.autograd.grad(_loss(y, near).loss, y)
     torch.testing.assert_close(gradient(rounded, lambda t: t), want, rtol=2.0**-22, atol=1e-9)
+
+
+def test_mask_bytes_other_than_one_weigh_one(kernel_calls):
+    """A bool tensor made from bytes may hold any of them: the differentiable form weighs a kept token with one, as the
+    kernels do."""
+    cur, old, ref, adv, mask = _case()
+    want = grpo._elementwise_gradient(cur, old, ref, adv, mask.view(torch.uint8), torch.tensor(1.0), None, None, CLIP, BETA)
+    got = grpo._elementwise_gradient(cur, old, ref, adv, mask.to(torch.uint8) * 255, torch.tensor(1.0), None, None, CLIP, BETA)
+    assert torch.equal(got, want)
