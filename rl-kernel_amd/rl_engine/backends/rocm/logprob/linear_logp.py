@@ -11,13 +11,20 @@ entry points for this op:
   (rl_engine/reference/logprob/linear_logp.py:731-773).
 
 Unlike the reference's ROCm route (bf16 logits written to HBM, then a tile-stats
-scan, rl_engine/integrations/common/linear_logp.py:1083-1102) the logits stay in
-registers and the target logit is the fp32 accumulator value.
+scan, rl_engine/integrations/common/linear_logp.py:1083-1102) the log-probs come from
+the fp32 accumulators in registers. Without gradients no logits are written at all; a
+differentiable call keeps a copy of them in fp32 for its backward where the device has
+the memory to spare (``recompute_logits`` switches that off).
 """
 
 from __future__ import annotations
 
-from typing import Any, Optional
+import weakref
+from contextlib import contextmanager
+from contextvars import ContextVar
+from itertools import count
+from threading import Lock
+from typing import Any, Iterator, Optional
 
 import torch
 
@@ -84,31 +91,62 @@ _SAVED_LOGITS_MAX_BYTES = 8 << 30
 _SAVED_LOGITS_UNCHECKED_BYTES = 64 << 20
 
 
+# The kept logits that are alive, over all graphs: key -> (weak reference, device, bytes). An entry goes when its buffer
+# does, which is when the graph it belongs to is freed (the callback may run in any thread, so it only pops).
+_saved_logits_alive: dict[int, tuple[weakref.ref, torch.device, int]] = {}
+_saved_logits_keys = count()
+_saved_logits_lock = Lock()
+_recompute: ContextVar[bool] = ContextVar("recompute_logits", default=False)
+
+
+@contextmanager
+def recompute_logits() -> Iterator[None]:
+    """Within it (in this thread) a differentiable linear-LogP saves its inputs only, and its backward computes the logits
+    again: the same bits for 4 bytes per logit less from the forward to the backward, and a shorter forward."""
+    token = _recompute.set(True)
+    try:
+        yield
+    finally:
+        _recompute.reset(token)
+
+
 def _logits_to_save(hidden_2d: torch.Tensor, vocab: int) -> Optional[torch.Tensor]:
     """A buffer for the forward's logits, or None where the backward computes them again (the same bits).
 
-    Only memory that the device can spare is taken: at most 8 GiB and a quarter of what is free. Under saved-tensor
-    hooks (activation checkpointing, offloading) and under graph capture nothing more is saved than the inputs."""
+    Only memory that the device can spare is taken: at most 8 GiB for all graphs alive together, and for each buffer, with
+    the bf16 d(logits) that its backward needs beside it, at most a quarter of what the driver has free (what the
+    allocator has cached may be pieces: to ask it for more than it has in one piece costs it the whole cache). Under
+    saved-tensor hooks (activation checkpointing, offloading), under :func:`recompute_logits` and under graph capture
+    nothing more is saved than the inputs."""
     n, d = hidden_2d.shape
     shape = (n, _C.linear_logp_logits_row_stride(vocab))
     size = 4 * shape[0] * shape[1]
-    if n == 0 or d < _SAVED_LOGITS_MIN_HIDDEN or size > _SAVED_LOGITS_MAX_BYTES:
+    if n == 0 or d < _SAVED_LOGITS_MIN_HIDDEN or size > _SAVED_LOGITS_MAX_BYTES or _recompute.get():
         return None
     if torch._C._autograd._top_saved_tensors_default_hooks(True) is not None or torch.cuda.is_current_stream_capturing():
         return None
     if n < _SAVED_LOGITS_MIN_TOKENS and d < _SAVED_LOGITS_ANY_TOKENS_HIDDEN and 2 * vocab * d <= _MEMORY_SIDE_CACHE_BYTES:
         return None
     device = hidden_2d.device
-    if size > _SAVED_LOGITS_UNCHECKED_BYTES:
-        spare = torch.cuda.mem_get_info(device)[0]
-        if size > spare // 4:
-            spare += torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
-            if size > spare // 4:
-                return None
-    try:
-        return torch.empty(shape, dtype=torch.float32, device=device)
-    except torch.cuda.OutOfMemoryError:
-        return None
+    with _saved_logits_lock:
+        total = size + sum(held for _, where, held in list(_saved_logits_alive.values()) if where == device)
+        if total > _SAVED_LOGITS_MAX_BYTES or (total > _SAVED_LOGITS_UNCHECKED_BYTES and 4 * (size + size // 2) > _spare(device)):
+            return None
+        try:
+            logits = torch.empty(shape, dtype=torch.float32, device=device)
+        except torch.cuda.OutOfMemoryError:
+            return None
+        key = next(_saved_logits_keys)
+        gone = weakref.ref(logits, lambda _ref, key=key: _saved_logits_alive.pop(key, None))
+        _saved_logits_alive[key] = (gone, device, size)
+    return logits
+
+
+def _spare(device: torch.device) -> int:
+    """Bytes that the allocator can still get from the driver."""
+    free, total = torch.cuda.mem_get_info(device)
+    share = torch.cuda.get_per_process_memory_fraction(device)
+    return free if share >= 1.0 else min(free, int(share * total) - torch.cuda.memory_reserved(device))
 
 
 class _HipLinearLogpAutograd(torch.autograd.Function):
@@ -325,4 +363,5 @@ __all__ = [
     "LinearLogpOp",
     "hip_deterministic_linear_logp",
     "linear_logp_contract_version",
+    "recompute_logits",
 ]

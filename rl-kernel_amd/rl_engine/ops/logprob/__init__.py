@@ -11,6 +11,7 @@ from rl_engine.ops.logprob.linear_logp import (
     deterministic_linear_logp,
     linear_logp,
     linear_logp_contract_version,
+    recompute_logits,
 )
 
 __all__ = [
@@ -21,4 +22,5 @@ __all__ = [
     "linear_logp",
     "linear_logp_contract_version",
     "merge_tile_partials",
+    "recompute_logits",
 ]

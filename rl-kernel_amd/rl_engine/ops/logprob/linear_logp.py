@@ -10,6 +10,7 @@ from rl_engine.backends.rocm.logprob.linear_logp import (
     HipLinearLogpOp as LinearLogpOp,
     hip_deterministic_linear_logp as deterministic_linear_logp,
     linear_logp_contract_version,
+    recompute_logits,
 )
 
 _OP: LinearLogpOp | None = None
@@ -28,4 +29,4 @@ def linear_logp(
     return _OP(hidden, lm_head_weight, target_ids, bias)
 
 
-__all__ = ["LinearLogpOp", "deterministic_linear_logp", "linear_logp", "linear_logp_contract_version"]
+__all__ = ["LinearLogpOp", "deterministic_linear_logp", "linear_logp", "linear_logp_contract_version", "recompute_logits"]
