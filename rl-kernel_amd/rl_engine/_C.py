@@ -493,6 +493,15 @@ def linear_logp_logits_row_stride(vocab: int) -> int:
     return (vocab + 63) // 64 * 64
 
 
+def _check_kept_logits(who: str, logits: torch.Tensor, hidden: torch.Tensor, vocab: int) -> None:
+    """The kernels see a pointer and a row stride: a buffer of another type, size or device would be written past."""
+    if (
+        logits.dtype != torch.float32 or logits.device != hidden.device or not logits.is_contiguous()
+        or tuple(logits.shape) != (hidden.size(0), linear_logp_logits_row_stride(vocab))
+    ):  # fmt: skip
+        raise RuntimeError(f"{who}: logits must be contiguous fp32 [N, {linear_logp_logits_row_stride(vocab)}] beside hidden")
+
+
 def fused_linear_logp_into(
     hidden: torch.Tensor,
     weight: torch.Tensor,
@@ -506,6 +515,7 @@ def fused_linear_logp_into(
     config: int = 0,
 ) -> List[torch.Tensor]:
     """:func:`fused_linear_logp` that also stores its fp32 logits in ``logits`` for :func:`fused_linear_logp_bwd`."""
+    _check_kept_logits("fused_linear_logp_into", logits, hidden, weight.size(0))
     logp, lse, _ = _linear_logp_forward(
         "fused_linear_logp", "rlk_linear_logp_fwd", hidden, weight, target, bias, temperature,
         real_vocab_size, vocab_start_index, config, logits=logits,
@@ -590,11 +600,8 @@ def fused_linear_logp_bwd(
     if not 0 < real_vocab <= v:
         raise RuntimeError(f"fused_linear_logp_bwd: real_vocab_size must be in [1, {v}]")
 
-    if logits is not None and (
-        logits.dtype != torch.float32 or logits.device != hidden.device or not logits.is_contiguous()
-        or tuple(logits.shape) != (n, linear_logp_logits_row_stride(v))
-    ):  # fmt: skip
-        raise RuntimeError("fused_linear_logp_bwd: logits must be the fp32 tensor the forward stored")
+    if logits is not None:
+        _check_kept_logits("fused_linear_logp_bwd", logits, hidden, v)
 
     def _per_row(t: Optional[torch.Tensor], name: str) -> Optional[torch.Tensor]:
         if t is None:

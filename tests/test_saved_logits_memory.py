@@ -128,3 +128,19 @@ def test_switched_off_for_a_block(device):
     with pytest.raises(KeyError), module.recompute_logits():
         raise KeyError
     assert module._logits_to_save(_hidden(), VOCAB) is not None
+
+
+@pytest.mark.parametrize("wrong", ["rows", "columns", "stride", "dtype", "device"])
+def test_the_forward_refuses_a_buffer_that_it_would_write_past(wrong):
+    """Refused by its shape, before anything reaches a device (the operands here are on none)."""
+    hidden, weight = _hidden(), torch.empty((VOCAB, module._SAVED_LOGITS_MIN_HIDDEN), dtype=torch.bfloat16)
+    columns = _C.linear_logp_logits_row_stride(VOCAB)
+    logits = {
+        "rows": torch.empty((TOKENS - 1, columns)),
+        "columns": torch.empty((TOKENS, VOCAB)),
+        "stride": torch.empty((columns, TOKENS)).t(),
+        "dtype": torch.empty((TOKENS, columns), dtype=torch.bfloat16),
+        "device": torch.empty((TOKENS, columns), device="meta"),
+    }[wrong]
+    with pytest.raises(RuntimeError, match="logits must be"):
+        _C.fused_linear_logp_into(hidden, weight, torch.zeros(TOKENS, dtype=torch.long), None, None, VOCAB, logits)
