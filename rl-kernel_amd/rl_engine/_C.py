@@ -855,9 +855,11 @@ class RowChecks:
     __slots__ = ("_flags", "_event")
 
     def __init__(self, ids: torch.Tensor, lo: int, hi: int, temperature: Optional[torch.Tensor] = None) -> None:
-        self._flags = torch.zeros((2,), dtype=torch.int32, pin_memory=True)
-        self._event = torch.cuda.Event()
         with _on(ids.device):
+            if torch.cuda.is_current_stream_capturing():  # a replay would store to the flags long after they are gone
+                raise RuntimeError("values that are read back to be checked cannot be captured into a graph")
+            self._flags = torch.zeros((2,), dtype=torch.int32, pin_memory=True)
+            self._event = torch.cuda.Event()
             status = _lib.load().rlk_check_rows(
                 ids.data_ptr(), temperature.data_ptr() if temperature is not None else None, ids.numel(), int(lo), int(hi),
                 self._flags.data_ptr(), _stream_handle(ids.device),
