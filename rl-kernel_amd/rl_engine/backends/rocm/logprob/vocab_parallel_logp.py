@@ -127,14 +127,14 @@ def hip_deterministic_logp_from_logits(
     target_1d = target_1d.contiguous()
     temp = _temperature_rows(temperature, rows, local_logits.device)
     fits = temp is None or temp.numel() == rows
-    checks = _C.RowChecks(target_1d, 0, real, temp if fits else None)
+    checks = _C.RowChecks(target_1d, 0, real, temp if fits else None) if rows else None
     try:
         if fits:  # runs behind the checks; the wait below is for them alone
             logp, lse = _HipLogpFromLogits.apply(
                 local_logits, target_1d, temp, int(vocab_start_index), real, int(num_vocab_tiles)
             )
     finally:  # the kernel writes to host memory that `checks` owns: never left behind unfinished
-        bad_id, bad_temperature = checks.results()
+        bad_id, bad_temperature = checks.results() if checks is not None else (False, False)
     if bad_id:
         raise ValueError(f"target_ids must be in the real vocabulary [0, {real})")
     if bad_temperature or not fits:

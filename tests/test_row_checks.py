@@ -42,3 +42,20 @@ def test_a_capture_goes_on_after_the_refusal():
         torch.cuda.synchronize()
         assert bool((y == start + 1).all())
     assert all(torch.equal(a, b) for a, b in zip(want, deterministic_logp_from_logits(z, ids)))
+
+
+@pytest.mark.gpu
+def test_no_rows_have_nothing_to_check(monkeypatch):
+    """No launch, no host memory and no wait; the temperature's size still counts."""
+    from rl_engine.ops.logprob import deterministic_logp_from_logits
+
+    def unused(*args):
+        raise AssertionError("nothing to check")
+
+    monkeypatch.setattr(_C, "RowChecks", unused)
+    z, ids = torch.empty((0, 640), device="cuda"), torch.empty(0, dtype=torch.long, device="cuda")
+    for temperature in (None, 0.7, torch.empty(0)):
+        logp, lse = deterministic_logp_from_logits(z, ids, temperature=temperature)
+        assert logp.shape == lse.shape == (0,)
+    with pytest.raises(ValueError, match="temperature"):
+        deterministic_logp_from_logits(z, ids, temperature=torch.ones(3))
