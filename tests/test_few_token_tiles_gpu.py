@@ -10,8 +10,8 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-# tokens: below, at and above the edges of the tiles, and of the one and a half tiles that bring in the prefetching wave; features: less than a tile, whole tiles, a last tile that
-# is not whole; reductions: the fewest stages, fewer stages than the ring holds, more
+# tokens: below, at and above the edges of the tiles, and of the one and a half tiles that bring in the prefetching wave;
+# features: less than a tile, whole tiles, a last tile that is not whole; reductions: the fewest stages, fewer stages than the ring holds, more
 @pytest.mark.parametrize("config,stage", [("32x32_deep", 128), ("32x64_deep", 256), ("64x32_deep", 256), ("64x96_deep", 128), ("64x160_deep", 128),
                                           ("128x64_deep", 128)])
 @pytest.mark.parametrize("tokens", [1, 31, 32, 33, 65, 95, 96, 97, 129, 144, 145, 160, 161, 193, 241])
@@ -33,17 +33,26 @@ def test_same_bits_as_the_one_wave_tile(config, stage, tokens, features):
             assert torch.equal(out.view(bits), want.view(bits)), (stages, dtype)
 
 
-# Shapes that the automatic choice gives to them, with a padded row pitch: 32 x 32, with the weight read past the caches
-# too; 32 x 64 without and (from 96 MiB of weight, an odd number of stages among them) with the prefetching wave; 64 x 32;
-# 64 x 96 with the wave and with the weight read past the caches; 128 x 64 and 64 x 160 with the wave.
+# Shapes that the automatic choice gives to them, with a padded row pitch, for every form that it reaches: the plain loop,
+# the weight read past the caches (one token tile, from 96 MiB of weight), the prefetching wave (several token tiles: from
+# 96 MiB and with the last tile more than half full for 32 x 64 and 64 x 32, else always); each with a ragged neighbour
+# (a last tile that is not whole, an odd number of stages).
 @pytest.mark.parametrize(
-    "tokens,features,k",
-    [(20, 6144, 4096), (30, 6144, 8320), (50, 4096, 4096), (65, 4096, 4096), (200, 1536, 4096), (80, 4096, 12288),
-     (128, 4096, 12544), (20, 12288, 4096), (333, 4096, 12288), (90, 12288, 4096), (500, 4096, 4096), (600, 4096, 4096)],
+    "config,tokens,features,k",
+    [("32x32_deep", 20, 6144, 4096), ("32x32_deep", 50, 4096, 4096), ("32x32_deep", 30, 6144, 8320),
+     ("32x64_deep", 65, 4096, 4096), ("32x64_deep", 200, 1536, 4096), ("32x64_deep", 80, 4096, 12288),
+     ("32x64_deep", 64, 8192, 8192), ("32x64_deep", 61, 8190, 8448), ("32x64_deep", 128, 4096, 12544), ("32x64_deep", 101, 4090, 12544),
+     ("64x32_deep", 20, 9000, 1280), ("64x32_deep", 20, 12288, 4096), ("64x32_deep", 66, 5120, 25600),
+     ("64x32_deep", 96, 5120, 25600), ("64x32_deep", 85, 5118, 25856),
+     ("64x96_deep", 140, 8190, 1152), ("64x96_deep", 90, 12288, 4096), ("64x96_deep", 333, 4096, 12288), ("64x96_deep", 150, 8190, 1152),
+     ("64x160_deep", 150, 12288, 2048), ("64x160_deep", 150, 12288, 4096), ("64x160_deep", 129, 12346, 4224),
+     ("64x160_deep", 600, 4096, 4096), ("64x160_deep", 651, 3250, 4224),
+     ("128x64_deep", 500, 4096, 4096), ("128x64_deep", 120, 12288, 4096)],
 )  # fmt: skip
-def test_chosen_shapes(tokens, features, k):
+def test_chosen_shapes(config, tokens, features, k):
     from rl_engine import _C, _lib
 
+    assert _C.det_gemm_pick_config(tokens, features, k) == _lib.GEMM_CONFIGS[config]
     gen = torch.Generator(device=DEV).manual_seed(tokens)
     x = torch.randn((tokens, k + 8), generator=gen, device=DEV, dtype=torch.bfloat16)[:, :k]
     w = torch.randn((features, k), generator=gen, device=DEV, dtype=torch.bfloat16)

@@ -1,8 +1,9 @@
 """A CPU model of the lane addresses of the native-layout direct-to-LDS loader (DmaLoader in csrc/det_gemm_tile.h):
 its row maps, chunk swizzle and edge clamping, with the widths the kernel computes in (64-bit pointers, 32-bit lane
-offsets), and of its K-major weight form. Walks launch grids of the GEMM, the gated projection and the stream-group LogP kernel - including the
-workgroups whose origin lies past the last vocabulary row - and asserts that every lane reads 16 bytes inside its
-operand, at the row and K position the stage layout expects. As a control, the same walk with the edge path's row
+offsets), of its K-major weight form, of the four-wave loop's loads (tile_mainloop_quad) and of the two prefetching waves
+(prefetch_quad_panel, prefetch_kmajor_panel). Walks launch grids of the GEMM, the gated projection and the stream-group LogP
+kernel - including the workgroups whose origin lies past the last vocabulary row - and asserts that every lane reads 16
+bytes inside its operand, at the row and K position the stage layout expects. As a control, the same walk with the edge path's row
 distance computed in 32 bits (a form that once faulted the GPU) must leave the operand."""
 
 from __future__ import annotations
@@ -148,3 +149,132 @@ def test_kmajor_weight_tiles_read_inside_the_weight(bn, n, k, ld):
                 seen.add((k_row, feat))
             if n0 + bn <= n:  # an interior tile: every 8-feature chunk of every K row exactly once
                 assert len(seen) == 64 * (bn // 8)
+
+
+QUAD_TILES = [  # features, tokens, K tiles per stage, stages of the ring
+    (32, 32, 2, 8), (32, 64, 4, 3), (64, 32, 4, 3), (64, 96, 2, 3), (64, 160, 1, 5), (128, 64, 1, 6),
+]  # fmt: skip
+K_TILE, PREFETCH_TILES, XCDS = 64, 4, 8
+
+
+def quad_addresses(rows_of_tile: int, origin: int, rows: int, ld: int, is_weight: bool):
+    """(LDS byte of the stage's operand part, element address at K = 0, row, first K value) of every lane of the four
+    waves; the addresses are 64-bit sums of a clamped row's start and the lane's chunk."""
+    tn = rows_of_tile // 32  # two waves along the features
+    for wave, j, lane in itertools.product(range(4), range(rows_of_tile // 32), range(64)):
+        block, rib = 4 * j + wave, lane >> 3
+        chunk = ((lane & 7) ^ rib) * 8
+        if is_weight:
+            want = origin + plain_block_offset(block, tn) + lane_offset(wave & 1, rib, 4 * tn)
+        else:
+            want = origin + 8 * block + rib
+        row = min(want, rows - 1)
+        yield block * 1024 + lane * 16, row * ld + chunk, row, chunk
+
+
+@pytest.mark.parametrize("bn,bm,ks,ns", QUAD_TILES)
+@pytest.mark.parametrize("rows", [1, 31, 200, 321])
+def test_the_four_wave_loop_reads_inside_its_operands(bn, bm, ks, ns, rows):
+    for size, is_weight in ((bn, True), (bm, False)):
+        for stages in (1, 2, ns + 1):
+            k = stages * ks * K_TILE
+            ld = k + 8
+            # stage t's first K value, past the last stage the last one again
+            starts = {min(t, stages - 1) * ks * K_TILE for t in range(stages + ns)}
+            for origin in sorted({0, (rows - 1) // size * size}):
+                lanes = list(quad_addresses(size, origin, rows, ld, is_weight))
+                assert sorted(lds for lds, *_ in lanes) == list(range(0, size * 128, 16))  # the operand's part of a K tile
+                for _, addr, row, chunk in lanes:
+                    assert addr == row * ld + chunk and origin <= row < rows
+                    for at in (start + s * K_TILE for start in starts for s in range(ks)):
+                        assert addr + at + 8 <= (rows - 1) * ld + k and chunk + at + 8 <= k
+                if origin + size <= rows:  # an interior tile: every row's eight chunks exactly once
+                    assert sorted((row - origin, chunk) for _, _, row, chunk in lanes) == [
+                        (r, c * 8) for r in range(size) for c in range(8)
+                    ]
+
+
+def xcd_compact_id(wg: int, total: int) -> int:
+    per, rem, xcd, slot = total // XCDS, total % XCDS, wg % XCDS, wg // XCDS
+    return xcd * per + min(xcd, rem) + slot
+
+
+def panel_shares(tiles_m: int, tiles_n: int):
+    """workgroup -> (XCD, weight panel, group of token tiles, share, shares), as det_gemm_kernel computes them."""
+    total, group_m = tiles_m * tiles_n, min(tiles_m, 8)
+    for wg in range(total):
+        tile = xcd_compact_id(wg, total)
+        group, within = divmod(tile, group_m * tiles_n)
+        width = min(tiles_m - group * group_m, group_m)
+        panel = tile - within % width
+        first = xcd_compact_id(wg % XCDS, total)
+        owned = total // XCDS + (1 if wg % XCDS < total % XCDS else 0)
+        lo, hi = max(panel, first), min(panel + width, first + owned)
+        yield wg % XCDS, within // width, group, tile - lo, hi - lo
+
+
+@pytest.mark.parametrize("tiles_m,tiles_n", [(2, 128), (4, 64), (6, 37), (3, 5), (9, 20), (17, 3), (1, 7), (8, 1)])
+def test_the_workgroups_of_an_xcd_share_a_panel_without_gap_or_overlap(tiles_m, tiles_n):
+    shares: dict = {}
+    for xcd, tile_n, group, index, of in panel_shares(tiles_m, tiles_n):
+        shares.setdefault((xcd, tile_n, group), []).append((index, of))
+    for got in shares.values():
+        assert sorted(got) == [(i, len(got)) for i in range(len(got))]
+
+
+def bursts(k: int, ks: int, ns: int):
+    """(first K tile, K tiles) of every burst of a prefetching wave beside a ring of ns stages of ks K tiles."""
+    k_tiles = k // (ks * K_TILE) * ks
+    for t in range(k_tiles // ks):
+        first = t * ks + ns * ks + 1
+        if t * ks % PREFETCH_TILES == 0 and first < k_tiles:
+            yield first, min(k_tiles - first, PREFETCH_TILES)
+
+
+def quad_prefetch(bn: int, n0: int, rows: int, first_tile: int, lines: int, index: int, count: int):
+    per = -(-bn // count)
+    mine = min(bn - index * per, per)
+    for lane in range(64):
+        for i in range(lane, mine * PREFETCH_TILES, 64):
+            line = min(i % PREFETCH_TILES, lines - 1)
+            yield min(n0 + index * per + i // PREFETCH_TILES, rows - 1), (first_tile + line) * K_TILE
+
+
+@pytest.mark.parametrize("bn,ks,ns", [(bn, ks, ns) for bn, _, ks, ns in QUAD_TILES if bn > 32 or ks == 4])
+@pytest.mark.parametrize("rows", [40, 64, 1000])
+def test_the_four_wave_loops_prefetch_touches_the_whole_panel_and_nothing_else(bn, ks, ns, rows):
+    assert PREFETCH_TILES % ks == 0
+    for k in (ks * K_TILE, 7 * ks * K_TILE, 25 * ks * K_TILE):
+        for n0, count in itertools.product(sorted({0, (rows - 1) // bn * bn}), (1, 2, 3, 5, 8)):
+            ahead = list(bursts(k, ks, ns))
+            for first, lines in ahead:
+                touched = {t for i in range(count) for t in quad_prefetch(bn, n0, rows, first, lines, i, count)}
+                assert touched == {
+                    (row, (first + line) * K_TILE) for row in range(n0, min(n0 + bn, rows)) for line in range(lines)
+                }  # 4 bytes at each: two values
+                assert all(0 <= row < rows and at + 2 <= k for row, at in touched)
+            # from the first burst on, no K tile of the whole stages is left out
+            tiles = [tile for first, lines in ahead for tile in range(first, first + lines)]
+            assert tiles == list(range(ns * ks + 1, k // K_TILE))
+
+
+def kmajor_prefetch(bn: int, n0: int, rows: int, first_tile: int, tiles: int, index: int, count: int):
+    lines, k_rows = bn // 64, tiles * K_TILE
+    per = -(-k_rows // count)
+    mine = min(k_rows - index * per, per)
+    for lane in range(64):
+        for i in range(lane, mine * lines, 64):
+            n = n0 + (i % lines) * 64
+            yield first_tile * K_TILE + index * per + i // lines, n if n < rows else rows - 8
+
+
+@pytest.mark.parametrize("bn,ks,ns", [(64, 2, 4), (128, 2, 3), (128, 2, 2)])
+@pytest.mark.parametrize("rows", [8, 72, 1000, 4096])
+def test_the_kmajor_prefetch_touches_the_whole_panel_and_nothing_else(bn, ks, ns, rows):
+    for k in (ns * ks * K_TILE, 13 * ks * K_TILE + 48):
+        for n0, count in itertools.product(sorted({0, (rows - 1) // bn * bn}), (1, 2, 3, 5, 8)):
+            for first, tiles in bursts(k, ks, ns):
+                touched = {t for i in range(count) for t in kmajor_prefetch(bn, n0, rows, first, tiles, i, count)}
+                starts = {n if n < rows else rows - 8 for n in range(n0, n0 + bn, 64)}
+                assert touched == {(row, n) for row in range(first * K_TILE, (first + tiles) * K_TILE) for n in starts}
+                assert all(row < k // (ks * K_TILE) * ks * K_TILE and 0 <= n and n + 2 <= rows for row, n in touched)
