@@ -389,9 +389,10 @@ static hipError_t launch_deep(const MatView& W, const MatView& X, void* C, int64
 //   128 x 64, 512 tokens: 78.1 / 65.6 -> 86.9 / 63.9 -> 69.8 / 62.2 (six stages of one K tile)
 //   32 x 64, 128 tokens:  45.2 / 29.6 -> 42.0 / 32.8 with the wave            80 tokens:  33.4 / 28.7 -> 36.1 / 30.8
 // (64 x 64, 256 tokens: 49.2 / 41.4 -> 59.2 / 39.3 -> 50.2 / 41.2, 128 x 128: 99 / 93 -> 117 / 107: they stay with eight
-// waves.) The 64 x 96, 64 x 160 and 128 x 64 tiles always run with it, the smaller ones where the weight is larger than what the
-// memory-side cache holds beside others (96 MiB) and the last token tile is more than half full, 32 x 32 never (two readers
-// at most: 64 tokens 33.2 -> 35.1).
+// waves.) A panel that several workgroups read always has the wave on 64 x 96 and 64 x 160 tiles (and on 128 x 64, which
+// are launched without this rule), on the smaller ones where the weight is larger than what the memory-side cache holds
+// beside others (96 MiB) and the last token tile is more than half full, on 32 x 32 never (two readers at most: 64 tokens
+// 33.2 -> 35.1).
 template <class S, int KS, int NS, bool PREFETCH = true>
 static hipError_t launch_quad(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K, bool out_f32,
                               hipStream_t stream) {
@@ -408,15 +409,14 @@ static hipError_t launch_quad(const MatView& W, const MatView& X, void* C, int64
   return launch_tile<S, kLoopQuad, false, KS, NS>(W, X, C, ldc, M, N, K, stream);
 }
 
-// The register-staged K-major-weight loop of a small tile with as many K tiles per stage as 128 KiB of LDS
-// hold (four for 64 x 64, two for the 128-token tiles): a long reduction wants several K tiles in flight per
-// workgroup. (Reductions that 128 does not divide run the ping-pong loop too: LogP grad_hidden, 1024 tokens, V = 18992,
-// 250 us register-staged, 154 us with the rest of 48 values behind the ring.)
+// The loops of a small tile for a K-major weight: from one ring on (512 / 384 / 256 values of K for 64 x 64 / 128 x 64 /
+// 128 x 128) the direct-to-LDS ping-pong loop, with the rest that its stages do not divide behind it (LogP grad_hidden,
+// 1024 tokens, V = 18992, whose rest is 48 values: 154 us, register-staged 250); below that the register-staged loop, whose
+// two stages hold all or most of so short a reduction.
 template <class S>
-static hipError_t launch_staged_kmajor(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
+static hipError_t launch_small_kmajor(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
                                        bool out_f32, hipStream_t stream) {
-  // The direct-to-LDS ping-pong loop over stages of two K tiles with a ring of as many stages as 128 KiB (144 for the
-  // 128 x 64 tile) hold, and the rest of the reduction behind it; below one ring the register-staged loop.
+  // Stages of two K tiles, as many of them as 128 KiB (144 for the 128 x 64 tile) hold.
   constexpr int kDmaKs = 2;
   constexpr int kDmaNs = S::kStageBytes <= 16 * 1024 ? 4 : S::kStageBytes <= 24 * 1024 ? 3 : 2;
   if (K >= kTileK * kDmaKs * kDmaNs)
@@ -658,13 +658,13 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
         if (!x_kmajor) return launch_shape<Shape256x64>(W, X, C, ldc, M, N, K, false, loop, true, out_f32, stream);
         break;
       case RLK_GEMM_CFG_64x64:
-        if (w_kmajor && x_native) return launch_staged_kmajor<Shape64x64>(W, X, C, ldc, M, N, K, out_f32, stream);
+        if (w_kmajor && x_native) return launch_small_kmajor<Shape64x64>(W, X, C, ldc, M, N, K, out_f32, stream);
         break;
       case RLK_GEMM_CFG_128x64:
-        if (w_kmajor && x_native) return launch_staged_kmajor<Shape128x64>(W, X, C, ldc, M, N, K, out_f32, stream);
+        if (w_kmajor && x_native) return launch_small_kmajor<Shape128x64>(W, X, C, ldc, M, N, K, out_f32, stream);
         break;
       case RLK_GEMM_CFG_128x128:
-        if (w_kmajor && x_native) return launch_staged_kmajor<Shape128x128>(W, X, C, ldc, M, N, K, out_f32, stream);
+        if (w_kmajor && x_native) return launch_small_kmajor<Shape128x128>(W, X, C, ldc, M, N, K, out_f32, stream);
         break;
       default:
         break;  // an explicitly requested other shape runs the element-wise loader below
@@ -698,8 +698,9 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
       if (config == RLK_GEMM_CFG_128x64_DEEP) {
         // Two token tiles only (12288 outputs at 97 ... 128 tokens) gain nothing from HBM and lose from the cache (K = 4096,
         // 100 tokens: 31.7 / 23.7 us with eight waves, 32.0 / 26.5 with four and the prefetch).
-        return M <= 2 * Shape128x64::BM ? launch_deep<Shape128x64, kDeep128, 3>(W, X, C, ldc, M, N, K, out_f32, stream)
-                                        : launch_quad<Quad128x64, 1, 6>(W, X, C, ldc, M, N, K, out_f32, stream);
+        if (M <= 2 * Shape128x64::BM) return launch_deep<Shape128x64, kDeep128, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
+        return out_f32 ? launch_tile<Quad128x64, kLoopQuadPrefetch, true, 1, 6>(W, X, C, ldc, M, N, K, stream)
+                       : launch_tile<Quad128x64, kLoopQuadPrefetch, false, 1, 6>(W, X, C, ldc, M, N, K, stream);
       }
       if (config == RLK_GEMM_CFG_64x64_DEEP) return launch_deep<Shape64x64, kDeep64>(W, X, C, ldc, M, N, K, out_f32, stream);
       return launch_deep<Shape128x128, kDeep128>(W, X, C, ldc, M, N, K, out_f32, stream);
