@@ -99,7 +99,7 @@ struct Stager {
       const int k = k0 + chunk_k[i];
       if (VEC) {
         if (TAIL) {
-          const bool ok = k < K;  // K % 8 == 0 on this path: a chunk is all in or all out
+          const bool ok = k < K;  // a chunk that starts inside is read whole: K % 8 == 0, or MatView::k_padded
           u32x4_t v = *reinterpret_cast<const u32x4_t*>(src[i] + (ok ? k : 0));
           const u32x4_t z = {0u, 0u, 0u, 0u};
           regs[i] = ok ? v : z;
@@ -225,18 +225,18 @@ struct IntTag {
   static constexpr int value = V;
 };
 
-// The register-staged loop with a K-major weight operand (B[K, N], N contiguous) for the small tiles, which
-// have no direct-to-LDS K-major loop: 16-byte loads of eight features at one k, the K-major stage layout and
-// transposing fragment reads; activations as in tile_mainloop_staged. With this operand MFMA tile jn of a
+// The register-staged loop with a K-major weight operand (B[K, N], N contiguous) for small tiles whose reduction is
+// shorter than one ring of the direct-to-LDS K-major loop: 16-byte loads of eight features at one k, the K-major stage
+// layout and transposing fragment reads; activations as in tile_mainloop_staged. With this operand MFMA tile jn of a
 // wave holds features (wave_n * TN + jn) * 16 + (lane >> 4) * 4 + q. Same MFMA chain: same bits.
 // A stage holds KS consecutive K tiles, and the loads of two stages are in flight while a third is
-// multiplied: these tiles serve long reductions against few outputs (one workgroup per CU), where one K
-// tile in flight per workgroup would make every iteration a memory round trip. Every load is issued
+// multiplied: with few workgroups per CU, one K tile in flight per workgroup would make every iteration a
+// memory round trip (the whole of such a reduction is one to three stages). Every load is issued
 // unconditionally (past the end it repeats the last K tile and its data is dropped), so the waits the
 // compiler places count loads on one straight path.
 // The last stage may hold fewer than KS tiles, and the last K tile fewer than 64 K values (the rest is
-// filled with zeros in both operands, as in every other loop). Needs BN % 64 == 0, N % 8 == 0, K % 8 == 0
-// (the activation chunks); 2 * KS * kStageBytes of LDS.
+// filled with zeros in both operands, as in every other loop). Needs BN % 64 == 0, N % 8 == 0, whole activation
+// chunks (K % 8 == 0, or MatView::k_padded); 2 * KS * kStageBytes of LDS.
 template <class S, int KS, bool RAGGED>
 __device__ __forceinline__ void tile_mainloop_staged_kmajor(const MatView& W, const MatView& X, int n0, int m0, int K,
                                                             char* lds, f32x4_t (&acc)[S::TN][S::TM]) {
@@ -290,7 +290,7 @@ __device__ __forceinline__ void tile_mainloop_staged_kmajor(const MatView& W, co
       }
 #pragma unroll
       for (int i = 0; i < S::kXIters; ++i) {
-        const int k = k0 + sx.chunk_k[i];  // K % 8 == 0: a chunk is all in or all out
+        const int k = k0 + sx.chunk_k[i];  // a chunk that starts inside is read whole (K % 8 == 0, or k_padded)
         if constexpr (RAGGED) {
           const u32x4_t v = *reinterpret_cast<const u32x4_t*>(sx.src[i] + (k < K ? k : 0));
           xr[R][q][i] = k < K ? v : zero;
@@ -762,7 +762,8 @@ constexpr bool pingpong_supported() {
 // Measured with weights from HBM, without -> with (dX = dY W, 4096 outputs): K = 12288 at 128 / 256 / 512 / 1024 tokens
 // 69.0 / 67.0 / 87.0 / 122 -> 56.3 / 52.7 / 75.5 / 110 us, K = 151936 at 256 / 512 / 1024 tokens 792 / 1032 / 1464 ->
 // 643 / 899 / 1282 us. Bursts of 8 and 16 K tiles: equal to 4 % slower; leads of 1 to 4 K tiles beyond the ring: equal.
-// (The native-layout loops do not gain: their small tiles take as long from the caches.)
+// (The eight-wave loops of the native layout do not gain: their small tiles take as long from the caches. The four-wave
+// loop does, see prefetch_quad_panel.)
 // The wave takes part in the loop's barriers, all 2 K / (64 KS) + 3 of them, and loads into `dump` (256 bytes of LDS).
 constexpr int kPrefetchTiles = 4;
 
@@ -1013,7 +1014,8 @@ __device__ __forceinline__ void tile_mainloop_pingpong(const MatView& W, const M
 // K values [k0, K) go through registers (16-byte chunks, zeros at and past K, addresses clamped into the
 // matrix), into stage 0 in the layout the loop uses, and through the same fragment reads and two MFMA steps.
 // The chain of an output element is the one every other loop runs: K tiles ascending, the tail zero-filled
-// to a multiple of 64 in both operands. A native operand needs K % 8 == 0 (a chunk is all in or all out).
+// to a multiple of 64 in both operands. A native operand is read in whole chunks: K % 8 == 0, or MatView::k_padded beside a
+// K-major operand, whose own rows past K are the zeros.
 // Call it after the loop (which ends on a barrier); it ends on a barrier as well.
 // ---------------------------------------------------------------------------
 // Everything here is derived from a thread index the compiler cannot see through, so that none of the step's
