@@ -24,6 +24,10 @@ def _stream_handle(device: torch.device) -> int:
     return torch._C._cuda_getCurrentRawStream(device.index)
 
 
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return t.data_ptr() if t is not None else None
+
+
 class _NoSwitch:
     """A context manager that does nothing: the device is already current."""
 
@@ -629,9 +633,6 @@ def fused_linear_logp_bwd(
     # torch's allocator hands out 512-byte aligned blocks, which covers the 256 the library asks for
     workspace = torch.empty((max(ws_bytes, 256),), dtype=torch.uint8, device=hidden.device)
 
-    def _ptr(t: Optional[torch.Tensor]):
-        return t.data_ptr() if t is not None else None
-
     if n == 0:  # no tokens: the token-summed gradients are zero
         if grad_weight is not None:
             grad_weight.zero_()
@@ -1122,9 +1123,8 @@ def grpo_ratio_kl_loss_bwd(
     grad = torch.empty_like(logp)
     with _on(logp.device):
         status = _lib.load().rlk_grpo_ratio_kl_loss_bwd(
-            logp.data_ptr(), old.data_ptr(), ref.data_ptr(), adv.data_ptr(), mask.data_ptr() if mask is not None else None,
-            workspace.data_ptr(), workspace.numel() * 4,
-            *(g.data_ptr() if g is not None else None for g in (g_loss, g_policy, g_kl)),
+            logp.data_ptr(), old.data_ptr(), ref.data_ptr(), adv.data_ptr(), _ptr(mask), workspace.data_ptr(), workspace.numel() * 4,
+            _ptr(g_loss), _ptr(g_policy), _ptr(g_kl),
             rollouts, tokens, 1.0 - clip_eps, 1.0 + clip_eps, beta, grad.data_ptr(), _stream_handle(logp.device),
         )  # fmt: skip
     _lib.check(status, "rlk_grpo_ratio_kl_loss_bwd failed")

@@ -55,32 +55,32 @@ def _elementwise_gradient(cur, old, ref, adv, mask, g_loss, g_policy, g_kl, clip
     return (w_policy * d_policy + w_kl * d_kl) * keep / count
 
 
-def _plain_values(tensors) -> bool:
-    """Whether the tensors are their values and nothing else, so that a kernel may read their memory: no batch of
+_is_batch = torch._C._functorch.is_legacy_batchedtensor
+_is_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+
+
+def _only_values(g_loss, g_policy, g_kl) -> bool:
+    """Whether the gradients are their values and nothing else, so that a kernel may read their memory: no batch of
     gradients (``is_grads_batched``, a vectorised Jacobian), no forward-mode tangent, no subclass, nothing that records
     the operations on them."""
-    if forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack():
+    if forward_ad._current_level >= 0 or _dispatch_modes():
         return False
-    for t in tensors:
-        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
-            return False
-        if torch._C._functorch.is_legacy_batchedtensor(t) or torch._C._functorch.is_functorch_wrapped_tensor(t):
+    for g in (g_loss, g_policy, g_kl):
+        if g is not None and (type(g) is not torch.Tensor or _is_batch(g) or _is_wrapped(g)):
             return False
     return True
 
 
-def _as_saved(inputs, shape, device) -> bool:
-    """Whether the saved tensors still are what the forward saved, in kind, type, shape and layout: a caller's
-    saved-tensor hooks may hand back anything that has the values."""
-    cur, old, ref, adv, mask = inputs
-    for t, dtype, size in ((cur, torch.float32, shape), (old, torch.float32, shape), (ref, torch.float32, shape),
-                           (adv, torch.float32, shape[:1]), (mask, torch.uint8, shape)):  # fmt: skip
-        if t is not None and not (
-            t.dtype is dtype and t.shape == size and t.is_contiguous() and t.device == device
-            and (type(t) is torch.Tensor or type(t) is torch.nn.Parameter)
-        ):  # fmt: skip
-            return False
-    return True
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def _in_memory_as(t, dtype, numel: int, gpu: int) -> bool:
+    """Whether ``t`` lies in memory as the forward saved it: a caller's saved-tensor hooks may hand back anything that has
+    the values."""
+    return (
+        t.dtype is dtype and t.is_contiguous() and t.numel() == numel and t.get_device() == gpu and type(t) in _PLAIN_TYPES
+    )
 
 
 class _GrpoLossAutograd(torch.autograd.Function):
@@ -98,8 +98,8 @@ class _GrpoLossAutograd(torch.autograd.Function):
         ctx.has_mask = mask is not None
         # `cur` itself, not the contiguous copy that the kernel read: a gradient of the gradient flows to it
         ctx.save_for_backward(cur, *(inputs[1:] if ctx.has_mask else inputs[1:4]))
-        ctx.shape, ctx.device = inputs[0].shape, inputs[0].device
-        ctx.workspace = workspace  # the kernel's own numbers, no values of the caller's: not for saved-tensor hooks
+        # the workspace holds the kernel's own numbers, no values of the caller's: it is not for saved-tensor hooks
+        ctx.forward = (cur.shape, cur.get_device(), workspace)
         ctx.clip_eps, ctx.beta = float(clip_eps), float(beta)
         ctx.mark_non_differentiable(ratio, k3)
         ctx.set_materialize_grads(False)  # an unused output costs no zero tensor
@@ -110,15 +110,20 @@ class _GrpoLossAutograd(torch.autograd.Function):
     def backward(ctx, g_loss, g_policy, g_kl, _g_ratio, _g_k3):
         if g_loss is None and g_policy is None and g_kl is None:
             return (None,) * 7
-        inputs = ctx.saved_tensors if ctx.has_mask else (*ctx.saved_tensors, None)
-        given = [g for g in (g_loss, g_policy, g_kl) if g is not None]
-        if not torch.is_grad_enabled() and _plain_values(given):
-            memory = (inputs[0].contiguous(), *inputs[1:])
-            if _as_saved(memory, ctx.shape, ctx.device):
-                grad = _C.grpo_ratio_kl_loss_bwd(memory, ctx.workspace, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
+        cur, old, ref, adv, mask = ctx.saved_tensors if ctx.has_mask else (*ctx.saved_tensors, None)
+        if not torch.is_grad_enabled() and _only_values(g_loss, g_policy, g_kl):
+            shape, gpu, workspace = ctx.forward
+            rows, numel, f32 = cur.contiguous(), shape.numel(), torch.float32
+            if (
+                rows.shape == shape and _in_memory_as(rows, f32, numel, gpu) and _in_memory_as(old, f32, numel, gpu)
+                and _in_memory_as(ref, f32, numel, gpu) and _in_memory_as(adv, f32, shape[0], gpu)
+                and (mask is None or _in_memory_as(mask, torch.uint8, numel, gpu))
+            ):  # fmt: skip
+                memory = (rows, old, ref, adv, mask)
+                grad = _C.grpo_ratio_kl_loss_bwd(memory, workspace, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
                 return grad, None, None, None, None, None, None
         # the gradient itself is to be differentiated (create_graph), or more than values came in
-        grad = _elementwise_gradient(*inputs, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
+        grad = _elementwise_gradient(cur, old, ref, adv, mask, g_loss, g_policy, g_kl, ctx.clip_eps, ctx.beta)
         return grad, None, None, None, None, None, None
 
 

@@ -102,6 +102,10 @@ def test_the_tangent_of_an_incoming_gradient(kernel_calls):
     torch.testing.assert_close(tangent, want, rtol=2.0**-22, atol=1e-9)
 
 
+class _Tagged(torch.Tensor):
+    pass
+
+
 def _hooks(pack, unpack):
     return torch.autograd.graph.saved_tensors_hooks(pack, unpack)
 
@@ -122,6 +126,8 @@ def test_saved_tensors_that_hooks_hand_back(kernel_calls):
 
     torch.testing.assert_close(gradient(lambda t: t, turned), want, rtol=2.0**-22, atol=1e-9)
     torch.testing.assert_close(gradient(lambda t: t, torch.Tensor.double), want, rtol=2.0**-19, atol=1e-9)
+    torch.testing.assert_close(gradient(lambda t: t, lambda t: t.as_subclass(_Tagged)), want, rtol=2.0**-22, atol=1e-9)
+    assert len(kernel_calls) == 1  # the gradient to compare with
 
     # values rounded to bf16: the gradient of the rounded values, over the tokens that are really there
     def rounded(t):
