@@ -319,7 +319,9 @@ static hipError_t launch_tile(const MatView& W, const MatView& X, void* C, int64
   // A weight that the forward has just left in the memory-side cache costs 3 to 9 % with the wave (dX of 6144 outputs, 4096
   // inputs at 333 tokens 33.3 -> 35.1 us, of 14336 outputs 71.9 -> 76.7), where it saves 10 to 20 % from HBM (42.6 -> 38.1,
   // 94.3 -> 79.8): it runs where the weight is too large to still be there, from 128 MiB, or from 96 MiB with many tokens,
-  // whose activations displace it (14336 outputs at 700 / 1000 tokens right behind the forward 117 / 132 -> 103 / 114).
+  // whose activations displace it. Right behind the forward / from HBM, in % of the time at 300 / 500 / 700 / 1000 tokens,
+  // 4096 inputs: 48 MiB of weight +6 / +2 / +2 / -2 and -14 / -13 / -23 / -17, 96 MiB +1 / -3 / -2 / +1 and -16 / -13 / -25 /
+  // -15, 112 MiB +3 / 0 / -8 / -14 and -19 / -15 / -25 / -16, 128 MiB -13 / -11 / -21 / -17 and -19 / -14 / -25 / -16.
   const bool shared_panel = tiles_m > 2 || M > S::BM + S::BM / 2;
   const int64_t weight_bytes = (int64_t)N * K * 2;
   const bool from_hbm = weight_bytes >= ((int64_t)128 << 20) || (weight_bytes >= ((int64_t)96 << 20) && M > 512);
@@ -596,7 +598,10 @@ static bool remainder_launch_pays(int M, int N, int K, int rest, bool fast_few_t
   const double round_us = 11.0 + 21.0 * K / 1024.0;
   double rest_us;
   if (w_kmajor) {
-    rest_us = 10.0 + 0.4 * (K / 64.0);  // register-staged small tiles: a chain of K tiles
+    // A chain of K tiles on the small tiles, an upper estimate: 0.27 to 0.41 us each at 1 to 64 tokens from HBM (4096
+    // inputs, K = 4096 / 12288 / 24576: 20 to 26, 53 to 71, 103 to 142 us), 0.2 from the cache. Either way it pays from two
+    // K tiles on.
+    rest_us = 10.0 + 0.4 * (K / 64.0);
   } else if (fast_few_tokens) {
     rest_us = 8.0 + 2.0 * N * (double)K / 4.5e6 * (rest <= 16 ? 1.0 : 1.5);  // the weight once at 4.5 TB/s
   } else {

@@ -1265,7 +1265,10 @@ __device__ __forceinline__ void tile_mainloop_solo_impl(const MatView& W, const 
 //
 // What bounds a small tile whose operands are in the L2 is LDS bandwidth: a wave reads its 16 TN weight and 16 TM token
 // rows of every K tile, so eight waves in a 4 x 2 layout read each weight row twice and each token row four times. Four
-// waves in a 2 x 2 layout read every row twice.
+// waves in a 2 x 2 layout read every row twice. (64 x 96, 4096 outputs, K = 12288, 333 tokens, weight in the memory-side
+// cache: 7760 fragment reads of 1 KiB per CU, which at 128 bytes a cycle are 58 % of its 107000 busy cycles, beside 3.9 MB
+// that arrive; no bank conflicts, the matrix pipe busy in 35 %. From HBM the reads are 44 % of 142000: there the arrivals
+// bound it.)
 //
 //   iteration t (fragments of stage t in registers, all of them read before the barrier)
 //     wait: my loads of stage t + 1 landed; barrier

@@ -54,11 +54,13 @@ inline double rounds_of_workgroups(int64_t tiles, int cus) {
 // memory-side cache for its next use once the other layers have passed through, and reads that leave nothing there are
 // faster: pure reads of 1.2 GB, 5.2 -> 5.9 TB/s in the kernels' pattern. Measured with weights from HBM: gate_up (201 MB) at
 // 1 / 32 / 64 / 128 tokens 37.1 / 45.6 / 46.8 / 52.2 -> 35.4 / 42.3 / 44.3 / 48.4 us, gated at 256 tokens 67.8 -> 62.9, down
-// (101 MB) at 1 token 20.1 -> 18.3, LogP (1.2 GB) at 16 tokens 258 -> 243. Below 96 MiB it gains nothing (qkv, 50 MB:
-// 12.3 / 11.9 at one token, equal at 16) and takes the cache from a weight that would have stayed (11.9 -> 13.3 us). Readers
-// that drift apart miss a line that the first of them has had: gate_up at 160 tokens (128 + 32) 60 -> 66 us, at 256
-// (128 + 128) 63 -> 60. Two readers of a weight between the two (12288 outputs, K = 4096, 256 tokens, three weights in turn:
-// 36.6 -> 38.6 us) are better served by what the cache still holds: they want 128 MiB.
+// (101 MB) at 1 token 20.1 -> 18.3, LogP (1.2 GB) at 16 tokens 258 -> 243. Readers that drift apart miss a line that the
+// first of them has had: gate_up at 160 tokens (128 + 32) 60 -> 66 us, at 256 (128 + 128) 63 -> 60.
+// Where the lines lie is what the cache still holds. From HBM one token tile gains at any size (K = 4096, 8192 ... 16384
+// outputs: 3 to 5 % at one token, 0 to 9 at 64, 0 to 5 at 128); three weights in turn lose where the cache would have held
+// all three and gain where it would not (1 / 16 / 64 / 128 tokens, in % of the time: 48 MiB 0 / +15 / +44 / +28, 64 MiB -1 /
+// +10 / +39 / +20, 80 MiB +1 / +12 / +20 / +37, 88 MiB 0 / +10 / +9 / +8, 96 MiB -4 / 0 / 0 / +3, 112 MiB -5 / -2 / -7 / -5,
+// 128 MiB -6 / -2 / -10 / -6). Two whole token tiles (256 tokens): +31 % at 80 MiB, +7 at 88, +3 at 96, -3 at 112, -4 at 128.
 inline bool streamed_weight(int64_t rows, int64_t k, int M, int bm) {
   const int64_t bytes = rows * k * 2;
   return (M <= bm && bytes >= ((int64_t)96 << 20)) || (M == 2 * bm && bytes >= ((int64_t)128 << 20));

@@ -54,6 +54,7 @@ def _saved_and_gradients(h, w, ids, g):
 
 
 def test_what_is_saved(monkeypatch):
+    """On the device, with its own answers about its memory."""
     h, w, ids, g = _inputs(module._SAVED_LOGITS_MIN_TOKENS, 1031, module._SAVED_LOGITS_MIN_HIDDEN)
     kept, grads = _saved_and_gradients(h, w, ids, g)
     assert kept == 1
@@ -69,9 +70,11 @@ def test_what_is_saved(monkeypatch):
             patch.setattr(module, name, value)
             count, want = _saved_and_gradients(h, w, ids, g)
             assert count == 0 and all(torch.equal(a, b) for a, b in zip(grads, want))
-    # little memory left: nothing is kept; an allocation that fails all the same is not an error either
+    # switched off, and with little memory left (tests/test_saved_logits_memory.py has the limits themselves)
+    with module.recompute_logits():
+        count, want = _saved_and_gradients(h, w, ids, g)
+    assert count == 0 and all(torch.equal(a, b) for a, b in zip(grads, want))
     monkeypatch.setattr(module, "_SAVED_LOGITS_UNCHECKED_BYTES", 0)
     monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (1 << 20, 1 << 20))
-    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda device: 0)
-    monkeypatch.setattr(torch.cuda, "memory_allocated", lambda device: 0)
-    assert module._logits_to_save(h, 1031) is None
+    count, want = _saved_and_gradients(h, w, ids, g)
+    assert count == 0 and all(torch.equal(a, b) for a, b in zip(grads, want))
