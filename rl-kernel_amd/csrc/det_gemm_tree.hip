@@ -25,11 +25,12 @@
 //     rounding as the fused multiply-add, at twice the vector rate; operands staged in LDS
 //     as fp32, [row][k].
 //
-// Two more kernels split K along the contract's own tree: the 16 nodes at depth 4 (8 at depth 3) are
+// Three more kernels split K along the contract's own tree: the nodes at depth 2, 3 or 4 are
 // independent, a wave evaluates one of them for a block of outputs, and the bf16 nodes are folded in tree
-// order: det_gemm_tree_nodes_kernel (fp32 matrix pipe, any row count; the fastest of all on K-contiguous aligned
-// operands with equal leaves, and what RLK_TREE_CFG_AUTO picks for them) and det_gemm_tree_skinny_kernel (up to
-// 16 rows, vector ALU; trees of 11 and 12 levels, which the former has no register slots for).
+// order: det_gemm_tree_rows_kernel and, for small grids, det_gemm_tree_nodes_kernel (fp32 matrix pipe, any row count; the
+// fastest of all on K-contiguous aligned operands with equal leaves, and what RLK_TREE_CFG_AUTO picks for them), and
+// det_gemm_tree_skinny_kernel (up to 16 rows, vector ALU; trees of 11 and 12 levels, which those have no register slots
+// for).
 //
 // Tiled kernels: a workgroup owns a 64 x 128 output tile. Leaves are visited left to right, the next leaf
 // is fetched while the current one is summed. The tree is evaluated on the
@@ -707,72 +708,64 @@ __global__ __launch_bounds__(64 * kTreeSkinnyWaves) void det_gemm_tree_skinny_ke
   }
 }
 
-// The same split for more rows, on the matrix pipe: a workgroup of 8 waves takes 16 rows, wave w evaluates
-// node w at depth 3 with one v_mfma_f32_16x16x1_4b_f32 per k, and wave 0 folds the 8 bf16 nodes in tree order.
-// Many more workgroups than the tiled kernel has tiles: for row counts whose tiles do not fill the chip. Two
-// workgroups fit a CU (LDS, registers), so one computes while the other starts or folds. The four 16 x 16
-// blocks of the instruction are
-//   KB = 1: four groups of 16 columns (64 columns per workgroup), the row operand of block 0 broadcast;
-//   KB = 4: the four grandchildren (depth 5) of the wave's node for one group of 16 columns, every block
-//           with its own k range; the lane then folds its four blocks in tree order. Four times the
-//           workgroups and a quarter of the leaves per lane: for narrow N, where 64-column workgroups
-//           would leave most CUs idle and a lane's chain of leaves (one memory round trip each) decides.
-// CHUNKS = leaf length / 8.
+// The same split on the matrix pipe for grids that would leave half of the CUs idle: a workgroup of 8 waves takes 16 rows
+// and 16 columns, wave w evaluates node w at depth 3 with one v_mfma_f32_16x16x1_4b_f32 per k, whose four 16 x 16 blocks are
+// the four grandchildren (depth 5) of the wave's node, every block with its own k range; the lane then folds its four blocks
+// in tree order, and wave 0 the 8 bf16 nodes. A quarter of the leaves per lane and four times the workgroups of the kernel
+// behind this one: a lane's chain of leaves (one memory round trip each) decides there. Two workgroups fit a CU (LDS,
+// registers), so one computes while the other starts or folds. CHUNKS = leaf length / 8.
 // Operand path: a lane's operand is 16 bytes per 8 k of ITS column, so loads into registers would touch 64
 // different lines per instruction and the address pipe, not memory or the matrix pipe, would set the pace. A
-// wave therefore brings its leaf in through LDS: direct-to-LDS loads whose lanes walk the 16-byte granules
+// wave therefore brings its leaf of the weight in through LDS: direct-to-LDS loads whose lanes walk the 16-byte granules
 // (column, chunk) in order - 4 / CHUNKS columns' worth of contiguous bytes per line touched - into a region of
 // LDS that belongs to the wave alone (two leaves: one landing while the other is read), then every lane reads
-// its own column back with ds_read_b128. No barrier: the wave waits for its own loads. The rows of A go the
-// same way for KB = 1 (16 rows of one k range: one load instruction per leaf); for KB = 4 the four blocks
-// need four k ranges of A, which would not fit beside the weight, and those stay register loads.
+// its own column back with ds_read_b128. No barrier: the wave waits for its own loads. The four blocks need four k ranges
+// of A, which would not fit beside the weight, and those are register loads.
 // Every load is issued unconditionally (past the node's end it repeats the last leaf), so that the waits
 // count loads along one straight path.
 // Workgroup ids are dealt so that the row groups of one column group run on the same XCD at the same time and
 // share that L2's copy of the weight.
 constexpr int kTreeNodeSplit = 3;                     // depth of the nodes the waves take
 constexpr int kTreeNodeWaves = 1 << kTreeNodeSplit;   // 8: two workgroups per CU, one starts while the other folds
-constexpr int kTreeNodeLevels = 7;                    // tree levels below a node, KB = 1 (K <= 32768)
+constexpr int kTreeNodeMaxDepth = 10;                 // K <= 32768: register slots
+constexpr int kTreeNodeCols = 16;
 
-template <int KB, int CHUNKS>
+template <int CHUNKS>
 struct TreeNodesLds {
-  static constexpr int kABytes = KB == 1 ? 1024 : 0;  // a leaf of the 16 rows: one load instruction whatever CHUNKS
-  static constexpr int kWBytes = 1024 * CHUNKS;       // a leaf of the wave's 64 (column, k range) pairs, behind the rows
-  static constexpr int kLeafBytes = kABytes + kWBytes;
+  static constexpr int kLeafBytes = 1024 * CHUNKS;  // a leaf of the wave's 64 (column, k range) pairs
   static constexpr int kWaveBytes = 2 * kLeafBytes;
-  static constexpr int kNodesBytes = kTreeNodeWaves * (KB == 4 ? 2 : 8) * 64 * 4;
-  static constexpr int kStageBytes = kTreeNodeWaves * kWaveBytes;
-  static constexpr int kBytes = kStageBytes > kNodesBytes ? kStageBytes : kNodesBytes;
+  static constexpr int kBytes = kTreeNodeWaves * kWaveBytes;
+  static_assert(kBytes >= kTreeNodeWaves * 2 * 64 * 4, "the fold's table takes the place of the staging regions");
 };
 
 // On this chip a vector-ALU instruction is not hidden behind the fp32 matrix instructions of the other waves of
-// its SIMD: each one adds about three cycles to the 32 of a 16x16x1 step. The leaf loop is therefore written
+// its SIMD: each one adds about four cycles to the 33 of a 16x16x1 step (three to four in a probe, four by the kernels'
+// instruction counts and times). The leaf loop is therefore written
 // for few of them: two per step to widen the bf16 operands, addresses as a scalar base plus a lane offset that
 // never changes, LDS reads at immediate offsets (the loop handles an even and an odd leaf per turn, so the
 // staging region of each is known at compile time), and the tree bookkeeping once per pair of leaves.
-template <int KB, int CHUNKS>
+template <int CHUNKS>
 __global__ __launch_bounds__(64 * kTreeNodeWaves, 4) void det_gemm_tree_nodes_kernel(
     MatView A, MatView B, bf16_bits* __restrict__ C, int64_t ldc, int M, int N, int K, int depth, int row_groups) {
-  using L = TreeNodesLds<KB, CHUNKS>;
-  constexpr int kLevels = KB == 4 ? kTreeNodeLevels - 2 : kTreeNodeLevels;
-  constexpr int kKeep = KB == 4 ? 2 : 8;  // packed registers a wave hands to the fold
-  constexpr int kAAhead = 2;              // KB = 4: leaves of A in flight in registers
-  constexpr int kLoadsPerLeaf = CHUNKS + (KB == 1 ? 1 : CHUNKS);
+  using L = TreeNodesLds<CHUNKS>;
+  constexpr int kSlots = kTreeNodeMaxDepth - kTreeNodeSplit - 2 - 1;  // levels below a block's node but the lowest
+  constexpr int kKeep = 2;   // packed registers a wave hands to the fold
+  constexpr int kAAhead = 2;  // leaves of A in flight in registers
+  constexpr int kLoadsPerLeaf = 2 * CHUNKS;
   extern __shared__ __attribute__((aligned(16))) char tree_lds[];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int id = xcd_compact_id(blockIdx.x, gridDim.x);
-  const int n0 = (id / row_groups) * (KB == 4 ? 16 : 64), m0 = (id % row_groups) * 16;
+  const int n0 = (id / row_groups) * kTreeNodeCols, m0 = (id % row_groups) * 16;
   constexpr int len = 8 * CHUNKS;  // leaf length
-  const int node_depth = kTreeNodeSplit + (KB == 4 ? 2 : 0);
-  const int leaves = 1 << (depth - node_depth);  // leaves under one block's node: a power of two, at least 2
-  // The k range of block b of this wave starts at (KB * wave + b) * leaves * len; block_k = leaves * len.
+  const int leaves = 1 << (depth - kTreeNodeSplit - 2);  // leaves under one block's node: a power of two, at least 2
+  // The k range of block b of this wave starts at (4 * wave + b) * leaves * len; block_k = leaves * len.
   const int block_k = leaves * len;
-  const int wave_k = (KB == 4 ? 4 * wave : wave) * block_k;  // uniform
+  const int wave_k = 4 * wave * block_k;  // uniform
 
-  // Granule g = 64 j + lane of a leaf: pair g / CHUNKS (KB = 1: column; KB = 4: column % 16 and block), position
-  // g % CHUNKS, which holds chunk position ^ swizzle(pair): the lanes of a ds_read_b128 then spread over the banks.
+  // Granule g = 64 j + lane of a leaf: pair g / CHUNKS (column % 16 and block), position g % CHUNKS, which holds chunk
+  // position ^ swizzle(pair): the lanes of a ds_read_b128 then spread over the banks.
   // Addresses are a uniform base (the workgroup's first column or row, the wave's k range, the leaf) plus a lane
   // offset in bytes that fits 32 bits (the launcher checks the strides).
   static_assert(CHUNKS == 3 || CHUNKS == 4, "leaves of 24 or 32");
@@ -783,28 +776,19 @@ __global__ __launch_bounds__(64 * kTreeNodeWaves, 4) void det_gemm_tree_nodes_ke
 #pragma unroll
   for (int j = 0; j < CHUNKS; ++j) {
     const int g = 64 * j + lane, pair = g / CHUNKS, chunk = (g % CHUNKS) ^ swizzle(pair);
-    const int col = KB == 4 ? (pair & 15) : pair;
+    const int col = pair & 15;
     const int col_in = n0 + col < N ? col : N - 1 - n0;
-    w_off[j] = 2u * (uint32_t)(col_in * (int)B.row_stride + (KB == 4 ? (pair >> 4) * block_k : 0) + 8 * chunk);
+    w_off[j] = 2u * (uint32_t)(col_in * (int)B.row_stride + (pair >> 4) * block_k + 8 * chunk);
   }
-  uint32_t a_off;
-  if constexpr (KB == 1) {  // lanes past the 16 rows repeat the last granule; their 16 bytes land in the spare of the region
-    const int g = lane < 16 * CHUNKS ? lane : 16 * CHUNKS - 1, row = g / CHUNKS;
-    const int row_in = m0 + row < M ? row : M - 1 - m0;
-    a_off = 2u * (uint32_t)(row_in * (int)A.row_stride + 8 * ((g % CHUNKS) ^ swizzle(row)));
-  } else {
-    const int row = lane & 15;
-    const int row_in = m0 + row < M ? row : M - 1 - m0;
-    a_off = 2u * (uint32_t)(row_in * (int)A.row_stride + (lane >> 4) * block_k);
-  }
+  const int row = lane & 15;
+  const int row_in = m0 + row < M ? row : M - 1 - m0;
+  const uint32_t a_off = 2u * (uint32_t)(row_in * (int)A.row_stride + (lane >> 4) * block_k);
   char* const mine = tree_lds + wave * L::kWaveBytes;
-  // Lane l reads chunk c of its pair l at read_at[c] (+ kABytes for the weight): rows and columns use the same
-  // lane offsets, lanes 16 .. 63 read rows that do not exist (inside the region; the instruction broadcasts block 0).
-  const char* read_at[CHUNKS];
+  const char* read_at[CHUNKS];  // lane l reads chunk c of its pair l
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) read_at[c] = mine + lane * (16 * CHUNKS) + 16 * (c ^ swizzle(lane));
 
-  u32x4_t wq[CHUNKS], aq[KB == 1 ? 1 : kAAhead + 1][CHUNKS];
+  u32x4_t wq[CHUNKS], aq[kAAhead + 1][CHUNKS];
   // leaf: which leaf of the node (past the end: the last one again); stage: 0 or 1
   auto issue = [&](int leaf, int stage_index, u32x4_t (&a)[CHUNKS]) __attribute__((always_inline)) {
     const int lo = (leaf < leaves ? leaf : leaves - 1) * (2 * len);  // uniform, bytes
@@ -819,30 +803,23 @@ __global__ __launch_bounds__(64 * kTreeNodeWaves, 4) void det_gemm_tree_nodes_ke
     for (int j = 0; j < CHUNKS; ++j) {
       uint32_t off = w_off[j];
       asm volatile("" : "+v"(off));  // widened here, next to the scalar base, not once outside the loop
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(w_leaf + off), (lds_ptr_t)(stage + L::kABytes + 1024 * j), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(w_leaf + off), (lds_ptr_t)(stage + 1024 * j), 16, 0, 0);
     }
     uint32_t off = a_off;
     asm volatile("" : "+v"(off));
-    if constexpr (KB == 1) {
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(a_leaf + off), (lds_ptr_t)stage, 16, 0, 0);
-    } else {
 #pragma unroll
-      for (int c = 0; c < CHUNKS; ++c) a[c] = *reinterpret_cast<const u32x4_t*>(a_leaf + off + 16 * c);
-    }
+    for (int c = 0; c < CHUNKS; ++c) a[c] = *reinterpret_cast<const u32x4_t*>(a_leaf + off + 16 * c);
   };
   auto take = [&](int stage_index) __attribute__((always_inline)) {  // the landed leaf out of LDS into registers
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) {
-      wq[c] = *reinterpret_cast<const u32x4_t*>(read_at[c] + stage_index * L::kLeafBytes + L::kABytes);
-      if constexpr (KB == 1) aq[0][c] = *reinterpret_cast<const u32x4_t*>(read_at[c] + stage_index * L::kLeafBytes);
-    }
+    for (int c = 0; c < CHUNKS; ++c) wq[c] = *reinterpret_cast<const u32x4_t*>(read_at[c] + stage_index * L::kLeafBytes);
   };
   // Leaf i (stage i & 1, a compile-time constant at every call): start the load of leaf i + 2 into the region leaf i
   // came from, sum the leaf, round it to bf16, and bring leaf i + 1 into registers.
   auto leaf_sum = [&](int i, int stage_index, uint32_t (&node)[8]) __attribute__((always_inline)) {
     __builtin_amdgcn_s_waitcnt(kWaitLgkm0);  // leaf i is in registers: its region is free
     asm volatile("" ::: "memory");
-    issue(i + 2, stage_index, aq[KB == 1 ? 0 : kAAhead]);
+    issue(i + 2, stage_index, aq[kAAhead]);
     f32x16_t acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
@@ -853,11 +830,7 @@ __global__ __launch_bounds__(64 * kTreeNodeWaves, 4) void det_gemm_tree_nodes_ke
         const uint32_t wb = wq[c][e >> 1], ab = aq[0][c][e >> 1];
         const float b = __uint_as_float((e & 1) ? (wb & 0xffff0000u) : (wb << 16));
         const float a = __uint_as_float((e & 1) ? (ab & 0xffff0000u) : (ab << 16));
-        if constexpr (KB == 4) {
-          acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, acc, 0, 0, 0);
-        } else {
-          acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, acc, 2, 0, 0);
-        }
+        acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, acc, 0, 0, 0);
       }
     }
 #pragma unroll
@@ -865,18 +838,16 @@ __global__ __launch_bounds__(64 * kTreeNodeWaves, 4) void det_gemm_tree_nodes_ke
     __builtin_amdgcn_s_waitcnt(wait_vmcnt(kLoadsPerLeaf));  // leaf i + 1 has landed (leaf i + 2 may be on its way)
     asm volatile("" ::: "memory");
     take(stage_index ^ 1);
-    if constexpr (KB == 4) {
 #pragma unroll
-      for (int p = 0; p < kAAhead; ++p)
+    for (int p = 0; p < kAAhead; ++p)
 #pragma unroll
-        for (int c = 0; c < CHUNKS; ++c) aq[p][c] = aq[p + 1][c];
-    }
+      for (int c = 0; c < CHUNKS; ++c) aq[p][c] = aq[p + 1][c];
   };
 
-  uint32_t slot[kLevels - 1][8];  // slot[l]: a finished left child l + 1 levels above the leaves
+  uint32_t slot[kSlots][8];  // slot[l]: a finished left child l + 1 levels above the leaves
   uint32_t left[8], cur[8];
   issue(0, 0, aq[0]);
-  issue(1, 1, aq[KB == 1 ? 0 : 1]);
+  issue(1, 1, aq[1]);
   __builtin_amdgcn_s_waitcnt(wait_vmcnt(kLoadsPerLeaf));  // leaf 0 has landed
   asm volatile("" ::: "memory");
   take(0);
@@ -889,7 +860,7 @@ __global__ __launch_bounds__(64 * kTreeNodeWaves, 4) void det_gemm_tree_nodes_ke
     int level = 0;
     for (int j = i >> 1; j & 1; j >>= 1, ++level) {
 #pragma unroll
-      for (int l = 0; l < kLevels - 1; ++l) {
+      for (int l = 0; l < kSlots; ++l) {
         if (l == level) {
 #pragma unroll
           for (int r = 0; r < 8; ++r) cur[r] = bf16x2_add(slot[l][r], cur[r]);
@@ -898,7 +869,7 @@ __global__ __launch_bounds__(64 * kTreeNodeWaves, 4) void det_gemm_tree_nodes_ke
     }
     if (i + 2 < leaves) {
 #pragma unroll
-      for (int l = 0; l < kLevels - 1; ++l) {
+      for (int l = 0; l < kSlots; ++l) {
         if (l == level) {
 #pragma unroll
           for (int r = 0; r < 8; ++r) slot[l][r] = cur[r];
@@ -912,18 +883,13 @@ __global__ __launch_bounds__(64 * kTreeNodeWaves, 4) void det_gemm_tree_nodes_ke
   uint32_t(*nodes)[kKeep][64] = reinterpret_cast<uint32_t(*)[kKeep][64]>(tree_lds);
   // Accumulator r: block r / 4; row 4 (lane / 16) + r % 4, column lane % 16 of the block.
   // cur[q] packs accumulators 2 q, 2 q + 1 (two consecutive rows of one column), block q / 2.
-  if constexpr (KB == 4) {
-    // blocks 0..3 are the node's grandchildren left to right: (0 + 1) + (2 + 3)
+  // Blocks 0..3 are the node's grandchildren left to right: (0 + 1) + (2 + 3).
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      nodes[wave][h][lane] = bf16x2_add(bf16x2_add(cur[h], cur[2 + h]), bf16x2_add(cur[4 + h], cur[6 + h]));
-  } else {
-#pragma unroll
-    for (int r = 0; r < 8; ++r) nodes[wave][r][lane] = cur[r];
-  }
+  for (int h = 0; h < 2; ++h)
+    nodes[wave][h][lane] = bf16x2_add(bf16x2_add(cur[h], cur[2 + h]), bf16x2_add(cur[4 + h], cur[6 + h]));
   __syncthreads();
   if (wave != 0) return;
-  const int out_col = n0 + (lane & 15);
+  const int c = n0 + (lane & 15);
   const int out_row = m0 + 4 * (lane >> 4);
 #pragma unroll
   for (int q = 0; q < kKeep; ++q) {
@@ -934,8 +900,7 @@ __global__ __launch_bounds__(64 * kTreeNodeWaves, 4) void det_gemm_tree_nodes_ke
     for (int width = kTreeNodeWaves / 2; width >= 1; width /= 2)
 #pragma unroll
       for (int w = 0; w < width; ++w) v[w] = bf16x2_add(v[2 * w], v[2 * w + 1]);
-    const int c = out_col + (KB == 4 ? 0 : 16 * (q >> 1));
-    const int r = out_row + 2 * (q & 1);
+    const int r = out_row + 2 * q;
     if (c < N) {
       if (r < M) C[(int64_t)r * ldc + c] = (bf16_bits)(v[0] & 0xffffu);
       if (r + 1 < M) C[(int64_t)(r + 1) * ldc + c] = (bf16_bits)(v[0] >> 16);
@@ -943,30 +908,291 @@ __global__ __launch_bounds__(64 * kTreeNodeWaves, 4) void det_gemm_tree_nodes_ke
   }
 }
 
-template <int KB, int CHUNKS>
+template <int CHUNKS>
 static hipError_t launch_nodes_leaf(const MatView& A, const MatView& B, bf16_bits* out, int64_t ldc, int M, int N, int K,
                                     int depth, hipStream_t stream) {
-  using L = TreeNodesLds<KB, CHUNKS>;
+  using L = TreeNodesLds<CHUNKS>;
   static PerDeviceOnce once;
-  auto kernel = det_gemm_tree_nodes_kernel<KB, CHUNKS>;
+  auto kernel = det_gemm_tree_nodes_kernel<CHUNKS>;
   hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), L::kBytes, once);
   if (err != hipSuccess) return err;
-  constexpr int kCols = KB == 4 ? 16 : 64;
   const int row_groups = (M + 15) / 16;
-  const int64_t groups = (int64_t)((N + kCols - 1) / kCols) * row_groups;
+  const int64_t groups = (int64_t)((N + kTreeNodeCols - 1) / kTreeNodeCols) * row_groups;
   if (groups > 0x7fffffff) return hipErrorInvalidValue;
   hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(64 * kTreeNodeWaves), L::kBytes, stream, A, B, out, ldc, M, N,
                      K, depth, row_groups);
   return hipGetLastError();
 }
 
-template <int KB>
 static hipError_t launch_nodes(const MatView& A, const MatView& B, bf16_bits* out, int64_t ldc, int M, int N, int K,
                                int depth, hipStream_t stream) {
   // equal leaves that are a multiple of 8 long are 24 or 32 long: a tree stops splitting at 32, so its leaves are
   // longer than 16
-  return (K >> depth) == 24 ? launch_nodes_leaf<KB, 3>(A, B, out, ldc, M, N, K, depth, stream)
-                            : launch_nodes_leaf<KB, 4>(A, B, out, ldc, M, N, K, depth, stream);
+  return (K >> depth) == 24 ? launch_nodes_leaf<3>(A, B, out, ldc, M, N, K, depth, stream)
+                            : launch_nodes_leaf<4>(A, B, out, ldc, M, N, K, depth, stream);
+}
+
+// Few vector instructions: what bounds a kernel of fp32 matrix instructions here (the note at the kernel above: each
+// vector instruction adds its four cycles to the 33 of a matrix instruction). R row groups of 16 per wave, 64 columns;
+// a workgroup of 8 / 4 waves takes the nodes at depth 3 / 2 for R = 1 / 2. Per matrix instruction, R = 1 / 2:
+//   * 1.25 / 0.75 conversions of operands (2 in the form above). The rows of A fill 16 R lanes, the lanes beside them hold
+//     the rows at later k: one widened register feeds 4 / R k steps, as the instruction broadcasts one of its 16-lane
+//     blocks (ABID) to all four column groups. The widened weight feeds R instructions.
+//   * 1.5 for the tree (2.25): a node is rounded in place, as the upper half of v_cvt_pk_bf16_f32(0, x), so a tree add is
+//     an add and a rounding instead of four unpackings, two adds and a packing per two outputs. The two lowest levels stay
+//     in that form (fp32 registers that hold bf16 values), the levels above, met once in eight leaves, are packed.
+// 4 / 2 waves per SIMD (128 / 256 registers). SLOTS: packed levels. Operands reach the lanes as above: a wave's own region
+// of LDS, two leaves, no barrier.
+template <int R>
+constexpr int tree_rows_split() {  // depth of the nodes the waves take
+  return R == 1 ? 3 : 2;
+}
+template <int R, int CHUNKS>
+struct TreeRowsLds {
+  static constexpr int kWaves = 1 << tree_rows_split<R>();
+  static constexpr int kABytes = 1024 * R;  // a leaf of the rows: R load instructions whatever CHUNKS
+  static constexpr int kLeafBytes = kABytes + 1024 * CHUNKS;
+  static constexpr int kWaveBytes = 2 * kLeafBytes;
+  static constexpr int kBytes = kWaves * kWaveBytes;
+  static_assert(kBytes >= kWaves * 8 * R * 64 * 4, "the fold's table takes the place of the staging regions");
+};
+
+// bf16(x), as the fp32 value: the upper half of one conversion of two values. `zero` is 0.f that the compiler cannot see
+// through (of a literal it makes a conversion of x alone and a byte permutation behind it).
+__device__ __forceinline__ float round_bf16(float zero, float x) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+  return __builtin_bit_cast(float, __builtin_convertvector((f32x2_t{zero, x}), bf16x2_t));
+}
+
+template <int R, int CHUNKS, int SLOTS>
+__global__ __launch_bounds__(64 << tree_rows_split<R>(), (R == 1 ? 4 : 2)) void det_gemm_tree_rows_kernel(
+    MatView A, MatView B, bf16_bits* __restrict__ C, int64_t ldc, int M, int N, int K, int depth, int row_groups) {
+  using L = TreeRowsLds<R, CHUNKS>;
+  static_assert(CHUNKS == 3 || CHUNKS == 4, "leaves of 24 or 32");
+  constexpr int kRows = 16 * R;
+  constexpr int kSets = 4 / R;                              // k steps that a widened register of A serves
+  constexpr int kAReads = (CHUNKS + kSets - 1) / kSets;     // of 16 bytes, per lane and leaf
+  constexpr int kLoadsPerLeaf = CHUNKS + R;
+  constexpr int len = 8 * CHUNKS;  // leaf length
+  extern __shared__ __attribute__((aligned(16))) char tree_lds[];
+
+  float zero = 0.f;
+  asm volatile("" : "+s"(zero));
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int id = xcd_compact_id(blockIdx.x, gridDim.x);
+  const int n0 = (id / row_groups) * 64, m0 = (id % row_groups) * kRows;
+  const int leaves = 1 << (depth - tree_rows_split<R>());  // of a wave's node: a power of two, at least 4
+  const int wave_k = wave * leaves * len;
+
+  // Granules, swizzle and addresses as in the kernel above.
+  auto swizzle = [](int pair) { return CHUNKS == 4 ? (pair >> 2) & 3 : 0; };
+  const char* const w_base = reinterpret_cast<const char*>(B.ptr + (int64_t)n0 * B.row_stride + wave_k);
+  const char* const a_base = reinterpret_cast<const char*>(A.ptr + (int64_t)m0 * A.row_stride + wave_k);
+  uint32_t w_off[CHUNKS], a_off[R];
+#pragma unroll
+  for (int j = 0; j < CHUNKS; ++j) {
+    const int g = 64 * j + lane, col = g / CHUNKS;
+    const int col_in = n0 + col < N ? col : N - 1 - n0;
+    w_off[j] = 2u * (uint32_t)(col_in * (int)B.row_stride + 8 * ((g % CHUNKS) ^ swizzle(col)));
+  }
+#pragma unroll
+  for (int j = 0; j < R; ++j) {  // lanes past the rows repeat the last granule, into the spare of the region
+    const int g = 64 * j + lane < kRows * CHUNKS ? 64 * j + lane : kRows * CHUNKS - 1, row = g / CHUNKS;
+    const int row_in = m0 + row < M ? row : M - 1 - m0;
+    a_off[j] = 2u * (uint32_t)(row_in * (int)A.row_stride + 8 * ((g % CHUNKS) ^ swizzle(row)));
+  }
+  char* const mine = tree_lds + wave * L::kWaveBytes;
+  // Lane l reads column l, and row l % kRows: chunk kSets i + l / kRows of it in read i (past the leaf: its last chunk,
+  // not used).
+  const char *w_at[CHUNKS], *a_at[kAReads];
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) w_at[c] = mine + L::kABytes + lane * (16 * CHUNKS) + 16 * (c ^ swizzle(lane));
+#pragma unroll
+  for (int i = 0; i < kAReads; ++i) {
+    const int row = lane % kRows;
+    const int chunk = kSets * i + lane / kRows < CHUNKS ? kSets * i + lane / kRows : CHUNKS - 1;
+    a_at[i] = mine + row * (16 * CHUNKS) + 16 * (chunk ^ swizzle(row));
+  }
+
+  // leaf: which leaf of the node (past the end: the last one again); stage: 0 or 1
+  auto issue = [&](int leaf, int stage_index) __attribute__((always_inline)) {
+    const int lo = (leaf < leaves ? leaf : leaves - 1) * (2 * len);  // uniform, bytes
+    char* const stage = mine + stage_index * L::kLeafBytes;
+    // the leaf's bases stay in scalar registers (the empty statements keep the compiler from folding the leaf
+    // into the lane offsets, which would cost a 64-bit vector add per load)
+    const char* w_leaf = w_base + lo;
+    const char* a_leaf = a_base + lo;
+    asm volatile("" : "+s"(w_leaf));
+    asm volatile("" : "+s"(a_leaf));
+#pragma unroll
+    for (int j = 0; j < CHUNKS; ++j) {
+      uint32_t off = w_off[j];
+      asm volatile("" : "+v"(off));  // widened here, next to the scalar base, not once outside the loop
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(w_leaf + off), (lds_ptr_t)(stage + L::kABytes + 1024 * j), 16, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      uint32_t off = a_off[j];
+      asm volatile("" : "+v"(off));
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(a_leaf + off), (lds_ptr_t)(stage + 1024 * j), 16, 0, 0);
+    }
+  };
+  u32x4_t wq[CHUNKS], aq[kAReads];
+  auto take = [&](int stage_index) __attribute__((always_inline)) {  // the landed leaf out of LDS into registers
+#pragma unroll
+    for (int i = 0; i < kAReads; ++i) aq[i] = *reinterpret_cast<const u32x4_t*>(a_at[i] + stage_index * L::kLeafBytes);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) wq[c] = *reinterpret_cast<const u32x4_t*>(w_at[c] + stage_index * L::kLeafBytes);
+  };
+  auto widen = [](const u32x4_t& v, int e) __attribute__((always_inline)) {
+    return __uint_as_float((e & 1) ? (v[e >> 1] & 0xffff0000u) : (v[e >> 1] << 16));
+  };
+  // Leaf i (stage i & 1, a compile-time constant at every call): start the load of leaf i + 2 into the region leaf i
+  // came from, sum the leaf, and bring leaf i + 1 into registers. node: the leaf's sum, rounded.
+  auto leaf_sum = [&](int i, int stage_index, float (&node)[16 * R]) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(kWaitLgkm0);  // leaf i is in registers: its region is free
+    asm volatile("" ::: "memory");
+    issue(i + 2, stage_index);
+    f32x16_t acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = f32x16_t{};
+#pragma unroll
+    for (int i2 = 0; i2 < kAReads; ++i2) {
+      float a[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a[e] = widen(aq[i2], e);
+#pragma unroll
+      for (int set = 0; set < kSets; ++set) {
+        const int c = kSets * i2 + set;
+        if (c >= CHUNKS) continue;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float b = widen(wq[c], e);
+          // the broadcast block is an immediate: block set * R + r holds row group r of this k
+          if constexpr (R == 1) {
+            if (set == 0) acc[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[e], b, acc[0], 2, 0, 0);
+            if (set == 1) acc[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[e], b, acc[0], 2, 1, 0);
+            if (set == 2) acc[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[e], b, acc[0], 2, 2, 0);
+            if (set == 3) acc[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[e], b, acc[0], 2, 3, 0);
+          } else {
+            if (set == 0) {
+              acc[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[e], b, acc[0], 2, 0, 0);
+              acc[1] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[e], b, acc[1], 2, 1, 0);
+            } else {
+              acc[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[e], b, acc[0], 2, 2, 0);
+              acc[1] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[e], b, acc[1], 2, 3, 0);
+            }
+          }
+        }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt(wait_vmcnt(kLoadsPerLeaf));  // leaf i + 1 has landed (leaf i + 2 may be on its way)
+    asm volatile("" ::: "memory");
+    take(stage_index ^ 1);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) node[16 * r + q] = round_bf16(zero, acc[r][q]);
+  };
+
+  uint32_t slot[SLOTS][8 * R];  // slot[l]: a finished left child l + 2 levels above the leaves, two registers packed
+  float left[16 * R], low[16 * R], cur[16 * R];
+  issue(0, 0);
+  issue(1, 1);
+  __builtin_amdgcn_s_waitcnt(wait_vmcnt(kLoadsPerLeaf));  // leaf 0 has landed
+  asm volatile("" ::: "memory");
+  take(0);
+  for (int i = 0; i < leaves; i += 4) {
+    leaf_sum(i, 0, left);
+    leaf_sum(i + 1, 1, cur);
+#pragma unroll
+    for (int q = 0; q < 16 * R; ++q) left[q] = round_bf16(zero, left[q] + cur[q]);
+    leaf_sum(i + 2, 0, low);
+    leaf_sum(i + 3, 1, cur);
+#pragma unroll
+    for (int q = 0; q < 16 * R; ++q) cur[q] = left[q] + round_bf16(zero, low[q] + cur[q]);
+    // Four leaves close one node per trailing one bit of i / 4; then it waits at the level of its lowest zero bit.
+    int level = 0;
+    for (int j = i >> 2; j & 1; j >>= 1, ++level) {
+#pragma unroll
+      for (int l = 0; l < SLOTS; ++l) {
+        if (l == level) {
+#pragma unroll
+          for (int q = 0; q < 8 * R; ++q) {
+            cur[2 * q] = __uint_as_float(slot[l][q] << 16) + round_bf16(zero, cur[2 * q]);
+            cur[2 * q + 1] = __uint_as_float(slot[l][q] & 0xffff0000u) + round_bf16(zero, cur[2 * q + 1]);
+          }
+        }
+      }
+    }
+    if (i + 4 < leaves) {
+#pragma unroll
+      for (int l = 0; l < SLOTS; ++l) {
+        if (l == level) {
+#pragma unroll
+          for (int q = 0; q < 8 * R; ++q) slot[l][q] = pack_bf16x2(cur[2 * q], cur[2 * q + 1]);
+        }
+      }
+    }
+  }
+  // The fold's table takes the place of the staging regions: every wave's loads must have landed first.
+  __builtin_amdgcn_s_waitcnt(kWaitAll0);
+  __syncthreads();
+  uint32_t(*nodes)[8 * R][64] = reinterpret_cast<uint32_t(*)[8 * R][64]>(tree_lds);
+#pragma unroll
+  for (int q = 0; q < 8 * R; ++q) nodes[wave][q][lane] = pack_bf16x2(cur[2 * q], cur[2 * q + 1]);
+  __syncthreads();
+  // Register x of a row group's accumulator: block x / 4; row 4 (lane / 16) + x % 4, column lane % 16 of the block.
+  // nodes[.][q] packs registers 2 q and 2 q + 1; every wave folds and stores its share of the 8 R.
+  const int out_col = n0 + (lane & 15);
+  constexpr int kShare = 8 * R / L::kWaves;
+#pragma unroll
+  for (int t = 0; t < kShare; ++t) {
+    const int q = kShare * wave + t;  // row group q / 8, block (q % 8) / 2
+    uint32_t v[L::kWaves];
+#pragma unroll
+    for (int w = 0; w < L::kWaves; ++w) v[w] = nodes[w][q][lane];
+#pragma unroll
+    for (int width = L::kWaves / 2; width >= 1; width /= 2)
+#pragma unroll
+      for (int w = 0; w < width; ++w) v[w] = bf16x2_add(v[2 * w], v[2 * w + 1]);
+    const int c = out_col + 16 * ((q & 7) >> 1);
+    const int r = m0 + 16 * (q >> 3) + 4 * (lane >> 4) + 2 * (q & 1);
+    if (c < N) {
+      if (r < M) C[(int64_t)r * ldc + c] = (bf16_bits)(v[0] & 0xffffu);
+      if (r + 1 < M) C[(int64_t)(r + 1) * ldc + c] = (bf16_bits)(v[0] >> 16);
+    }
+  }
+}
+
+template <int R, int CHUNKS, int SLOTS>
+static hipError_t launch_rows_kernel(const MatView& A, const MatView& B, bf16_bits* out, int64_t ldc, int M, int N, int K,
+                                     int depth, hipStream_t stream) {
+  using L = TreeRowsLds<R, CHUNKS>;
+  static PerDeviceOnce once;
+  auto kernel = det_gemm_tree_rows_kernel<R, CHUNKS, SLOTS>;
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), L::kBytes, once);
+  if (err != hipSuccess) return err;
+  const int row_groups = (M + 16 * R - 1) / (16 * R);
+  const int64_t groups = (int64_t)((N + 63) / 64) * row_groups;
+  if (groups > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(64 * L::kWaves), L::kBytes, stream, A, B, out, ldc, M, N, K,
+                     depth, row_groups);
+  return hipGetLastError();
+}
+
+// Trees of tree_rows_split<R>() + 2 to 10 levels. Packed levels: all below the nodes but the lowest two.
+template <int R>
+static hipError_t launch_rows(const MatView& A, const MatView& B, bf16_bits* out, int64_t ldc, int M, int N, int K,
+                              int depth, hipStream_t stream) {
+  constexpr int kFew = 7 - tree_rows_split<R>() - 2, kMany = 10 - tree_rows_split<R>() - 2;
+  if ((K >> depth) == 24)
+    return depth <= 7 ? launch_rows_kernel<R, 3, kFew>(A, B, out, ldc, M, N, K, depth, stream)
+                      : launch_rows_kernel<R, 3, kMany>(A, B, out, ldc, M, N, K, depth, stream);
+  return depth <= 7 ? launch_rows_kernel<R, 4, kFew>(A, B, out, ldc, M, N, K, depth, stream)
+                    : launch_rows_kernel<R, 4, kMany>(A, B, out, ldc, M, N, K, depth, stream);
 }
 
 int det_gemm_tree_max_k() { return kTreeLeaf << 20; }
@@ -1049,23 +1275,30 @@ hipError_t det_gemm_tree_launch(const MatView& A, const MatView& B, void* C, int
   const bool skinny_ok = M <= 16 && a_chunked && b_chunked && depth >= kTreeSkinnySplit &&
                          depth - kTreeSkinnySplit <= kTreeSkinnyLevels;
   if (config == RLK_TREE_CFG_SKINNY && !skinny_ok) return hipErrorInvalidValue;
-  // (at least two leaves under a wave's node; lane offsets of up to 64 rows and the reduction length in 32 bits)
-  const bool nodes_ok = a_chunked && b_chunked && depth > kTreeNodeSplit && depth - kTreeNodeSplit <= kTreeNodeLevels &&
+  // (lane offsets of up to 64 rows and the reduction length in 32 bits)
+  const bool nodes_ok = a_chunked && b_chunked && depth > 3 && depth <= kTreeNodeMaxDepth &&
                         ((K >> depth) == 24 || (K >> depth) == 32) && A.row_stride < (1 << 24) && B.row_stride < (1 << 24);
   if (config == RLK_TREE_CFG_NODES && !nodes_ok) return hipErrorInvalidValue;
-  // The node-per-wave kernel splits a node over the four blocks of its instruction where 64-column workgroups
-  // would not give every CU one; that needs two more tree levels above the leaves.
-  const int64_t wide_groups = (int64_t)((N + 63) / 64) * ((M + 15) / 16);
-  const bool split_blocks = nodes_ok && wide_groups < 256 && depth > kTreeNodeSplit + 2;
-  // The node-per-wave kernel wherever it is eligible. Measured on the Qwen3-8B projections it is ahead of the tiled
-  // kernel at every row count (gate_up: 58 against 279 us at 16 rows, 157 against 281 us at 64, 8.8 against 9.6 ms at
-  // 4096; down 4.7 against 6.2 ms at 4096): its waves never meet at a barrier inside a node and its operands need no
-  // conversion pass. Up to 8 rows it is ahead of the vector-ALU kernel below as well, with weights that come from HBM
-  // (gate_up at one token 59 against 84 us, the lm_head 287 against 403 us, down 33 against 75 us).
+  // The node-per-wave kernels wherever they are eligible. Measured on the Qwen3-8B projections they are ahead of the tiled
+  // kernel at every row count (gate_up: 55 against 279 us at 16 rows, 130 against 281 us at 64, 7.7 against 9.6 ms at
+  // 4096; down 4.2 against 6.2 ms at 4096): their waves never meet at a barrier inside a node and their operands need no
+  // conversion pass. Up to 8 rows they are ahead of the vector-ALU kernel below as well, with weights that come from HBM
+  // (gate_up at one token 57 against 84 us, the lm_head 287 against 403 us, down 33 against 75 us).
   if (config == RLK_TREE_CFG_AUTO && nodes_ok) config = RLK_TREE_CFG_NODES;
   if (config == RLK_TREE_CFG_NODES) {
-    return split_blocks ? launch_nodes<4>(A, B, out, ldc, M, N, K, depth, stream)
-                        : launch_nodes<1>(A, B, out, ldc, M, N, K, depth, stream);
+    // Which of them. Workgroups of 16 x 64 / 32 x 64 outputs that the busiest CU runs one after the other (pairs of them
+    // side by side), K = 4096: one 26 / 48 us, two 46 / 84, every further one 21 / 41. So 32 rows from two on where that
+    // is at least 4 % less than 16 rows (o_proj at 256 rows 88 / 85 us, qkv at 509 263 / 246, but qkv at 384, five against
+    // nine, 192 / 204). With up to a workgroup of 16 x 64 for every second CU the kernel that splits a node over the blocks
+    // of its instruction: o_proj at 32 rows 21 against 26 us, at 48 rows 29 against 26; it needs six levels, and the
+    // 16-row kernel five.
+    const int64_t cus = device_cu_count();
+    const int64_t groups16 = (int64_t)((N + 63) / 64) * ((M + 15) / 16), groups32 = (int64_t)((N + 63) / 64) * ((M + 31) / 32);
+    const int64_t turns16 = (groups16 + cus - 1) / cus, turns32 = (groups32 + cus - 1) / cus;
+    if (2 * groups16 <= cus && depth > kTreeNodeSplit + 2) return launch_nodes(A, B, out, ldc, M, N, K, depth, stream);
+    if (depth == 4 || (turns32 >= 2 && 48 * turns32 < 25 * turns16))
+      return launch_rows<2>(A, B, out, ldc, M, N, K, depth, stream);
+    return launch_rows<1>(A, B, out, ldc, M, N, K, depth, stream);
   }
   // Up to 16 rows of a tree the node kernel does not take (11 or 12 levels): the vector-ALU node kernel.
   if (skinny_ok && (config == RLK_TREE_CFG_SKINNY || config == RLK_TREE_CFG_AUTO)) {
