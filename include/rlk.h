@@ -101,6 +101,33 @@ int rlk_det_gemm_bf16(const void* a, int64_t a_row_stride, int64_t a_k_stride, c
                       int64_t b_k_stride, int64_t b_n_stride, void* c, int64_t ldc, int M, int N, int K,
                       int out_fp32, int config, void* stream);
 
+/* How rlk_linear_bwd_bf16 launches its two products. The choice never changes a result bit. */
+typedef enum rlk_linear_bwd_config {
+  RLK_LINEAR_BWD_CFG_AUTO = 0,
+  RLK_LINEAR_BWD_CFG_SEPARATE = 1,        /* one launch each */
+  RLK_LINEAR_BWD_CFG_256x256_256x256 = 2, /* one launch: tiles of 256 inputs x 256 tokens of dx, 256 x 256 of dw */
+  RLK_LINEAR_BWD_CFG_256x128_256x256 = 3,
+  RLK_LINEAR_BWD_CFG_256x256_256x128 = 4,
+  RLK_LINEAR_BWD_CFG_256x128_256x128 = 5,
+  RLK_LINEAR_BWD_CFG_128x128_256x256 = 6,
+  RLK_LINEAR_BWD_CFG_64x64_256x256 = 7,
+  RLK_LINEAR_BWD_CFG_COUNT = 8
+} rlk_linear_bwd_config;
+
+/*
+ * Both gradients of y = x @ w^T:
+ *   dx[tokens, inputs] = dy[tokens, outputs] @ w[outputs, inputs],   dw[outputs, inputs] = dy^T @ x[tokens, inputs]
+ * with the bits of two calls of rlk_det_gemm_bf16, in one launch where the second product's tiles can fill the compute
+ * units that the first leaves idle. bf16, contiguous columns, row strides in elements; no operand layout is refused, the
+ * one launch needs the K-major fast layout of rlk_det_gemm_bf16 for all three operands. dx and dw must not overlap each
+ * other or an operand.
+ *
+ * Stands in for the two GEMMs of the reference's MFMA linear backward (rl_engine/backends/rocm/gemm/mfma_gemm.py:404-458).
+ */
+int rlk_linear_bwd_bf16(const void* dy, int64_t dy_row_stride, const void* x, int64_t x_row_stride, const void* w,
+                        int64_t w_row_stride, void* dx, int64_t dx_row_stride, void* dw, int64_t dw_row_stride, int tokens,
+                        int inputs, int outputs, int config, void* stream);
+
 /*
  * C[M,N] = A[M,K] @ B[K,N] under the k-tree contract (rlk_det_gemm_tree_contract_id):
  *   T(lo,hi) = bf16(sum of a_k*b_k, k = lo..hi-1, fp32 from +0, k ascending, fused multiply-add)

@@ -1,0 +1,242 @@
+// The two products of a linear layer's backward in one launch:
+//   dX[M, K_in]     = dY[M, N_out] W[N_out, K_in]      (weight read K-major)
+//   dW[N_out, K_in] = dY^T X                           (both operands read K-major)
+// Neither waits for the other, and each has its own number of tiles, so launched one after the other each pays for a last
+// round of workgroups that leaves compute units idle. In one launch the workgroups of the second product take the compute
+// units that the first has no tile for. The tiles, loops and so the bits are those of det_gemm.hip.
+#include "det_gemm_body.h"
+#include "rlk_host.h"
+
+namespace rlk {
+
+struct PairProblem {
+  MatView W, X;
+  void* C;
+  int64_t ldc;
+  int M, N, K;
+  int tiles_m, tiles_n, group_m;
+};
+
+// Workgroups [0, first_blocks) own the tiles of the product that starts first, the others those of the second.
+// first_blocks is a whole multiple of the XCD count, so that both products keep their XCD-compact tile order; the
+// workgroups behind the first product's last tile have nothing to do.
+// (dX in small tiles keeps the stages of launch_small_kmajor, without its prefetching wave: a ninth wave has no registers
+// beside eight of the dW tile's.)
+template <class SX, int KSX, int NSX, class SW>
+__global__ __launch_bounds__(SX::kThreads) void det_gemm_pair_kernel(PairProblem dx, PairProblem dw, int first_blocks,
+                                                                     bool dx_first) {
+  static_assert(SX::kThreads == SW::kThreads, "one workgroup size");
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const bool second = (int)blockIdx.x >= first_blocks;
+  const int block = second ? (int)blockIdx.x - first_blocks : (int)blockIdx.x;
+  if (second != dx_first) {
+    if (block < dx.tiles_m * dx.tiles_n)
+      det_gemm_tile<SX, kLoopPingPongKMajor, false, KSX, NSX, false>(dx.W, dx.X, dx.C, dx.ldc, dx.M, dx.N, dx.K,
+                                                                     dx.tiles_m, dx.tiles_n, dx.group_m, block, lds);
+  } else {
+    if (block < dw.tiles_m * dw.tiles_n)
+      det_gemm_tile<SW, kLoopPingPongBothKMajor, false, 1, 2, false>(dw.W, dw.X, dw.C, dw.ldc, dw.M, dw.N, dw.K,
+                                                                     dw.tiles_m, dw.tiles_n, dw.group_m, block, lds);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Host side
+// ---------------------------------------------------------------------------
+
+using Pair256x256 = TileShape<256, 256, 4, 2>;
+using Pair256x128 = TileShape<256, 128, 4, 2>;
+using Pair128x128 = TileShape<128, 128, 4, 2>;
+using Pair64x64 = TileShape<64, 64, 4, 2>;
+
+// The tiles of a configuration, features x tokens for dX, inputs x outputs for dW, and their relative throughput on a full
+// chip (the K-major column of kTileCandidates; 128 x 128 falls behind it beside the dW tiles, 0.62 -> 0.53).
+struct PairTiles {
+  int dx_bn, dx_bm;
+  double dx_quality;
+  int dw_bn, dw_bm;
+  double dw_quality;
+};
+static const PairTiles kPairTiles[RLK_LINEAR_BWD_CFG_COUNT] = {
+    {}, {},  // automatic, two launches
+    {256, 256, 1.00, 256, 256, 1.00}, {256, 128, 0.70, 256, 256, 1.00}, {256, 256, 1.00, 256, 128, 0.70},
+    {256, 128, 0.70, 256, 128, 0.70}, {128, 128, 0.53, 256, 256, 1.00}, {64, 64, 0.25, 256, 256, 1.00},
+};
+
+template <class S>
+static PairProblem pair_problem(const GemmProblem& p) {
+  PairProblem r{p.W, p.X, p.C, p.ldc, p.M, p.N, p.K, (p.M + S::BM - 1) / S::BM, (p.N + S::BN - 1) / S::BN, 1};
+  r.group_m = r.tiles_m < 8 ? r.tiles_m : 8;
+  return r;
+}
+
+template <class SX, int KSX, int NSX, class SW>
+static hipError_t launch_pair(const GemmProblem& dx, const GemmProblem& dw, bool dx_first, hipStream_t stream) {
+  auto kernel = det_gemm_pair_kernel<SX, KSX, NSX, SW>;
+  constexpr int kLdsX = KSX * NSX * SX::kStageBytes, kLdsW = 2 * SW::kStageBytes;
+  constexpr int kLds = kLdsX > kLdsW ? kLdsX : kLdsW;
+  static PerDeviceOnce once;
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds, once);
+  if (err != hipSuccess) return err;
+  const PairProblem a = pair_problem<SX>(dx), b = pair_problem<SW>(dw);
+  const int tiles_dx = a.tiles_m * a.tiles_n, tiles_dw = b.tiles_m * b.tiles_n;
+  const int first = ((dx_first ? tiles_dx : tiles_dw) + kXcds - 1) / kXcds * kXcds;
+  const int second = dx_first ? tiles_dw : tiles_dx;
+  hipLaunchKernelGGL(kernel, dim3(first + second), dim3(SX::kThreads), kLds, stream, a, b, first, dx_first);
+  return hipGetLastError();
+}
+
+// When the last of the workgroups of two products ends, first product first, each compute unit taking the next tile when it
+// is free: n1 tiles of t1, then n2 of t2, on `cus` compute units.
+static double pair_span(int64_t n1, double t1, int64_t n2, double t2, int cus) {
+  const int64_t full = n1 / cus, late = n1 % cus;  // `late` compute units have one tile of the first product more
+  const double base = full * t1;
+  int64_t early_rounds = 0, late_rounds = 0, done = 0;
+  double span = late ? base + t1 : base;
+  while (done < n2) {  // the next round to start is the earlier of the two groups'
+    const double early_at = base + early_rounds * t2, late_at = base + t1 + late_rounds * t2;
+    const bool early = late == 0 || early_at <= late_at;
+    const int64_t group = early ? cus - late : late;
+    (early ? early_rounds : late_rounds) += 1;
+    done += group;
+    const double end = (early ? early_at : late_at) + t2;
+    if (end > span) span = end;
+  }
+  return span;
+}
+
+// The estimate of a launch, fitted to 282 shapes (64 to 8192 tokens, 21 layers and vocabularies, every configuration and
+// the two launches measured): the choice takes 0.6 % longer than the best configuration of each shape, 0.870 of the two
+// launches' time over all shapes, and is never more than 2 % slower than them.
+//
+// A tile on a full chip, us: 11 + 21 K / 1024 for 256 x 256 outputs (see remainder_launch_pays), other shapes by area and
+// quality; a tile of dW, whose reduction is short, starts faster.
+constexpr double kStartUs = 11.0, kStartDwUs = 9.0, kLaunchUs = 5.0;  // the last: a second launch
+static double tile_us(int bn, int bm, double quality, double start, int K) {
+  return (start + 21.0 * K / 1024.0) * bn * bm / 65536.0 / quality;
+}
+// dX reads its weight from HBM where the memory-side cache cannot still hold it from the forward. Its small tiles miss
+// their prefetching wave then (304 tokens, 24576 outputs: 255 us as two launches, 279 as one; 201 tokens, 14336 outputs, 112
+// MiB: 126 and 160).
+static bool weight_from_hbm(const GemmProblem& dx) { return (int64_t)dx.N * dx.K * 2 >= ((int64_t)112 << 20); }
+static double dx_tile_us(const PairTiles& t, const GemmProblem& dx) {
+  return tile_us(t.dx_bn, t.dx_bm, t.dx_quality, kStartUs, dx.K) * (t.dx_bn < 256 && weight_from_hbm(dx) ? 1.2 : 1.0);
+}
+static double dw_tile_us(const PairTiles& t, const GemmProblem& dw) {
+  return tile_us(t.dw_bn, t.dw_bm, t.dw_quality, kStartDwUs, dw.K);
+}
+
+static int64_t tile_count(const GemmProblem& p, int bn, int bm) { return (int64_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); }
+
+// The time of the one launch: the work of all tiles at the full chip's rate, or the span of tiles of which some run with
+// much of the chip idle. A tile takes 0.6 of its time alone (256 x 256, K = 4096: 95 -> 65 us, 256 x 128: 68 -> 48.5), the
+// whole of it on a full chip and wherever its weight comes at the HBM latency (256 x 256 at K = 37984 / 151936: 790 / 3127
+// -> 740 / 2900).
+static double pair_us(const GemmProblem& dx, const GemmProblem& dw, const PairTiles& t, int cus) {
+  const double tx = dx_tile_us(t, dx), tw = dw_tile_us(t, dw);
+  const int64_t nx = tile_count(dx, t.dx_bn, t.dx_bm), nw = tile_count(dw, t.dw_bn, t.dw_bm);
+  const double work = (nx * tx + nw * tw) / cus;
+  const double span = tx >= tw ? pair_span(nx, tx, nw, tw, cus) : pair_span(nw, tw, nx, tx, cus);
+  const double alone = weight_from_hbm(dx) ? 1.0 : 0.6;
+  const double us = span * (alone + (1.0 - alone) * (work / span));
+  return work > us ? work : us;
+}
+
+static bool one_launch_serves(const GemmProblem& dx, const GemmProblem& dw) {
+  return dx.X.k_stride == 1 && dx.W.k_stride != 1 && dw.X.k_stride != 1 && dw.W.k_stride != 1 &&
+         det_gemm_takes_kmajor(dx.W, dx.X, dx.K) && det_gemm_takes_kmajor(dw.W, dw.X, dw.K);
+}
+
+static double best_pair_us(const GemmProblem& dx, const GemmProblem& dw, int cus, int* config) {
+  double best = 1e300;
+  for (int c = RLK_LINEAR_BWD_CFG_SEPARATE + 1; c < RLK_LINEAR_BWD_CFG_COUNT; ++c) {
+    const double us = pair_us(dx, dw, kPairTiles[c], cus);
+    if (us < best) {
+      best = us;
+      *config = c;
+    }
+  }
+  return best;
+}
+
+// The rows [0, rows) of dX, and the ones behind them.
+static GemmProblem head_of(GemmProblem dx, int rows) {
+  dx.M = dx.X.rows = rows;
+  return dx;
+}
+static GemmProblem tail_of(GemmProblem dx, int rows) {
+  dx.X.ptr += (int64_t)rows * dx.X.row_stride;
+  dx.C = reinterpret_cast<bf16_bits*>(dx.C) + (int64_t)rows * dx.ldc;
+  dx.M = dx.X.rows = dx.M - rows;
+  return dx;
+}
+
+// One launch where the estimate says 2 % less than the two launches' own. Both sides measured, us, 256 CUs, weights and
+// activations of three layers in turn (tokens, inputs, outputs: two launches -> one):
+//   128, 4096, 4096: 31 -> 22        300, 4096, 4096: 45 -> 35      700, 4096, 4096: 62 -> 56     1400, 4096, 4096: 97 -> 85
+//   2047, 4096, 4096: 117 -> 110     300, 4096, 6144: 66 -> 50      1400, 4096, 6144: 157 -> 132  2047, 4096, 6144: 190 -> 163
+//   6000, 4096, 6144: 500 -> 445     128, 4096, 1536: 17 -> 12      2047, 4096, 1536: 58 -> 50    200, 12288, 4096: 96 -> 79
+//   500, 12288, 4096: 130 -> 113     300, 1024, 4096: 26 -> 18      4120, 1024, 4096: 103 -> 73
+// where the rounds are whole it stays with two (4096, 4096, 4096: 205 = 205), and with up to 256 tokens against a large
+// weight, whose dW is a stream of stores of its own (det_gemm_shortk_kernel; 128, 4096, 24576: 153 as two, 184 as one; 136:
+// 199 as two, 160 as one).
+// A token count just above a multiple of 256 (see remainder_launch_pays): the whole tiles of dX first, then the few tokens
+// behind them beside dW.
+LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem& dw) {
+  LinearBackwardPlan plan{RLK_LINEAR_BWD_CFG_SEPARATE, 0};
+  if (!one_launch_serves(dx, dw)) return plan;
+  if (weight_from_hbm(dx) && det_gemm_shortk_supported(dw.W, dw.X, dw.M, dw.N, dw.K) && det_gemm_shortk_pays(dw.M, dw.N)) return plan;
+  const int cus = device_cu_count();
+  const double partial = weight_from_hbm(dx) ? 1.0 : 0.9;
+  double best = 0.98 * (det_gemm_kmajor_us(dx.M, dx.N, dx.K, true, false, partial) +
+                        det_gemm_kmajor_us(dw.M, dw.N, dw.K, true, true, partial) + kLaunchUs);
+  int config;
+  const double together = best_pair_us(dx, dw, cus, &config);
+  if (together < best) {
+    best = together;
+    plan.config = config;
+  }
+  const int rest = dx.M % 256;
+  if (dx.M > 256 && rest >= 1 && rest <= 64) {
+    const int whole = dx.M - rest;
+    const double head = det_gemm_kmajor_us(whole, dx.N, dx.K, true, false, partial);
+    const double with_rest = head + kLaunchUs + best_pair_us(tail_of(dx, whole), dw, cus, &config);
+    if (with_rest < best) plan = {config, whole};
+  }
+  return plan;
+}
+
+hipError_t linear_backward_launch(GemmProblem dx, const GemmProblem& dw, LinearBackwardPlan plan, hipStream_t stream) {
+  if (plan.config != RLK_LINEAR_BWD_CFG_SEPARATE && !one_launch_serves(dx, dw)) plan = {RLK_LINEAR_BWD_CFG_SEPARATE, 0};
+  if (plan.head_rows > 0) {
+    const GemmProblem head = head_of(dx, plan.head_rows);
+    const hipError_t err = det_gemm_launch(head.W, head.X, head.C, head.ldc, head.M, head.N, head.K, false, RLK_GEMM_CFG_AUTO, stream);
+    if (err != hipSuccess) return err;
+    dx = tail_of(dx, plan.head_rows);
+  }
+  const PairTiles& t = kPairTiles[plan.config];
+  const bool dx_first = plan.config != RLK_LINEAR_BWD_CFG_SEPARATE && dx_tile_us(t, dx) >= dw_tile_us(t, dw);
+  switch (plan.config) {
+    case RLK_LINEAR_BWD_CFG_SEPARATE: {
+      const hipError_t err = det_gemm_launch(dx.W, dx.X, dx.C, dx.ldc, dx.M, dx.N, dx.K, false, RLK_GEMM_CFG_AUTO, stream);
+      if (err != hipSuccess) return err;
+      return det_gemm_launch(dw.W, dw.X, dw.C, dw.ldc, dw.M, dw.N, dw.K, false, RLK_GEMM_CFG_AUTO, stream);
+    }
+    case RLK_LINEAR_BWD_CFG_256x256_256x256:
+      return launch_pair<Pair256x256, 1, 2, Pair256x256>(dx, dw, dx_first, stream);
+    case RLK_LINEAR_BWD_CFG_256x128_256x256:
+      return launch_pair<Pair256x128, 1, 2, Pair256x256>(dx, dw, dx_first, stream);
+    case RLK_LINEAR_BWD_CFG_256x256_256x128:
+      return launch_pair<Pair256x256, 1, 2, Pair256x128>(dx, dw, dx_first, stream);
+    case RLK_LINEAR_BWD_CFG_256x128_256x128:
+      return launch_pair<Pair256x128, 1, 2, Pair256x128>(dx, dw, dx_first, stream);
+    case RLK_LINEAR_BWD_CFG_128x128_256x256:
+      return launch_pair<Pair128x128, 2, 2, Pair256x256>(dx, dw, dx_first, stream);
+    case RLK_LINEAR_BWD_CFG_64x64_256x256:
+      return launch_pair<Pair64x64, 2, 4, Pair256x256>(dx, dw, dx_first, stream);
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace rlk

@@ -457,9 +457,22 @@ hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int6
   // at 80 tokens 257 / 1763, now 80 / 230.)
   const int v_chunks = (V + kChunkElems - 1) / kChunkElems * kChunkElems;
   const int gemm_config = force_staged ? (RLK_GEMM_CFG_AUTO | RLK_GEMM_CFG_FORCE_STAGED) : RLK_GEMM_CFG_AUTO;
+  const MatView dz_by_column{a.dz, 1, a.ld_dz, v_chunks};  // rows = v, reduction index = t
+  const MatView dz_by_token{a.dz, a.ld_dz, 1, T, true};
+  const MatView w_by_feature{W.ptr, 1, W.row_stride, D};  // rows = d, reduction index = v
+  const MatView h_by_feature{H.ptr, 1, H.row_stride, D};  // rows = d, reduction index = t
+  const GemmProblem to_hidden{w_by_feature, dz_by_token, grad_hidden, gh_row_stride, T, D, V};
+  const GemmProblem to_weight{h_by_feature, dz_by_column, grad_weight, gw_row_stride, V, D, T};
+  const LinearBackwardPlan plan = grad_hidden && grad_weight && !force_staged
+                                      ? linear_backward_plan(to_hidden, to_weight)
+                                      : LinearBackwardPlan{RLK_LINEAR_BWD_CFG_SEPARATE, 0};
+  if (plan.config != RLK_LINEAR_BWD_CFG_SEPARATE) {
+    err = linear_backward_launch(to_hidden, to_weight, plan, stream);
+    if (err != hipSuccess) return err;
+    grad_hidden = grad_weight = nullptr;  // done
+  }
   if (grad_weight) {
     // grad_weight[v, d] = sum over t ascending of dz[t, v] * H[t, d]
-    const MatView dz_by_column{a.dz, 1, a.ld_dz, v_chunks};  // rows = v, reduction index = t
     // Both operands are K-major as they lie. From 512 tokens on the hidden states are transposed first (into the
     // grad_hidden buffer, which has exactly their size and is written only afterwards), so that the feature operand
     // runs the plain ping-pong loads: lm_head at 8192 tokens 8.32 -> 7.79 ms plus 0.04 ms for the transposition.
@@ -476,15 +489,12 @@ hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int6
       const MatView h_rows{hidden_t, T, 1, D};  // rows = d, reduction index = t contiguous
       err = det_gemm_launch(h_rows, dz_by_column, grad_weight, gw_row_stride, V, D, T, false, gemm_config, stream);
     } else {
-      const MatView h_by_feature{H.ptr, 1, H.row_stride, D};  // rows = d, reduction index = t
       err = det_gemm_launch(h_by_feature, dz_by_column, grad_weight, gw_row_stride, V, D, T, false, gemm_config, stream);
     }
     if (err != hipSuccess) return err;
   }
   if (grad_hidden) {
     // grad_hidden[t, d] = sum over v ascending of dz[t, v] * W[v, d]
-    const MatView w_by_feature{W.ptr, 1, W.row_stride, D};  // rows = d, reduction index = v
-    const MatView dz_by_token{a.dz, a.ld_dz, 1, T, true};
     err = det_gemm_launch(w_by_feature, dz_by_token, grad_hidden, gh_row_stride, T, D, V, false, gemm_config, stream);
     if (err != hipSuccess) return err;
   }

@@ -113,6 +113,36 @@ int rlk_det_gemm_bf16(const void* a, int64_t a_row_stride, int64_t a_k_stride, c
   return err == hipSuccess ? RLK_OK : device_error("rlk_det_gemm_bf16", err);
 }
 
+int rlk_linear_bwd_bf16(const void* dy, int64_t dy_row_stride, const void* x, int64_t x_row_stride, const void* w,
+                        int64_t w_row_stride, void* dx, int64_t dx_row_stride, void* dw, int64_t dw_row_stride, int tokens,
+                        int inputs, int outputs, int config, void* stream) {
+  if (tokens < 1 || inputs < 1 || outputs < 1) {
+    set_last_error("rlk_linear_bwd_bf16: tokens=%d inputs=%d outputs=%d must be positive", tokens, inputs, outputs);
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  if (config < 0 || config >= RLK_LINEAR_BWD_CFG_COUNT) {
+    set_last_error("rlk_linear_bwd_bf16: unknown config %d", config);
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  if (dy == nullptr || x == nullptr || w == nullptr || dx == nullptr || dw == nullptr) {
+    set_last_error("rlk_linear_bwd_bf16: null pointer");
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  if (dy_row_stride < 0 || x_row_stride < 0 || w_row_stride < 0 || dx_row_stride < inputs || dw_row_stride < inputs) {
+    set_last_error("rlk_linear_bwd_bf16: row strides must not be negative, those of dx and dw not below %d", inputs);
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  const bf16_bits* g = reinterpret_cast<const bf16_bits*>(dy);
+  const GemmProblem to_dx{{reinterpret_cast<const bf16_bits*>(w), 1, w_row_stride, inputs}, {g, dy_row_stride, 1, tokens},
+                          dx, dx_row_stride, tokens, inputs, outputs};
+  const GemmProblem to_dw{{reinterpret_cast<const bf16_bits*>(x), 1, x_row_stride, inputs}, {g, 1, dy_row_stride, outputs},
+                          dw, dw_row_stride, outputs, inputs, tokens};
+  const LinearBackwardPlan plan =
+      config == RLK_LINEAR_BWD_CFG_AUTO ? linear_backward_plan(to_dx, to_dw) : LinearBackwardPlan{config, 0};
+  hipError_t err = linear_backward_launch(to_dx, to_dw, plan, reinterpret_cast<hipStream_t>(stream));
+  return err == hipSuccess ? RLK_OK : device_error("rlk_linear_bwd_bf16", err);
+}
+
 const char* rlk_det_gemm_tree_contract_id(void) { return "rlkernel.det_gemm.hip_ktree32_gfx950.v1"; }
 const char* rlk_det_gemm_tree_leaf_space_contract_id(void) { return "rlkernel.det_gemm.hip_ktree32_leafspace_gfx950.v1"; }
 

@@ -43,10 +43,10 @@ int device_cu_count();
 // What a launch of `tiles` equal workgroups costs in rounds of one workgroup per compute unit: the whole rounds plus
 // a last, partly filled one priced at max(0.9, its share) - the chip is power limited and a round that keeps fewer
 // compute units busy runs at a higher clock, so its cost is little more than its share, but never free.
-inline double rounds_of_workgroups(int64_t tiles, int cus) {
+inline double rounds_of_workgroups(int64_t tiles, int cus, double partial_floor = 0.9) {
   const int64_t full = tiles / cus;
   const double part = (double)(tiles - full * cus) / cus;
-  return (double)full + (part > 0.0 ? (part > 0.9 ? part : 0.9) : 0.0);
+  return (double)full + (part > 0.0 ? (part > partial_floor ? part : partial_floor) : 0.0);
 }
 
 // Whether a kernel loads the weight past the caches (non-temporal): its M tokens are one token tile of `bm`, or two whole
@@ -72,6 +72,26 @@ int pick_det_gemm_config(int M, int N, int K);
 // rows are tokens; C[m*ldc + n].
 hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
                            bool out_f32, int config, hipStream_t stream);
+
+// What a launch with K-major operands takes in the tile estimate, us, a last round that is partly filled priced at
+// max(partial_floor, its share); whether the direct-to-LDS loops take these operands, one or both of them K-major.
+double det_gemm_kmajor_us(int M, int N, int K, bool w_kmajor, bool x_kmajor, double partial_floor);
+bool det_gemm_takes_kmajor(const MatView& W, const MatView& X, int K);
+
+// Both products of a linear layer's backward, in one launch where that is faster.
+struct GemmProblem {
+  MatView W, X;
+  void* C;
+  int64_t ldc;
+  int M, N, K;
+};
+struct LinearBackwardPlan {
+  int config;     // rlk_linear_bwd_config, not AUTO
+  int head_rows;  // rows of dx that a launch of their own computes first
+};
+LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem& dw);
+// A plan whose one launch does not serve the operands runs as two.
+hipError_t linear_backward_launch(GemmProblem dx, const GemmProblem& dw, LinearBackwardPlan plan, hipStream_t stream);
 
 // The k-tree contract (fp32 leaves of at most 32 K values, bf16 midpoint tree). A[M, K]; B holds
 // one row per output column (B.rows == N); any strides. K <= det_gemm_tree_max_k().

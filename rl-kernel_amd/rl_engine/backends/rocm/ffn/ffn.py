@@ -26,6 +26,7 @@ from rl_engine.backends.rocm.gemm.det_gemm import (
     det_gemm_linear,
     det_gemm_linear_input_gradient,
     det_gemm_linear_weight_gradient,
+    mfma_linear_gradients,
 )
 
 QWEN3_8B_HIDDEN_SIZE = 4096
@@ -130,6 +131,16 @@ def qwen3_ffn_packed_inference(
 # ---------------------------------------------------------------------------
 
 
+def _linear_gradients(a: Tensor, weight: Tensor, grad: Tensor, need_a: bool, need_weight: bool) -> tuple:
+    """The gradients of ``a @ weight.T`` that are wanted, ``None`` for the others; both at once where both are."""
+    if need_a and need_weight:
+        return mfma_linear_gradients(a, weight, grad)
+    return (
+        det_gemm_linear_input_gradient(grad, weight) if need_a else None,
+        det_gemm_linear_weight_gradient(a, grad) if need_weight else None,
+    )
+
+
 class _DeterministicFFNFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, rmsnorm_output, gate_weight, up_weight, down_weight, fused_gate_up_weight):
@@ -157,19 +168,16 @@ class _DeterministicFFNFunction(torch.autograd.Function):
         else:
             x, gate, up, activated, gate_weight, up_weight, down_weight = ctx.saved_tensors
         grad_output = grad_output.reshape(-1, grad_output.size(-1)).to(torch.bfloat16).contiguous()
-        grad_activated = det_gemm_linear_input_gradient(grad_output, down_weight)
+        need = ctx.needs_input_grad
+        grad_activated, grad_down_weight = _linear_gradients(activated, down_weight, grad_output, True, need[3])
         if ctx.packed:
             grad_gate, grad_up = _C.swiglu_packed_backward(grad_activated, gate_up)
         else:
             grad_gate, grad_up = _C.swiglu_backward(grad_activated, gate, up)
-        need = ctx.needs_input_grad
-        grad_down_weight = det_gemm_linear_weight_gradient(activated, grad_output) if need[3] else None
-        grad_gate_weight = det_gemm_linear_weight_gradient(x, grad_gate) if need[1] else None
-        grad_up_weight = det_gemm_linear_weight_gradient(x, grad_up) if need[2] else None
-        grad_x = None
+        grad_x, grad_gate_weight = _linear_gradients(x, gate_weight, grad_gate, need[0], need[1])
+        from_up, grad_up_weight = _linear_gradients(x, up_weight, grad_up, need[0], need[2])
         if need[0]:
-            grad_x = det_gemm_linear_input_gradient(grad_gate, gate_weight)
-            grad_x.add_(det_gemm_linear_input_gradient(grad_up, up_weight))
+            grad_x.add_(from_up)
             grad_x = grad_x.reshape(ctx.input_shape)
         return grad_x, grad_gate_weight, grad_up_weight, grad_down_weight, None
 
