@@ -60,7 +60,9 @@ typedef enum rlk_gemm_config {
   RLK_GEMM_CFG_32x32_DEEP = 21,   /* 32 features x 32 tokens, 128 K values per barrier */
   RLK_GEMM_CFG_32x64_DEEP = 22,   /* 32 features x 64 tokens, 256 K values per barrier */
   RLK_GEMM_CFG_64x160_DEEP = 23,  /* 64 features x 160 tokens; K % 128 == 0 */
-  RLK_GEMM_CFG_COUNT = 24,
+  RLK_GEMM_CFG_256x192 = 24,      /* 256 features x 192 tokens; K % 64 == 0 */
+  RLK_GEMM_CFG_192x192 = 25,      /* 192 features x 192 tokens, three stages; K % 64 == 0 */
+  RLK_GEMM_CFG_COUNT = 26,
   /* OR-ed into a configuration: use the register-staged main loop even where the
    * direct-to-LDS ping-pong loop applies. Bit-neutral; exists so tests can
    * compare the two loops. */
@@ -111,7 +113,8 @@ typedef enum rlk_linear_bwd_config {
   RLK_LINEAR_BWD_CFG_256x128_256x128 = 5,
   RLK_LINEAR_BWD_CFG_128x128_256x256 = 6,
   RLK_LINEAR_BWD_CFG_64x64_256x256 = 7,
-  RLK_LINEAR_BWD_CFG_COUNT = 8
+  RLK_LINEAR_BWD_CFG_256x192_256x256 = 8,
+  RLK_LINEAR_BWD_CFG_COUNT = 9
 } rlk_linear_bwd_config;
 
 /*

@@ -159,6 +159,8 @@ static hipError_t launch_small_kmajor(const MatView& W, const MatView& X, void* 
 using Shape256x256 = TileShape<256, 256, 4, 2>;
 using Shape256x256Solo = TileShape<256, 256, 2, 2>;
 using Shape192x256 = TileShape<192, 256, 4, 2>;  // 192 features x 256 tokens: three MFMA tiles per wave along N
+using Shape256x192 = TileShape<256, 192, 4, 2>;
+using Shape192x192 = TileShape<192, 192, 4, 2>;  // 192 features x 192 tokens
 using Shape192x128 = TileShape<192, 128, 4, 2>;  // 192 features x 128 tokens
 using Shape256x128 = TileShape<256, 128, 4, 2>;
 using Shape256x64 = TileShape<256, 64, 4, 2>;
@@ -217,10 +219,16 @@ int device_cu_count() {
 // N = 10240 at 2048 tokens 190 -> 162 us) and loses the tie against 256 x 128 at N = 4096, 2048 tokens. 192 x 128
 // (three stages) does the same one size down (weights from HBM: gate_up at 256 tokens 65.0 -> 62.2 us, N = 6144 at 768
 // tokens 55.1 -> 49.1 us).
+// 192-token tiles where two of them, or three, hold what 128- and 256-token tiles do not divide well; they read 144 and
+// 160 rows per wave and K tile from LDS for 36 and 48 matrix instructions a step, between 256 x 128 (128 for 32) and 256 x
+// 256. Weights of three layers in turn, before -> with them: gate_up at 360 / 700 / 900 tokens 89.9 / 156 / 169 -> 72.0 / 134 /
+// 157 us, 12288 outputs at 700 / 1500 tokens 78.8 / 153 -> 65.2 / 133, 14336 at 540 / 1300 tokens 81.3 / 158 -> 65.1 / 144,
+// qkv at 1300 tokens 67.4 -> 58.3, down at 2600 tokens 224 -> 206.
 // K-major-weight column (`dY @ W`, `a @ b`, prepared weights): the 64- and 128-feature tiles give a long reduction
 // against few output tiles - grad_hidden of the LogP backward up to about a thousand tokens (N = 4096, K = 151936) - a
 // workgroup per CU, each streaming a narrow slice of the weight instead of a 256-column one (1.9 -> 0.8 ms at 256
-// tokens, 1.8 -> 1.03 ms at 512, 1.65 -> 1.45 ms at 1024); their qualities are those of the direct-to-LDS loop.
+// tokens, 1.8 -> 1.03 ms at 512, 1.65 -> 1.45 ms at 1024); their qualities are those of the direct-to-LDS loop. 256 x 192:
+// dX of 14336 inputs, 4096 outputs at 540 / 1300 tokens 106 / 169 -> 68 / 142 us, of 4096, 6144 at 2300 tokens 108 -> 95.
 struct TileCandidate {
   int config, bn, bm;
   double native, ragged192, w_kmajor;
@@ -228,6 +236,7 @@ struct TileCandidate {
 };
 static const TileCandidate kTileCandidates[] = {
     {RLK_GEMM_CFG_256x256, 256, 256, 1.00, 0.00, 1.00, true},  {RLK_GEMM_CFG_192x256, 192, 256, 0.89, 0.85, 0.00, false},
+    {RLK_GEMM_CFG_256x192, 256, 192, 0.87, 0.00, 0.87, false}, {RLK_GEMM_CFG_192x192, 192, 192, 0.75, 0.68, 0.00, false},
     {RLK_GEMM_CFG_256x128, 256, 128, 0.65, 0.00, 0.70, true},  {RLK_GEMM_CFG_192x128, 192, 128, 0.56, 0.53, 0.00, false},
     {RLK_GEMM_CFG_256x64, 256, 64, 0.50, 0.00, 0.56, false},   {RLK_GEMM_CFG_128x128, 128, 128, 0.65, 0.00, 0.62, false},
     {RLK_GEMM_CFG_128x64, 128, 64, 0.45, 0.00, 0.40, false},   {RLK_GEMM_CFG_64x64, 64, 64, 0.42, 0.00, 0.25, false},
@@ -247,7 +256,7 @@ static int pick_tile_candidate(int M, int N, int K, bool w_kmajor, bool x_kmajor
       quality = c.w_kmajor;
     } else {
       const bool wide192 = c.ragged192 != 0.0;
-      if (wide192 && K % kTileK != 0) continue;
+      if ((wide192 || c.bm == 192) && K % kTileK != 0) continue;  // the direct-to-LDS loop only
       quality = (wide192 && N % 192 != 0) ? c.ragged192 : c.native;
     }
     const double t = rounds_of_workgroups(tile_count(M, N, c.bm, c.bn), cus, partial_floor) * (double)(c.bn * c.bm) / quality;
@@ -394,6 +403,9 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     switch (config) {
       case RLK_GEMM_CFG_256x256:
         return launch_shape<Shape256x256>(W, X, C, ldc, M, N, K, false, loop, true, out_f32, stream);
+      case RLK_GEMM_CFG_256x192:
+        if (!x_kmajor) return launch_shape<Shape256x192>(W, X, C, ldc, M, N, K, false, loop, true, out_f32, stream);
+        break;
       case RLK_GEMM_CFG_256x128:
         return launch_shape<Shape256x128>(W, X, C, ldc, M, N, K, false, loop, true, out_f32, stream);
       case RLK_GEMM_CFG_256x64:
@@ -463,6 +475,16 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
   if (config == RLK_GEMM_CFG_192x128) {
     if (vec && allow_pingpong && K % kTileK == 0)
       return launch_loop<Shape192x128, kLoopPingPong, pingpong_stages<Shape192x128>()>(W, X, C, ldc, M, N, K, out_f32, stream);
+    config = RLK_GEMM_CFG_256x128;
+  }
+  if (config == RLK_GEMM_CFG_256x192) {
+    if (vec && allow_pingpong && K % kTileK == 0)
+      return launch_loop<Shape256x192, kLoopPingPong>(W, X, C, ldc, M, N, K, out_f32, stream);
+    config = RLK_GEMM_CFG_256x256;
+  }
+  if (config == RLK_GEMM_CFG_192x192) {
+    if (vec && allow_pingpong && K % kTileK == 0)
+      return launch_loop<Shape192x192, kLoopPingPong, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
     config = RLK_GEMM_CFG_256x128;
   }
   if (config == RLK_GEMM_CFG_192x256) {

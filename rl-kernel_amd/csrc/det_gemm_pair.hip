@@ -45,6 +45,7 @@ __global__ __launch_bounds__(SX::kThreads) void det_gemm_pair_kernel(PairProblem
 // ---------------------------------------------------------------------------
 
 using Pair256x256 = TileShape<256, 256, 4, 2>;
+using Pair256x192 = TileShape<256, 192, 4, 2>;
 using Pair256x128 = TileShape<256, 128, 4, 2>;
 using Pair128x128 = TileShape<128, 128, 4, 2>;
 using Pair64x64 = TileShape<64, 64, 4, 2>;
@@ -61,6 +62,7 @@ static const PairTiles kPairTiles[RLK_LINEAR_BWD_CFG_COUNT] = {
     {}, {},  // automatic, two launches
     {256, 256, 1.00, 256, 256, 1.00}, {256, 128, 0.70, 256, 256, 1.00}, {256, 256, 1.00, 256, 128, 0.70},
     {256, 128, 0.70, 256, 128, 0.70}, {128, 128, 0.53, 256, 256, 1.00}, {64, 64, 0.25, 256, 256, 1.00},
+    {256, 192, 0.90, 256, 256, 1.00},
 };
 
 template <class S>
@@ -234,6 +236,8 @@ hipError_t linear_backward_launch(GemmProblem dx, const GemmProblem& dw, LinearB
       return launch_pair<Pair128x128, 2, 2, Pair256x256>(dx, dw, dx_first, stream);
     case RLK_LINEAR_BWD_CFG_64x64_256x256:
       return launch_pair<Pair64x64, 2, 4, Pair256x256>(dx, dw, dx_first, stream);
+    case RLK_LINEAR_BWD_CFG_256x192_256x256:
+      return launch_pair<Pair256x192, 1, 2, Pair256x256>(dx, dw, dx_first, stream);
     default:
       return hipErrorInvalidValue;
   }

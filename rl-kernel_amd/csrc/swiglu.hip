@@ -230,6 +230,7 @@ __global__ __launch_bounds__(S::kThreads) void det_gemm_swiglu_kernel(MatView W,
 }
 
 using GatedShape256 = TileShape<256, 256, 4, 2>;
+using GatedShape192 = TileShape<256, 192, 4, 2>;
 using GatedShape128 = TileShape<256, 128, 4, 2>;
 using GatedShape64 = TileShape<256, 64, 4, 2>;
 
@@ -274,14 +275,19 @@ hipError_t det_gemm_swiglu_launch(const MatView& W, const MatView& X, void* Y, i
   if (det_gemm_swiglu_fused_supported(W, X, M, K)) {
     if (streams_gated(M, K)) return det_gemm_stream_gated_launch(W, X, Y, ldy, M, I, K, stream);
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((I + 127) / 128);
+    const int64_t t192 = (int64_t)((M + 191) / 192) * ((I + 127) / 128);
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((I + 127) / 128);
     // Rounds of workgroups x tokens per tile / relative throughput, as in pick_det_gemm_config:
-    // a partly filled last round costs little more than its share, so the large tile wins early.
+    // a partly filled last round costs little more than its share, so the large tile wins early. 192-token tiles, K = 4096,
+    // before -> with them: I = 12288 at 308 / 778 / 1492 tokens 85.8 / 163 / 249 -> 72.0 / 144 / 220 us, 6144 at 722 tokens 78.6
+    // -> 68.2, 3072 at 1908 tokens 76.8 -> 69.6.
     const int cus = device_cu_count();
     auto cost = [cus](int64_t tiles, double tokens, double quality) {
       return rounds_of_workgroups(tiles, cus) * tokens / quality;
     };
-    if (M > 128 && cost(t256, 256.0, 1.0) <= cost(t128, 128.0, 0.65))
+    const double c256 = cost(t256, 256.0, 1.0), c192 = cost(t192, 192.0, 0.87), c128 = cost(t128, 128.0, 0.65);
+    if (M > 128 && c192 < c256 && c192 < c128) return launch_gated<GatedShape192>(W, X, Y, ldy, M, I, K, stream);
+    if (M > 128 && c256 <= c128)
       return launch_gated<GatedShape256>(W, X, Y, ldy, M, I, K, stream);
     if (M > 64 && t128 >= 128) return launch_gated<GatedShape128>(W, X, Y, ldy, M, I, K, stream);
     return launch_gated<GatedShape64>(W, X, Y, ldy, M, I, K, stream);

@@ -46,6 +46,8 @@ GEMM_CONFIGS = {
     "32x32_deep": 21,
     "32x64_deep": 22,
     "64x160_deep": 23,
+    "256x192": 24,
+    "192x192": 25,
 }
 # OR-ed into a GEMM or LogP configuration: register-staged main loop (bit-neutral).
 FORCE_STAGED = 0x100

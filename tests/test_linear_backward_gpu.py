@@ -9,7 +9,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda"
-CONFIGS = range(2, 8)  # rlk_linear_bwd_config: every one-launch configuration
+CONFIGS = range(2, 9)  # rlk_linear_bwd_config: every one-launch configuration
 # (tokens, inputs, outputs): one tile and less, a token more than a tile of each height, ragged everything, reductions of
 # dX that no stage divides, many tiles of one product beside few of the other, both orders of the two
 SHAPES = [
@@ -91,7 +91,7 @@ def test_few_tokens_behind_whole_tiles(rest):
     got = _backward(g, x, w, 0)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     assert _lib.load().rlk_linear_bwd_bf16(None, n, x.data_ptr(), k, w.data_ptr(), k, x.data_ptr(), k, w.data_ptr(), k, m, k, n, 0, None) < 0
-    assert _lib.load().rlk_linear_bwd_bf16(g.data_ptr(), n, x.data_ptr(), k, w.data_ptr(), k, x.data_ptr(), k, w.data_ptr(), k, m, k, n, 8, None) < 0
+    assert _lib.load().rlk_linear_bwd_bf16(g.data_ptr(), n, x.data_ptr(), k, w.data_ptr(), k, x.data_ptr(), k, w.data_ptr(), k, m, k, n, 9, None) < 0
 
 
 def test_a_captured_backward_replays():
