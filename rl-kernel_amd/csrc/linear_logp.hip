@@ -492,7 +492,6 @@ hipError_t linear_logp_launch(const MatView& H, const MatView& W, const int64_t*
   config &= ~RLK_LOGP_CFG_FORCE_STAGED;
   const int requested = config;
   if (config == RLK_LOGP_CFG_AUTO) config = pick_linear_logp_config(T, V);
-  if (!vec && config == RLK_LOGP_CFG_256) config = RLK_LOGP_CFG_128;
   const int loop = !vec ? 0 : (D % kTileK == 0 && !force_staged) ? 2 : 1;
   // The stream-group kernels have the direct-to-LDS loop only and a bounded workspace.
   if (loop != 2 || T > kStreamGroupMaxTokens) {
@@ -500,6 +499,7 @@ hipError_t linear_logp_launch(const MatView& H, const MatView& W, const int64_t*
     if (config == RLK_LOGP_CFG_128_STREAMS) config = RLK_LOGP_CFG_128;
     if (config == RLK_LOGP_CFG_256_STREAMS) config = RLK_LOGP_CFG_256;
   }
+  if (!vec && config == RLK_LOGP_CFG_256) config = RLK_LOGP_CFG_128;  // which has the element-wise loader
   hipError_t err;
   switch (config) {
     case RLK_LOGP_CFG_64_STREAMS:
