@@ -202,11 +202,12 @@ typedef enum rlk_logp_config {
   RLK_LOGP_CFG_128 = 2,
   RLK_LOGP_CFG_64 = 3,
   RLK_LOGP_CFG_16 = 4,
-  /* up to 1024 tokens: four workgroups per vocabulary split, four streams each (64 / 128 / 256-token tiles) */
+  /* up to 1024 tokens: four workgroups per vocabulary split, four streams each (64- to 256-token tiles) */
   RLK_LOGP_CFG_64_STREAMS = 5,
   RLK_LOGP_CFG_128_STREAMS = 6,
   RLK_LOGP_CFG_256_STREAMS = 7,
-  RLK_LOGP_CFG_COUNT = 8,
+  RLK_LOGP_CFG_192_STREAMS = 8,
+  RLK_LOGP_CFG_COUNT = 9,
   /* OR-ed into a configuration: register-staged main loop instead of the
    * direct-to-LDS ping-pong loop (bit-neutral; for tests). */
   RLK_LOGP_CFG_FORCE_STAGED = 0x100

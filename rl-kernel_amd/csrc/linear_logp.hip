@@ -370,6 +370,7 @@ hipError_t linear_logp_merge_launch(const float* part, float* logp, float* lse, 
 // ---------------------------------------------------------------------------
 
 using LogpShape256 = TileShape<256, 256, 4, 2>;
+using LogpShape192 = TileShape<256, 192, 4, 2>;
 using LogpShape128 = TileShape<256, 128, 4, 2>;
 using LogpShape64 = TileShape<256, 64, 4, 2>;
 using LogpShape16 = TileShape<256, 16, 4, 1>;
@@ -420,6 +421,14 @@ static hipError_t launch_streamgroup_range(LogpArgs a, float* spart, int split_f
   return hipGetLastError();
 }
 
+// A 256-token launch whose last round would fill at most half of the chip ends in 128-token tiles: the splits those cover.
+static int balanced_tail_splits(int T, int n_split, int cus) {
+  const int per_split = (T + 255) / 256 * (kLogpStreams / 4);
+  if (per_split > cus || cus % per_split != 0) return 0;
+  const int tail = n_split % (cus / per_split);
+  return tail * per_split * 2 <= cus && n_split > tail ? tail : 0;
+}
+
 // `balance`: with the 256-token tile, a last round that would fill at most half of the chip
 // runs as 128-token tiles instead (twice the workgroups, each about 0.57 of the time): for
 // 256 tokens and V = 151936, 596 workgroups are 2.33 rounds of 256; 512 of them plus 168
@@ -427,16 +436,9 @@ static hipError_t launch_streamgroup_range(LogpArgs a, float* spart, int split_f
 // is not part of the contract.
 template <class S>
 static hipError_t launch_streamgroup(LogpArgs a, bool balance, hipStream_t stream) {
-  const int kCus = device_cu_count();
   float* spart = a.part + (size_t)3 * a.n_split * a.T;  // behind the per-split partials
-  const int tiles_m = (a.T + S::BM - 1) / S::BM;
-  const int per_split = tiles_m * (kLogpStreams / 4);
   int main_splits = a.n_split;
-  if (balance && S::BM == 256 && per_split <= kCus && kCus % per_split == 0) {
-    const int per_round = kCus / per_split;
-    const int tail = a.n_split % per_round;
-    if (tail * per_split * 2 <= kCus && a.n_split > tail) main_splits = a.n_split - tail;
-  }
+  if (balance && S::BM == 256) main_splits -= balanced_tail_splits(a.T, a.n_split, device_cu_count());
   hipError_t err = launch_streamgroup_range<S>(a, spart, 0, main_splits, stream);
   if (err != hipSuccess) return err;
   if (main_splits < a.n_split) {
@@ -450,17 +452,26 @@ static hipError_t launch_streamgroup(LogpArgs a, bool balance, hipStream_t strea
 }
 
 int pick_linear_logp_config(int T, int V) {
-  (void)V;
   // Measured at V = 151936, D = 4096: the 64-token tile (two workgroups per CU, direct-to-LDS
-  // loop) is the fastest from decode sizes up to 64 tokens, the 256-token tile from 256 tokens on
+  // loop) is the fastest from decode sizes up to 64 tokens, the 256-token tile from 1024 tokens on
   // even where it leaves the last round of workgroups part empty.
   if (T <= 64) return RLK_LOGP_CFG_64_STREAMS;
   if (T <= 128) return RLK_LOGP_CFG_128_STREAMS;
-  // 257 ... 384 tokens are three 128-token tiles or two 256-token ones, a third of them padding (544 against 582 us
-  // at 384 tokens); wherever 128-token tiles save no padded tile the 256-token tile wins (798 against 966 us at 768).
-  if (T > 256 && T <= 384) return RLK_LOGP_CFG_128_STREAMS;
-  if (T <= 1024) return RLK_LOGP_CFG_256_STREAMS;
-  return RLK_LOGP_CFG_256;
+  if (T <= 256) return RLK_LOGP_CFG_256_STREAMS;
+  if (T > kStreamGroupMaxTokens) return RLK_LOGP_CFG_256;
+  // Between them by rounds of workgroups x tokens per tile / relative throughput. 128 / 256 / 192 tokens, us: V = 151936, D =
+  // 4096 at 300 tokens 482 / 523 / 432, 540: 779 / 737 / 608, 700: 914 / 746 / 811; V = 37984 at 300: 137 / 199 / 161, 450: 193
+  // / 203 / 166, 800: 307 / 303 / 256; V = 32768, D = 2048 at 300: 84 / 74 / 62, 700: 122 / 128 / 109.
+  const int cus = device_cu_count();
+  const int n_split = linear_logp_split_count(V);
+  auto cost = [&](int splits, int bm, double quality) {
+    return rounds_of_workgroups((int64_t)((T + bm - 1) / bm) * splits * (kLogpStreams / 4), cus) * bm / quality;
+  };
+  const int tail = balanced_tail_splits(T, n_split, cus);
+  const double c256 = tail ? cost(n_split - tail, 256, 1.0) + cost(tail, 128, 0.76) : cost(n_split, 256, 1.0);
+  const double c192 = cost(n_split, 192, 0.945), c128 = cost(n_split, 128, 0.76);
+  if (c192 < c256 && c192 < c128) return RLK_LOGP_CFG_192_STREAMS;
+  return c128 < c256 ? RLK_LOGP_CFG_128_STREAMS : RLK_LOGP_CFG_256_STREAMS;
 }
 
 hipError_t linear_logp_launch(const MatView& H, const MatView& W, const int64_t* target, const float* bias,
@@ -497,7 +508,7 @@ hipError_t linear_logp_launch(const MatView& H, const MatView& W, const int64_t*
   if (loop != 2 || T > kStreamGroupMaxTokens) {
     if (config == RLK_LOGP_CFG_64_STREAMS) config = RLK_LOGP_CFG_64;
     if (config == RLK_LOGP_CFG_128_STREAMS) config = RLK_LOGP_CFG_128;
-    if (config == RLK_LOGP_CFG_256_STREAMS) config = RLK_LOGP_CFG_256;
+    if (config == RLK_LOGP_CFG_192_STREAMS || config == RLK_LOGP_CFG_256_STREAMS) config = RLK_LOGP_CFG_256;
   }
   if (!vec && config == RLK_LOGP_CFG_256) config = RLK_LOGP_CFG_128;  // which has the element-wise loader
   hipError_t err;
@@ -507,6 +518,9 @@ hipError_t linear_logp_launch(const MatView& H, const MatView& W, const int64_t*
       break;
     case RLK_LOGP_CFG_128_STREAMS:
       err = launch_streamgroup<LogpShape128>(a, false, stream);
+      break;
+    case RLK_LOGP_CFG_192_STREAMS:
+      err = launch_streamgroup<LogpShape192>(a, false, stream);
       break;
     case RLK_LOGP_CFG_256_STREAMS:
       err = launch_streamgroup<LogpShape256>(a, requested == RLK_LOGP_CFG_AUTO, stream);

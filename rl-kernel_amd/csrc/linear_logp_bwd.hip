@@ -410,11 +410,13 @@ hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int6
                    pitch_fits_lane_offsets(W.row_stride) && pitch_fits_lane_offsets(H.row_stride);
   const bool force_staged = (config & RLK_LOGP_CFG_FORCE_STAGED) != 0;
   config &= ~RLK_LOGP_CFG_FORCE_STAGED;
-  if (config == RLK_LOGP_CFG_AUTO) config = pick_linear_logp_config(T, V);
+  // 257 ... 384 tokens are three 128-token tiles or two 256-token ones, a third of them padding
+  if (config == RLK_LOGP_CFG_AUTO)
+    config = T <= 64 ? RLK_LOGP_CFG_64 : (T <= 128 || (T > 256 && T <= 384)) ? RLK_LOGP_CFG_128 : RLK_LOGP_CFG_256;
   // the stream-group configurations are forward-only work splits
   if (config == RLK_LOGP_CFG_64_STREAMS) config = RLK_LOGP_CFG_64;
   if (config == RLK_LOGP_CFG_128_STREAMS) config = RLK_LOGP_CFG_128;
-  if (config == RLK_LOGP_CFG_256_STREAMS) config = RLK_LOGP_CFG_256;
+  if (config == RLK_LOGP_CFG_192_STREAMS || config == RLK_LOGP_CFG_256_STREAMS) config = RLK_LOGP_CFG_256;
   if (!vec && config == RLK_LOGP_CFG_256) config = RLK_LOGP_CFG_128;
   // the bias-gradient partials of 16-token tiles only fit the workspace up to kBiasSmallTileMaxTokens
   if (grad_bias && config == RLK_LOGP_CFG_16 && T > kBiasSmallTileMaxTokens) config = RLK_LOGP_CFG_64;

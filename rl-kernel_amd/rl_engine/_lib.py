@@ -56,7 +56,9 @@ NOALLOC_SCRATCH_BYTES = 32 << 20  # RLK_NOALLOC_SCRATCH_BYTES
 # rlk_dtype (element types of materialised logits)
 DTYPE_BF16, DTYPE_FP16, DTYPE_FP32 = 0, 1, 2
 # rlk_logp_config
-LOGP_CONFIGS = {"auto": 0, "256": 1, "128": 2, "64": 3, "16": 4, "64_streams": 5, "128_streams": 6, "256_streams": 7}
+LOGP_CONFIGS = {
+    "auto": 0, "256": 1, "128": 2, "64": 3, "16": 4, "64_streams": 5, "128_streams": 6, "256_streams": 7, "192_streams": 8,
+}  # fmt: skip
 
 EXPORTED_SYMBOLS = (
     "rlk_contract_id",
