@@ -558,6 +558,21 @@ struct GatedRowMap {
   }
 };
 
+// The same for four waves that share all weight rows (1 x 4): the first TN / 2 MFMA tiles hold gate features
+// (lane>>4) * 2 TN + jn * 4 + q, the others the up projection of the same features.
+template <class S>
+struct GatedSharedRowMap {
+  static_assert(S::WN == 1 && S::TN % 2 == 0, "one wave column, as many gate tiles as up tiles");
+  static constexpr bool kGated = true;
+  static constexpr int kTiles = S::TN / 2;
+  static __device__ __forceinline__ int block_offset(int b) { return (b / 2 % kTiles) * 4; }
+  static __device__ __forceinline__ int block_half(int b) { return b / 2 / kTiles; }
+  static __device__ __forceinline__ int lane_offset(int parity, int rib) {
+    const int i = parity * 8 + rib;
+    return (i >> 2) * (4 * kTiles) + (i & 3);
+  }
+};
+
 // StridedColumnRowMap<S, STRIDE>: wave column c of the stage holds the 64 weight rows that
 // start STRIDE * c after the tile origin (same order inside a column as PlainRowMap), so one
 // workgroup covers a 64-row slice of four blocks of rows STRIDE apart.
@@ -1279,14 +1294,13 @@ __device__ __forceinline__ void tile_mainloop_solo_impl(const MatView& W, const 
 // ---------------------------------------------------------------------------
 template <class S>
 constexpr bool quad_supported() {
-  return S::WN == 2 && S::WM == 2 && S::BN % 32 == 0 && S::BM % 32 == 0;
+  return S::WN * S::WM == 4 && S::BN % 32 == 0 && S::BM % 32 == 0;
 }
 
-template <class S, int KS, int NS, bool WSTREAM>
+template <class S, int KS, int NS, bool WSTREAM, class Map = PlainRowMap<S>>
 __device__ __forceinline__ void tile_mainloop_quad(const MatView& W, const MatView& X, int n0, int m0, int K, char* lds,
                                                    f32x4_t (&acc)[S::TN][S::TM]) {
-  static_assert(quad_supported<S>() && NS >= 2, "2 x 2 waves");
-  using Map = PlainRowMap<S>;
+  static_assert(quad_supported<S>() && NS >= 2, "four waves");
   constexpr int kLoadsW = S::BN / 32, kLoadsX = S::BM / 32;  // blocks of 8 rows per wave and K tile
   constexpr int kLoads = KS * (kLoadsW + kLoadsX);
   static_assert((NS - 1) * kLoads <= 63, "loads in flight must fit vmcnt");
@@ -1305,9 +1319,10 @@ __device__ __forceinline__ void tile_mainloop_quad(const MatView& W, const MatVi
   auto block = [&](int j) { return 4 * j + wave; };
 #pragma unroll
   for (int j = 0; j < kLoadsW; ++j) {
+    const int n_rows = Map::kGated ? W.rows / 2 : W.rows;  // of one half of a packed gate/up weight
     int g = n0 + Map::block_offset(block(j)) + Map::lane_offset(wave & 1, rib);
-    g = g < W.rows ? g : W.rows - 1;
-    w_src[j] = W.ptr + (int64_t)g * W.row_stride + chunk_elems;
+    g = g < n_rows ? g : n_rows - 1;
+    w_src[j] = W.ptr + ((int64_t)(Map::block_half(block(j)) * n_rows) + g) * W.row_stride + chunk_elems;
   }
 #pragma unroll
   for (int j = 0; j < kLoadsX; ++j) {

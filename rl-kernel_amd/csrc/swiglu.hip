@@ -229,6 +229,66 @@ __global__ __launch_bounds__(S::kThreads) void det_gemm_swiglu_kernel(MatView W,
   }
 }
 
+// The same for few tokens: four waves over one wave column of BN / 2 gate rows and the up rows of the same features, all of
+// the tokens of a launch in one tile.
+// Bound by HBM: the weight is read once (201 MB of gate_up in 39 us, 5.2 TB/s), four waves read every weight row from LDS
+// (448 + 160 rows a K tile of 96 x 64, 608 of about 1300 cycles that its 12 KiB of weight take at that rate).
+template <class S, int KS, int NS, bool WSTREAM>
+__global__ __launch_bounds__(S::kThreads) void det_gemm_swiglu_few_kernel(MatView W, MatView X, bf16_bits* __restrict__ Y,
+                                                                           int64_t ldy, int M, int I, int K) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  constexpr int kTiles = S::TN / 2;
+  const int f0 = xcd_compact_id(blockIdx.x, gridDim.x) * (S::BN / 2);
+
+  f32x4_t acc[S::TN][S::TM];
+  tile_mainloop_quad<S, KS, NS, WSTREAM, GatedSharedRowMap<S>>(W, X, f0, 0, K, lds, acc);
+
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int f_run = f0 + (lane >> 4) * 4 * kTiles;  // first of this lane's 4 kTiles consecutive features
+#pragma unroll
+  for (int jm = 0; jm < S::TM; ++jm) {
+    const int m = (wave * S::TM + jm) * 16 + (lane & 15);
+    if (m >= M) continue;
+    bf16_bits* out = Y + (int64_t)m * ldy + f_run;
+    const bool whole = f_run + 4 * kTiles <= I && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      float y[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        y[q] = swiglu_f32(round_through_bf16(acc[t][jm][q]), round_through_bf16(acc[t + kTiles][jm][q]));
+      const uint32_t packed[2] = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+      if (whole) {
+        *reinterpret_cast<u32x2_t*>(out + t * 4) = u32x2_t{packed[0], packed[1]};
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (f_run + t * 4 + q < I) out[t * 4 + q] = (bf16_bits)((packed[q >> 1] >> ((q & 1) * 16)) & 0xffffu);
+      }
+    }
+  }
+}
+
+// BN rows (BN / 2 features), 64 TM tokens, KS K tiles a stage, NS stages.
+template <int BN, int TM, int KS, int NS, bool WSTREAM = false>
+static hipError_t launch_gated_few(const MatView& W, const MatView& X, void* Y, int64_t ldy, int M, int I, int K,
+                                   hipStream_t stream) {
+  using S = TileShape<BN, 64 * TM, 1, 4>;
+  if constexpr (!WSTREAM) {
+    if (streamed_weight(2 * (int64_t)I, K, M, S::BM)) return launch_gated_few<BN, TM, KS, NS, true>(W, X, Y, ldy, M, I, K, stream);
+  }
+  auto kernel = det_gemm_swiglu_few_kernel<S, KS, NS, WSTREAM>;
+  constexpr int kLds = NS * KS * S::kStageBytes;
+  static_assert(kLds <= 160 * 1024, "stages exceed the LDS");
+  static PerDeviceOnce once;
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds, once);
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL(kernel, dim3((I + BN / 2 - 1) / (BN / 2)), dim3(S::kThreads), kLds, stream, W, X,
+                     reinterpret_cast<bf16_bits*>(Y), ldy, M, I, K);
+  return hipGetLastError();
+}
+
 using GatedShape256 = TileShape<256, 256, 4, 2>;
 using GatedShape192 = TileShape<256, 192, 4, 2>;
 using GatedShape128 = TileShape<256, 128, 4, 2>;
@@ -253,27 +313,45 @@ static hipError_t launch_gated(const MatView& W, const MatView& X, void* Y, int6
 }
 
 // Up to 16 tokens the streaming kernel serves the packed projection (the same panels of 16 weight
-// rows, eight gate and eight up), from 129 tokens on the gated tile kernels; between them the
-// projection and the activation run as two kernels (the weight read bounds the time there and the
-// GEMM kernels for few tokens spread it over more CUs than a gated 128-feature tile).
+// rows, eight gate and eight up), from 129 tokens on the gated tile kernels.
 static bool streams_gated(int M, int K) { return M <= 16 && K >= 1024; }
+// From 17 to 128 tokens a gated tile on four waves, no wider than gives every CU one: gate_up of 12288 at 64 tokens ran on 192
+// of 256 CUs as 128-row tiles, and the projection was written, read again and activated by a second launch. Weights from
+// HBM, two launches -> one, us (K = 4096, I = 12288 / 6144 / 3072): 17 tokens 42.1 / 23.6 / 15.0 -> 37.1 / 20.8 / 13.7, 64: 45.4
+// / 27.6 / 20.8 -> 39.1 / 25.8 / 17.6, 128: 50.5 / 37.4 / 23.4 -> 45.0 / 32.6 / 25.0 (not used: the many token rows beside 32
+// weight rows per tile; K = 2048: 12.6 -> 10.5).
+static bool few_gated(int M, int I, int K) {
+  return M > 16 && M <= 128 && K % 128 == 0 && K >= 512 && (M <= 96 || K <= 2048 || I > 16 * device_cu_count());
+}
 
 bool det_gemm_swiglu_fused_supported(const MatView& W, const MatView& X, int M, int K) {
   auto native = [](const MatView& v) {
     return v.k_stride == 1 && (v.row_stride % kChunkElems) == 0 && pitch_fits_lane_offsets(v.row_stride) &&
            (reinterpret_cast<uintptr_t>(v.ptr) & 15) == 0;
   };
-  return native(W) && native(X) && (K % kTileK) == 0 && (M > 128 || streams_gated(M, K));
+  return native(W) && native(X) && (K % kTileK) == 0 && (M > 128 || streams_gated(M, K) || few_gated(M, W.rows / 2, K));
 }
 
 // Y[M, I] = swiglu(X @ W[0:I]^T, X @ W[I:2I]^T). `workspace` ([M, 2 I] bf16) is used only when
-// the fused kernel does not apply (other layouts, ragged K, up to 128 tokens: there the weight read bounds the time and the
-// GEMM kernels for few tokens spread it over more CUs than a gated 128-feature tile), where the
+// the fused kernels do not apply (other layouts, ragged K, 97 to 128 tokens of a small weight), where the
 // projection and the activation run as two kernels with the same result.
 hipError_t det_gemm_swiglu_launch(const MatView& W, const MatView& X, void* Y, int64_t ldy, void* workspace, int M,
                                   int I, int K, hipStream_t stream) {
   if (det_gemm_swiglu_fused_supported(W, X, M, K)) {
     if (streams_gated(M, K)) return det_gemm_stream_gated_launch(W, X, Y, ldy, M, I, K, stream);
+    if (few_gated(M, I, K)) {
+      const int cus = device_cu_count();
+      if (M <= 64) {
+        if (I <= 16 * cus) return launch_gated_few<32, 1, 2, 6>(W, X, Y, ldy, M, I, K, stream);
+        if (I <= 32 * cus) return launch_gated_few<64, 1, 2, 4>(W, X, Y, ldy, M, I, K, stream);
+        if (I <= 48 * cus) return launch_gated_few<96, 1, 1, 7>(W, X, Y, ldy, M, I, K, stream);
+        return launch_gated_few<128, 1, 1, 6>(W, X, Y, ldy, M, I, K, stream);
+      }
+      if (I <= 16 * cus) return launch_gated_few<32, 2, 1, 7>(W, X, Y, ldy, M, I, K, stream);
+      if (I <= 32 * cus) return launch_gated_few<64, 2, 1, 6>(W, X, Y, ldy, M, I, K, stream);
+      if (I <= 48 * cus) return launch_gated_few<96, 2, 1, 5>(W, X, Y, ldy, M, I, K, stream);
+      return launch_gated_few<128, 2, 1, 4>(W, X, Y, ldy, M, I, K, stream);
+    }
     const int64_t t256 = (int64_t)((M + 255) / 256) * ((I + 127) / 128);
     const int64_t t192 = (int64_t)((M + 191) / 192) * ((I + 127) / 128);
     const int64_t t128 = (int64_t)((M + 127) / 128) * ((I + 127) / 128);
