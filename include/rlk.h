@@ -62,7 +62,8 @@ typedef enum rlk_gemm_config {
   RLK_GEMM_CFG_64x160_DEEP = 23,  /* 64 features x 160 tokens; K % 128 == 0 */
   RLK_GEMM_CFG_256x192 = 24,      /* 256 features x 192 tokens; K % 64 == 0 */
   RLK_GEMM_CFG_192x192 = 25,      /* 192 features x 192 tokens, three stages; K % 64 == 0 */
-  RLK_GEMM_CFG_COUNT = 26,
+  RLK_GEMM_CFG_96x64_DEEP = 26,   /* 96 features x 64 tokens, seven stages; K % 128 == 0 */
+  RLK_GEMM_CFG_COUNT = 27,
   /* OR-ed into a configuration: use the register-staged main loop even where the
    * direct-to-LDS ping-pong loop applies. Bit-neutral; exists so tests can
    * compare the two loops. */

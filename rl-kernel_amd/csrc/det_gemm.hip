@@ -170,6 +170,7 @@ using Shape64x64 = TileShape<64, 64, 4, 2>;
 using Shape64x16 = TileShape<64, 16, 4, 1>;
 using Quad128x64 = TileShape<128, 64, 2, 2>;
 using Quad64x160 = TileShape<64, 160, 2, 2>;
+using Quad96x64 = TileShape<96, 64, 2, 2>;
 using Quad64x96 = TileShape<64, 96, 2, 2>;
 using Quad64x32 = TileShape<64, 32, 2, 2>;
 using Quad32x64 = TileShape<32, 64, 2, 2>;
@@ -298,6 +299,8 @@ int pick_det_gemm_config(int M, int N, int K) {
   //   64 x 32: N = 12288 at 17 tokens 22.1 / 17.0 -> 21.6 / 16.9
   //   64 x 96: down at 288 / 384 tokens 74.6 / 60.2, 76.7 / 60.5 (128 x 64) -> 59.0 / 49.1, 59.4 / 51.4; N = 6144 at 192 tokens
   //            29.1 / 23.6 -> 23.3 / 20.2
+  //   96 x 64: N = 24576 at 64 tokens 42.4 / 39.0 (128 x 64) -> 40.3 / 36.1, 12288 at 100 tokens 32.6 / 24.0 -> 29.0 / 23.0, 6144
+  //            at 200 tokens 30.2 / 23.0 -> 24.7 / 19.0, K = 12288 at 256 tokens 92.6 / 62.2 -> 77.0 / 52.0
   //   128 x 64 with the prefetch: down at 512 tokens 76.6 / 65.0 -> 70.1 / 60.7, N = K = 4096 at 512 tokens 27.6 / 24.8 -> 25.0 / 22.6
   //   64 x 160: down at 600 tokens 90.6 / 75.1 (128 x 128) -> 80.2 / 74.1, N = K = 4096 at 600 tokens 32.0 / 28.1 -> 29.3 / 27.6
   if (deep && tile_count(M, N, 32, 32) <= cus) return RLK_GEMM_CFG_32x32_DEEP;
@@ -307,7 +310,13 @@ int pick_det_gemm_config(int M, int N, int K) {
     if (tile_count(M, N, 64, 64) <= cus) return RLK_GEMM_CFG_64x64_DEEP;
   }
   if (deep) {
+    // 160 rows both. 96 x 64 first where its three token tiles hold what two of 96 leave partly empty (N = 6144 at 160 tokens 27.0
+    // / 20.3 as 64 x 96, 24.5 / 18.1 as 96 x 64; with K = 12288 77.9 / 51.6, 70.1 / 46.8); two of its token tiles are the 128 x 64
+    // configuration, which runs as 96 x 64 by the same rule.
+    const bool fits96x64 = tile_count(M, N, 64, 96) <= cus;
+    if (fits96x64 && M > 128 && M <= 192) return RLK_GEMM_CFG_96x64_DEEP;
     if (tile_count(M, N, 96, 64) <= cus) return RLK_GEMM_CFG_64x96_DEEP;
+    if (fits96x64 && (M <= 64 || M > 192)) return RLK_GEMM_CFG_96x64_DEEP;
     if (tile_count(M, N, 64, 128) <= cus) return RLK_GEMM_CFG_128x64_DEEP;
     if (tile_count(M, N, 160, 64) <= cus) return RLK_GEMM_CFG_64x160_DEEP;
     if (tile_count(M, N, 128, 128) <= cus) return RLK_GEMM_CFG_128x128_DEEP;
@@ -437,7 +446,7 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
   // Deep-stage variants need the fast layout and whole stages; otherwise the plain shape
   // computes the same bits.
   if (config == RLK_GEMM_CFG_32x32_DEEP || config == RLK_GEMM_CFG_32x64_DEEP || config == RLK_GEMM_CFG_64x32_DEEP ||
-      config == RLK_GEMM_CFG_64x64_DEEP || config == RLK_GEMM_CFG_64x96_DEEP || config == RLK_GEMM_CFG_64x160_DEEP ||
+      config == RLK_GEMM_CFG_64x64_DEEP || config == RLK_GEMM_CFG_64x96_DEEP || config == RLK_GEMM_CFG_96x64_DEEP || config == RLK_GEMM_CFG_64x160_DEEP ||
       config == RLK_GEMM_CFG_128x64_DEEP || config == RLK_GEMM_CFG_128x128_DEEP) {
     const int ks = config == RLK_GEMM_CFG_32x64_DEEP || config == RLK_GEMM_CFG_64x32_DEEP || config == RLK_GEMM_CFG_64x64_DEEP
                        ? kDeep64
@@ -448,10 +457,15 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
       if (config == RLK_GEMM_CFG_32x64_DEEP) return launch_quad<Quad32x64, kDeep64, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
       if (config == RLK_GEMM_CFG_64x32_DEEP) return launch_quad<Quad64x32, kDeep64, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
       if (config == RLK_GEMM_CFG_64x96_DEEP) return launch_quad<Quad64x96, kDeep128, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
+      // (the prefetching wave loses here: four readers at most)
+      if (config == RLK_GEMM_CFG_96x64_DEEP) return launch_quad<Quad96x64, 1, 7, false>(W, X, C, ldc, M, N, K, out_f32, stream);
       if (config == RLK_GEMM_CFG_64x160_DEEP) return launch_quad<Quad64x160, 1, 5>(W, X, C, ldc, M, N, K, out_f32, stream);
       if (config == RLK_GEMM_CFG_128x64_DEEP) {
-        // Two token tiles only (12288 outputs at 97 ... 128 tokens) gain nothing from HBM and lose from the cache (K = 4096,
+        // 96 x 64 where it gives every CU at most one (12288 outputs at 97 ... 128 tokens, see pick_det_gemm_config). Two token
+        // tiles of 128 x 64 gain nothing from HBM and lose from the cache (K = 4096,
         // 100 tokens: 31.7 / 23.7 us with eight waves, 32.0 / 26.5 with four and the prefetch).
+        if (M <= 2 * Shape128x64::BM && tile_count(M, N, 64, 96) <= device_cu_count())
+          return launch_quad<Quad96x64, 1, 7, false>(W, X, C, ldc, M, N, K, out_f32, stream);
         if (M <= 2 * Shape128x64::BM) return launch_deep<Shape128x64, kDeep128, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
         return out_f32 ? launch_tile<Quad128x64, kLoopQuadPrefetch, true, 1, 6>(W, X, C, ldc, M, N, K, stream)
                        : launch_tile<Quad128x64, kLoopQuadPrefetch, false, 1, 6>(W, X, C, ldc, M, N, K, stream);
@@ -460,7 +474,7 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
       return launch_deep<Shape128x128, kDeep128>(W, X, C, ldc, M, N, K, out_f32, stream);
     }
     config = config == RLK_GEMM_CFG_128x128_DEEP || config == RLK_GEMM_CFG_64x160_DEEP     ? RLK_GEMM_CFG_128x128
-             : config == RLK_GEMM_CFG_128x64_DEEP || config == RLK_GEMM_CFG_64x96_DEEP ? RLK_GEMM_CFG_128x64
+             : config == RLK_GEMM_CFG_128x64_DEEP || config == RLK_GEMM_CFG_64x96_DEEP || config == RLK_GEMM_CFG_96x64_DEEP ? RLK_GEMM_CFG_128x64
                                                                                        : RLK_GEMM_CFG_64x64;
   }
   // The element-wise loader of the generic path keeps eight values per chunk in

@@ -48,6 +48,7 @@ GEMM_CONFIGS = {
     "64x160_deep": 23,
     "256x192": 24,
     "192x192": 25,
+    "96x64_deep": 26,
 }
 # OR-ed into a GEMM or LogP configuration: register-staged main loop (bit-neutral).
 FORCE_STAGED = 0x100
