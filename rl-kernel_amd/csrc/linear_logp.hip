@@ -46,23 +46,10 @@ struct LogpArgs {
   int tiles_m, n_split, group_m;
 };
 
-// LOOP: 0 generic element loader, 1 register-staged 16-byte loads, 2 direct-to-LDS ping-pong.
+// One (token tile, split). LOOP: 0 generic element loader, 1 register-staged 16-byte loads, 2 direct-to-LDS ping-pong.
 template <class S, int LOOP>
-__global__ __launch_bounds__(S::kThreads) void linear_logp_partial_kernel(LogpArgs a) {
+__device__ __forceinline__ void logp_partial_tile(const LogpArgs& a, int m0, int split, char* lds) {
   static_assert(S::BN == kLogpTileCols && S::kRun == 16 && S::WN == 4, "stream layout is pinned");
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-
-  const int total = a.tiles_m * a.n_split;
-  const int id = xcd_compact_id(blockIdx.x, total);
-  const int per_group = a.group_m * a.n_split;
-  const int group = id / per_group;
-  const int first_m = group * a.group_m;
-  const int width = (a.tiles_m - first_m) < a.group_m ? (a.tiles_m - first_m) : a.group_m;
-  const int within = id - group * per_group;
-  const int tile_m = first_m + within % width;
-  const int split = within / width;
-  const int m0 = tile_m * S::BM;
-
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wave_n = wave % S::WN;
@@ -154,6 +141,31 @@ __global__ __launch_bounds__(S::kThreads) void linear_logp_partial_kernel(LogpAr
     a.part[plane + at] = sum;
     a.part[2 * plane + at] = zt;
   }
+}
+
+// ST: the tile of a last row of token tiles that has at most ST::BM tokens left (S where it is not smaller).
+template <class S, class ST, int LOOP>
+__global__ __launch_bounds__(S::kThreads) void linear_logp_partial_kernel(LogpArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+
+  const int total = a.tiles_m * a.n_split;
+  const int id = xcd_compact_id(blockIdx.x, total);
+  const int per_group = a.group_m * a.n_split;
+  const int group = id / per_group;
+  const int first_m = group * a.group_m;
+  const int width = (a.tiles_m - first_m) < a.group_m ? (a.tiles_m - first_m) : a.group_m;
+  const int within = id - group * per_group;
+  const int tile_m = first_m + within % width;
+  const int split = within / width;
+  const int m0 = tile_m * S::BM;
+
+  if constexpr (ST::BM < S::BM) {
+    if (m0 + ST::BM >= a.T) {
+      logp_partial_tile<ST, LOOP>(a, m0, split, lds);
+      return;
+    }
+  }
+  logp_partial_tile<S, LOOP>(a, m0, split, lds);
 }
 
 // Few token tiles: a split of 1024 columns gives the chip only tiles_m * ceil(V / 1024)
@@ -386,18 +398,31 @@ size_t linear_logp_workspace_bytes(int T, int V) {
   return T <= kStreamGroupMaxTokens ? per_split * (1 + kLogpStreams) : per_split;
 }
 
-template <class S, int LOOP>
+template <class S, int LOOP, class ST = S>
 static hipError_t launch_logp(LogpArgs a, hipStream_t stream) {
-  auto kernel = linear_logp_partial_kernel<S, LOOP>;
+  auto kernel = linear_logp_partial_kernel<S, ST, LOOP>;
   constexpr int kMergeBytes = 3 * kLogpStreams * S::BM * (int)sizeof(float);
   constexpr int kLds = S::kLdsBytes > kMergeBytes ? S::kLdsBytes : kMergeBytes;
   static PerDeviceOnce once;
   hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds, once);
   if (err != hipSuccess) return err;
   a.tiles_m = (a.T + S::BM - 1) / S::BM;
-  a.group_m = a.tiles_m < 8 ? a.tiles_m : 8;
+  // Groups of eight token tiles share the weight's panels in an XCD's L2. Up to eleven tiles are one group and 17 or 18 two of
+  // nine: a last group of one to three tiles would read the whole weight again (V = 131072, D = 2048: 2600 tokens 1195 -> 1161
+  // us, 4120: 1932 -> 1758). Beyond, groups of other widths cost as much as they save (21 tiles as three of seven: 2197 -> 2258).
+  a.group_m = a.tiles_m <= 11 ? a.tiles_m : a.tiles_m == 17 || a.tiles_m == 18 ? 9 : 8;
   hipLaunchKernelGGL(kernel, dim3(a.tiles_m * a.n_split), dim3(S::kThreads), kLds, stream, a);
   return hipGetLastError();
+}
+
+// 256-token tiles; a last one with few tokens runs as a tile of its size. With the groups above, us: V = 151936, D = 4096 at
+// 2100 tokens 2179 -> 2051 (with stored logits 2491 -> 2343), 4120: 3812 -> 3775 (4381 -> 4319); V = 131072, D = 2048 at 1030
+// tokens 597 -> 529, 2100: 1046 -> 988; V = 18992, D = 4096 at 1100 tokens 302 -> 271.
+static hipError_t launch_logp_256(const LogpArgs& a, hipStream_t stream) {
+  const int rest = a.T % LogpShape256::BM;
+  if (rest >= 1 && rest <= LogpShape64::BM) return launch_logp<LogpShape256, 2, LogpShape64>(a, stream);
+  if (rest >= 1 && rest <= LogpShape128::BM) return launch_logp<LogpShape256, 2, LogpShape128>(a, stream);
+  return launch_logp<LogpShape256, 2>(a, stream);
 }
 
 // Up to 128 tokens every weight tile is used by one workgroup only: three stages for the
@@ -526,7 +551,7 @@ hipError_t linear_logp_launch(const MatView& H, const MatView& W, const int64_t*
       err = launch_streamgroup<LogpShape256>(a, requested == RLK_LOGP_CFG_AUTO, stream);
       break;
     case RLK_LOGP_CFG_256:
-      err = loop == 2 ? launch_logp<LogpShape256, 2>(a, stream) : launch_logp<LogpShape256, 1>(a, stream);
+      err = loop == 2 ? launch_logp_256(a, stream) : launch_logp<LogpShape256, 1>(a, stream);
       break;
     case RLK_LOGP_CFG_128:
       err = loop == 2   ? launch_logp<LogpShape128, 2>(a, stream)
