@@ -1015,8 +1015,8 @@ def det_gemm_swiglu(a: torch.Tensor, weight: torch.Tensor, out: Optional[torch.T
     """``swiglu(a @ weight[:I].T, a @ weight[I:].T)`` for a packed ``[2 I, K]`` gate/up weight.
 
     Equals ``swiglu_packed_forward(det_gemm_fwd_rhs_transposed(a, weight))`` bit for bit; with
-    contiguous operands, ``K % 64 == 0`` and more than 16 rows the ``[M, 2 I]`` projection is
-    never written (rl_engine/backends/rocm/gemm/swiglu_gemm.py:36-86).
+    contiguous operands, ``K % 128 == 0`` and ``K >= 1024`` the ``[M, 2 I]`` projection is never
+    written, but for 97 to 128 rows of a small weight (rl_engine/backends/rocm/gemm/swiglu_gemm.py:36-86).
     """
     _check_in(a, "A")
     _check_in(weight, "weight")

@@ -4,8 +4,9 @@ Stands in for rl_engine/backends/rocm/gemm/swiglu_gemm.py:36-86 of the reference
 fused path serves decode-sized batches through split-K partials. Here one MFMA tile kernel
 serves every batch above 128 rows (a workgroup owns the gate and the up projection of the
 same 128 features, so the ``[M, 2 I]`` projection is never written), the streaming kernel
-serves up to 16 rows the same way (eight gate and eight up rows per weight panel), and the
-batches between run the GEMM for few tokens and the elementwise kernel. All three orders of
+serves up to 16 rows the same way (eight gate and eight up rows per weight panel), and from
+17 to 128 rows four waves share a narrow tile's weight rows; 97 to 128 rows of a small weight
+run the GEMM and the elementwise kernel. All these orders of
 work give the same bits.
 """
 
