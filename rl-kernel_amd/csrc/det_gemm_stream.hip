@@ -71,61 +71,114 @@ __global__ __launch_bounds__(64 * (MT + 4)) void det_gemm_stream_kernel(MatView 
     x_base[t] = X.ptr + (int64_t)xr * X.row_stride + chunk_elems;
   }
 
-  auto issue_stage = [&](int s) {
-    if (producer < 0) return;
-    char* base = lds + (s % RING) * kStageBytes;
-#pragma unroll
-    for (int j = 0; j < kLoads; ++j) {
-      const int q = (producer >> 1) + 2 * j;  // pair: [0, KT) weights, then KT per token tile
-      const bool is_w = j < kWLoads;
-      const int tile = is_w ? 0 : (q - KT) / KT;
-      const int sub = is_w ? q : (q - KT) % KT;
-      int ks = s * KT + sub;
-      ks = ks < nsub ? ks : nsub - 1;  // past the end: re-fetch the last sub-tile (never consumed)
-      const bf16_bits* row = w_base;
-#pragma unroll
-      for (int t = 0; t < MT; ++t) row = (!is_w && tile == t) ? x_base[t] : row;
-      const global_ptr_t src = (global_ptr_t)(row + ks * kTileK);
-      const lds_ptr_t dst = (lds_ptr_t)(base + (2 * q + half) * 1024);
-      if (WSTREAM && j < kWLoads)
-        __builtin_amdgcn_global_load_lds(src, dst, 16, 0, kLoadNonTemporal);
-      else
-        __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
-    }
+  // Load j of this producer for a stage: its half of the pair (producer >> 1) + 2 j.
+  auto load = [&](int j, const bf16_bits* src, int slot) {
+    const lds_ptr_t dst = (lds_ptr_t)(lds + slot + (2 * ((producer >> 1) + 2 * j) + half) * 1024);
+    if (WSTREAM && j < kWLoads)
+      __builtin_amdgcn_global_load_lds((global_ptr_t)src, dst, 16, 0, kLoadNonTemporal);
+    else
+      __builtin_amdgcn_global_load_lds((global_ptr_t)src, dst, 16, 0, 0);
   };
-
+  auto next_slot = [](int slot) { return slot == (RING - 1) * kStageBytes ? 0 : slot + kStageBytes; };
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   const int l16 = lane & 15;
   const int grp = lane >> 4;
   const int frag_lo = l16 * kRowBytes + ((grp ^ (l16 & 7)) << 4);  // K step 0 of a sub-tile
   const int frag_hi = frag_lo ^ 64;                                 // K step 1
 
+  // Both kinds of waves meet at one barrier per stage and do little else there. With the stage's fragments read in front of
+  // their MFMAs, and the refills' clamps and addresses in every stage, one took 0.18 us, which is what bounds panels that HBM
+  // does not; now about 0.1. Weights from HBM, us, K -> outputs: 4096 -> 1536 at one token 7.8 -> 5.2, 6144 -> 2048 10.7 -> 8.3,
+  // 1024 -> 4096 4.5 -> 4.0, 4096 -> 6144 13.0 -> 12.2, 4096 -> 24576 at 1 / 16 tokens 35.7 / 40.8 -> 33.8 / 38.0.
+  if (wave >= MT) {
+    // Stage t, of which the sub-tiles behind the reduction's end fetch the last one again (never consumed). Behind the last
+    // stage one lane of each load goes on, for the counts that the wait relies on (whole loads there took the CU's load path
+    // from its next workgroup: 4096 -> 24576 at 16 tokens 39.7 us, with one lane 38.0; no loads and a wait by the number of
+    // stages left cost more in the short panels).
+    auto issue_last = [&](int t, int slot) {
+      if (t >= nstage && lane != 0) return;
 #pragma unroll
-  for (int s = 0; s < RING - 1; ++s) issue_stage(s);
-  for (int s = 0; s < nstage; ++s) {
-    __builtin_amdgcn_s_waitcnt(wait_vmcnt((RING - 2) * kLoads));  // my loads of stage s have landed
-    wg_barrier();  // stage s is complete; the consumers are done with stage s - 1
-    issue_stage(s + RING - 1);
-    if (wave < MT) {
-      const char* base = lds + (s % RING) * kStageBytes;
-      const int remaining = nsub - s * KT;
-      const int count = remaining < KT ? remaining : KT;
-      u32x4_t wf[2 * KT], xf[2 * KT];
+      for (int j = 0; j < kLoads; ++j) {
+        const int q = (producer >> 1) + 2 * j;  // pair: [0, KT) weights, then KT per token tile
+        const int ks = t * KT + q % KT;
+        load(j, (j < kWLoads ? w_base : x_base[(2 * j - KT) / KT]) + (ks < nsub ? ks : nsub - 1) * kTileK, slot);
+      }
+    };
+    auto step = [&] {
+      __builtin_amdgcn_s_waitcnt(wait_vmcnt((RING - 2) * kLoads));  // my loads of stage s have landed
+      wg_barrier();  // stage s is complete; the consumers hold the fragments of stage s - 1
+    };
+    int64_t k = (producer >> 1) * kTileK;
+    int slot = 0;
+    auto issue_whole = [&] {  // the next stage, all of it inside the reduction
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j)
+        load(j, (j < kWLoads ? w_base : x_base[(2 * j - KT) / KT]) + k + 2 * j % KT * kTileK, slot);
+      k += KT * kTileK;
+      slot = next_slot(slot);
+    };
+    const int whole = nsub / KT - (RING - 1);  // stages of the loop whose refill is a whole one
+    if (whole >= 0) {
+#pragma unroll
+      for (int t = 0; t < RING - 1; ++t) issue_whole();
+    } else {
+#pragma nounroll
+      for (int t = 0; t < RING - 1; ++t) {
+        issue_last(t, slot);
+        slot = next_slot(slot);
+      }
+    }
+    int s = 0;
+    for (; s < whole; ++s) {
+      step();
+      issue_whole();
+    }
+    for (; s < nstage; ++s) {
+      step();
+      issue_last(s + RING - 1, slot);
+      slot = next_slot(slot);
+    }
+  } else {
+    // The fragments of stage s are read under the MFMAs of stage s - 1.
+    struct Fragments {
+      u32x4_t w[2 * KT], x[2 * KT];
+    };
+    auto multiply = [&](const Fragments& f, int steps) {
+#pragma unroll
+      for (int i = 0; i < 2 * KT; ++i)
+        if (i < steps) acc = mfma_16x16x32(f.w[i], f.x[i], acc);
+    };
+    int slot = 0;
+    auto stage = [&](Fragments& next, const Fragments& now) {
+      wg_barrier();
+      const char* base = lds + slot;
 #pragma unroll
       for (int sub = 0; sub < KT; ++sub) {
         const char* wt = base + sub * kSubBytes;
         const char* xt = base + (KT + wave * KT + sub) * kSubBytes;
-        wf[2 * sub] = *reinterpret_cast<const u32x4_t*>(wt + frag_lo);
-        xf[2 * sub] = *reinterpret_cast<const u32x4_t*>(xt + frag_lo);
-        wf[2 * sub + 1] = *reinterpret_cast<const u32x4_t*>(wt + frag_hi);
-        xf[2 * sub + 1] = *reinterpret_cast<const u32x4_t*>(xt + frag_hi);
+        next.w[2 * sub] = *reinterpret_cast<const u32x4_t*>(wt + frag_lo);
+        next.x[2 * sub] = *reinterpret_cast<const u32x4_t*>(xt + frag_lo);
+        next.w[2 * sub + 1] = *reinterpret_cast<const u32x4_t*>(wt + frag_hi);
+        next.x[2 * sub + 1] = *reinterpret_cast<const u32x4_t*>(xt + frag_hi);
       }
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(now, 2 * KT);
+      __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < 2 * KT; ++i)
-        if (i < 2 * count) acc = mfma_16x16x32(wf[i], xf[i], acc);
-      __builtin_amdgcn_sched_barrier(0);
+      slot = next_slot(slot);
+    };
+    Fragments even, odd = {};  // (the first stage multiplies zeros: the accumulator stays +0)
+    int s = 0;
+    for (; s + 1 < nstage; s += 2) {
+      stage(even, odd);
+      stage(odd, even);
+    }
+    const int last_steps = 2 * (nsub - (nstage - 1) * KT);
+    if (s < nstage) {
+      stage(even, odd);
+      multiply(even, last_steps);
+    } else {
+      multiply(odd, last_steps);
     }
   }
   __builtin_amdgcn_s_waitcnt(kWaitAll0);
