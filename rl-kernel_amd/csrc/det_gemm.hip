@@ -311,12 +311,11 @@ int pick_det_gemm_config(int M, int N, int K) {
   }
   if (deep) {
     // 160 rows both. 96 x 64 first where its three token tiles hold what two of 96 leave partly empty (N = 6144 at 160 tokens 27.0
-    // / 20.3 as 64 x 96, 24.5 / 18.1 as 96 x 64; with K = 12288 77.9 / 51.6, 70.1 / 46.8); two of its token tiles are the 128 x 64
-    // configuration, which runs as 96 x 64 by the same rule.
+    // / 20.3 as 64 x 96, 24.5 / 18.1 as 96 x 64; with K = 12288 77.9 / 51.6, 70.1 / 46.8).
     const bool fits96x64 = tile_count(M, N, 64, 96) <= cus;
     if (fits96x64 && M > 128 && M <= 192) return RLK_GEMM_CFG_96x64_DEEP;
     if (tile_count(M, N, 96, 64) <= cus) return RLK_GEMM_CFG_64x96_DEEP;
-    if (fits96x64 && (M <= 64 || M > 192)) return RLK_GEMM_CFG_96x64_DEEP;
+    if (fits96x64) return RLK_GEMM_CFG_96x64_DEEP;
     if (tile_count(M, N, 64, 128) <= cus) return RLK_GEMM_CFG_128x64_DEEP;
     if (tile_count(M, N, 160, 64) <= cus) return RLK_GEMM_CFG_64x160_DEEP;
     if (tile_count(M, N, 128, 128) <= cus) return RLK_GEMM_CFG_128x128_DEEP;
@@ -461,11 +460,8 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
       if (config == RLK_GEMM_CFG_96x64_DEEP) return launch_quad<Quad96x64, 1, 7, false>(W, X, C, ldc, M, N, K, out_f32, stream);
       if (config == RLK_GEMM_CFG_64x160_DEEP) return launch_quad<Quad64x160, 1, 5>(W, X, C, ldc, M, N, K, out_f32, stream);
       if (config == RLK_GEMM_CFG_128x64_DEEP) {
-        // 96 x 64 where it gives every CU at most one (12288 outputs at 97 ... 128 tokens, see pick_det_gemm_config). Two token
-        // tiles of 128 x 64 gain nothing from HBM and lose from the cache (K = 4096,
-        // 100 tokens: 31.7 / 23.7 us with eight waves, 32.0 / 26.5 with four and the prefetch).
-        if (M <= 2 * Shape128x64::BM && tile_count(M, N, 64, 96) <= device_cu_count())
-          return launch_quad<Quad96x64, 1, 7, false>(W, X, C, ldc, M, N, K, out_f32, stream);
+        // Four waves gain nothing from HBM with two token tiles and lose from the cache (12288 outputs, K = 4096, 100 tokens:
+        // 31.7 / 23.7 us with eight waves, 32.0 / 26.5 with four and the prefetch).
         if (M <= 2 * Shape128x64::BM) return launch_deep<Shape128x64, kDeep128, 3>(W, X, C, ldc, M, N, K, out_f32, stream);
         return out_f32 ? launch_tile<Quad128x64, kLoopQuadPrefetch, true, 1, 6>(W, X, C, ldc, M, N, K, stream)
                        : launch_tile<Quad128x64, kLoopQuadPrefetch, false, 1, 6>(W, X, C, ldc, M, N, K, stream);

@@ -47,7 +47,8 @@ def test_same_bits_as_the_one_wave_tile(config, stage, tokens, features):
      ("64x96_deep", 140, 8190, 1152), ("64x96_deep", 90, 12288, 4096), ("64x96_deep", 333, 4096, 12288), ("64x96_deep", 150, 8190, 1152),
      ("64x160_deep", 150, 12288, 2048), ("64x160_deep", 150, 12288, 4096), ("64x160_deep", 129, 12346, 4224),
      ("64x160_deep", 600, 4096, 4096), ("64x160_deep", 651, 3250, 4224),
-     ("128x64_deep", 500, 4096, 4096), ("128x64_deep", 120, 12288, 4096)],
+     ("128x64_deep", 500, 4096, 4096), ("128x64_deep", 120, 14336, 4096), ("128x64_deep", 97, 16380, 1152),
+     ("96x64_deep", 120, 12288, 4096)],
 )  # fmt: skip
 def test_chosen_shapes(config, tokens, features, k):
     from rl_engine import _C, _lib

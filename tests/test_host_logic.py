@@ -71,6 +71,20 @@ def test_config_pick_is_deterministic_and_in_range(rlk_lib):
     assert rlk_lib.rlk_det_gemm_pick_config(4096, 24576, 4096) == _lib.GEMM_CONFIGS["256x256"]
 
 
+# where 96 x 64 gives every one of 256 CUs at most one tile, from 17 to 256 tokens, and just beyond; all of them with a whole
+# number of stages
+@pytest.mark.parametrize(
+    "m,n,k,name",
+    [(64, 24576, 4096, "96x64_deep"), (65, 24576, 4096, "128x128_deep"), (80, 12288, 4096, "64x96_deep"), (97, 12288, 4096, "96x64_deep"),
+     (120, 12288, 4096, "96x64_deep"), (128, 12288, 1152, "96x64_deep"), (120, 12289, 4096, "128x64_deep"),
+     (120, 14336, 4096, "128x64_deep"), (160, 6144, 4096, "96x64_deep"), (256, 6144, 4096, "96x64_deep")],
+)  # fmt: skip
+def test_the_pick_names_the_few_token_tile_that_runs(rlk_lib, m, n, k, name):
+    from rl_engine import _lib
+
+    assert rlk_lib.rlk_det_gemm_pick_config(m, n, k) == _lib.GEMM_CONFIGS[name]
+
+
 def test_argument_errors_are_reported_without_touching_the_gpu(rlk_lib):
     # Invalid arguments are rejected before any HIP call, so this runs on a CPU-only host.
     rc = rlk_lib.rlk_det_gemm_bf16(None, 4, 1, None, 1, 4, None, 4, -1, 4, 4, 0, 0, None)
