@@ -473,8 +473,11 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
              : config == RLK_GEMM_CFG_128x64_DEEP || config == RLK_GEMM_CFG_64x96_DEEP || config == RLK_GEMM_CFG_96x64_DEEP ? RLK_GEMM_CFG_128x64
                                                                                        : RLK_GEMM_CFG_64x64;
   }
-  // The element-wise loader of the generic path keeps eight values per chunk in
-  // flight; the largest shapes would spill registers with it.
+  // The element-wise loader keeps eight values per chunk in flight, and a picked 256-feature tile gives way to 128 x 128, which
+  // holds them without spilling. The 192-feature and 192-token tiles, which have no such loader, become 256-feature tiles
+  // behind this line and keep them: spilled registers (98 of 256 x 256) cost less there than twice the loads. Odd pitch, as
+  // the large tile / as 128 x 128, us: 4096 outputs at 2817 tokens, K = 4096 604 / 829, 14336 at 3456 2459 / 3285, 24576 at 300
+  // 565 / 779, 6144 at 768 (192 x 128) 295 / 567; K = 128: 36.5 / 35.4, 64: 26.5 / 25.2.
   if (!vec && (config == RLK_GEMM_CFG_256x256 || config == RLK_GEMM_CFG_256x128 || config == RLK_GEMM_CFG_256x64))
     config = RLK_GEMM_CFG_128x128;
   if (config == RLK_GEMM_CFG_256x256_SOLO) {
