@@ -115,8 +115,15 @@ typedef enum rlk_linear_bwd_config {
   RLK_LINEAR_BWD_CFG_128x128_256x256 = 6,
   RLK_LINEAR_BWD_CFG_64x64_256x256 = 7,
   RLK_LINEAR_BWD_CFG_256x192_256x256 = 8,
-  RLK_LINEAR_BWD_CFG_COUNT = 9
+  RLK_LINEAR_BWD_CFG_COUNT = 9,
+  /* OR-ed into a one-launch configuration: the whole multiples of 256 tokens of dx in a launch of their own first, its
+   * other tokens (tokens % 256) in the one launch beside dw. */
+  RLK_LINEAR_BWD_CFG_REST_BESIDE = 0x100
 } rlk_linear_bwd_config;
+
+/* The configuration RLK_LINEAR_BWD_CFG_AUTO resolves to for contiguous operands of a shape, or, with logp != 0, the one that
+ * the fused linear-LogP backward runs both its gradients in (tokens x hidden size x vocabulary); host only, no GPU call. */
+int rlk_linear_bwd_pick_config(int tokens, int inputs, int outputs, int logp);
 
 /*
  * Both gradients of y = x @ w^T:

@@ -244,10 +244,10 @@ static const TileCandidate kTileCandidates[] = {
 };
 
 // The cheapest candidate by the estimate above. `w_kmajor` / `x_kmajor`: the operand layouts of the call.
-static int pick_tile_candidate(int M, int N, int K, bool w_kmajor, bool x_kmajor, double partial_floor = 0.9,
-                               double* estimate = nullptr) {
+static const TileCandidate& best_tile_candidate(int M, int N, int K, bool w_kmajor, bool x_kmajor, double partial_floor,
+                                                double* estimate) {
   const int cus = device_cu_count();
-  int best = RLK_GEMM_CFG_64x64;
+  const TileCandidate* best = kTileCandidates;
   double best_time = 1e300;
   for (const TileCandidate& c : kTileCandidates) {
     double quality;
@@ -263,16 +263,22 @@ static int pick_tile_candidate(int M, int N, int K, bool w_kmajor, bool x_kmajor
     const double t = rounds_of_workgroups(tile_count(M, N, c.bm, c.bn), cus, partial_floor) * (double)(c.bn * c.bm) / quality;
     if (t < best_time * 0.999) {
       best_time = t;
-      best = c.config;
+      best = &c;
     }
   }
-  if (estimate) *estimate = best_time;
-  return best;
+  *estimate = best_time;
+  return *best;
 }
 
-double det_gemm_kmajor_us(int M, int N, int K, bool w_kmajor, bool x_kmajor, double partial_floor) {
+static int pick_tile_candidate(int M, int N, int K, bool w_kmajor, bool x_kmajor) {
+  double estimate;
+  return best_tile_candidate(M, N, K, w_kmajor, x_kmajor, 0.9, &estimate).config;
+}
+
+double det_gemm_kmajor_us(int M, int N, int K, bool w_kmajor, bool x_kmajor, double partial_floor, int* tile_outputs) {
   double outputs;  // of 256 x 256 tiles at the native rate, 11 + 21 K / 1024 us each (see remainder_launch_pays)
-  pick_tile_candidate(M, N, K, w_kmajor, x_kmajor, partial_floor, &outputs);
+  const TileCandidate& tile = best_tile_candidate(M, N, K, w_kmajor, x_kmajor, partial_floor, &outputs);
+  if (tile_outputs) *tile_outputs = tile.bn * tile.bm;
   return (11.0 + 21.0 * K / 1024.0) * outputs / 65536.0;
 }
 

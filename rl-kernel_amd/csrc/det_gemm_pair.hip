@@ -134,8 +134,16 @@ static int64_t tile_count(const GemmProblem& p, int bn, int bm) { return (int64_
 // much of the chip idle. A tile takes 0.6 of its time alone (256 x 256, K = 4096: 95 -> 65 us, 256 x 128: 68 -> 48.5), the
 // whole of it on a full chip and wherever its weight comes at the HBM latency (256 x 256 at K = 37984 / 151936: 790 / 3127
 // -> 740 / 2900).
-static double pair_us(const GemmProblem& dx, const GemmProblem& dw, const PairTiles& t, int cus) {
-  const double tx = dx_tile_us(t, dx), tw = dw_tile_us(t, dw);
+// Up to kFewTokens a weight from HBM keeps the small tiles of dX waiting, and the dW tiles beside them run at 0.7 of their
+// time: 37984 outputs, 4096 inputs, 128 x 128 tiles of dX, us at 520 / 688 / 784 / 1024 tokens: 429 / 484 / 548 / 641, by this
+// estimate 447 / 486 / 554 / 643, with the whole time 472 / 563 / 645 / 741. (Not beside the rest of a dX whose whole tiles
+// ran before: too few tiles of it.) Right behind the LogP forward part of a weight of up to 180 MiB still lies in the
+// memory-side cache: 18992 outputs at 400 / 512 tokens 170 / 174 us, by this estimate 208, 227 from HBM.
+constexpr int kFewTokens = 1024;
+static double pair_us(const GemmProblem& dx, const GemmProblem& dw, const PairTiles& t, int cus, bool logp) {
+  const bool waiting = t.dx_bn < 256 && weight_from_hbm(dx) && dw.K <= kFewTokens && dx.M == dw.K;
+  const bool partly_cached = waiting && logp && (int64_t)dx.N * dx.K * 2 < ((int64_t)180 << 20);
+  const double tx = dx_tile_us(t, dx) * (partly_cached ? 0.92 : 1.0), tw = dw_tile_us(t, dw) * (waiting ? 0.7 : 1.0);
   const int64_t nx = tile_count(dx, t.dx_bn, t.dx_bm), nw = tile_count(dw, t.dw_bn, t.dw_bm);
   const double work = (nx * tx + nw * tw) / cus;
   const double span = tx >= tw ? pair_span(nx, tx, nw, tw, cus) : pair_span(nw, tw, nx, tx, cus);
@@ -149,10 +157,10 @@ static bool one_launch_serves(const GemmProblem& dx, const GemmProblem& dw) {
          det_gemm_takes_kmajor(dx.W, dx.X, dx.K) && det_gemm_takes_kmajor(dw.W, dw.X, dw.K);
 }
 
-static double best_pair_us(const GemmProblem& dx, const GemmProblem& dw, int cus, int* config) {
+static double best_pair_us(const GemmProblem& dx, const GemmProblem& dw, int cus, bool logp, int* config) {
   double best = 1e300;
   for (int c = RLK_LINEAR_BWD_CFG_SEPARATE + 1; c < RLK_LINEAR_BWD_CFG_COUNT; ++c) {
-    const double us = pair_us(dx, dw, kPairTiles[c], cus);
+    const double us = pair_us(dx, dw, kPairTiles[c], cus, logp);
     if (us < best) {
       best = us;
       *config = c;
@@ -184,16 +192,32 @@ static GemmProblem tail_of(GemmProblem dx, int rows) {
 // 199 as two, 160 as one).
 // A token count just above a multiple of 256 (see remainder_launch_pays): the whole tiles of dX first, then the few tokens
 // behind them beside dW.
-LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem& dw) {
+//
+// The LogP's own two launches take less than the estimate up to kFewTokens where the weight comes from HBM: dX in 128 x 64
+// tiles 0.84 of it (priced at 0.93), dW of whole K tiles, with a native feature operand from 512 tokens on, 0.82 to 0.93.
+// Gradients right behind the forward, us, two launches / as chosen before these two, the 0.7 and the 0.92 above / now (tokens,
+// inputs, outputs):
+//   512, 4096, 37984: 416 / 439 / 416      304, 5120, 32000: 347 / 387 / 347      400, 4096, 18992: 210 / 210 / 170
+//   768, 4096, 37984: 530 / 557 / 499      600, 5120, 32000: 497 / 530 / 476      768, 4096, 18992: 266 / 266 / 235
+//   768, 5120, 32000: 520 / 546 / 546      800, 4096, 64000: 982 / 932 / 959      520, 4096, 16384: 215 / 172 / 172
+// 396 measured forms of 12 layers take 0.920 of the two launches' time (0.935), and are up to 5 % slower than them (13).
+constexpr double kFewTokensDx = 0.93, kFewTokensDw = 0.92;
+LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem& dw, bool logp) {
   LinearBackwardPlan plan{RLK_LINEAR_BWD_CFG_SEPARATE, 0};
   if (!one_launch_serves(dx, dw)) return plan;
   if (weight_from_hbm(dx) && det_gemm_shortk_supported(dw.W, dw.X, dw.M, dw.N, dw.K) && det_gemm_shortk_pays(dw.M, dw.N)) return plan;
   const int cus = device_cu_count();
   const double partial = weight_from_hbm(dx) ? 1.0 : 0.9;
-  double best = 0.98 * (det_gemm_kmajor_us(dx.M, dx.N, dx.K, true, false, partial) +
-                        det_gemm_kmajor_us(dw.M, dw.N, dw.K, true, true, partial) + kLaunchUs);
+  int dx_outputs;
+  double us_dx = det_gemm_kmajor_us(dx.M, dx.N, dx.K, true, false, partial, &dx_outputs);
+  double us_dw = det_gemm_kmajor_us(dw.M, dw.N, dw.K, true, true, partial);
+  if (logp && weight_from_hbm(dx) && dx.M <= kFewTokens) {
+    if (dx_outputs == 128 * 64) us_dx *= kFewTokensDx;
+    if (dx.M % kTileK == 0) us_dw *= kFewTokensDw;
+  }
+  double best = 0.98 * (us_dx + us_dw + kLaunchUs);
   int config;
-  const double together = best_pair_us(dx, dw, cus, &config);
+  const double together = best_pair_us(dx, dw, cus, logp, &config);
   if (together < best) {
     best = together;
     plan.config = config;
@@ -202,14 +226,14 @@ LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem
   if (dx.M > 256 && rest >= 1 && rest <= 64) {
     const int whole = dx.M - rest;
     const double head = det_gemm_kmajor_us(whole, dx.N, dx.K, true, false, partial);
-    const double with_rest = head + kLaunchUs + best_pair_us(tail_of(dx, whole), dw, cus, &config);
+    const double with_rest = head + kLaunchUs + best_pair_us(tail_of(dx, whole), dw, cus, logp, &config);
     if (with_rest < best) plan = {config, whole};
   }
   return plan;
 }
 
 hipError_t linear_backward_launch(GemmProblem dx, const GemmProblem& dw, LinearBackwardPlan plan, hipStream_t stream) {
-  if (plan.config != RLK_LINEAR_BWD_CFG_SEPARATE && !one_launch_serves(dx, dw)) plan = {RLK_LINEAR_BWD_CFG_SEPARATE, 0};
+  if (!one_launch_serves(dx, dw)) plan = {RLK_LINEAR_BWD_CFG_SEPARATE, 0};
   if (plan.head_rows > 0) {
     const GemmProblem head = head_of(dx, plan.head_rows);
     const hipError_t err = det_gemm_launch(head.W, head.X, head.C, head.ldc, head.M, head.N, head.K, false, RLK_GEMM_CFG_AUTO, stream);

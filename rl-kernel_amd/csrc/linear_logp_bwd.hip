@@ -379,6 +379,29 @@ __global__ __launch_bounds__(256) void transpose_bf16_kernel(const bf16_bits* __
   }
 }
 
+// dz rows are zero from V to their end (a multiple of 64), so the gradients read them in whole chunks at any V: the
+// transposed operand shows up to seven rows more than are stored, the reduction ends in a chunk padded with zeros. (The
+// element-wise loader at V = 50257, D = 2048: grad_weight / grad_hidden at 1000 tokens 1781 / 4037 us, now 224 / 297;
+// at 80 tokens 257 / 1763, now 80 / 230.)
+// grad_hidden[t, d] = sum over v ascending of dz[t, v] * W[v, d], grad_weight[v, d] = sum over t ascending of dz[t, v] * H[t, d]
+static GemmProblem hidden_gradient(const MatView& W, const bf16_bits* dz, void* grad_hidden, int64_t ld, int T, int D, int V) {
+  const MatView dz_by_token{dz, linear_logp_dz_row_stride(V), 1, T, true};
+  const MatView w_by_feature{W.ptr, 1, W.row_stride, D};  // rows = d, reduction index = v
+  return {w_by_feature, dz_by_token, grad_hidden, ld, T, D, V};
+}
+static GemmProblem weight_gradient(const MatView& H, const bf16_bits* dz, void* grad_weight, int64_t ld, int T, int D, int V) {
+  const int v_chunks = (V + kChunkElems - 1) / kChunkElems * kChunkElems;
+  const MatView dz_by_column{dz, 1, linear_logp_dz_row_stride(V), v_chunks};  // rows = v, reduction index = t
+  const MatView h_by_feature{H.ptr, 1, H.row_stride, D};                      // rows = d, reduction index = t
+  return {h_by_feature, dz_by_column, grad_weight, ld, V, D, T};
+}
+
+LinearBackwardPlan linear_logp_bwd_plan(int T, int D, int V) {
+  const bf16_bits* any = reinterpret_cast<const bf16_bits*>(uintptr_t{256});  // its alignment is all that is looked at
+  const MatView W{any, D, 1, V}, H{any, D, 1, T};
+  return linear_backward_plan(hidden_gradient(W, any, nullptr, D, T, D, V), weight_gradient(H, any, nullptr, D, T, D, V), true);
+}
+
 hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int64_t* target, const float* bias,
                                   const float* temperature, const float* lse, const float* logits,
                                   int64_t logits_ld, const float* grad_logp, const float* grad_lse, void* grad_hidden, int64_t gh_row_stride, void* grad_weight,
@@ -453,20 +476,11 @@ hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int6
   }
   if (err != hipSuccess) return err;
 
-  // dz rows are zero from V to their end (a multiple of 64), so the gradients read them in whole chunks at any V: the
-  // transposed operand shows up to seven rows more than are stored, the reduction ends in a chunk padded with zeros. (The
-  // element-wise loader at V = 50257, D = 2048: grad_weight / grad_hidden at 1000 tokens 1781 / 4037 us, now 224 / 297;
-  // at 80 tokens 257 / 1763, now 80 / 230.)
-  const int v_chunks = (V + kChunkElems - 1) / kChunkElems * kChunkElems;
   const int gemm_config = force_staged ? (RLK_GEMM_CFG_AUTO | RLK_GEMM_CFG_FORCE_STAGED) : RLK_GEMM_CFG_AUTO;
-  const MatView dz_by_column{a.dz, 1, a.ld_dz, v_chunks};  // rows = v, reduction index = t
-  const MatView dz_by_token{a.dz, a.ld_dz, 1, T, true};
-  const MatView w_by_feature{W.ptr, 1, W.row_stride, D};  // rows = d, reduction index = v
-  const MatView h_by_feature{H.ptr, 1, H.row_stride, D};  // rows = d, reduction index = t
-  const GemmProblem to_hidden{w_by_feature, dz_by_token, grad_hidden, gh_row_stride, T, D, V};
-  const GemmProblem to_weight{h_by_feature, dz_by_column, grad_weight, gw_row_stride, V, D, T};
+  const GemmProblem to_hidden = hidden_gradient(W, a.dz, grad_hidden, gh_row_stride, T, D, V);
+  const GemmProblem to_weight = weight_gradient(H, a.dz, grad_weight, gw_row_stride, T, D, V);
   const LinearBackwardPlan plan = grad_hidden && grad_weight && !force_staged
-                                      ? linear_backward_plan(to_hidden, to_weight)
+                                      ? linear_backward_plan(to_hidden, to_weight, true)
                                       : LinearBackwardPlan{RLK_LINEAR_BWD_CFG_SEPARATE, 0};
   if (plan.config != RLK_LINEAR_BWD_CFG_SEPARATE) {
     err = linear_backward_launch(to_hidden, to_weight, plan, stream);
@@ -474,7 +488,6 @@ hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int6
     grad_hidden = grad_weight = nullptr;  // done
   }
   if (grad_weight) {
-    // grad_weight[v, d] = sum over t ascending of dz[t, v] * H[t, d]
     // Both operands are K-major as they lie. From 512 tokens on the hidden states are transposed first (into the
     // grad_hidden buffer, which has exactly their size and is written only afterwards), so that the feature operand
     // runs the plain ping-pong loads: lm_head at 8192 tokens 8.32 -> 7.79 ms plus 0.04 ms for the transposition.
@@ -489,15 +502,14 @@ hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int6
       err = hipGetLastError();
       if (err != hipSuccess) return err;
       const MatView h_rows{hidden_t, T, 1, D};  // rows = d, reduction index = t contiguous
-      err = det_gemm_launch(h_rows, dz_by_column, grad_weight, gw_row_stride, V, D, T, false, gemm_config, stream);
+      err = det_gemm_launch(h_rows, to_weight.X, grad_weight, gw_row_stride, V, D, T, false, gemm_config, stream);
     } else {
-      err = det_gemm_launch(h_by_feature, dz_by_column, grad_weight, gw_row_stride, V, D, T, false, gemm_config, stream);
+      err = det_gemm_launch(to_weight.W, to_weight.X, grad_weight, gw_row_stride, V, D, T, false, gemm_config, stream);
     }
     if (err != hipSuccess) return err;
   }
   if (grad_hidden) {
-    // grad_hidden[t, d] = sum over v ascending of dz[t, v] * W[v, d]
-    err = det_gemm_launch(w_by_feature, dz_by_token, grad_hidden, gh_row_stride, T, D, V, false, gemm_config, stream);
+    err = det_gemm_launch(to_hidden.W, to_hidden.X, grad_hidden, gh_row_stride, T, D, V, false, gemm_config, stream);
     if (err != hipSuccess) return err;
   }
   if (grad_bias) {

@@ -113,6 +113,33 @@ int rlk_det_gemm_bf16(const void* a, int64_t a_row_stride, int64_t a_k_stride, c
   return err == hipSuccess ? RLK_OK : device_error("rlk_det_gemm_bf16", err);
 }
 
+static GemmProblem linear_dx(const void* dy, int64_t dy_ld, const void* w, int64_t w_ld, void* dx, int64_t dx_ld, int tokens,
+                             int inputs, int outputs) {
+  return {{reinterpret_cast<const bf16_bits*>(w), 1, w_ld, inputs}, {reinterpret_cast<const bf16_bits*>(dy), dy_ld, 1, tokens},
+          dx, dx_ld, tokens, inputs, outputs};
+}
+static GemmProblem linear_dw(const void* dy, int64_t dy_ld, const void* x, int64_t x_ld, void* dw, int64_t dw_ld, int tokens,
+                             int inputs, int outputs) {
+  return {{reinterpret_cast<const bf16_bits*>(x), 1, x_ld, inputs}, {reinterpret_cast<const bf16_bits*>(dy), 1, dy_ld, outputs},
+          dw, dw_ld, outputs, inputs, tokens};
+}
+
+int rlk_linear_bwd_pick_config(int tokens, int inputs, int outputs, int logp) {
+  if (tokens < 1 || inputs < 1 || outputs < 1) {
+    set_last_error("rlk_linear_bwd_pick_config: tokens=%d inputs=%d outputs=%d must be positive", tokens, inputs, outputs);
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  LinearBackwardPlan plan;
+  if (logp) {
+    plan = linear_logp_bwd_plan(tokens, inputs, outputs);
+  } else {
+    const void* any = reinterpret_cast<const void*>(uintptr_t{256});  // its alignment is all that is looked at
+    plan = linear_backward_plan(linear_dx(any, outputs, any, inputs, nullptr, inputs, tokens, inputs, outputs),
+                                linear_dw(any, outputs, any, inputs, nullptr, inputs, tokens, inputs, outputs), false);
+  }
+  return plan.config | (plan.head_rows > 0 ? RLK_LINEAR_BWD_CFG_REST_BESIDE : 0);
+}
+
 int rlk_linear_bwd_bf16(const void* dy, int64_t dy_row_stride, const void* x, int64_t x_row_stride, const void* w,
                         int64_t w_row_stride, void* dx, int64_t dx_row_stride, void* dw, int64_t dw_row_stride, int tokens,
                         int inputs, int outputs, int config, void* stream) {
@@ -120,7 +147,9 @@ int rlk_linear_bwd_bf16(const void* dy, int64_t dy_row_stride, const void* x, in
     set_last_error("rlk_linear_bwd_bf16: tokens=%d inputs=%d outputs=%d must be positive", tokens, inputs, outputs);
     return RLK_ERR_INVALID_ARGUMENT;
   }
-  if (config < 0 || config >= RLK_LINEAR_BWD_CFG_COUNT) {
+  const int rest_beside = config & RLK_LINEAR_BWD_CFG_REST_BESIDE;
+  if (config < 0 || (config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE) >= RLK_LINEAR_BWD_CFG_COUNT ||
+      (rest_beside && (config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE) <= RLK_LINEAR_BWD_CFG_SEPARATE)) {
     set_last_error("rlk_linear_bwd_bf16: unknown config %d", config);
     return RLK_ERR_INVALID_ARGUMENT;
   }
@@ -132,13 +161,13 @@ int rlk_linear_bwd_bf16(const void* dy, int64_t dy_row_stride, const void* x, in
     set_last_error("rlk_linear_bwd_bf16: row strides must not be negative, those of dx and dw not below %d", inputs);
     return RLK_ERR_INVALID_ARGUMENT;
   }
-  const bf16_bits* g = reinterpret_cast<const bf16_bits*>(dy);
-  const GemmProblem to_dx{{reinterpret_cast<const bf16_bits*>(w), 1, w_row_stride, inputs}, {g, dy_row_stride, 1, tokens},
-                          dx, dx_row_stride, tokens, inputs, outputs};
-  const GemmProblem to_dw{{reinterpret_cast<const bf16_bits*>(x), 1, x_row_stride, inputs}, {g, 1, dy_row_stride, outputs},
-                          dw, dw_row_stride, outputs, inputs, tokens};
-  const LinearBackwardPlan plan =
-      config == RLK_LINEAR_BWD_CFG_AUTO ? linear_backward_plan(to_dx, to_dw) : LinearBackwardPlan{config, 0};
+  const GemmProblem to_dx = linear_dx(dy, dy_row_stride, w, w_row_stride, dx, dx_row_stride, tokens, inputs, outputs);
+  const GemmProblem to_dw = linear_dw(dy, dy_row_stride, x, x_row_stride, dw, dw_row_stride, tokens, inputs, outputs);
+  // (without a rest, or with nothing else, the whole is one launch)
+  const int head = rest_beside && tokens > 256 && tokens % 256 != 0 ? tokens - tokens % 256 : 0;
+  const LinearBackwardPlan plan = config == RLK_LINEAR_BWD_CFG_AUTO
+                                      ? linear_backward_plan(to_dx, to_dw, false)
+                                      : LinearBackwardPlan{config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE, head};
   hipError_t err = linear_backward_launch(to_dx, to_dw, plan, reinterpret_cast<hipStream_t>(stream));
   return err == hipSuccess ? RLK_OK : device_error("rlk_linear_bwd_bf16", err);
 }

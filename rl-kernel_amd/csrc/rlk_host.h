@@ -74,8 +74,9 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
                            bool out_f32, int config, hipStream_t stream);
 
 // What a launch with K-major operands takes in the tile estimate, us, a last round that is partly filled priced at
-// max(partial_floor, its share); whether the direct-to-LDS loops take these operands, one or both of them K-major.
-double det_gemm_kmajor_us(int M, int N, int K, bool w_kmajor, bool x_kmajor, double partial_floor);
+// max(partial_floor, its share), and the outputs of one of its tiles; whether the direct-to-LDS loops take these operands,
+// one or both of them K-major.
+double det_gemm_kmajor_us(int M, int N, int K, bool w_kmajor, bool x_kmajor, double partial_floor, int* tile_outputs = nullptr);
 bool det_gemm_takes_kmajor(const MatView& W, const MatView& X, int K);
 
 // Both products of a linear layer's backward, in one launch where that is faster.
@@ -89,7 +90,8 @@ struct LinearBackwardPlan {
   int config;     // rlk_linear_bwd_config, not AUTO
   int head_rows;  // rows of dx that a launch of their own computes first
 };
-LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem& dw);
+// logp: the two launches that the one competes with are those of the LogP backward.
+LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem& dw, bool logp);
 // A plan whose one launch does not serve the operands runs as two.
 hipError_t linear_backward_launch(GemmProblem dx, const GemmProblem& dw, LinearBackwardPlan plan, hipStream_t stream);
 
@@ -174,6 +176,7 @@ hipError_t logits_backward_launch(const void* logits, int dtype, int64_t row_str
 // grad_hidden / grad_weight / grad_bias may each be null. logits [T, logits_ld >= V]: what linear_logp_launch stored for
 // the same inputs, or null (the logits are computed again, and always where a bias gradient is wanted).
 int64_t linear_logp_dz_row_stride(int V);
+LinearBackwardPlan linear_logp_bwd_plan(int T, int D, int V);  // of both its gradients, contiguous operands
 size_t linear_logp_bwd_workspace_bytes(int T, int V, bool with_bias);
 hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int64_t* target, const float* bias,
                                   const float* temperature, const float* lse, const float* logits,

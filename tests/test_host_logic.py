@@ -85,6 +85,18 @@ def test_the_pick_names_the_few_token_tile_that_runs(rlk_lib, m, n, k, name):
     assert rlk_lib.rlk_det_gemm_pick_config(m, n, k) == _lib.GEMM_CONFIGS[name]
 
 
+# (tokens, hidden size, vocabulary): two launches where they are faster (whole token tiles and whole K tiles of a weight from
+# HBM), one launch in the tiles that are the faster ones, the rest behind whole tiles beside the weight gradient
+@pytest.mark.parametrize(
+    "t,d,v,config",
+    [(512, 4096, 37984, 1), (512, 4096, 151936, 1), (304, 5120, 32000, 1), (384, 5120, 32000, 1), (1024, 2048, 131072, 1),
+     (400, 4096, 18992, 6), (512, 4096, 18992, 6), (520, 4096, 37984, 6), (768, 4096, 37984, 6), (768, 4096, 151936, 6),
+     (600, 5120, 32000, 6), (960, 4096, 37984, 3), (1040, 4096, 18992, 3), (2112, 4096, 37984, 2), (4120, 4096, 151936, 0x103)],
+)  # fmt: skip
+def test_the_launches_of_the_logp_backward(rlk_lib, t, d, v, config):
+    assert rlk_lib.rlk_linear_bwd_pick_config(t, d, v, 1) == config
+
+
 def test_argument_errors_are_reported_without_touching_the_gpu(rlk_lib):
     # Invalid arguments are rejected before any HIP call, so this runs on a CPU-only host.
     rc = rlk_lib.rlk_det_gemm_bf16(None, 4, 1, None, 1, 4, None, 4, -1, 4, 4, 0, 0, None)

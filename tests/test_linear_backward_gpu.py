@@ -79,19 +79,71 @@ def test_gradients_of_every_operand_form(form, operand, tokens, inputs, outputs)
     assert torch.equal(dw.view(torch.int16), want_dw.view(torch.int16))
 
 
-@pytest.mark.parametrize("rest", [24, 64, 65])
-def test_few_tokens_behind_whole_tiles(rest):
-    """A long reduction (an lm_head) with a token count just above whole tiles: dX in two parts, the second beside dW."""
+REST_BESIDE = 0x100  # RLK_LINEAR_BWD_CFG_REST_BESIDE
+
+
+@pytest.mark.parametrize("config", CONFIGS)
+@pytest.mark.parametrize("tokens", [257, 280, 576, 577, 1279])  # rests of 1, 24, 64, 65 and 255 behind one, two and four tiles
+def test_the_rest_of_dx_beside_dw(config, tokens):
+    """dX in two parts, the second in the launch of dW: operands and results with pitches of their own."""
+    k, n = 264, 1032
+    gen = torch.Generator(device=DEV).manual_seed(tokens)
+    g, x, w = (_rand(gen, rows, cols + pad)[:, :cols] for rows, cols, pad in ((tokens, n, 8), (tokens, k, 24), (n, k, 16)))
+    want = _backward(g, x, w, 1)
+    got = _backward(g, x, w, config | REST_BESIDE, dx_pitch=8, dw_pitch=16)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("tokens", [4097, 4120, 4160, 4161])
+def test_few_tokens_behind_whole_tiles(tokens):
+    """A token count just above whole tiles: up to 64 tokens beside dW, by the automatic choice."""
     from rl_engine import _lib
 
-    m, k, n = 4096 + rest, 4096, 16448
-    gen = torch.Generator(device=DEV).manual_seed(rest)
-    g, x, w = _rand(gen, m, n), _rand(gen, m, k), _rand(gen, n, k)
+    k = n = 4096
+    lib = _lib.load()
+    assert bool(lib.rlk_linear_bwd_pick_config(tokens, k, n, 0) & REST_BESIDE) == (tokens <= 4160)
+    gen = torch.Generator(device=DEV).manual_seed(tokens)
+    g, x, w = _rand(gen, tokens, n), _rand(gen, tokens, k), _rand(gen, n, k)
     want = _backward(g, x, w, 1)
     got = _backward(g, x, w, 0)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
-    assert _lib.load().rlk_linear_bwd_bf16(None, n, x.data_ptr(), k, w.data_ptr(), k, x.data_ptr(), k, w.data_ptr(), k, m, k, n, 0, None) < 0
-    assert _lib.load().rlk_linear_bwd_bf16(g.data_ptr(), n, x.data_ptr(), k, w.data_ptr(), k, x.data_ptr(), k, w.data_ptr(), k, m, k, n, 9, None) < 0
+
+
+@pytest.mark.parametrize("tokens", [4097, 4120, 4160])
+@pytest.mark.parametrize("vocab", [4093, 4096])
+def test_few_tokens_behind_whole_tiles_in_the_logp_backward(tokens, vocab):
+    """The same in the LogP backward, whose d(logits) rows go on to a whole chunk behind the vocabulary: the bits of each
+    gradient asked for alone."""
+    from rl_engine import _C, _lib
+
+    assert _lib.load().rlk_linear_bwd_pick_config(tokens, 4096, vocab, 1) & REST_BESIDE
+    gen = torch.Generator(device=DEV).manual_seed(tokens)
+    h, w = _rand(gen, tokens, 4096), _rand(gen, vocab, 4096).mul_(0.02)
+    ids = torch.randint(0, vocab, (tokens,), generator=gen, device=DEV)
+    _, lse = _C.fused_linear_logp(h, w, ids)
+    g = torch.randn((tokens,), generator=gen, device=DEV)
+    both = _C.fused_linear_logp_bwd(h, w, ids, lse, g, None)
+    hidden = _C.fused_linear_logp_bwd(h, w, ids, lse, g, None, need_grad_weight=False)
+    weight = _C.fused_linear_logp_bwd(h, w, ids, lse, g, None, need_grad_hidden=False)
+    assert torch.equal(both[0].view(torch.int16), hidden[0].view(torch.int16))
+    assert torch.equal(both[1].view(torch.int16), weight[1].view(torch.int16))
+
+
+def test_refused_arguments():
+    from rl_engine import _lib
+
+    m, k, n = 8, 8, 16
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    g, x, w = _rand(gen, m, n), _rand(gen, m, k), _rand(gen, n, k)
+    dx, dw = torch.empty_like(x), torch.empty_like(w)
+    lib = _lib.load()
+
+    def call(grad, config):
+        return lib.rlk_linear_bwd_bf16(grad, n, x.data_ptr(), k, w.data_ptr(), k, dx.data_ptr(), k, dw.data_ptr(), k, m, k, n, config, None)
+
+    assert call(None, 0) < 0
+    for config in (-1, 9, REST_BESIDE, REST_BESIDE | 1, REST_BESIDE | 9, 2 * REST_BESIDE):
+        assert call(g.data_ptr(), config) < 0, config
 
 
 def test_a_captured_backward_replays():
