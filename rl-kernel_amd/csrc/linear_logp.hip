@@ -398,6 +398,21 @@ size_t linear_logp_workspace_bytes(int T, int V) {
   return T <= kStreamGroupMaxTokens ? per_split * (1 + kLogpStreams) : per_split;
 }
 
+// Groups of eight token tiles share the weight's panels in an XCD's L2. One to three tiles behind one or two whole groups would
+// read the whole weight again and are spread over the groups instead (256-token tiles, the only ones that come in such
+// numbers by the automatic choice). Groups of eight / spread, us, a last tile of 40 / of 250 tokens: V = 131072, D = 2048 with 9
+// tiles 1062 / 1006, 1055 / 1032, 11: 1237 / 1195, 1227 / 1244, 17: 1866 / 1823, 1889 / 1867, 19: 2092 / 2074, 2103 / 2077; V =
+// 151936, D = 4096 with 9: 2261 / 2087, 2241 / 2226, 11: 2671 / 2547, 2638 / 2640, 18: 4229 / 4149, 4244 / 4184, 19: 4603 / 4617,
+// 4549 / 4560. Behind three groups it is no gain: 25 tiles 2730 / 2716, 5925 / 5963, 26: 2763 / 2748, 6309 / 6325, 27: 2938 / 2980,
+// 6306 / 6384; nor with four to seven tiles (21 as three groups of seven: 2197 / 2258).
+template <class S>
+static int token_tiles_per_group(int tiles) {
+  if (tiles < 8) return tiles;
+  const int groups = tiles / 8, rest = tiles % 8;
+  const bool spread = S::BM == 256 && groups <= 2 && rest >= 1 && rest <= 3;
+  return spread ? (tiles + groups - 1) / groups : 8;
+}
+
 template <class S, int LOOP, class ST = S>
 static hipError_t launch_logp(LogpArgs a, hipStream_t stream) {
   auto kernel = linear_logp_partial_kernel<S, ST, LOOP>;
@@ -407,10 +422,7 @@ static hipError_t launch_logp(LogpArgs a, hipStream_t stream) {
   hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds, once);
   if (err != hipSuccess) return err;
   a.tiles_m = (a.T + S::BM - 1) / S::BM;
-  // Groups of eight token tiles share the weight's panels in an XCD's L2. Up to eleven tiles are one group and 17 or 18 two of
-  // nine: a last group of one to three tiles would read the whole weight again (V = 131072, D = 2048: 2600 tokens 1195 -> 1161
-  // us, 4120: 1932 -> 1758). Beyond, groups of other widths cost as much as they save (21 tiles as three of seven: 2197 -> 2258).
-  a.group_m = a.tiles_m <= 11 ? a.tiles_m : a.tiles_m == 17 || a.tiles_m == 18 ? 9 : 8;
+  a.group_m = token_tiles_per_group<S>(a.tiles_m);
   hipLaunchKernelGGL(kernel, dim3(a.tiles_m * a.n_split), dim3(S::kThreads), kLds, stream, a);
   return hipGetLastError();
 }

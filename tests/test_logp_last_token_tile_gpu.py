@@ -9,8 +9,9 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# tokens: the last tile with 1, 64, 65, 128, 129 and 256 of them; one group of 5 to 11 tiles, two (6 + 6, 9 + 8), three
-@pytest.mark.parametrize("tokens", [1025, 1088, 1089, 1152, 1153, 1280, 2600, 2817, 2880, 3009, 4120, 5000])
+# tokens: the last tile with 1, 64, 65, 128, 129 and 256 of them; one group of 5 to 11 tiles, two (8 + 4,
+# 9 + 8, 10 + 9), three (8 + 8 + 4), four (8 + 8 + 8 + 1)
+@pytest.mark.parametrize("tokens", [1025, 1088, 1089, 1152, 1153, 1280, 2600, 2817, 2880, 3009, 4120, 4700, 5000, 6300])
 def test_rows_do_not_depend_on_the_tile(tokens):
     from rl_engine import _C
 
