@@ -71,28 +71,33 @@ constexpr int pingpong_stages() {
   return (S::BN >= 192 && S::BM <= 128) ? 3 : 2;
 }
 
-// kmajor_loop: 0, or the K-major ping-pong variant the operand layouts call for.
+// `loop`: the K-major ping-pong variant the operand layouts call for.
 template <class S>
-static hipError_t launch_shape(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
-                               bool vec, int kmajor_loop, bool allow_pingpong, bool out_f32, hipStream_t stream) {
-  if constexpr (pingpong_supported<S>() && S::TN == 4) {
-    if (kmajor_loop == kLoopPingPongKMajor)
-      return launch_loop<S, kLoopPingPongKMajor>(W, X, C, ldc, M, N, K, out_f32, stream);
-    if constexpr (S::BM % 128 == 0) {
-      if (kmajor_loop == kLoopPingPongXKMajor)
-        return launch_loop<S, kLoopPingPongXKMajor>(W, X, C, ldc, M, N, K, out_f32, stream);
-      if (kmajor_loop == kLoopPingPongBothKMajor)
-        return launch_loop<S, kLoopPingPongBothKMajor>(W, X, C, ldc, M, N, K, out_f32, stream);
-    }
+static hipError_t launch_kmajor(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K, int loop,
+                                bool out_f32, hipStream_t stream) {
+  static_assert(pingpong_supported<S>() && S::TN == 4, "64-feature wave columns");
+  if (loop == kLoopPingPongKMajor) return launch_loop<S, kLoopPingPongKMajor>(W, X, C, ldc, M, N, K, out_f32, stream);
+  if constexpr (S::BM % 128 == 0) {
+    if (loop == kLoopPingPongXKMajor) return launch_loop<S, kLoopPingPongXKMajor>(W, X, C, ldc, M, N, K, out_f32, stream);
+    if (loop == kLoopPingPongBothKMajor)
+      return launch_loop<S, kLoopPingPongBothKMajor>(W, X, C, ldc, M, N, K, out_f32, stream);
   }
-  if (kmajor_loop != 0) return hipErrorInvalidValue;
+  return hipErrorInvalidValue;
+}
+
+// ELEMENTS: whether operands that are not 16-byte aligned come here (`vec` is true otherwise).
+template <class S, bool ELEMENTS = true>
+static hipError_t launch_shape(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
+                               bool vec, bool allow_pingpong, bool out_f32, hipStream_t stream) {
   if constexpr (pingpong_supported<S>()) {
     if (vec && allow_pingpong && K % kTileK == 0) {
       return launch_loop<S, kLoopPingPong, pingpong_stages<S>()>(W, X, C, ldc, M, N, K, out_f32, stream);
     }
   }
-  if (vec) return launch_loop<S, kLoopStaged>(W, X, C, ldc, M, N, K, out_f32, stream);
-  return launch_loop<S, kLoopGeneric>(W, X, C, ldc, M, N, K, out_f32, stream);
+  if constexpr (ELEMENTS) {
+    if (!vec) return launch_loop<S, kLoopGeneric>(W, X, C, ldc, M, N, K, out_f32, stream);
+  }
+  return vec ? launch_loop<S, kLoopStaged>(W, X, C, ldc, M, N, K, out_f32, stream) : hipErrorInvalidValue;
 }
 
 // Deep-stage variant (KS K tiles per barrier pair) of a small tile; native layout only. Two stages of 64 KiB, three of 48
@@ -416,14 +421,14 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     if (config == RLK_GEMM_CFG_AUTO) config = pick_tile_candidate(M, N, K, w_kmajor, x_kmajor);
     switch (config) {
       case RLK_GEMM_CFG_256x256:
-        return launch_shape<Shape256x256>(W, X, C, ldc, M, N, K, false, loop, true, out_f32, stream);
+        return launch_kmajor<Shape256x256>(W, X, C, ldc, M, N, K, loop, out_f32, stream);
       case RLK_GEMM_CFG_256x192:
-        if (!x_kmajor) return launch_shape<Shape256x192>(W, X, C, ldc, M, N, K, false, loop, true, out_f32, stream);
+        if (!x_kmajor) return launch_kmajor<Shape256x192>(W, X, C, ldc, M, N, K, loop, out_f32, stream);
         break;
       case RLK_GEMM_CFG_256x128:
-        return launch_shape<Shape256x128>(W, X, C, ldc, M, N, K, false, loop, true, out_f32, stream);
+        return launch_kmajor<Shape256x128>(W, X, C, ldc, M, N, K, loop, out_f32, stream);
       case RLK_GEMM_CFG_256x64:
-        if (!x_kmajor) return launch_shape<Shape256x64>(W, X, C, ldc, M, N, K, false, loop, true, out_f32, stream);
+        if (!x_kmajor) return launch_kmajor<Shape256x64>(W, X, C, ldc, M, N, K, loop, out_f32, stream);
         break;
       case RLK_GEMM_CFG_64x64:
         if (w_kmajor && x_native) return launch_small_kmajor<Shape64x64>(W, X, C, ldc, M, N, K, out_f32, stream);
@@ -513,21 +518,21 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
   }
   switch (config) {
     case RLK_GEMM_CFG_256x256:
-      return launch_shape<Shape256x256>(W, X, C, ldc, M, N, K, vec, 0, allow_pingpong, out_f32, stream);
+      return launch_shape<Shape256x256>(W, X, C, ldc, M, N, K, vec, allow_pingpong, out_f32, stream);
     case RLK_GEMM_CFG_256x128:
-      return launch_shape<Shape256x128>(W, X, C, ldc, M, N, K, vec, 0, allow_pingpong, out_f32, stream);
+      return launch_shape<Shape256x128>(W, X, C, ldc, M, N, K, vec, allow_pingpong, out_f32, stream);
     case RLK_GEMM_CFG_256x64:
-      return launch_shape<Shape256x64>(W, X, C, ldc, M, N, K, vec, 0, allow_pingpong, out_f32, stream);
+      return launch_shape<Shape256x64, false>(W, X, C, ldc, M, N, K, vec, allow_pingpong, out_f32, stream);
     case RLK_GEMM_CFG_128x128:
-      return launch_shape<Shape128x128>(W, X, C, ldc, M, N, K, vec, 0, allow_pingpong, out_f32, stream);
+      return launch_shape<Shape128x128>(W, X, C, ldc, M, N, K, vec, allow_pingpong, out_f32, stream);
     case RLK_GEMM_CFG_128x64:
-      return launch_shape<Shape128x64>(W, X, C, ldc, M, N, K, vec, 0, allow_pingpong, out_f32, stream);
+      return launch_shape<Shape128x64>(W, X, C, ldc, M, N, K, vec, allow_pingpong, out_f32, stream);
     case RLK_GEMM_CFG_64x64:
-      return launch_shape<Shape64x64>(W, X, C, ldc, M, N, K, vec, 0, allow_pingpong, out_f32, stream);
+      return launch_shape<Shape64x64>(W, X, C, ldc, M, N, K, vec, allow_pingpong, out_f32, stream);
     case RLK_GEMM_CFG_64x16:
-      return launch_shape<Shape64x16>(W, X, C, ldc, M, N, K, vec, 0, allow_pingpong, out_f32, stream);
+      return launch_shape<Shape64x16>(W, X, C, ldc, M, N, K, vec, allow_pingpong, out_f32, stream);
     case RLK_GEMM_CFG_16x16:
-      return launch_shape<Shape16x16>(W, X, C, ldc, M, N, K, vec, 0, allow_pingpong, out_f32, stream);
+      return launch_shape<Shape16x16>(W, X, C, ldc, M, N, K, vec, allow_pingpong, out_f32, stream);
     default:
       return hipErrorInvalidValue;
   }
