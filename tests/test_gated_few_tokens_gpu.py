@@ -30,14 +30,18 @@ def test_projection_and_activation_in_one(tokens, inter):
     assert torch.equal(_C.det_gemm_swiglu(x, w).view(torch.int16), want)
 
 
-@pytest.mark.parametrize("k", [64, 384, 448, 640, 1024, 2048, 4096])
-def test_reduction_lengths_around_the_rule(k):
+# one intermediate size of each tile width (16, 32, 48 and 64 features), both tile heights; reductions below the rule, of fewer
+# stages than the ring holds, of as many and of more (a slot is used again)
+@pytest.mark.parametrize("tokens", [40, 100])
+@pytest.mark.parametrize("inter", [3000, 4096, 8190, 12283, 12400])
+@pytest.mark.parametrize("k", [64, 384, 448, 512, 640, 896, 1024, 1152, 2048, 4096])
+def test_reduction_lengths_around_the_rule(k, inter, tokens):
     from rl_engine import _C
 
     gen = torch.Generator(device=DEV).manual_seed(k)
-    x = torch.randn((40, k), generator=gen, device=DEV, dtype=torch.bfloat16)
-    w = torch.randn((2 * 3000, k), generator=gen, device=DEV, dtype=torch.bfloat16).mul_(0.05)
-    gate_up = torch.empty((40, 6000), device=DEV, dtype=torch.bfloat16)
+    x = torch.randn((tokens, k), generator=gen, device=DEV, dtype=torch.bfloat16)
+    w = torch.randn((2 * inter, k), generator=gen, device=DEV, dtype=torch.bfloat16).mul_(0.05)
+    gate_up = torch.empty((tokens, 2 * inter), device=DEV, dtype=torch.bfloat16)
     _C.gemm_strided(x, w.t(), gate_up)
     assert torch.equal(_C.det_gemm_swiglu(x, w).view(torch.int16), _C.swiglu_packed_forward(gate_up).view(torch.int16))
     # infinities and NaN stay in their rows

@@ -31,14 +31,17 @@ def test_gemm_rows_equal_those_of_a_small_weight(operands, tokens):
         assert torch.equal(out[:, lo:hi].view(torch.int16), part.view(torch.int16))
 
 
-@pytest.mark.parametrize("tokens", [1, 16, 128, 129, 256, 257])
-def test_gated_projection_equals_gemm_and_activation(operands, tokens):
+# up to 128 tokens in tiles of 16, 32, 48 and 64 features: weights of 96 to 194 MiB
+@pytest.mark.parametrize("tokens", [1, 16, 17, 63, 64, 65, 96, 97, 128, 129, 256, 257])
+@pytest.mark.parametrize("rows,k", [(8190, 6272), (16384, 4096), (N, 4096), (24800, 4096)])
+def test_gated_projection_equals_gemm_and_activation(operands, tokens, rows, k):
     from rl_engine import _C
     from rl_engine.backends.rocm.gemm import swiglu_gemm
 
-    x, w = operands
-    fused = swiglu_gemm.forward(x[:tokens], w)
-    two = _C.swiglu_packed_forward(_C.det_gemm_fwd_rhs_transposed(x[:tokens], w))
+    x, w = (t.flatten()[: n * k].view(n, k) if t.numel() >= n * k else t.flatten().repeat(2)[: n * k].view(n, k)
+            for t, n in zip(operands, (tokens, rows)))  # fmt: skip
+    fused = swiglu_gemm.forward(x, w)
+    two = _C.swiglu_packed_forward(_C.det_gemm_fwd_rhs_transposed(x, w))
     assert torch.equal(fused.view(torch.int16), two.view(torch.int16))
 
 
