@@ -118,12 +118,17 @@ typedef enum rlk_linear_bwd_config {
   RLK_LINEAR_BWD_CFG_COUNT = 9,
   /* OR-ed into a one-launch configuration: the whole multiples of 256 tokens of dx in a launch of their own first, its
    * other tokens (tokens % 256) in the one launch beside dw. */
-  RLK_LINEAR_BWD_CFG_REST_BESIDE = 0x100
+  RLK_LINEAR_BWD_CFG_REST_BESIDE = 0x100,
+  /* The automatic choice for one of several weights that are together more than the memory-side cache holds from their forward
+   * to their backward (a gated FFN's). */
+  RLK_LINEAR_BWD_CFG_MANY_WEIGHTS = 0x400
 } rlk_linear_bwd_config;
 
-/* The configuration RLK_LINEAR_BWD_CFG_AUTO resolves to for contiguous operands of a shape, or, with logp != 0, the one that
- * the fused linear-LogP backward runs both its gradients in (tokens x hidden size x vocabulary); host only, no GPU call. */
-int rlk_linear_bwd_pick_config(int tokens, int inputs, int outputs, int logp);
+/* The configuration that the automatic choice resolves to for contiguous operands of a shape: RLK_LINEAR_BWD_CFG_AUTO's,
+ * the one that the fused linear-LogP backward runs both its gradients in (tokens x hidden size x vocabulary), or
+ * RLK_LINEAR_BWD_CFG_MANY_WEIGHTS's; host only, no GPU call. */
+enum { RLK_LINEAR_BWD_OF_LINEAR = 0, RLK_LINEAR_BWD_OF_LOGP = 1, RLK_LINEAR_BWD_OF_MANY_WEIGHTS = 2 };
+int rlk_linear_bwd_pick_config(int tokens, int inputs, int outputs, int of);
 
 /*
  * Both gradients of y = x @ w^T:

@@ -119,10 +119,20 @@ static double tile_us(int bn, int bm, double quality, double start, int K) {
 }
 // dX reads its weight from HBM where the memory-side cache cannot still hold it from the forward. Its small tiles miss
 // their prefetching wave then (304 tokens, 24576 outputs: 255 us as two launches, 279 as one; 201 tokens, 14336 outputs, 112
-// MiB: 126 and 160).
-static bool weight_from_hbm(const GemmProblem& dx) { return (int64_t)dx.N * dx.K * 2 >= ((int64_t)112 << 20); }
-static double dx_tile_us(const PairTiles& t, const GemmProblem& dx) {
-  return tile_us(t.dx_bn, t.dx_bm, t.dx_quality, kStartUs, dx.K) * (t.dx_bn < 256 && weight_from_hbm(dx) ? 1.2 : 1.0);
+// MiB: 126 and 160). Up to 256 tokens from 96 MiB on, which the forward of so few reads past the caches (streamed_weight), and
+// where other weights were read in between: 128 x 128 tiles of dX then take longer than 64 x 64 ones, and the two launches'
+// dW by the short-reduction kernel is the faster one. Forward and backward, us, two launches / priced as cached / as from HBM:
+// 4096 inputs, 12288 outputs at 128 / 193 / 256 tokens 106 / 117 / 106, 139 / 176 / 139, 139 / 174 / 139; a gated FFN of 4096 x
+// 12288 at 193 / 256 tokens 438 / 505 / 424, 459 / 519 / 449, of 4096 x 6144 253 / 268 / 247, 262 / 280 / 253. Above, the same
+// price chose the slower form (257 to 512 tokens up to 6 %, 1600 tokens 4 %).
+static bool weight_from_hbm(const GemmProblem& dx, int tokens, BackwardOf of) {
+  const int64_t bytes = (int64_t)dx.N * dx.K * 2;
+  if (of != BackwardOf::kLogp && tokens <= 256 && (of == BackwardOf::kManyWeights || bytes >= ((int64_t)96 << 20))) return true;
+  return bytes >= ((int64_t)112 << 20);
+}
+static double dx_tile_us(const PairTiles& t, const GemmProblem& dx, int tokens, BackwardOf of) {
+  const bool waits = t.dx_bn < 256 && weight_from_hbm(dx, tokens, of);
+  return tile_us(t.dx_bn, t.dx_bm, t.dx_quality, kStartUs, dx.K) * (waits ? 1.2 : 1.0);
 }
 static double dw_tile_us(const PairTiles& t, const GemmProblem& dw) {
   return tile_us(t.dw_bn, t.dw_bm, t.dw_quality, kStartDwUs, dw.K);
@@ -140,14 +150,15 @@ static int64_t tile_count(const GemmProblem& p, int bn, int bm) { return (int64_
 // ran before: too few tiles of it.) Right behind the LogP forward part of a weight of up to 180 MiB still lies in the
 // memory-side cache: 18992 outputs at 400 / 512 tokens 170 / 174 us, by this estimate 208, 227 from HBM.
 constexpr int kFewTokens = 1024;
-static double pair_us(const GemmProblem& dx, const GemmProblem& dw, const PairTiles& t, int cus, bool logp) {
-  const bool waiting = t.dx_bn < 256 && weight_from_hbm(dx) && dw.K <= kFewTokens && dx.M == dw.K;
-  const bool partly_cached = waiting && logp && (int64_t)dx.N * dx.K * 2 < ((int64_t)180 << 20);
-  const double tx = dx_tile_us(t, dx) * (partly_cached ? 0.92 : 1.0), tw = dw_tile_us(t, dw) * (waiting ? 0.7 : 1.0);
+static double pair_us(const GemmProblem& dx, const GemmProblem& dw, const PairTiles& t, int cus, BackwardOf of) {
+  const bool from_hbm = weight_from_hbm(dx, dw.K, of);
+  const bool waiting = t.dx_bn < 256 && from_hbm && dw.K <= kFewTokens && dx.M == dw.K;
+  const bool partly_cached = waiting && of == BackwardOf::kLogp && (int64_t)dx.N * dx.K * 2 < ((int64_t)180 << 20);
+  const double tx = dx_tile_us(t, dx, dw.K, of) * (partly_cached ? 0.92 : 1.0), tw = dw_tile_us(t, dw) * (waiting ? 0.7 : 1.0);
   const int64_t nx = tile_count(dx, t.dx_bn, t.dx_bm), nw = tile_count(dw, t.dw_bn, t.dw_bm);
   const double work = (nx * tx + nw * tw) / cus;
   const double span = tx >= tw ? pair_span(nx, tx, nw, tw, cus) : pair_span(nw, tw, nx, tx, cus);
-  const double alone = weight_from_hbm(dx) ? 1.0 : 0.6;
+  const double alone = from_hbm ? 1.0 : 0.6;
   const double us = span * (alone + (1.0 - alone) * (work / span));
   return work > us ? work : us;
 }
@@ -157,10 +168,10 @@ static bool one_launch_serves(const GemmProblem& dx, const GemmProblem& dw) {
          det_gemm_takes_kmajor(dx.W, dx.X, dx.K) && det_gemm_takes_kmajor(dw.W, dw.X, dw.K);
 }
 
-static double best_pair_us(const GemmProblem& dx, const GemmProblem& dw, int cus, bool logp, int* config) {
+static double best_pair_us(const GemmProblem& dx, const GemmProblem& dw, int cus, BackwardOf of, int* config) {
   double best = 1e300;
   for (int c = RLK_LINEAR_BWD_CFG_SEPARATE + 1; c < RLK_LINEAR_BWD_CFG_COUNT; ++c) {
-    const double us = pair_us(dx, dw, kPairTiles[c], cus, logp);
+    const double us = pair_us(dx, dw, kPairTiles[c], cus, of);
     if (us < best) {
       best = us;
       *config = c;
@@ -202,22 +213,25 @@ static GemmProblem tail_of(GemmProblem dx, int rows) {
 //   768, 5120, 32000: 520 / 546 / 546      800, 4096, 64000: 982 / 932 / 959      520, 4096, 16384: 215 / 172 / 172
 // 396 measured forms of 12 layers take 0.920 of the two launches' time (0.935), and are up to 5 % slower than them (13).
 constexpr double kFewTokensDx = 0.93, kFewTokensDw = 0.92;
-LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem& dw, bool logp) {
+LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem& dw, BackwardOf of) {
   LinearBackwardPlan plan{RLK_LINEAR_BWD_CFG_SEPARATE, 0};
   if (!one_launch_serves(dx, dw)) return plan;
-  if (weight_from_hbm(dx) && det_gemm_shortk_supported(dw.W, dw.X, dw.M, dw.N, dw.K) && det_gemm_shortk_pays(dw.M, dw.N)) return plan;
+  const bool from_hbm = weight_from_hbm(dx, dw.K, of);
+  if (of != BackwardOf::kManyWeights && from_hbm && det_gemm_shortk_supported(dw.W, dw.X, dw.M, dw.N, dw.K) &&
+      det_gemm_shortk_pays(dw.M, dw.N))
+    return plan;
   const int cus = device_cu_count();
-  const double partial = weight_from_hbm(dx) ? 1.0 : 0.9;
+  const double partial = from_hbm ? 1.0 : 0.9;
   int dx_outputs;
   double us_dx = det_gemm_kmajor_us(dx.M, dx.N, dx.K, true, false, partial, &dx_outputs);
   double us_dw = det_gemm_kmajor_us(dw.M, dw.N, dw.K, true, true, partial);
-  if (logp && weight_from_hbm(dx) && dx.M <= kFewTokens) {
+  if (of == BackwardOf::kLogp && from_hbm && dx.M <= kFewTokens) {
     if (dx_outputs == 128 * 64) us_dx *= kFewTokensDx;
     if (dx.M % kTileK == 0) us_dw *= kFewTokensDw;
   }
   double best = 0.98 * (us_dx + us_dw + kLaunchUs);
   int config;
-  const double together = best_pair_us(dx, dw, cus, logp, &config);
+  const double together = best_pair_us(dx, dw, cus, of, &config);
   if (together < best) {
     best = together;
     plan.config = config;
@@ -226,7 +240,7 @@ LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem
   if (dx.M > 256 && rest >= 1 && rest <= 64) {
     const int whole = dx.M - rest;
     const double head = det_gemm_kmajor_us(whole, dx.N, dx.K, true, false, partial);
-    const double with_rest = head + kLaunchUs + best_pair_us(tail_of(dx, whole), dw, cus, logp, &config);
+    const double with_rest = head + kLaunchUs + best_pair_us(tail_of(dx, whole), dw, cus, of, &config);
     if (with_rest < best) plan = {config, whole};
   }
   return plan;
@@ -241,7 +255,8 @@ hipError_t linear_backward_launch(GemmProblem dx, const GemmProblem& dw, LinearB
     dx = tail_of(dx, plan.head_rows);
   }
   const PairTiles& t = kPairTiles[plan.config];
-  const bool dx_first = plan.config != RLK_LINEAR_BWD_CFG_SEPARATE && dx_tile_us(t, dx) >= dw_tile_us(t, dw);
+  const bool dx_first =
+      plan.config != RLK_LINEAR_BWD_CFG_SEPARATE && dx_tile_us(t, dx, dw.K, BackwardOf::kLinear) >= dw_tile_us(t, dw);
   switch (plan.config) {
     case RLK_LINEAR_BWD_CFG_SEPARATE: {
       const hipError_t err = det_gemm_launch(dx.W, dx.X, dx.C, dx.ldc, dx.M, dx.N, dx.K, false, RLK_GEMM_CFG_AUTO, stream);

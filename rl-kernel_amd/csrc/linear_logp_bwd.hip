@@ -399,7 +399,8 @@ static GemmProblem weight_gradient(const MatView& H, const bf16_bits* dz, void* 
 LinearBackwardPlan linear_logp_bwd_plan(int T, int D, int V) {
   const bf16_bits* any = reinterpret_cast<const bf16_bits*>(uintptr_t{256});  // its alignment is all that is looked at
   const MatView W{any, D, 1, V}, H{any, D, 1, T};
-  return linear_backward_plan(hidden_gradient(W, any, nullptr, D, T, D, V), weight_gradient(H, any, nullptr, D, T, D, V), true);
+  return linear_backward_plan(hidden_gradient(W, any, nullptr, D, T, D, V), weight_gradient(H, any, nullptr, D, T, D, V),
+                              BackwardOf::kLogp);
 }
 
 hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int64_t* target, const float* bias,
@@ -480,7 +481,7 @@ hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int6
   const GemmProblem to_hidden = hidden_gradient(W, a.dz, grad_hidden, gh_row_stride, T, D, V);
   const GemmProblem to_weight = weight_gradient(H, a.dz, grad_weight, gw_row_stride, T, D, V);
   const LinearBackwardPlan plan = grad_hidden && grad_weight && !force_staged
-                                      ? linear_backward_plan(to_hidden, to_weight, true)
+                                      ? linear_backward_plan(to_hidden, to_weight, BackwardOf::kLogp)
                                       : LinearBackwardPlan{RLK_LINEAR_BWD_CFG_SEPARATE, 0};
   if (plan.config != RLK_LINEAR_BWD_CFG_SEPARATE) {
     err = linear_backward_launch(to_hidden, to_weight, plan, stream);

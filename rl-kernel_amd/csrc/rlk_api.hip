@@ -124,18 +124,23 @@ static GemmProblem linear_dw(const void* dy, int64_t dy_ld, const void* x, int64
           dw, dw_ld, outputs, inputs, tokens};
 }
 
-int rlk_linear_bwd_pick_config(int tokens, int inputs, int outputs, int logp) {
+int rlk_linear_bwd_pick_config(int tokens, int inputs, int outputs, int of) {
   if (tokens < 1 || inputs < 1 || outputs < 1) {
     set_last_error("rlk_linear_bwd_pick_config: tokens=%d inputs=%d outputs=%d must be positive", tokens, inputs, outputs);
     return RLK_ERR_INVALID_ARGUMENT;
   }
+  if (of < RLK_LINEAR_BWD_OF_LINEAR || of > RLK_LINEAR_BWD_OF_MANY_WEIGHTS) {
+    set_last_error("rlk_linear_bwd_pick_config: unknown backward %d", of);
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
   LinearBackwardPlan plan;
-  if (logp) {
+  if (of == RLK_LINEAR_BWD_OF_LOGP) {
     plan = linear_logp_bwd_plan(tokens, inputs, outputs);
   } else {
     const void* any = reinterpret_cast<const void*>(uintptr_t{256});  // its alignment is all that is looked at
     plan = linear_backward_plan(linear_dx(any, outputs, any, inputs, nullptr, inputs, tokens, inputs, outputs),
-                                linear_dw(any, outputs, any, inputs, nullptr, inputs, tokens, inputs, outputs), false);
+                                linear_dw(any, outputs, any, inputs, nullptr, inputs, tokens, inputs, outputs),
+                                of == RLK_LINEAR_BWD_OF_LINEAR ? BackwardOf::kLinear : BackwardOf::kManyWeights);
   }
   return plan.config | (plan.head_rows > 0 ? RLK_LINEAR_BWD_CFG_REST_BESIDE : 0);
 }
@@ -148,8 +153,9 @@ int rlk_linear_bwd_bf16(const void* dy, int64_t dy_row_stride, const void* x, in
     return RLK_ERR_INVALID_ARGUMENT;
   }
   const int rest_beside = config & RLK_LINEAR_BWD_CFG_REST_BESIDE;
-  if (config < 0 || (config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE) >= RLK_LINEAR_BWD_CFG_COUNT ||
-      (rest_beside && (config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE) <= RLK_LINEAR_BWD_CFG_SEPARATE)) {
+  if (config != RLK_LINEAR_BWD_CFG_MANY_WEIGHTS &&
+      (config < 0 || (config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE) >= RLK_LINEAR_BWD_CFG_COUNT ||
+       (rest_beside && (config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE) <= RLK_LINEAR_BWD_CFG_SEPARATE))) {
     set_last_error("rlk_linear_bwd_bf16: unknown config %d", config);
     return RLK_ERR_INVALID_ARGUMENT;
   }
@@ -165,9 +171,11 @@ int rlk_linear_bwd_bf16(const void* dy, int64_t dy_row_stride, const void* x, in
   const GemmProblem to_dw = linear_dw(dy, dy_row_stride, x, x_row_stride, dw, dw_row_stride, tokens, inputs, outputs);
   // (without a rest, or with nothing else, the whole is one launch)
   const int head = rest_beside && tokens > 256 && tokens % 256 != 0 ? tokens - tokens % 256 : 0;
-  const LinearBackwardPlan plan = config == RLK_LINEAR_BWD_CFG_AUTO
-                                      ? linear_backward_plan(to_dx, to_dw, false)
-                                      : LinearBackwardPlan{config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE, head};
+  const LinearBackwardPlan plan =
+      config == RLK_LINEAR_BWD_CFG_AUTO ? linear_backward_plan(to_dx, to_dw, BackwardOf::kLinear)
+      : config == RLK_LINEAR_BWD_CFG_MANY_WEIGHTS
+          ? linear_backward_plan(to_dx, to_dw, BackwardOf::kManyWeights)
+          : LinearBackwardPlan{config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE, head};
   hipError_t err = linear_backward_launch(to_dx, to_dw, plan, reinterpret_cast<hipStream_t>(stream));
   return err == hipSuccess ? RLK_OK : device_error("rlk_linear_bwd_bf16", err);
 }

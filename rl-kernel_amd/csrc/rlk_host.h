@@ -90,8 +90,10 @@ struct LinearBackwardPlan {
   int config;     // rlk_linear_bwd_config, not AUTO
   int head_rows;  // rows of dx that a launch of their own computes first
 };
-// logp: the two launches that the one competes with are those of the LogP backward.
-LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem& dw, bool logp);
+// Whose backward it is: a linear layer's right behind its forward; the LogP's, whose own two launches are what the one competes
+// with; or that of a layer with more weights than the memory-side cache holds from the forward to the backward.
+enum class BackwardOf { kLinear, kLogp, kManyWeights };
+LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem& dw, BackwardOf of);
 // A plan whose one launch does not serve the operands runs as two.
 hipError_t linear_backward_launch(GemmProblem dx, const GemmProblem& dw, LinearBackwardPlan plan, hipStream_t stream);
 

@@ -183,9 +183,11 @@ def linear_weight_gradient_plain(a: torch.Tensor, grad: torch.Tensor) -> Optiona
     return _launch_plain(grad, 1, grad.stride(0), a, a.stride(0), out, n, k, m)
 
 
-def linear_backward_plain(grad: torch.Tensor, weight: torch.Tensor, a: torch.Tensor) -> Optional[tuple]:
+def linear_backward_plain(grad: torch.Tensor, weight: torch.Tensor, a: torch.Tensor, many_weights: bool = False) -> Optional[tuple]:
     """``(grad[M,N] @ weight[N,K], grad.T @ a[M,K])`` in one library call, one launch where that is faster, under the
-    conditions of :func:`linear_input_gradient_plain` and :func:`linear_weight_gradient_plain`, or ``None``."""
+    conditions of :func:`linear_input_gradient_plain` and :func:`linear_weight_gradient_plain`, or ``None``.
+    ``many_weights``: ``weight`` is one of several that the memory-side cache cannot hold from their forward on (a choice of
+    launches, never of bits)."""
     if not _plain_pair(grad, weight) or not _plain_pair(grad, a) or grad.size(1) != weight.size(0) or a.size(0) != grad.size(0):
         return None
     (m, n), k = grad.shape, weight.size(1)
@@ -197,7 +199,8 @@ def linear_backward_plain(grad: torch.Tensor, weight: torch.Tensor, a: torch.Ten
     with _on(device):
         status = _lib.load().rlk_linear_bwd_bf16(
             grad.data_ptr(), grad.stride(0), a.data_ptr(), a.stride(0), weight.data_ptr(), weight.stride(0),
-            da.data_ptr(), k, dw.data_ptr(), k, m, k, n, 0, torch._C._cuda_getCurrentRawStream(device.index),
+            da.data_ptr(), k, dw.data_ptr(), k, m, k, n, _lib.LINEAR_BWD_MANY_WEIGHTS if many_weights else 0,
+            torch._C._cuda_getCurrentRawStream(device.index),
         )  # fmt: skip
     if status:
         _lib.check(status, "rlk_linear_bwd_bf16 failed")

@@ -52,6 +52,8 @@ GEMM_CONFIGS = {
 }
 # OR-ed into a GEMM or LogP configuration: register-staged main loop (bit-neutral).
 FORCE_STAGED = 0x100
+# rlk_linear_bwd_config: the automatic choice for one of many weights
+LINEAR_BWD_MANY_WEIGHTS = 0x400
 TREE_LEAF_SPACE = 0x100  # RLK_TREE_CFG_LEAF_SPACE: OR-ed into rlk_tree_config 0 (auto) or 2 (matrix pipe)
 NOALLOC_SCRATCH_BYTES = 32 << 20  # RLK_NOALLOC_SCRATCH_BYTES
 # rlk_dtype (element types of materialised logits)

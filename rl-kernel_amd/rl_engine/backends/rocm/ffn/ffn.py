@@ -131,10 +131,15 @@ def qwen3_ffn_packed_inference(
 # ---------------------------------------------------------------------------
 
 
+# Three weights of 48 MiB come from HBM again in the backward (193 tokens of 4096 x 6144: 268 -> 247 us when told so), three of 24
+# MiB do not.
+_MANY_WEIGHTS_BYTES = 128 << 20
+
+
 def _linear_gradients(a: Tensor, weight: Tensor, grad: Tensor, need_a: bool, need_weight: bool) -> tuple:
     """The gradients of ``a @ weight.T`` that are wanted, ``None`` for the others; both at once where both are."""
     if need_a and need_weight:
-        return mfma_linear_gradients(a, weight, grad)
+        return mfma_linear_gradients(a, weight, grad, 3 * weight.nbytes >= _MANY_WEIGHTS_BYTES)
     return (
         det_gemm_linear_input_gradient(grad, weight) if need_a else None,
         det_gemm_linear_weight_gradient(a, grad) if need_weight else None,

@@ -97,6 +97,23 @@ def test_the_launches_of_the_logp_backward(rlk_lib, t, d, v, config):
     assert rlk_lib.rlk_linear_bwd_pick_config(t, d, v, 1) == config
 
 
+# (whose backward, tokens, inputs, outputs): a layer of 96 MiB right behind its forward (0) and one of an FFN's three weights (2)
+# read their weight from HBM up to 256 tokens, a layer of 48 MiB right behind its forward does not
+@pytest.mark.parametrize(
+    "of,m,k,n,config",
+    [(0, 100, 4096, 12288, 7), (0, 128, 4096, 12288, 1), (0, 193, 4096, 12288, 7), (0, 225, 4096, 12288, 7),
+     (0, 256, 4096, 12288, 1), (0, 257, 4096, 12288, 6), (0, 400, 4096, 12288, 6), (0, 193, 4096, 6144, 6),
+     (2, 128, 4096, 12288, 7), (2, 193, 4096, 12288, 7), (2, 256, 4096, 12288, 7), (2, 257, 4096, 12288, 6),
+     (2, 193, 4096, 6144, 7), (2, 256, 4096, 6144, 7), (2, 300, 4096, 6144, 6), (2, 193, 12288, 4096, 3)],
+)  # fmt: skip
+def test_the_launches_of_a_linear_backward(rlk_lib, of, m, k, n, config):
+    assert rlk_lib.rlk_linear_bwd_pick_config(m, k, n, of) == config
+
+
+def test_unknown_backwards_have_no_choice(rlk_lib):
+    assert rlk_lib.rlk_linear_bwd_pick_config(64, 64, 64, -1) < 0 and rlk_lib.rlk_linear_bwd_pick_config(64, 64, 64, 3) < 0
+
+
 def test_argument_errors_are_reported_without_touching_the_gpu(rlk_lib):
     # Invalid arguments are rejected before any HIP call, so this runs on a CPU-only host.
     rc = rlk_lib.rlk_det_gemm_bf16(None, 4, 1, None, 1, 4, None, 4, -1, 4, 4, 0, 0, None)

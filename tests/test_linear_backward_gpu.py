@@ -94,6 +94,18 @@ def test_the_rest_of_dx_beside_dw(config, tokens):
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+@pytest.mark.parametrize("tokens,inputs,outputs", [(193, 1024, 6144), (256, 1032, 2056), (300, 264, 1032), (4120, 1024, 4096)])
+def test_one_of_many_weights(tokens, inputs, outputs):
+    """The choice for weights that come from HBM again: the same bits."""
+    from rl_engine import _lib
+
+    gen = torch.Generator(device=DEV).manual_seed(tokens)
+    g, x, w = _rand(gen, tokens, outputs), _rand(gen, tokens, inputs), _rand(gen, outputs, inputs)
+    want = _backward(g, x, w, 1)
+    got = _backward(g, x, w, _lib.LINEAR_BWD_MANY_WEIGHTS)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("tokens", [4097, 4120, 4160, 4161])
 def test_few_tokens_behind_whole_tiles(tokens):
     """A token count just above whole tiles: up to 64 tokens beside dW, by the automatic choice."""
@@ -142,7 +154,7 @@ def test_refused_arguments():
         return lib.rlk_linear_bwd_bf16(grad, n, x.data_ptr(), k, w.data_ptr(), k, dx.data_ptr(), k, dw.data_ptr(), k, m, k, n, config, None)
 
     assert call(None, 0) < 0
-    for config in (-1, 9, REST_BESIDE, REST_BESIDE | 1, REST_BESIDE | 9, 2 * REST_BESIDE):
+    for config in (-1, 9, REST_BESIDE, REST_BESIDE | 1, REST_BESIDE | 9, 2 * REST_BESIDE, 0x401, 0x500):
         assert call(g.data_ptr(), config) < 0, config
 
 
