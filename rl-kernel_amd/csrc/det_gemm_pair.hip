@@ -119,15 +119,16 @@ static double tile_us(int bn, int bm, double quality, double start, int K) {
 }
 // dX reads its weight from HBM where the memory-side cache cannot still hold it from the forward. Its small tiles miss
 // their prefetching wave then (304 tokens, 24576 outputs: 255 us as two launches, 279 as one; 201 tokens, 14336 outputs, 112
-// MiB: 126 and 160). Up to 256 tokens from 96 MiB on, which the forward of so few reads past the caches (streamed_weight), and
+// MiB: 126 and 160). Up to 272 tokens from 96 MiB on, which the forward of so few reads past the caches (streamed_weight), and
 // where other weights were read in between: 128 x 128 tiles of dX then take longer than 64 x 64 ones, and the two launches'
 // dW by the short-reduction kernel is the faster one. Forward and backward, us, two launches / priced as cached / as from HBM:
 // 4096 inputs, 12288 outputs at 128 / 193 / 256 tokens 106 / 117 / 106, 139 / 176 / 139, 139 / 174 / 139; a gated FFN of 4096 x
 // 12288 at 193 / 256 tokens 438 / 505 / 424, 459 / 519 / 449, of 4096 x 6144 253 / 268 / 247, 262 / 280 / 253. Above, the same
-// price chose the slower form (257 to 512 tokens up to 6 %, 1600 tokens 4 %).
+// price chooses the slower form (4096 inputs, 12288 outputs, two launches / one: 257 tokens 179 / 183, 272: 182 / 182, 288: 185 /
+// 184, 512: 205 / 193).
 static bool weight_from_hbm(const GemmProblem& dx, int tokens, BackwardOf of) {
   const int64_t bytes = (int64_t)dx.N * dx.K * 2;
-  if (of != BackwardOf::kLogp && tokens <= 256 && (of == BackwardOf::kManyWeights || bytes >= ((int64_t)96 << 20))) return true;
+  if (of != BackwardOf::kLogp && tokens <= 272 && (of == BackwardOf::kManyWeights || bytes >= ((int64_t)96 << 20))) return true;
   return bytes >= ((int64_t)112 << 20);
 }
 static double dx_tile_us(const PairTiles& t, const GemmProblem& dx, int tokens, BackwardOf of) {
