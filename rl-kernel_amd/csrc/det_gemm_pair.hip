@@ -108,8 +108,9 @@ static double pair_span(int64_t n1, double t1, int64_t n2, double t2, int cus) {
 }
 
 // The estimate of a launch, fitted to 282 shapes (64 to 8192 tokens, 21 layers and vocabularies, every configuration and
-// the two launches measured): the choice takes 0.6 % longer than the best configuration of each shape, 0.870 of the two
-// launches' time over all shapes, and is never more than 2 % slower than them.
+// the two launches measured, weights right behind their forward). Over them the choice takes 0.6 % longer than the best
+// configuration of each shape, 0.870 of the two launches' time, and is never more than 2 % slower than them; over 72 shapes of
+// 12 layers that it was not fitted to 1.4 % longer (at worst 38 %), 0.810, and never more than 2 % slower.
 //
 // A tile on a full chip, us: 11 + 21 K / 1024 for 256 x 256 outputs (see remainder_launch_pays), other shapes by area and
 // quality; a tile of dW, whose reduction is short, starts faster.
