@@ -51,7 +51,7 @@ typedef enum rlk_gemm_config {
   RLK_GEMM_CFG_128x64_DEEP = 12,  /* 128x64 tile; K % 128 == 0 */
   RLK_GEMM_CFG_128x128_DEEP = 13, /* 128x128 tile, 128 K values per barrier pair */
   RLK_GEMM_CFG_STREAM64 = 14,     /* M <= 64: 16-feature panels streamed through an LDS ring, one consumer wave per 16 tokens */
-  RLK_GEMM_CFG_256x256_SOLO = 15, /* 256 x 256 tile on four waves (one per SIMD, 128 x 128 each) */
+  RLK_GEMM_CFG_256x256_SOLO = 15, /* 256 x 256 tiles on four waves (one per SIMD, 128 x 128 each), a workgroup per CU */
   RLK_GEMM_CFG_192x256 = 16,      /* 192 features x 256 tokens (N / 192 tiles where N / 256 leaves a round half empty) */
   RLK_GEMM_CFG_SHORTK = 17,       /* K <= 256, K-major token operand: features stationary in registers, tokens streamed */
   RLK_GEMM_CFG_192x128 = 18,      /* 192 features x 128 tokens, three stages (N / 192 x M / 128 tiles that fill one round) */

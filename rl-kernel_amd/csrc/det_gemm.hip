@@ -5,6 +5,7 @@
 // rl_engine/backends/rocm/gemm/mfma_gemm.py:135-274. No split-K, no atomics, no
 // stream-K: one workgroup owns an output tile for the whole K range.
 #include "det_gemm_body.h"
+#include "det_gemm_solo.h"
 #include "rlk_host.h"
 
 namespace rlk {
@@ -17,9 +18,70 @@ __global__ __launch_bounds__(S::kThreads + (has_prefetch_wave<LOOP, KS>() ? kWav
   det_gemm_tile<S, LOOP, OUT_F32, KS, NS>(W, X, C, ldc, M, N, K, tiles_m, tiles_n, group_m, blockIdx.x, lds);
 }
 
+// 256 x 256 tiles, one workgroup per CU that goes through its share of them (det_gemm_solo.h).
+__global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_solo_kernel(MatView W, MatView X, bf16_bits* __restrict__ C,
+                                                                            int64_t ldc, int M, int N, int K, int tiles_m,
+                                                                            int tiles_n, int group_m) {
+  using S = SoloShape;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto tile_at = [&](int block, int& n0, int& m0) __attribute__((always_inline)) {
+    const TileOrder at = tile_order(block, tiles_m, tiles_n, group_m);
+    n0 = at.tile_n * S::BN;
+    m0 = at.tile_m * S::BM;
+  };
+  auto done = [&](int block, SoloAcc& acc, char*) __attribute__((always_inline)) -> bool {
+    int n0, m0;
+    tile_at(block, n0, m0);
+    const int lane = solo_lane(), grp = lane >> 4;
+    const int n_wave = n0 + wave % S::WN * 128, m_wave = m0 + wave / S::WN * 128;
+    const int m_lane = m_wave + (lane & 15);
+    if (n_wave + 128 <= N && (reinterpret_cast<uintptr_t>(C) & 15) == 0 && (ldc & 7) == 0) {
+#pragma unroll
+      for (int jm = 0; jm < S::TM; ++jm) {
+        bf16_bits* const row = C + (int64_t)(m_lane + jm * 16) * ldc + n_wave;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          solo_store_span(row + h * 64, grp, m_lane + jm * 16 < M, acc[4 * h][jm], acc[4 * h + 1][jm], acc[4 * h + 2][jm],
+                          acc[4 * h + 3][jm]);
+      }
+      return m_wave + 128 <= M;
+    }
+#pragma unroll
+    for (int jm = 0; jm < S::TM; ++jm) {
+      const int m = m_lane + jm * 16;
+      if (m >= M) continue;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int n = n_wave + h * 64 + grp * 16;
+        bf16_bits* const dst = C + (int64_t)m * ldc + n;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (n + e < N) dst[e] = to_bf16_bits(acc[4 * h + (e >> 2)][jm][e & 3]);
+      }
+    }
+    return false;
+  };
+  solo_tiles<SoloPlainRows, 4 * S::TM>(W, X, K, blockIdx.x, gridDim.x, tiles_m * tiles_n, lds, tile_at, done);
+}
+
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
+
+static hipError_t launch_solo(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
+                              hipStream_t stream) {
+  static PerDeviceOnce once;
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(det_gemm_solo_kernel), kSoloLdsBytes, once);
+  if (err != hipSuccess) return err;
+  const int tiles_m = (M + SoloShape::BM - 1) / SoloShape::BM;
+  const int tiles_n = (N + SoloShape::BN - 1) / SoloShape::BN;
+  const int cus = device_cu_count();
+  const int grid = tiles_m * tiles_n < cus ? tiles_m * tiles_n : cus;
+  hipLaunchKernelGGL(det_gemm_solo_kernel, dim3(grid), dim3(SoloShape::kThreads), kSoloLdsBytes, stream, W, X,
+                     reinterpret_cast<bf16_bits*>(C), ldc, M, N, K, tiles_m, tiles_n, tiles_m < 8 ? tiles_m : 8);
+  return hipGetLastError();
+}
 
 template <class S, int LOOP, bool OUT_F32, int KS = 1, int NS = 2>
 static hipError_t launch_tile(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
@@ -162,7 +224,6 @@ static hipError_t launch_small_kmajor(const MatView& W, const MatView& X, void* 
 
 // Tile shapes. Which one runs is a pure performance choice (see det_gemm_tile.h).
 using Shape256x256 = TileShape<256, 256, 4, 2>;
-using Shape256x256Solo = TileShape<256, 256, 2, 2>;
 using Shape192x256 = TileShape<192, 256, 4, 2>;  // 192 features x 256 tokens: three MFMA tiles per wave along N
 using Shape256x192 = TileShape<256, 192, 4, 2>;
 using Shape192x192 = TileShape<192, 192, 4, 2>;  // 192 features x 192 tokens
@@ -331,7 +392,9 @@ int pick_det_gemm_config(int M, int N, int K) {
     if (tile_count(M, N, 160, 64) <= cus) return RLK_GEMM_CFG_64x160_DEEP;
     if (tile_count(M, N, 128, 128) <= cus) return RLK_GEMM_CFG_128x128_DEEP;
   }
-  return pick_tile_candidate(M, N, K, false, false);
+  const int config = pick_tile_candidate(M, N, K, false, false);
+  const bool solo = config == RLK_GEMM_CFG_256x256 && K % kTileK == 0 && solo_tiles_pay(tile_count(M, N, 256, 256), cus);
+  return solo ? RLK_GEMM_CFG_256x256_SOLO : config;
 }
 
 // A K-major view (element [row, k] at ptr[k * k_stride + row], rows contiguous: B[K,N] as the
@@ -484,6 +547,11 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
              : config == RLK_GEMM_CFG_128x64_DEEP || config == RLK_GEMM_CFG_64x96_DEEP || config == RLK_GEMM_CFG_96x64_DEEP ? RLK_GEMM_CFG_128x64
                                                                                        : RLK_GEMM_CFG_64x64;
   }
+  if (config == RLK_GEMM_CFG_256x256_SOLO) {
+    if (vec && allow_pingpong && K % kTileK == 0 && !out_f32 && solo_offsets_fit(W) && solo_offsets_fit(X))
+      return launch_solo(W, X, C, ldc, M, N, K, stream);
+    config = RLK_GEMM_CFG_256x256;
+  }
   // The element-wise loader keeps eight values per chunk in flight, and a picked 256-feature tile gives way to 128 x 128, which
   // holds them without spilling. The 192-feature and 192-token tiles, which have no such loader, become 256-feature tiles
   // behind this line and keep them: spilled registers (98 of 256 x 256) cost less there than twice the loads. Odd pitch, as
@@ -491,11 +559,6 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
   // 565 / 779, 6144 at 768 (192 x 128) 295 / 567; K = 128: 36.5 / 35.4, 64: 26.5 / 25.2.
   if (!vec && (config == RLK_GEMM_CFG_256x256 || config == RLK_GEMM_CFG_256x128 || config == RLK_GEMM_CFG_256x64))
     config = RLK_GEMM_CFG_128x128;
-  if (config == RLK_GEMM_CFG_256x256_SOLO) {
-    if (vec && allow_pingpong && K % kTileK == 0)
-      return launch_loop<Shape256x256Solo, kLoopSolo>(W, X, C, ldc, M, N, K, out_f32, stream);
-    config = RLK_GEMM_CFG_256x256;
-  }
   if (config == RLK_GEMM_CFG_192x128) {
     if (vec && allow_pingpong && K % kTileK == 0)
       return launch_loop<Shape192x128, kLoopPingPong, pingpong_stages<Shape192x128>()>(W, X, C, ldc, M, N, K, out_f32, stream);

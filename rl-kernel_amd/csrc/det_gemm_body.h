@@ -19,7 +19,6 @@ enum : int {
   kLoopPingPongKMajor = 3,   // weight K-major
   kLoopPingPongXKMajor = 4,  // activation K-major
   kLoopPingPongBothKMajor = 5,
-  kLoopSolo = 6,  // four waves, one per SIMD
   kLoopStagedKMajor = 7,     // register-staged, weight K-major (the small tiles), K % 64 == 0
   kLoopStagedKMajorTail = 8, // the same with a zero-filled last K tile
   kLoopPingPongWStream = 9,  // kLoopPingPong with the weight read past the caches
@@ -40,21 +39,31 @@ constexpr bool has_prefetch_wave() {
 }
 constexpr int kPrefetchDumpBytes = kWave * 4;
 
+// Tile raster: XCD-compact ids, then column groups of group_m token tiles so
+// the tiles resident on one XCD share weight and activation panels in its L2.
+struct TileOrder {
+  int id, within, width, tile_m, tile_n;
+};
+__device__ __forceinline__ TileOrder tile_order(int block, int tiles_m, int tiles_n, int group_m) {
+  TileOrder o;
+  o.id = xcd_compact_id(block, tiles_m * tiles_n);
+  const int per_group = group_m * tiles_n;
+  const int group = o.id / per_group;
+  const int first_m = group * group_m;
+  o.width = (tiles_m - first_m) < group_m ? (tiles_m - first_m) : group_m;
+  o.within = o.id - group * per_group;
+  o.tile_m = first_m + o.within % o.width;
+  o.tile_n = o.within / o.width;
+  return o;
+}
+
 // One tile of a launch: workgroup `block` of the tiles_m x tiles_n that the problem consists of.
 template <class S, int LOOP, bool OUT_F32, int KS, int NS, bool PREFETCH = has_prefetch_wave<LOOP, KS>()>
 __device__ __forceinline__ void det_gemm_tile(const MatView& W, const MatView& X, void* __restrict__ C, int64_t ldc, int M,
                                               int N, int K, int tiles_m, int tiles_n, int group_m, int block, char* lds) {
-  // Tile raster: XCD-compact ids, then column groups of group_m token tiles so
-  // the tiles resident on one XCD share weight and activation panels in its L2.
   const int total = tiles_m * tiles_n;
-  const int id = xcd_compact_id(block, total);
-  const int per_group = group_m * tiles_n;
-  const int group = id / per_group;
-  const int first_m = group * group_m;
-  const int width = (tiles_m - first_m) < group_m ? (tiles_m - first_m) : group_m;
-  const int within = id - group * per_group;
-  const int tile_m = first_m + within % width;
-  const int tile_n = within / width;
+  const TileOrder at = tile_order(block, tiles_m, tiles_n, group_m);
+  const int id = at.id, within = at.within, width = at.width, tile_m = at.tile_m, tile_n = at.tile_n;
   const int n0 = tile_n * S::BN;
   const int m0 = tile_m * S::BM;
 
@@ -74,8 +83,6 @@ __device__ __forceinline__ void det_gemm_tile(const MatView& W, const MatView& X
   f32x4_t acc[S::TN][S::TM];
   if constexpr (LOOP == kLoopQuad || LOOP == kLoopQuadWStream || LOOP == kLoopQuadPrefetch) {
     tile_mainloop_quad<S, KS, NS, LOOP == kLoopQuadWStream>(W, X, n0, m0, K, lds, acc);
-  } else if constexpr (LOOP == kLoopSolo) {
-    tile_mainloop_solo<S>(W, X, n0, m0, K, lds, acc);
   } else if constexpr (LOOP == kLoopStagedKMajor || LOOP == kLoopStagedKMajorTail) {
     tile_mainloop_staged_kmajor<S, KS, LOOP == kLoopStagedKMajorTail>(W, X, n0, m0, K, lds, acc);
   } else if constexpr (LOOP == kLoopPingPongWStream) {

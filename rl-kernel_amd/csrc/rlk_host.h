@@ -49,6 +49,16 @@ inline double rounds_of_workgroups(int64_t tiles, int cus, double partial_floor 
   return (double)full + (part > 0.0 ? (part > partial_floor ? part : partial_floor) : 0.0);
 }
 
+// Whether 256 x 256 tiles run with one wave per SIMD (det_gemm_solo.h) or in two groups of four waves (the ping-pong loop). The first
+// takes less energy and no time between tiles, which counts where all CUs are busy and the package is at its power cap; the
+// second takes 5 % fewer cycles a K tile, which counts where a round fills less than half of the chip. Ping-pong / one wave, 4096
+// outputs, K = 4096, us: 64 tiles 66.6 / 69.1, 96: 66.1 / 69.6, 128: 70.4 / 70.4, 160: 74.5 / 74.3, 192: 80.7 / 79.7, 256: 98.3 /
+// 97.1, 272: 155.9 / 157.9, 384: 165.4 / 170.4, 896: 359 / 352, 1024: 376 / 365, 1536: 558 / 539.
+inline bool solo_tiles_pay(int64_t tiles, int cus) {
+  const int64_t last = tiles % cus;
+  return tiles >= 2 * cus || last == 0 || last * 2 > cus;
+}
+
 // Whether a kernel loads the weight past the caches (non-temporal): its M tokens are one token tile of `bm`, or two whole
 // ones, whose workgroups read a weight line at the same time. A weight of 96 MiB or more does not wait in the 256 MB
 // memory-side cache for its next use once the other layers have passed through, and reads that leave nothing there are

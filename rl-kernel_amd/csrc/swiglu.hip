@@ -17,6 +17,8 @@
 // The fused kernel rounds its two fp32 accumulators to bf16 before the activation, so it
 // returns exactly what the GEMM followed by the elementwise kernel returns.
 #include "linear_logp_common.h"
+#include "det_gemm_body.h"
+#include "det_gemm_solo.h"
 #include "rlk_host.h"
 
 namespace rlk {
@@ -229,6 +231,50 @@ __global__ __launch_bounds__(S::kThreads) void det_gemm_swiglu_kernel(MatView W,
   }
 }
 
+// The same on 256 weight rows x 256 tokens with one wave per SIMD, a workgroup per CU (det_gemm_solo.h).
+__global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_swiglu_solo_kernel(MatView W, MatView X,
+                                                                                   bf16_bits* __restrict__ Y, int64_t ldy,
+                                                                                   int M, int I, int K, int tiles_m,
+                                                                                   int tiles_n, int group_m) {
+  using S = SoloShape;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto tile_at = [&](int block, int& f0, int& m0) __attribute__((always_inline)) {
+    const TileOrder at = tile_order(block, tiles_m, tiles_n, group_m);
+    f0 = at.tile_n * (S::BN / 2);
+    m0 = at.tile_m * S::BM;
+  };
+  auto done = [&](int block, SoloAcc& acc, char*) __attribute__((always_inline)) -> bool {
+    int f0, m0;
+    tile_at(block, f0, m0);
+    const int lane = solo_lane(), grp = lane >> 4;
+    const int f_wave = f0 + wave % S::WN * 64, m_wave = m0 + wave / S::WN * 128;
+    const int m_lane = m_wave + (lane & 15);
+    const bool whole = f_wave + 64 <= I && (reinterpret_cast<uintptr_t>(Y) & 15) == 0 && (ldy & 7) == 0;
+#pragma unroll
+    for (int jm = 0; jm < S::TM; ++jm) {
+      f32x4_t y[4];
+#pragma unroll
+      for (int jn = 0; jn < 4; ++jn)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          y[jn][q] = swiglu_f32(round_through_bf16(acc[jn][jm][q]), round_through_bf16(acc[jn + 4][jm][q]));
+      const int m = m_lane + jm * 16;
+      bf16_bits* const row = Y + (int64_t)m * ldy;
+      if (whole) {
+        solo_store_span(row + f_wave, grp, m < M, y[0], y[1], y[2], y[3]);
+      } else if (m < M) {
+        const int f = f_wave + grp * 16;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (f + e < I) row[f + e] = to_bf16_bits(y[e >> 2][e & 3]);
+      }
+    }
+    return whole && m_wave + 128 <= M;
+  };
+  solo_tiles<SoloGatedRows, 2 * S::TM>(W, X, K, blockIdx.x, gridDim.x, tiles_m * tiles_n, lds, tile_at, done);
+}
+
 // The same for few tokens: four waves over one wave column of BN / 2 gate rows and the up rows of the same features, all of
 // the tokens of a launch in one tile.
 // Bound by HBM: the weight is read once (201 MB of gate_up in 39 us, 5.2 TB/s), four waves read every weight row from LDS
@@ -286,6 +332,20 @@ static hipError_t launch_gated_few(const MatView& W, const MatView& X, void* Y, 
   if (err != hipSuccess) return err;
   hipLaunchKernelGGL(kernel, dim3((I + BN / 2 - 1) / (BN / 2)), dim3(S::kThreads), kLds, stream, W, X,
                      reinterpret_cast<bf16_bits*>(Y), ldy, M, I, K);
+  return hipGetLastError();
+}
+
+static hipError_t launch_gated_solo(const MatView& W, const MatView& X, void* Y, int64_t ldy, int M, int I, int K,
+                                    hipStream_t stream) {
+  static PerDeviceOnce once;
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(det_gemm_swiglu_solo_kernel), kSoloLdsBytes, once);
+  if (err != hipSuccess) return err;
+  const int tiles_m = (M + SoloShape::BM - 1) / SoloShape::BM;
+  const int tiles_n = (I + SoloShape::BN / 2 - 1) / (SoloShape::BN / 2);
+  const int cus = device_cu_count();
+  const int grid = tiles_m * tiles_n < cus ? tiles_m * tiles_n : cus;
+  hipLaunchKernelGGL(det_gemm_swiglu_solo_kernel, dim3(grid), dim3(SoloShape::kThreads), kSoloLdsBytes, stream, W, X,
+                     reinterpret_cast<bf16_bits*>(Y), ldy, M, I, K, tiles_m, tiles_n, tiles_m < 8 ? tiles_m : 8);
   return hipGetLastError();
 }
 
@@ -365,8 +425,12 @@ hipError_t det_gemm_swiglu_launch(const MatView& W, const MatView& X, void* Y, i
     };
     const double c256 = cost(t256, 256.0, 1.0), c192 = cost(t192, 192.0, 0.87), c128 = cost(t128, 128.0, 0.65);
     if (M > 128 && c192 < c256 && c192 < c128) return launch_gated<GatedShape192>(W, X, Y, ldy, M, I, K, stream);
-    if (M > 128 && c256 <= c128)
+    if (M > 128 && c256 <= c128) {
+      // (a weight that is read past the caches has the ping-pong loop only)
+      if (solo_tiles_pay(t256, cus) && !streamed_weight(2 * (int64_t)I, K, M, 256) && solo_offsets_fit(W, (int64_t)I + 128) && solo_offsets_fit(X))
+        return launch_gated_solo(W, X, Y, ldy, M, I, K, stream);
       return launch_gated<GatedShape256>(W, X, Y, ldy, M, I, K, stream);
+    }
     if (M > 64 && t128 >= 128) return launch_gated<GatedShape128>(W, X, Y, ldy, M, I, K, stream);
     return launch_gated<GatedShape64>(W, X, Y, ldy, M, I, K, stream);
   }
