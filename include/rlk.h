@@ -37,7 +37,7 @@ typedef enum rlk_status {
  * bit; RLK_GEMM_CFG_AUTO picks by shape. Exposed so tests can prove that. */
 typedef enum rlk_gemm_config {
   RLK_GEMM_CFG_AUTO = 0,
-  RLK_GEMM_CFG_256x256 = 1,
+  RLK_GEMM_CFG_256x256 = 1, /* picked, it runs as 256x256_SOLO where that is faster */
   RLK_GEMM_CFG_256x128 = 2,
   RLK_GEMM_CFG_128x128 = 3,
   RLK_GEMM_CFG_128x64 = 4,

@@ -1,4 +1,5 @@
-"""Build librlk_gfx950.so (the C-ABI HIP library) in-tree with hipcc.
+"""Build librlk_gfx950.so (the C-ABI HIP library) in-tree with hipcc, and rl_engine/_torch_host.so (the host side of the
+smallest calls, no device code) with the host compiler.
 
 Usage: python rl-kernel_amd/build.py            (or __graft_entry__.build())
 """
@@ -14,6 +15,8 @@ from pathlib import Path
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "librlk_gfx950.so"
+HOST_SOURCE = CSRC / "torch_host.cpp"
+HOST_MODULE = PKG_DIR / "rl_engine" / "_torch_host.so"
 OBJ_DIR = PKG_DIR / "build"  # object files (git-ignored)
 SOURCES = ["det_gemm.hip", "det_gemm_pair.hip", "det_gemm_stream.hip", "det_gemm_shortk.hip", "det_gemm_tree.hip", "det_gemm_seq.hip", "linear_logp.hip",
     "linear_logp_bwd.hip", "logits_logp.hip", "swiglu.hip", "grpo.hip", "rlk_api.hip"]
@@ -51,6 +54,20 @@ def _run(cmd: list[str]) -> str:
     return out
 
 
+def host_module_command() -> list[str]:
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    includes = [*include_paths(), sysconfig.get_paths()["include"], os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")]
+    return [
+        shutil.which(os.environ.get("CXX", "g++")) or "g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", *(f"-I{d}" for d in includes), str(HOST_SOURCE), "-o", str(HOST_MODULE),
+        *(f"-L{d}" for d in library_paths()), "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+    ]  # fmt: skip
+
+
 def build(verbose: bool = True, only: list[str] | None = None) -> Path:
     """Compile every HIP source for gfx950 (one hipcc per source, side by side) and link them into
     one shared library. `only` names the sources to recompile; the objects of the others are reused
@@ -70,6 +87,9 @@ def build(verbose: bool = True, only: list[str] | None = None) -> Path:
         if only is not None and src not in only and fresh:
             continue
         jobs.append([hipcc, *compile_flags, "-c", "-o", str(obj), str(CSRC / src)])
+    host_newest = max(HOST_SOURCE.stat().st_mtime, (PKG_DIR.parent / "include" / "rlk.h").stat().st_mtime)
+    if only is None or HOST_SOURCE.name in only or not HOST_MODULE.exists() or HOST_MODULE.stat().st_mtime < host_newest:
+        jobs.insert(0, host_module_command())
     if verbose:
         for cmd in jobs:
             print("[rlk build]", " ".join(cmd), flush=True)

@@ -392,9 +392,7 @@ int pick_det_gemm_config(int M, int N, int K) {
     if (tile_count(M, N, 160, 64) <= cus) return RLK_GEMM_CFG_64x160_DEEP;
     if (tile_count(M, N, 128, 128) <= cus) return RLK_GEMM_CFG_128x128_DEEP;
   }
-  const int config = pick_tile_candidate(M, N, K, false, false);
-  const bool solo = config == RLK_GEMM_CFG_256x256 && K % kTileK == 0 && solo_tiles_pay(tile_count(M, N, 256, 256), cus);
-  return solo ? RLK_GEMM_CFG_256x256_SOLO : config;
+  return pick_tile_candidate(M, N, K, false, false);
 }
 
 // A K-major view (element [row, k] at ptr[k * k_stride + row], rows contiguous: B[K,N] as the
@@ -506,7 +504,12 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
         break;  // an explicitly requested other shape runs the element-wise loader below
     }
   }
-  if (config == RLK_GEMM_CFG_AUTO) config = pick_det_gemm_config(M, N, K);
+  if (config == RLK_GEMM_CFG_AUTO) {
+    config = pick_det_gemm_config(M, N, K);
+    // the picked shape with one wave per SIMD (which a call can ask for, and which is 256 x 256 again for what it does not take)
+    if (config == RLK_GEMM_CFG_256x256 && solo_tiles_pay(tile_count(M, N, 256, 256), device_cu_count()))
+      config = RLK_GEMM_CFG_256x256_SOLO;
+  }
   if (config == RLK_GEMM_CFG_STREAM16_DEEP || config == RLK_GEMM_CFG_STREAM16 || config == RLK_GEMM_CFG_STREAM64) {
     // The streaming kernel serves up to 16 (STREAM16*) or 64 tokens and needs the fast layout;
     // otherwise a tile kernel computes the same bits.

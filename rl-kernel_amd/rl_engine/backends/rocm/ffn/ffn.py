@@ -19,10 +19,11 @@ from typing import Any
 import torch
 from torch import Tensor
 
-from rl_engine import _C, _lib
+from rl_engine import _C, _host, _lib
 from rl_engine._checks import enforce
 from rl_engine.backends.rocm.gemm import swiglu_gemm
 from rl_engine.backends.rocm.gemm.det_gemm import (
+    det_gemm_backend,
     det_gemm_linear,
     det_gemm_linear_input_gradient,
     det_gemm_linear_weight_gradient,
@@ -118,6 +119,10 @@ def qwen3_ffn_packed_inference(
     del collective_handle, collective
     if tp_world_size != 1:
         raise RuntimeError("packed rollout FFN with tensor parallelism needs a collective; this build runs on one GPU")
+    if not torch.compiler.is_compiling() and det_gemm_backend() == "hip_mfma":
+        y = _host.native().packed_ffn(rmsnorm_output, fused_gate_up_weight, down_weight)  # everyday operands, natively
+        if y is not None:
+            return y
     operands = {"rmsnorm_output": rmsnorm_output, "fused_gate_up_weight": fused_gate_up_weight, "down_weight": down_weight}
     enforce(
         (t.dtype == torch.bfloat16, TypeError, f"{name} must have dtype bfloat16, got {t.dtype}.")
@@ -146,6 +151,24 @@ def _linear_gradients(a: Tensor, weight: Tensor, grad: Tensor, need_a: bool, nee
     )
 
 
+def ffn_gradients(
+    x, gate, up, activated, gate_weight, up_weight, down_weight, grad_output, need_x, need_gate, need_up, need_down, *, gate_up=None,
+) -> tuple:
+    """``(dx [tokens, hidden], d gate, d up, d down)``, ``None`` for the weights and inputs not wanted; ``gate_up``: the packed
+    projection in place of ``gate`` and ``up``."""
+    grad_output = grad_output.reshape(-1, grad_output.size(-1)).to(torch.bfloat16).contiguous()
+    grad_activated, grad_down_weight = _linear_gradients(activated, down_weight, grad_output, True, need_down)
+    if gate_up is not None:
+        grad_gate, grad_up = _C.swiglu_packed_backward(grad_activated, gate_up)
+    else:
+        grad_gate, grad_up = _C.swiglu_backward(grad_activated, gate, up)
+    grad_x, grad_gate_weight = _linear_gradients(x, gate_weight, grad_gate, need_x, need_gate)
+    from_up, grad_up_weight = _linear_gradients(x, up_weight, grad_up, need_x, need_up)
+    if need_x:
+        grad_x.add_(from_up)
+    return grad_x, grad_gate_weight, grad_up_weight, grad_down_weight
+
+
 class _DeterministicFFNFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, rmsnorm_output, gate_weight, up_weight, down_weight, fused_gate_up_weight):
@@ -168,23 +191,13 @@ class _DeterministicFFNFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
+        gate = up = gate_up = None
         if ctx.packed:
-            x, gate_up, activated, gate_weight, up_weight, down_weight = ctx.saved_tensors
+            x, gate_up, activated, *weights = ctx.saved_tensors
         else:
-            x, gate, up, activated, gate_weight, up_weight, down_weight = ctx.saved_tensors
-        grad_output = grad_output.reshape(-1, grad_output.size(-1)).to(torch.bfloat16).contiguous()
-        need = ctx.needs_input_grad
-        grad_activated, grad_down_weight = _linear_gradients(activated, down_weight, grad_output, True, need[3])
-        if ctx.packed:
-            grad_gate, grad_up = _C.swiglu_packed_backward(grad_activated, gate_up)
-        else:
-            grad_gate, grad_up = _C.swiglu_backward(grad_activated, gate, up)
-        grad_x, grad_gate_weight = _linear_gradients(x, gate_weight, grad_gate, need[0], need[1])
-        from_up, grad_up_weight = _linear_gradients(x, up_weight, grad_up, need[0], need[2])
-        if need[0]:
-            grad_x.add_(from_up)
-            grad_x = grad_x.reshape(ctx.input_shape)
-        return grad_x, grad_gate_weight, grad_up_weight, grad_down_weight, None
+            x, gate, up, activated, *weights = ctx.saved_tensors
+        grad_x, *grads = ffn_gradients(x, gate, up, activated, *weights, grad_output, *ctx.needs_input_grad[:4], gate_up=gate_up)
+        return grad_x.reshape(ctx.input_shape) if grad_x is not None else None, *grads, None
 
 
 def qwen3_ffn(
@@ -209,6 +222,10 @@ def qwen3_ffn(
         raise ValueError("sequence_parallel requires a tensor-parallel group.")
     _single_rank(tp_group, "tensor")
     _single_rank(cp_group, "context")
+    if fused_gate_up_weight is None and not torch.compiler.is_compiling() and det_gemm_backend() == "hip_mfma":
+        y = _host.native().ffn(rmsnorm_output, gate_weight, up_weight, down_weight)  # everyday operands, natively
+        if y is not None:
+            return y
     _validate_ffn_inputs(rmsnorm_output, gate_weight, up_weight, down_weight, fused_gate_up_weight)
     _lib.load()
     return _DeterministicFFNFunction.apply(rmsnorm_output, gate_weight, up_weight, down_weight, fused_gate_up_weight)

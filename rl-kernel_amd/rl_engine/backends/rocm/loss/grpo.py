@@ -17,7 +17,7 @@ from typing import NamedTuple, Optional
 import torch
 from torch.autograd import forward_ad
 
-from rl_engine import _C
+from rl_engine import _C, _host
 
 
 class GrpoLossOutput(NamedTuple):
@@ -143,6 +143,10 @@ def grpo_ratio_kl_loss(
     the rollout's tokens; masked tokens contribute zero and do not count.
     Defaults follow the reference (clip_eps 0.2, beta 0.0, grpo_loss.py:33-34).
     """
+    if not torch.compiler.is_compiling():  # everyday arguments: the same kernels and autograd function, natively
+        native = _host.native().grpo(current_logps, old_logps, ref_logps, sample_advantages, completion_mask, clip_eps, beta)
+        if native is not None:
+            return GrpoLossOutput(*native)
     if current_logps.dim() not in (1, 2):
         raise ValueError("log-probs must be [tokens] or [rollouts, tokens]")
     shape = current_logps.shape

@@ -36,15 +36,16 @@ def test_same_bits_as_the_small_tiles(shape, pitch):
     assert bool((pad[m] == 7.0).all()) and bool((pad[:, n:] == 7.0).all())
 
 
-def test_where_the_automatic_choice_takes_them():
+@pytest.mark.parametrize("shape", [(4096, 4096, 256), (4100, 4300, 64), (9000, 4096, 128)])
+def test_the_automatic_choice_runs_them_and_gives_the_bits_of_the_other_loop(shape):
     from rl_engine import _C, _lib
 
-    solo, pingpong = _lib.GEMM_CONFIGS["256x256_solo"], _lib.GEMM_CONFIGS["256x256"]
-    assert _C.det_gemm_pick_config(16384, 6144, 4096) == solo
-    assert _C.det_gemm_pick_config(4096, 4096, 4096) == solo
-    assert _C.det_gemm_pick_config(4096, 4096, 4096 + 8) == pingpong  # no whole K tiles
-    x, w = _operands((4096, 4096, 256), 3)
-    a, b = (torch.empty((4096, 4096), device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    m, n, k = shape
+    pingpong = _lib.GEMM_CONFIGS["256x256"]
+    if shape == (4096, 4096, 256):
+        assert _C.det_gemm_pick_config(m, n, k) == pingpong  # the shape; how it runs is the launch's choice
+    x, w = _operands(shape, 3)
+    a, b = (torch.empty((m, n), device=DEV, dtype=torch.bfloat16) for _ in range(2))
     _C.gemm_strided(x, w.t(), a)
     _C.gemm_strided(x, w.t(), b, config=pingpong)
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
