@@ -89,14 +89,27 @@ __device__ __forceinline__ void solo_store_span(bf16_bits* span, int grp, bool l
   }
 }
 
+// One result out of its accumulator register, where it is wanted: the compiler brings all of them into others first, which in a long
+// epilogue it does not have.
+__device__ __forceinline__ float solo_result(float accumulator) {
+  float value;
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(value) : "a"(accumulator));
+  return value;
+}
+
 typedef f32x4_t SoloAcc[SoloShape::TN][SoloShape::TM];
 
 // Runs the tiles first, first + step, ... < total (at least one). tile_at(i, n0, m0) says where tile i lies; done(i, acc, scratch)
 // takes its results, may use the spare part of the LDS if it ends on a barrier then, and returns whether this wave has issued STORES
-// vector memory instructions, no fewer: so many more may then be in flight at the first wait of the next tile.
-template <class Rows, int STORES, class TileAt, class Done>
+// vector memory instructions, no fewer: so many more may then be in flight at the first wait of the next tile. LONG: done() wants
+// the registers of the next tile's first fragments, which are read again behind it. keep() runs once per K tile: an empty asm with the
+// values that done() carries from tile to tile as its operands keeps them in registers.
+struct SoloKeepsNothing {
+  __device__ __forceinline__ void operator()() const {}
+};
+template <class Rows, int STORES, bool LONG = false, class TileAt, class Done, class Keep = SoloKeepsNothing>
 __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, int K, int first, int step, int total, char* lds,
-                                           TileAt tile_at, Done done) {
+                                           TileAt tile_at, Done done, Keep keep = Keep()) {
   using S = SoloShape;
   constexpr int kBehind = STORES + kSoloLoads < 63 ? STORES + kSoloLoads : 63;
   const int lane = threadIdx.x & 63;
@@ -125,6 +138,7 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
       const uint32_t in_row = ((lane & 7) ^ (lane >> 3)) * 16 + (kBlocksPerBase - j % kBlocksPerBase) * kBlockBytes;
       off_w[j] = row_w * (uint32_t)W.row_stride * 2 + in_row;
       off_x[j] = row_x * (uint32_t)X.row_stride * 2 + in_row;
+      asm volatile("" : "+v"(off_w[j]), "+v"(off_x[j]));  // 32 bits each: as halves of 64-bit products they took two registers
     }
   };
   aim();
@@ -153,12 +167,14 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
     u32x4_t w[S::TN], x[S::TM];
   };
   const int frag = (grp ^ (l16 & 7)) << 4;  // of the first K step of a K tile; the second one flips bit 6
-  const char* const w_rows = lds + ((wave % S::WN) * 128 + l16) * kRowBytes;
-  const char* const x_rows = lds + ((wave / S::WN) * 128 + l16) * kRowBytes;
-  auto read = [&](const char* w, const char* x, int i, Frags& f) __attribute__((always_inline)) {  // in the order of their use
-    if (i == 0) f.w[0] = *reinterpret_cast<const u32x4_t*>(w);
-    else if (i <= S::TM) f.x[i - 1] = *reinterpret_cast<const u32x4_t*>(x + (i - 1) * 16 * kRowBytes);
-    else f.w[i - S::TM] = *reinterpret_cast<const u32x4_t*>(w + (i - S::TM) * 16 * kRowBytes);
+  typedef const __attribute__((address_space(3))) char* lds_bytes_t;  // 32 bits whatever the compiler knows of `lds`
+  typedef const __attribute__((address_space(3))) u32x4_t* lds_chunk_t;
+  const lds_bytes_t w_rows = (lds_bytes_t)lds + ((wave % S::WN) * 128 + l16) * kRowBytes;
+  const lds_bytes_t x_rows = (lds_bytes_t)lds + ((wave / S::WN) * 128 + l16) * kRowBytes;
+  auto read = [&](lds_bytes_t w, lds_bytes_t x, int i, Frags& f) __attribute__((always_inline)) {  // in the order of their use
+    if (i == 0) f.w[0] = *(lds_chunk_t)w;
+    else if (i <= S::TM) f.x[i - 1] = *(lds_chunk_t)(x + (i - 1) * 16 * kRowBytes);
+    else f.w[i - S::TM] = *(lds_chunk_t)(w + (i - S::TM) * 16 * kRowBytes);
   };
 
   auto next_part = [](int at) { return at + kSoloPartBytes < kSoloLdsBytes ? at + kSoloPartBytes : 0; };
@@ -195,8 +211,8 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
       __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
       to = lds + spare;
     }
-    const char* const w = w_rows + w_part + (kSecond ? frag : frag ^ 64);
-    const char* const x = x_rows + x_part + (kSecond ? frag : frag ^ 64);
+    const lds_bytes_t w = w_rows + w_part + (kSecond ? frag : frag ^ 64);
+    const lds_bytes_t x = x_rows + x_part + (kSecond ? frag : frag ^ 64);
     __builtin_amdgcn_sched_barrier(0);
     for_blocks([&](auto row) __attribute__((always_inline)) {
       constexpr int jn = decltype(row)::value;
@@ -219,6 +235,7 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
     k_step(a, b, IntTag<0>{}, IntTag<1>{}, behind);
     k_step(b, a, IntTag<1>{}, IntTag<1>{}, behind);
     for (int t = 1; t < nk; ++t) {
+      keep();
       k_step(a, b, IntTag<0>{}, IntTag<0>{}, false);
       k_step(b, a, IntTag<1>{}, IntTag<0>{}, false);
     }
@@ -228,6 +245,10 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
                  :
                  : "memory");
     behind = done(tile, acc, lds + spare);
+    if constexpr (LONG) {
+#pragma unroll
+      for (int i = 0; i < S::TN + S::TM; ++i) read(w_rows + w_part + frag, x_rows + x_part + frag, i, a);
+    }
   }
   __builtin_amdgcn_s_waitcnt(kWaitAll0);
 }

@@ -26,6 +26,7 @@
 //   final merge over splits ascending with the same formula;
 //   lse = M + log(S);  zt = y_target;  logp = min(zt - lse, 0)
 //   e(x) = v_exp_f32(x * log2(e)) with an unfused fp32 multiply.
+#include "det_gemm_solo.h"
 #include "linear_logp_common.h"
 #include "rlk_host.h"
 
@@ -166,6 +167,209 @@ __global__ __launch_bounds__(S::kThreads) void linear_logp_partial_kernel(LogpAr
     }
   }
   logp_partial_tile<S, LOOP>(a, m0, split, lds);
+}
+
+// One wave per SIMD (det_gemm_solo.h): the loads of a unit's vocabulary tile run ahead under the tile before and its fold, and
+// stored logits leave under the next tile's products. A lane holds two runs of 16 columns, i.e. two streams, of eight tokens.
+// Bound by the package's power cap, with stored logits also by HBM. Ping-pong -> this, us, V = 151936, D = 4096: 2048 tokens 1848 ->
+// 1808 (1410 TFLOP/s), 4200 3800 -> 3700, 8192 7027 -> 6870 (1484); with stored logits at 4120 tokens 4306 -> 4167. (A workgroup per CU
+// that goes through many units, as in the GEMM, measures the same up to 10 rounds of them; behind 18 the workgroups that share
+// panels have drifted apart: 1 % slower. The two runs of a token folded side by side: 4 % slower.)
+// ST: the tile of a last row of token tiles that has at most ST::BM tokens left, a four-wave loop over 256 columns x ST::BM tokens.
+template <bool LOGITS, class S>
+__device__ __forceinline__ void logp_fold_tile(const LogpArgs& a, const f32x4_t (&acc)[S::TN][S::TM], int jm, int h, int span0, int col0,
+                                               bool span_stores, int grp, int split, int m, int tgt, float inv_t, float& run_m,
+                                               float& run_s) {
+  __builtin_amdgcn_sched_barrier(0);  // one run of 16 at a time: the accumulators and the next fragments leave few registers
+  float y[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) y[c] = solo_result(acc[4 * h + (c >> 2)][jm][c & 3]);
+  if (span0 + 64 > a.vocab_limit) {  // uniform: the last columns
+#pragma unroll
+    for (int c = 0; c < 16; ++c) y[c] = col0 + c < a.vocab_limit ? y[c] : kNegInf;
+  }
+  if constexpr (LOGITS) {  // the same accumulators the reduction sees, stored before the temperature
+    float* row = a.logits + (int64_t)(m < a.T ? m : 0) * a.logits_ld;
+    if (span_stores) store_logit_span(row, span0, grp, m < a.T, y);
+    else if (m < a.T) store_logit_run(row, col0, a.V, y);
+  }
+  // by one without a temperature: a branch around it costs the compiler its grip on the accumulators (1000 spilled registers)
+#pragma unroll
+  for (int c = 0; c < 16; ++c) y[c] = y[c] * inv_t;
+  const int at = tgt - col0;
+  float zt = 0.f;
+  logp_fold_run(y, at, run_m, run_s, zt);
+  if (at >= 0 && at < 16) a.part[(2 * (int64_t)a.n_split + split) * a.T + m] = zt;  // (logp_store_units() writes the others' zeros)
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+__device__ __forceinline__ int logp_target(const LogpArgs& a, int m) {
+  if (m >= a.T) return -1;
+  const int64_t local = a.target[m] - a.vocab_start;
+  return local >= 0 && local < a.vocab_limit ? (int)local : -1;
+}
+__device__ __forceinline__ float logp_inverse_temperature(const LogpArgs& a, int m) {
+  return m < a.T && a.temperature ? 1.0f / a.temperature[m] : 1.0f;
+}
+
+// The stream merge of `tokens` tokens whose states lie in LDS, streams `tokens` floats apart; token i of them is row m_of(i). A target
+// among the columns [v_first, v_end) of the unit has had its logit stored by the fold.
+template <class RowOf>
+__device__ __forceinline__ void logp_store_units(const LogpArgs& a, int split, int v_first, int v_end, const float* xm, const float* xs,
+                                                 int tokens, RowOf m_of) {
+  const int64_t plane = (int64_t)a.n_split * a.T;
+  for (int i = threadIdx.x; i < tokens; i += SoloShape::kThreads) {
+    const int m = m_of(i);
+    if (m >= a.T) continue;
+    float big, sum, unused;
+    logp_merge_streams(xm + i, xs + i, xs + i, tokens, big, sum, unused);
+    const int64_t at = (int64_t)split * a.T + m;
+    a.part[at] = big;
+    a.part[plane + at] = sum;
+    const int tgt = logp_target(a, m);
+    if (tgt < v_first || tgt >= v_end) a.part[2 * plane + at] = 0.f;
+  }
+}
+
+template <bool LOGITS, class S, int NS>
+__device__ __forceinline__ void logp_small_unit(const LogpArgs& a, int m0, int split, char* lds) {
+  static_assert(S::WN == 2 && S::WM == 2 && S::TN == 8, "a lane holds two streams");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = lane >> 4;
+  const int wave_n = wave % S::WN;
+  const int tok_local = wave / S::WN * 16 * S::TM + (lane & 15);
+  float run_m[2][S::TM], run_s[2][S::TM];
+#pragma unroll
+  for (int jm = 0; jm < S::TM; ++jm) {
+    run_m[0][jm] = run_m[1][jm] = kNegInf;
+    run_s[0][jm] = run_s[1][jm] = 0.f;
+  }
+  for (int t = 0; t < kLogpSplitTiles; ++t) {
+    const int v0 = split * kLogpSplitCols + t * kLogpTileCols;
+    if (v0 >= a.V) break;
+    f32x4_t acc[S::TN][S::TM];
+    tile_mainloop_quad<S, 1, NS, false>(a.W, a.H, v0, m0, a.D, lds, acc);
+    const int col = v0 + wave_n * 128 + grp * 32;  // a lane's 32 consecutive columns
+#pragma unroll
+    for (int jm = 0; jm < S::TM; ++jm) {
+      const int m = m0 + tok_local + jm * 16;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        logp_fold_tile<LOGITS, S>(a, acc, jm, h, v0 + wave_n * 128 + 64, col + 16 * h, false, grp, split, m, logp_target(a, m),
+                                  logp_inverse_temperature(a, m), run_m[h][jm], run_s[h][jm]);
+    }
+  }
+  float* const xm = reinterpret_cast<float*>(lds);  // the loop ended on a barrier
+  float* const xs = xm + kLogpStreams * S::BM;
+#pragma unroll
+  for (int jm = 0; jm < S::TM; ++jm) {
+    const int tok = tok_local + jm * 16;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      xm[(wave_n * 8 + grp * 2 + h) * S::BM + tok] = run_m[h][jm];
+      xs[(wave_n * 8 + grp * 2 + h) * S::BM + tok] = run_s[h][jm];
+    }
+  }
+  __syncthreads();
+  const int v_first = split * kLogpSplitCols;
+  logp_store_units(a, split, v_first, v_first + kLogpSplitCols, xm, xs, S::BM, [&](int i) { return m0 + i; });
+  __syncthreads();
+}
+
+struct LogpNoRest {
+  static constexpr int BM = 0;
+};
+
+template <bool LOGITS, class ST>
+__global__ __launch_bounds__(SoloShape::kThreads) void linear_logp_solo_kernel(LogpArgs a) {
+  using S = SoloShape;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_n = wave % S::WN, wave_m = wave / S::WN;
+  const int units = a.tiles_m * a.n_split;
+  if constexpr (ST::BM > 0) {
+    if ((int)blockIdx.x >= units) {
+      logp_small_unit<LOGITS, ST, kSoloLdsBytes / ST::kStageBytes>(a, a.tiles_m * S::BM, blockIdx.x - units, lds);
+      return;
+    }
+  }
+  const int id = xcd_compact_id(blockIdx.x, units);
+  const int per_group = a.group_m * a.n_split;
+  const int group = id / per_group;
+  const int first_m = group * a.group_m;
+  const int width = (a.tiles_m - first_m) < a.group_m ? (a.tiles_m - first_m) : a.group_m;
+  const int within = id - group * per_group;
+  const int m0 = (first_m + within % width) * S::BM;
+  const int split = within / width;
+  if constexpr (ST::BM > 0) {
+    if (m0 + ST::BM >= a.T) {
+      logp_small_unit<LOGITS, ST, kSoloLdsBytes / ST::kStageBytes>(a, m0, split, lds);
+      return;
+    }
+  }
+  const int v_first = split * kLogpSplitCols;
+  const int tiles = min(kLogpSplitTiles, (a.V - v_first + kLogpTileCols - 1) / kLogpTileCols);
+
+  float run_m[2][S::TM], run_s[2][S::TM];
+#pragma unroll
+  for (int jm = 0; jm < S::TM; ++jm) {
+    run_m[0][jm] = run_m[1][jm] = kNegInf;
+    run_s[0][jm] = run_s[1][jm] = 0.f;
+  }
+  auto tile_at = [&](int t, int& v0, int& m) __attribute__((always_inline)) {
+    v0 = v_first + t * kLogpTileCols;
+    m = m0;
+  };
+  auto done = [&](int t, SoloAcc& acc, char* scratch) __attribute__((always_inline)) -> bool {
+    const int lane = solo_lane(), grp = lane >> 4;
+    const int tok_local = wave_m * 128 + (lane & 15);
+    const int span = v_first + t * kLogpTileCols + wave_n * 128;
+    // (read before the first logits are stored, or each would wait for the stores before it)
+    int tgt[S::TM];
+    float inv_t[S::TM];
+#pragma unroll
+    for (int jm = 0; jm < S::TM; ++jm) {
+      tgt[jm] = logp_target(a, m0 + tok_local + jm * 16);
+      inv_t[jm] = logp_inverse_temperature(a, m0 + tok_local + jm * 16);
+    }
+#pragma unroll
+    for (int jm = 0; jm < S::TM; ++jm)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        logp_fold_tile<LOGITS, S>(a, acc, jm, h, span + h * 64, span + h * 64 + grp * 16, span + h * 64 + 64 <= a.V, grp,
+                                  split, m0 + tok_local + jm * 16, tgt[jm], inv_t[jm], run_m[h][jm], run_s[h][jm]);
+    if (t + 1 < tiles) return LOGITS && span + 128 <= a.V && m0 + S::BM <= a.T;
+
+    // the 16 streams of the unit, 128 tokens at a time
+    constexpr int kTokens = 128, kRows = S::TM / 2;
+    float* const xm = reinterpret_cast<float*>(scratch);
+    float* const xs = xm + kLogpStreams * kTokens;
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) {
+        const int jm = pass * kRows + r, tok = wave_m * 64 + r * 16 + (lane & 15);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          xm[(wave_n * 8 + h * 4 + grp) * kTokens + tok] = run_m[h][jm];
+          xs[(wave_n * 8 + h * 4 + grp) * kTokens + tok] = run_s[h][jm];
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+      wg_barrier();
+      logp_store_units(a, split, v_first, v_first + kLogpSplitCols, xm, xs, kTokens, [&](int i) { return m0 + (i >> 6) * 128 + pass * 64 + (i & 63); });
+      __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+      wg_barrier();
+    }
+    return false;
+  };
+  auto keep = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int jm = 0; jm < S::TM; ++jm)
+      asm volatile("" : "+v"(run_m[0][jm]), "+v"(run_m[1][jm]), "+v"(run_s[0][jm]), "+v"(run_s[1][jm]));
+  };
+  solo_tiles<SoloPlainRows, LOGITS ? 55 : 0, true>(a.W, a.H, a.D, 0, 1, tiles, lds, tile_at, done, keep);
 }
 
 // Few token tiles: a split of 1024 columns gives the chip only tiles_m * ceil(V / 1024)
@@ -427,11 +631,50 @@ static hipError_t launch_logp(LogpArgs a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// A last token tile with few tokens is read beside the others (its workgroups share their weight panels) or behind them, in units of
+// their own: behind eight or more whole tiles, whose groups of eight it would widen (beside / behind, us, D = 4096, V = 151936: 2100
+// tokens 2044 / 1971, 3100 with logits 3390 / 3240, 5130 4832 / 4632, 8200 7497 / 7052; V = 32768, D = 2048, 4110 with logits 690 /
+// 626), behind fewer where the last round of workgroups has little room for units of the whole size (1290 tokens, 745 units: 1380 /
+// 1343, but 1030, 596 units, with logits 1224 / 1266; 1850, 1043 units, with logits 1983 / 2080).
+static bool logp_rest_behind(int whole_tiles, int n_split, int cus) {
+  return whole_tiles >= 8 || whole_tiles * n_split % cus * 4 >= 3 * cus;
+}
+
+template <class ST>
+static hipError_t launch_logp_solo(LogpArgs a, hipStream_t stream) {
+  auto kernel = a.logits != nullptr ? linear_logp_solo_kernel<true, ST> : linear_logp_solo_kernel<false, ST>;
+  static PerDeviceOnce once[2];
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kSoloLdsBytes, once[a.logits != nullptr]);
+  if (err != hipSuccess) return err;
+  const int whole = a.T / SoloShape::BM;
+  const bool behind = ST::BM > 0 && logp_rest_behind(whole, a.n_split, device_cu_count());
+  a.tiles_m = behind ? whole : (a.T + SoloShape::BM - 1) / SoloShape::BM;
+  a.group_m = token_tiles_per_group<LogpShape256>(a.tiles_m);
+  hipLaunchKernelGGL(kernel, dim3((a.tiles_m + (behind ? 1 : 0)) * a.n_split), dim3(SoloShape::kThreads), kSoloLdsBytes, stream, a);
+  return hipGetLastError();
+}
+
+// Where one wave per SIMD is the faster loop: as for the GEMM (ping-pong / one wave, us: V = 18992 at 2000 tokens, 152 units of four
+// tiles, 282 / 293, at 8192, 608 units, 991 / 992; V = 37984 at 1700 tokens, 266 units, 629 / 639, at 2560, 380 units, 674 / 653), and
+// with stored logits from a round on (V = 18992 at 4000 tokens, 304 units, 733 / 700).
+static bool logp_solo_pays(const LogpArgs& a) {
+  const bool spans = a.logits == nullptr || ((a.logits_ld & 3) == 0 && (reinterpret_cast<uintptr_t>(a.logits) & 15) == 0);
+  if (!spans || a.bias != nullptr || !solo_offsets_fit(a.W) || !solo_offsets_fit(a.H)) return false;
+  const int cus = device_cu_count();
+  const int64_t units = (int64_t)((a.T + 127) / SoloShape::BM) * a.n_split;
+  return solo_tiles_pay(units, cus) || (a.logits != nullptr && units >= cus);
+}
+
 // 256-token tiles; a last one with few tokens runs as a tile of its size. With the groups above, us: V = 151936, D = 4096 at
 // 2100 tokens 2179 -> 2051 (with stored logits 2491 -> 2343), 4120: 3812 -> 3775 (4381 -> 4319); V = 131072, D = 2048 at 1030
 // tokens 597 -> 529, 2100: 1046 -> 988; V = 18992, D = 4096 at 1100 tokens 302 -> 271.
 static hipError_t launch_logp_256(const LogpArgs& a, hipStream_t stream) {
   const int rest = a.T % LogpShape256::BM;
+  if (logp_solo_pays(a)) {
+    if (rest >= 1 && rest <= 64) return launch_logp_solo<TileShape<256, 64, 2, 2>>(a, stream);
+    if (rest >= 1 && rest <= 128) return launch_logp_solo<TileShape<256, 128, 2, 2>>(a, stream);
+    return launch_logp_solo<LogpNoRest>(a, stream);
+  }
   if (rest >= 1 && rest <= LogpShape64::BM) return launch_logp<LogpShape256, 2, LogpShape64>(a, stream);
   if (rest >= 1 && rest <= LogpShape128::BM) return launch_logp<LogpShape256, 2, LogpShape128>(a, stream);
   return launch_logp<LogpShape256, 2>(a, stream);
