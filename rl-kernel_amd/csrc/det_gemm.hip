@@ -4,8 +4,7 @@
 // csrc/cuda/gemm/det_gemm_kernel.cu:92-101, 250-402) and the Triton MFMA kernels of
 // rl_engine/backends/rocm/gemm/mfma_gemm.py:135-274. No split-K, no atomics, no
 // stream-K: one workgroup owns an output tile for the whole K range.
-#include "det_gemm_body.h"
-#include "det_gemm_solo.h"
+#include "det_gemm_solo_body.h"
 #include "rlk_host.h"
 
 namespace rlk {
@@ -19,67 +18,26 @@ __global__ __launch_bounds__(S::kThreads + (has_prefetch_wave<LOOP, KS>() ? kWav
 }
 
 // 256 x 256 tiles, one workgroup per CU that goes through its share of them (det_gemm_solo.h).
-__global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_solo_kernel(MatView W, MatView X, bf16_bits* __restrict__ C,
-                                                                            int64_t ldc, int M, int N, int K, int tiles_m,
-                                                                            int tiles_n, int group_m) {
-  using S = SoloShape;
+template <class Layout>
+__global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_solo_kernel(SoloProblem p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  auto tile_at = [&](int block, int& n0, int& m0) __attribute__((always_inline)) {
-    const TileOrder at = tile_order(block, tiles_m, tiles_n, group_m);
-    n0 = at.tile_n * S::BN;
-    m0 = at.tile_m * S::BM;
-  };
-  auto done = [&](int block, SoloAcc& acc, char*) __attribute__((always_inline)) -> bool {
-    int n0, m0;
-    tile_at(block, n0, m0);
-    const int lane = solo_lane(), grp = lane >> 4;
-    const int n_wave = n0 + wave % S::WN * 128, m_wave = m0 + wave / S::WN * 128;
-    const int m_lane = m_wave + (lane & 15);
-    if (n_wave + 128 <= N && (reinterpret_cast<uintptr_t>(C) & 15) == 0 && (ldc & 7) == 0) {
-#pragma unroll
-      for (int jm = 0; jm < S::TM; ++jm) {
-        bf16_bits* const row = C + (int64_t)(m_lane + jm * 16) * ldc + n_wave;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          solo_store_span(row + h * 64, grp, m_lane + jm * 16 < M, acc[4 * h][jm], acc[4 * h + 1][jm], acc[4 * h + 2][jm],
-                          acc[4 * h + 3][jm]);
-      }
-      return m_wave + 128 <= M;
-    }
-#pragma unroll
-    for (int jm = 0; jm < S::TM; ++jm) {
-      const int m = m_lane + jm * 16;
-      if (m >= M) continue;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int n = n_wave + h * 64 + grp * 16;
-        bf16_bits* const dst = C + (int64_t)m * ldc + n;
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          if (n + e < N) dst[e] = to_bf16_bits(acc[4 * h + (e >> 2)][jm][e & 3]);
-      }
-    }
-    return false;
-  };
-  solo_tiles<SoloPlainRows, 4 * S::TM>(W, X, K, blockIdx.x, gridDim.x, tiles_m * tiles_n, lds, tile_at, done);
+  solo_product<Layout>(p, blockIdx.x, gridDim.x, p.tiles_m * p.tiles_n, lds);
 }
 
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
 
+template <class Layout>
 static hipError_t launch_solo(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
                               hipStream_t stream) {
+  auto kernel = det_gemm_solo_kernel<Layout>;
   static PerDeviceOnce once;
-  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(det_gemm_solo_kernel), kSoloLdsBytes, once);
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kSoloLdsBytes, once);
   if (err != hipSuccess) return err;
-  const int tiles_m = (M + SoloShape::BM - 1) / SoloShape::BM;
-  const int tiles_n = (N + SoloShape::BN - 1) / SoloShape::BN;
-  const int cus = device_cu_count();
-  const int grid = tiles_m * tiles_n < cus ? tiles_m * tiles_n : cus;
-  hipLaunchKernelGGL(det_gemm_solo_kernel, dim3(grid), dim3(SoloShape::kThreads), kSoloLdsBytes, stream, W, X,
-                     reinterpret_cast<bf16_bits*>(C), ldc, M, N, K, tiles_m, tiles_n, tiles_m < 8 ? tiles_m : 8);
+  const SoloProblem p = solo_problem(W, X, C, ldc, M, N, K);
+  const int cus = device_cu_count(), tiles = p.tiles_m * p.tiles_n;
+  hipLaunchKernelGGL(kernel, dim3(tiles < cus ? tiles : cus), dim3(SoloShape::kThreads), kSoloLdsBytes, stream, p);
   return hipGetLastError();
 }
 
@@ -479,7 +437,18 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     // activation needs at least 128 tokens per tile.
     // With few token tiles against a long reduction (grad_hidden of the LogP backward at 1024 tokens: N = 4096,
     // K = 151936) a smaller token tile doubles the workgroups, every one of which still streams its whole weight panel.
-    if (config == RLK_GEMM_CFG_AUTO) config = pick_tile_candidate(M, N, K, w_kmajor, x_kmajor);
+    if (config == RLK_GEMM_CFG_AUTO) {
+      config = pick_tile_candidate(M, N, K, w_kmajor, x_kmajor);
+      if (config == RLK_GEMM_CFG_256x256 && solo_kmajor_pays(tile_count(M, N, 256, 256), device_cu_count(), w_kmajor && x_kmajor))
+        config = RLK_GEMM_CFG_256x256_SOLO;
+    }
+    if (config == RLK_GEMM_CFG_256x256_SOLO) {
+      if (!out_f32 && solo_kmajor_fits(W) && solo_kmajor_fits(X))
+        return !x_kmajor   ? launch_solo<SoloLayout<true, false>>(W, X, C, ldc, M, N, K, stream)
+               : w_kmajor ? launch_solo<SoloLayout<true, true>>(W, X, C, ldc, M, N, K, stream)
+                          : launch_solo<SoloLayout<false, true>>(W, X, C, ldc, M, N, K, stream);
+      config = RLK_GEMM_CFG_256x256;
+    }
     switch (config) {
       case RLK_GEMM_CFG_256x256:
         return launch_kmajor<Shape256x256>(W, X, C, ldc, M, N, K, loop, out_f32, stream);
@@ -552,7 +521,7 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
   }
   if (config == RLK_GEMM_CFG_256x256_SOLO) {
     if (vec && allow_pingpong && K % kTileK == 0 && !out_f32 && solo_offsets_fit(W) && solo_offsets_fit(X))
-      return launch_solo(W, X, C, ldc, M, N, K, stream);
+      return launch_solo<SoloLayout<false, false>>(W, X, C, ldc, M, N, K, stream);
     config = RLK_GEMM_CFG_256x256;
   }
   // The element-wise loader keeps eight values per chunk in flight, and a picked 256-feature tile gives way to 128 x 128, which

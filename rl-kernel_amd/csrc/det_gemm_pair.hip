@@ -3,8 +3,9 @@
 //   dW[N_out, K_in] = dY^T X                           (both operands read K-major)
 // Neither waits for the other, and each has its own number of tiles, so launched one after the other each pays for a last
 // round of workgroups that leaves compute units idle. In one launch the workgroups of the second product take the compute
-// units that the first has no tile for. The tiles, loops and so the bits are those of det_gemm.hip.
-#include "det_gemm_body.h"
+// units that the first has no tile for. The tiles, loops and so the bits are those of det_gemm.hip: workgroups of a tile each, or, where
+// there is enough for 256 x 256 tiles, one workgroup per CU that goes through a share of both products.
+#include "det_gemm_solo_body.h"
 #include "rlk_host.h"
 
 namespace rlk {
@@ -37,6 +38,45 @@ __global__ __launch_bounds__(SX::kThreads) void det_gemm_pair_kernel(PairProblem
     if (block < dw.tiles_m * dw.tiles_n)
       det_gemm_tile<SW, kLoopPingPongBothKMajor, false, 1, 2, false>(dw.W, dw.X, dw.C, dw.ldc, dw.M, dw.N, dw.K,
                                                                      dw.tiles_m, dw.tiles_n, dw.group_m, block, lds);
+  }
+}
+
+// The same in 256 x 256 tiles with one wave per SIMD (det_gemm_solo.h), one workgroup per CU with a share of both products fixed by the
+// host: the tiles of `first` in turn, then those of the other product, of which workgroups [0, late), which have one tile of the
+// first more, take late_tiles each and the others the rest.
+struct SoloShares {
+  bool dx_first;
+  int late, late_tiles;
+};
+struct SoloPair {
+  SoloProblem dx, dw;
+  SoloShares shares;
+};
+__global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_pair_solo_kernel(SoloPair pair) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const SoloShares shares = pair.shares;
+  const int group = blockIdx.x, groups = gridDim.x;
+  for (int product = 0; product < 2; ++product) {
+    const bool is_dx = (product == 0) == shares.dx_first;
+    // Read from the arguments when its turn comes: as values of the kernel, the two products are in scalar registers at once, and
+    // spill a hundred.
+    const __attribute__((address_space(4))) SoloPair* args = (const __attribute__((address_space(4))) SoloPair*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    SoloProblem p;
+    __builtin_memcpy(&p, is_dx ? &args->dx : &args->dw, sizeof(p));
+    const int tiles = p.tiles_m * p.tiles_n;
+    int at = group, step = groups, total = tiles;
+    if (product == 1) {
+      const int of_late = min(shares.late * shares.late_tiles, tiles);
+      const bool late = group < shares.late;
+      at = late ? group : of_late + group - shares.late;
+      step = late ? shares.late : groups - shares.late;
+      total = late ? of_late : tiles;
+    }
+    if (at >= total) continue;
+    if (is_dx) solo_product<SoloLayout<true, false>>(p, at, step, total, lds);
+    else solo_product<SoloLayout<true, true>>(p, at, step, total, lds);
+    wg_barrier();  // the next product's loads overwrite what the last reads are of
   }
 }
 
@@ -85,6 +125,67 @@ static hipError_t launch_pair(const GemmProblem& dx, const GemmProblem& dw, bool
   const int first = ((dx_first ? tiles_dx : tiles_dw) + kXcds - 1) / kXcds * kXcds;
   const int second = dx_first ? tiles_dw : tiles_dx;
   hipLaunchKernelGGL(kernel, dim3(first + second), dim3(SX::kThreads), kLds, stream, a, b, first, dx_first);
+  return hipGetLastError();
+}
+
+static int64_t tile_count(const GemmProblem& p, int bn, int bm) { return (int64_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); }
+
+constexpr int64_t kSoloTileCost = 6;  // of a tile beside its K tiles, in K tiles
+static int64_t solo_length(const GemmProblem& p) { return ((int64_t)p.K + kTileK - 1) / kTileK + kSoloTileCost; }
+
+// The shares of the one-wave-per-SIMD launch, and what the workgroup with the most to do has, in K tiles. The product with the longer
+// tiles comes first; `late` workgroups have one of its tiles more than the others, and late_tiles is what evens that out.
+static SoloShares solo_shares(const GemmProblem& dx, const GemmProblem& dw, int groups, int64_t* k_tiles) {
+  SoloShares s{solo_length(dx) >= solo_length(dw), 0, 0};
+  const GemmProblem &a = s.dx_first ? dx : dw, &b = s.dx_first ? dw : dx;
+  const int64_t na = tile_count(a, 256, 256), nb = tile_count(b, 256, 256), la = solo_length(a), lb = solo_length(b);
+  const int64_t rounds = na / groups, late = na % groups;
+  s.late = (int)late;
+  *k_tiles = 0;
+  const int64_t even = ((na * la + nb * lb) / groups - (rounds + 1) * la) / lb;  // late_tiles, if all had the same
+  for (int64_t t = even < 0 ? 0 : even; t <= (even < 0 ? 0 : even + 1); ++t) {
+    const int64_t of_late = late * t < nb ? late * t : nb;
+    const int64_t others = (nb - of_late + groups - late - 1) / (groups - late);
+    int64_t span = rounds * la + others * lb;
+    if (late > 0 && (rounds + 1) * la + t * lb > span) span = (rounds + 1) * la + t * lb;
+    if (*k_tiles == 0 || span < *k_tiles) {
+      *k_tiles = span;
+      s.late_tiles = (int)t;
+    }
+  }
+  return s;
+}
+static int solo_groups(const GemmProblem& dx, const GemmProblem& dw) {
+  const int64_t tiles = tile_count(dx, 256, 256) + tile_count(dw, 256, 256);
+  const int cus = device_cu_count();
+  return (int)(tiles < cus ? tiles : cus);
+}
+// What that launch takes, on the scale of pair_us() (whose figures are 8 to 10 % below what a chip at its power cap takes): the longest
+// share at a rate, and all the work at a rate that the package's power gives. Fitted to 62 shapes of 200 to 8000 tokens within
+// 4 %. The best other configuration -> this, us, where the rule takes it (tokens, inputs, outputs):
+//   2047, 4096, 4096: 110.8 -> 102.6    601, 14336, 4096: 165.8 -> 138.9    855, 12288, 4096: 182 -> 159     1882, 14336, 4096: 372 -> 339
+//   2325, 4096, 3072: 118.6 -> 104.3    2048, 4096, 12288: 327 -> 305       5872, 4096, 14336: 1023 -> 965   7438, 4096, 1536: 179.6 -> 162.0
+//   4120, 4096, 151936: 7524 -> 7230    4120, 1024, 4096: 80.4 -> 75.6      2064, 6144, 2048: 94.5 -> 95.4   1472, 4096, 14336: 291 -> 294
+// where it does not: 1024, 4096, 4096: 64.9 / 80.1    8192, 1024, 1024: 98 / 146    1407, 4096, 24576: 474 / 489   1478, 6144, 4096: 136 / 130.5
+static double solo_pair_us(const GemmProblem& dx, const GemmProblem& dw, int cus) {
+  int64_t k_tiles;
+  solo_shares(dx, dw, solo_groups(dx, dw), &k_tiles);
+  const double work = (double)(tile_count(dx, 256, 256) * solo_length(dx) + tile_count(dw, 256, 256) * solo_length(dw)) / cus;
+  return 0.805 * k_tiles + 0.435 * work;
+}
+static bool solo_pair_serves(const GemmProblem& dx, const GemmProblem& dw) {
+  return solo_kmajor_fits(dx.W) && solo_kmajor_fits(dx.X) && solo_kmajor_fits(dw.W) && solo_kmajor_fits(dw.X);
+}
+static hipError_t launch_pair_solo(const GemmProblem& dx, const GemmProblem& dw, hipStream_t stream) {
+  static PerDeviceOnce once;
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(det_gemm_pair_solo_kernel), kSoloLdsBytes, once);
+  if (err != hipSuccess) return err;
+  auto problem = [](const GemmProblem& p) { return solo_problem(p.W, p.X, p.C, p.ldc, p.M, p.N, p.K); };
+  const int groups = solo_groups(dx, dw);
+  int64_t k_tiles;
+  const SoloShares shares = solo_shares(dx, dw, groups, &k_tiles);
+  hipLaunchKernelGGL(det_gemm_pair_solo_kernel, dim3(groups), dim3(SoloShape::kThreads), kSoloLdsBytes, stream,
+                     SoloPair{problem(dx), problem(dw), shares});
   return hipGetLastError();
 }
 
@@ -139,8 +240,6 @@ static double dx_tile_us(const PairTiles& t, const GemmProblem& dx, int tokens, 
 static double dw_tile_us(const PairTiles& t, const GemmProblem& dw) {
   return tile_us(t.dw_bn, t.dw_bm, t.dw_quality, kStartDwUs, dw.K);
 }
-
-static int64_t tile_count(const GemmProblem& p, int bn, int bm) { return (int64_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); }
 
 // The time of the one launch: the work of all tiles at the full chip's rate, or the span of tiles of which some run with
 // much of the chip idle. A tile takes 0.6 of its time alone (256 x 256, K = 4096: 95 -> 65 us, 256 x 128: 68 -> 48.5), the
@@ -243,13 +342,19 @@ LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem
     const int whole = dx.M - rest;
     const double head = det_gemm_kmajor_us(whole, dx.N, dx.K, true, false, partial);
     const double with_rest = head + kLaunchUs + best_pair_us(tail_of(dx, whole), dw, cus, of, &config);
-    if (with_rest < best) plan = {config, whole};
+    if (with_rest < best) {
+      best = with_rest;
+      plan = {config, whole};
+    }
   }
+  const double solo = solo_pair_us(dx, dw, cus);
+  plan.solo = solo < best && solo_pair_serves(dx, dw);
   return plan;
 }
 
 hipError_t linear_backward_launch(GemmProblem dx, const GemmProblem& dw, LinearBackwardPlan plan, hipStream_t stream) {
   if (!one_launch_serves(dx, dw)) plan = {RLK_LINEAR_BWD_CFG_SEPARATE, 0};
+  if (plan.solo && solo_pair_serves(dx, dw)) return launch_pair_solo(dx, dw, stream);
   if (plan.head_rows > 0) {
     const GemmProblem head = head_of(dx, plan.head_rows);
     const hipError_t err = det_gemm_launch(head.W, head.X, head.C, head.ldc, head.M, head.N, head.K, false, RLK_GEMM_CFG_AUTO, stream);

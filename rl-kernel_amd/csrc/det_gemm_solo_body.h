@@ -1,0 +1,71 @@
+// A workgroup's share of a product's 256 x 256 tiles on the loop of det_gemm_solo.h, with the rounding and the stores.
+#pragma once
+
+#include "det_gemm_body.h"
+#include "det_gemm_solo.h"
+
+namespace rlk {
+
+// C[M, N] = X[M, K] W[N, K]^T in tiles_m x tiles_n tiles.
+struct SoloProblem {
+  MatView W, X;
+  bf16_bits* C;
+  int64_t ldc;
+  int M, N, K;
+  int tiles_m, tiles_n, group_m;
+};
+inline SoloProblem solo_problem(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K) {
+  SoloProblem p{W, X, reinterpret_cast<bf16_bits*>(C), ldc, M, N, K, (M + SoloShape::BM - 1) / SoloShape::BM,
+                (N + SoloShape::BN - 1) / SoloShape::BN, 1};
+  p.group_m = p.tiles_m < 8 ? p.tiles_m : 8;
+  return p;
+}
+
+// The tiles first, first + step, ... < total in the order of tile_order(); at least one.
+template <class Layout>
+__device__ __forceinline__ void solo_product(const SoloProblem& p, int first, int step, int total, char* lds) {
+  using S = SoloShape;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto tile_at = [&](int block, int& n0, int& m0) __attribute__((always_inline)) {
+    const TileOrder at = tile_order(block, p.tiles_m, p.tiles_n, p.group_m);
+    n0 = at.tile_n * S::BN;
+    m0 = at.tile_m * S::BM;
+  };
+  auto done = [&](int block, SoloAcc& acc, char*) __attribute__((always_inline)) -> bool {
+    int n0, m0;
+    tile_at(block, n0, m0);
+    const int lane = solo_lane(), grp = lane >> 4;
+    const int n_wave = n0 + wave % S::WN * 128, m_wave = m0 + wave / S::WN * 128;
+    const int m_lane = m_wave + (lane & 15);
+    if (n_wave + 128 <= p.N && (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 && (p.ldc & 7) == 0) {
+#pragma unroll
+      for (int jm = 0; jm < S::TM; ++jm) {
+        bf16_bits* const row = p.C + (int64_t)(m_lane + jm * 16) * p.ldc + n_wave;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const auto &a = acc[4 * h][jm], &b = acc[4 * h + 1][jm], &c = acc[4 * h + 2][jm], &d = acc[4 * h + 3][jm];
+          if constexpr (Layout::kW) solo_store_span_kmajor(row + h * 64, grp, m_lane + jm * 16 < p.M, a, b, c, d);
+          else solo_store_span(row + h * 64, grp, m_lane + jm * 16 < p.M, a, b, c, d);
+        }
+      }
+      return m_wave + 128 <= p.M;
+    }
+#pragma unroll
+    for (int jm = 0; jm < S::TM; ++jm) {
+      const int m = m_lane + jm * 16;
+      if (m >= p.M) continue;
+      bf16_bits* const row = p.C + (int64_t)m * p.ldc;
+#pragma unroll
+      for (int jn = 0; jn < S::TN; ++jn) {
+        const int n = n_wave + (Layout::kW ? jn * 16 + grp * 4 : jn / 4 * 64 + grp * 16 + jn % 4 * 4);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (n + q < p.N) row[n + q] = to_bf16_bits(acc[jn][jm][q]);
+      }
+    }
+    return false;
+  };
+  solo_tiles<SoloPlainRows, 4 * S::TM, false, Layout>(p.W, p.X, p.K, first, step, total, lds, tile_at, done);
+}
+
+}  // namespace rlk

@@ -59,6 +59,13 @@ inline bool solo_tiles_pay(int64_t tiles, int cus) {
   return tiles >= 2 * cus || last == 0 || last * 2 > cus;
 }
 
+// The same with a K-major operand, or two, whose ping-pong loops read 24 or 36 times from LDS per 32 MFMAs. Ping-pong / one wave, us:
+// both K-major, K = 4096, 4096 inputs, 96 tiles 77.8 / 76.7, 128: 79.0 / 78.1, 192: 87.8 / 85.4, 256: 103.0 / 100.9, 288: 171.3 /
+// 165.6, 384: 185.7 / 176.5, 768: 312 / 300, 9504 4060 / 3822, K = 12288 with 144 239 / 220, K = 1024 with 1536 195.2 / 175.6; a
+// K-major weight, K = 4096, 128 tiles 68.3 / 70.9, 160: 74.8 / 75.1, 176: 78.0 / 77.4, 256: 97.7 / 95.5, 288: 157.2 / 155.7, 768:
+// 299 / 288, K = 151936 with 256 3402 / 3340; K-major tokens, 9504 tiles 3826 / 3594. Few tiles lose 4 to 13 %.
+inline bool solo_kmajor_pays(int64_t tiles, int cus, bool both) { return 3 * tiles >= (both ? cus : 2 * cus); }
+
 // Whether a kernel loads the weight past the caches (non-temporal): its M tokens are one token tile of `bm`, or two whole
 // ones, whose workgroups read a weight line at the same time. A weight of 96 MiB or more does not wait in the 256 MB
 // memory-side cache for its next use once the other layers have passed through, and reads that leave nothing there are
@@ -99,6 +106,7 @@ struct GemmProblem {
 struct LinearBackwardPlan {
   int config;     // rlk_linear_bwd_config, not AUTO
   int head_rows;  // rows of dx that a launch of their own computes first
+  bool solo = false;  // instead, all of both products in 256 x 256 tiles with one wave per SIMD
 };
 // Whose backward it is: a linear layer's right behind its forward; the LogP's, whose own two launches are what the one competes
 // with; or that of a layer with more weights than the memory-side cache holds from the forward to the backward.

@@ -101,3 +101,83 @@ def test_no_part_is_overwritten_before_it_is_read(k_tiles, tiles):
         x = nxt(w)
         issue("x", old_w)
         head += 1
+
+
+def kmajor_swizzle(k_row):
+    return 4 * ((k_row >> 1) & 1) + 2 * (((k_row >> 3) ^ (k_row >> 4)) & 1)
+
+
+def kmajor_loads(rows, k_left, ld):
+    """The same of a K-major operand: rows its matrix has from the tile's first one on, K values left from the K tile's first one on."""
+    for wave in range(4):
+        for j in range(LOADS):
+            for lane in range(64):
+                rib = lane >> 3
+                first = wave * 64 + ((lane & 7) ^ (4 * ((rib >> 1) & 1))) * 8
+                off = (rib * ld * 2 + min(first ^ (((j ^ (j >> 1)) & 1) * 16), rows - 8) * 2) % U32
+                scalar = ld * 16 * j + 4 * 1024 - (j % 4) * 1024
+                lds = (wave * LOADS + j) * 1024 + lane * 16
+                outside = rib >= k_left - 8 * j
+                yield lds, (0x80000000 if outside else off), scalar, (j % 4) * 1024
+
+
+@pytest.mark.parametrize("rows", [256, 264, 200, 8])
+@pytest.mark.parametrize("k_left", [64, 24, 1, 63])
+@pytest.mark.parametrize("ld", [264, 4096, 151936, (1 << 23) - 8])
+def test_kmajor_columns_arrive_once_and_are_read_where_they_lie(rows, k_left, ld):
+    span = 0x7FFF0000  # what the hardware takes as inside the buffer, which begins 4 KiB before the operand
+    seen = {}
+    for lds, off, scalar, imm in kmajor_loads(rows, k_left, ld):
+        assert lds not in seen and 0 <= lds < PART
+        if off >= span - scalar - imm:
+            assert off == 0x80000000
+            seen[lds] = None  # zeros
+            continue
+        k_row, at = divmod(off + scalar + imm - 4 * 1024, ld * 2)
+        assert 0 <= k_row < min(64, k_left) and at % 16 == 0 and at // 2 + 8 <= rows
+        seen[lds] = (k_row, at // 2)
+    assert len(seen) == PART // 16
+    # a transposing read: eight bytes of a lane, row tile j16 of a column, K row of its step, lane group and half
+    for tile in range(16):
+        for k in range(64):
+            step, grp, half, a = k // 32, k // 8 % 4, k // 4 % 2, k % 4
+            for l4 in range(4):  # the lane's four rows: 4 l4 .. + 3 of the tile
+                tr_row = grp * 8 + a
+                tr_at = tr_row * 128 + (((l4 >> 1) ^ kmajor_swizzle(tr_row)) << 4) + (l4 & 1) * 8
+                place = tile // 4 * 8192 + (tr_at ^ (tile % 4) << 5) + step * 4096 + half * 512
+                first = tile * 16 + l4 // 2 * 8
+                want = (k, min(first, rows - 8)) if k < k_left else None
+                assert seen[place // 16 * 16] == want and place % 16 == (l4 & 1) * 8
+
+
+def shares(na, la, nb, lb, groups):
+    """solo_shares(): tiles of the first product and of the second, their lengths in K tiles."""
+    rounds, late = divmod(na, groups)
+    even = ((na * la + nb * lb) // groups - (rounds + 1) * la) / lb
+    best = None
+    for t in [0] if even < 0 else [int(even), int(even) + 1]:
+        of_late = min(late * t, nb)
+        others = -(-(nb - of_late) // (groups - late))
+        span = max(rounds * la + others * lb, (rounds + 1) * la + t * lb if late else 0)
+        if best is None or span < best[0]:
+            best = (span, late, t)
+    return best
+
+
+@pytest.mark.parametrize("na,la,nb,lb", [(128, 70, 256, 38), (272, 2380, 9504, 71), (1, 7, 1, 7), (256, 70, 256, 70), (3, 90, 700, 10), (700, 20, 1, 8)])
+def test_two_products_are_shared_out_whole(na, la, nb, lb):
+    groups = min(256, na + nb)
+    span, late, late_tiles = shares(na, la, nb, lb, groups)
+    first, second, longest = [], [], 0
+    for g in range(groups):
+        of_late = min(late * late_tiles, nb)
+        mine = list(range(g, na, groups))
+        if g < late:
+            more = list(range(g, of_late, late))
+        else:
+            more = list(range(of_late + g - late, nb, groups - late))
+        first += mine
+        second += more
+        longest = max(longest, len(mine) * la + len(more) * lb)
+    assert sorted(first) == list(range(na)) and sorted(second) == list(range(nb)) and longest <= span
+    assert span <= (na * la + nb * lb) / groups + la + lb

@@ -63,3 +63,99 @@ def test_gated_projection(tokens, inter, k):
     gate_up = torch.empty((tokens, 2 * inter), device=DEV, dtype=torch.bfloat16)
     _C.gemm_strided(x, w.t(), gate_up, config=3)  # 128 x 128
     assert torch.equal(y.view(torch.int16), _C.swiglu_packed_forward(gate_up).view(torch.int16))
+
+
+# (tokens, outputs, K): one K tile and less, a few values more than whole K tiles, odd ones, edges of tiles of either side, more
+# tiles than CUs
+KMAJOR_SHAPES = [(8, 8, 8), (256, 256, 24), (264, 520, 64), (248, 776, 72), (1000, 264, 200), (512, 512, 2056), (4360, 4360, 136)]
+
+
+@pytest.mark.parametrize("shape", KMAJOR_SHAPES)
+@pytest.mark.parametrize("w_kmajor,x_kmajor", [(True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("pitch", [8, 3])  # of the result beyond its columns: whole 16-byte stores, element stores
+def test_kmajor_operands(shape, w_kmajor, x_kmajor, pitch):
+    """The bits of the two-group loop of the same operands; with both K-major also reductions of odd length."""
+    from rl_engine import _C, _lib
+
+    m, n, k = shape
+    gen = torch.Generator(device=DEV).manual_seed(m + k)
+
+    def operand(rows, length, kmajor):
+        shape = (length, rows) if kmajor else (rows, length)
+        t = torch.randn(shape, generator=gen, device=DEV, dtype=torch.bfloat16)
+        return t.t() if kmajor else t
+
+    for length in (k, k + 1, k + 63) if w_kmajor and x_kmajor else (k,):
+        if not w_kmajor and length % 64 == 0 and x_kmajor:
+            length += 8
+        x, w = operand(m, length, x_kmajor), operand(n, length, w_kmajor)
+        want = torch.empty((m, n), device=DEV, dtype=torch.bfloat16)
+        _C.gemm_strided(x.contiguous(), w.contiguous().t(), want, config=3)  # 128 x 128, native operands
+        pad = torch.full((m + 1, n + pitch), 7.0, device=DEV, dtype=torch.bfloat16)
+        for _ in range(2):
+            _C.gemm_strided(x, w.t(), pad[:m, :n], config=_lib.GEMM_CONFIGS["256x256_solo"])
+            assert torch.equal(pad[:m, :n].contiguous().view(torch.int16), want.view(torch.int16)), length
+        assert bool((pad[m] == 7.0).all()) and bool((pad[:, n:] == 7.0).all())
+
+
+def test_nothing_past_a_reduction_is_used():
+    """The values behind the reduction's end, which lie in memory beside it, are NaN: the next K rows of K-major operands, the rest
+    of the rows of a native one."""
+    from rl_engine import _C, _lib
+
+    m, n, k = 520, 264, 136
+    x = torch.full((m, k + 64), float("nan"), device=DEV, dtype=torch.bfloat16)
+    xt = torch.full((k + 64, m), float("nan"), device=DEV, dtype=torch.bfloat16)
+    w = torch.full((k + 64, n), float("nan"), device=DEV, dtype=torch.bfloat16)
+    x[:, :k].normal_()
+    xt[:k] = x[:, :k].t()
+    w[:k].normal_()
+    want = torch.empty((m, n), device=DEV, dtype=torch.bfloat16)
+    _C.gemm_strided(x[:, :k].contiguous(), w[:k].t().contiguous().t(), want, config=3)
+    for a in (x[:, :k], xt[:k].t()):
+        got = torch.empty_like(want)
+        _C.gemm_strided(a, w[:k], got, config=_lib.GEMM_CONFIGS["256x256_solo"])
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# (tokens, inputs, outputs): one tile each, one of either and many of the other, both products longer, shares of two sizes
+PAIR_SHAPES = [(8, 8, 8), (64, 264, 8200), (2304, 256, 320), (1030, 1032, 2056), (2047, 4096, 4096), (4120, 4096, 1600), (300, 16384, 4160)]
+
+
+@pytest.mark.parametrize("tokens,inputs,outputs", PAIR_SHAPES)
+def test_both_gradients_of_a_linear_layer(tokens, inputs, outputs):
+    from rl_engine import _lib
+
+    lib = _lib.load()
+    gen = torch.Generator(device=DEV).manual_seed(tokens)
+    g, x, w = (torch.randn(s, generator=gen, device=DEV, dtype=torch.bfloat16) for s in ((tokens, outputs), (tokens, inputs), (outputs, inputs)))
+
+    def backward(config):
+        dx, dw = torch.full_like(x, 7.0), torch.full_like(w, 7.0)
+        stream = torch.cuda.current_stream().cuda_stream
+        assert lib.rlk_linear_bwd_bf16(g.data_ptr(), outputs, x.data_ptr(), inputs, w.data_ptr(), inputs, dx.data_ptr(), inputs,
+                                       dw.data_ptr(), inputs, tokens, inputs, outputs, config, stream) == 0  # fmt: skip
+        return dx.view(torch.int16), dw.view(torch.int16)
+
+    want = backward(1)
+    for config in (_lib.LINEAR_BWD_SOLO, 0):
+        got = backward(config)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("tokens,vocab", [(2050, 12337), (4120, 9000)])
+def test_gradients_of_the_logp_at_a_ragged_vocabulary(tokens, vocab):
+    """Sizes where they run in one launch of these tiles: the bits of each gradient asked for alone."""
+    from rl_engine import _C
+
+    gen = torch.Generator(device=DEV).manual_seed(tokens)
+    h = torch.randn((tokens, 2048), generator=gen, device=DEV, dtype=torch.bfloat16)
+    w = torch.randn((vocab, 2048), generator=gen, device=DEV, dtype=torch.bfloat16).mul_(0.02)
+    ids = torch.randint(0, vocab, (tokens,), generator=gen, device=DEV)
+    _, lse = _C.fused_linear_logp(h, w, ids)
+    grad = torch.randn(tokens, generator=gen, device=DEV)
+    both = _C.fused_linear_logp_bwd(h, w, ids, lse, grad, None)
+    hidden = _C.fused_linear_logp_bwd(h, w, ids, lse, grad, None, need_grad_weight=False)
+    weight = _C.fused_linear_logp_bwd(h, w, ids, lse, grad, None, need_grad_hidden=False)
+    assert torch.equal(both[0].view(torch.int16), hidden[0].view(torch.int16))
+    assert torch.equal(both[1].view(torch.int16), weight[1].view(torch.int16))
