@@ -67,7 +67,10 @@ typedef enum rlk_gemm_config {
   /* OR-ed into a configuration: use the register-staged main loop even where the
    * direct-to-LDS ping-pong loop applies. Bit-neutral; exists so tests can
    * compare the two loops. */
-  RLK_GEMM_CFG_FORCE_STAGED = 0x100
+  RLK_GEMM_CFG_FORCE_STAGED = 0x100,
+  /* OR-ed into 256x128 (K-major weight), 192x256, 192x128, 192x192 (native operands) or 256x192 (either): four waves, one per SIMD,
+   * instead of eight. The automatic choice runs a picked shape that way where it is faster. Other operands run the plain shape. */
+  RLK_GEMM_CFG_FOUR_WAVES = 0x200
 } rlk_gemm_config;
 
 /* Arithmetic contract identifier (provenance string).

@@ -33,12 +33,18 @@ static hipError_t launch_solo(const MatView& W, const MatView& X, void* C, int64
                               hipStream_t stream) {
   auto kernel = det_gemm_solo_kernel<Layout>;
   static PerDeviceOnce once;
-  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kSoloLdsBytes, once);
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), Layout::kLds, once);
   if (err != hipSuccess) return err;
-  const SoloProblem p = solo_problem(W, X, C, ldc, M, N, K);
+  const SoloProblem p = solo_problem<typename Layout::Shape>(W, X, C, ldc, M, N, K);
   const int cus = device_cu_count(), tiles = p.tiles_m * p.tiles_n;
-  hipLaunchKernelGGL(kernel, dim3(tiles < cus ? tiles : cus), dim3(SoloShape::kThreads), kSoloLdsBytes, stream, p);
+  hipLaunchKernelGGL(kernel, dim3(tiles < cus ? tiles : cus), dim3(SoloShape::kThreads), Layout::kLds, stream, p);
   return hipGetLastError();
+}
+
+// A smaller shape on four waves, native operands.
+template <int BN, int BM>
+static hipError_t launch_solo_shape(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K, hipStream_t stream) {
+  return launch_solo<SoloLayout<false, false, TileShape<BN, BM, 2, 2>>>(W, X, C, ldc, M, N, K, stream);
 }
 
 template <class S, int LOOP, bool OUT_F32, int KS = 1, int NS = 2>
@@ -254,18 +260,48 @@ int device_cu_count() {
 // workgroup per CU, each streaming a narrow slice of the weight instead of a 256-column one (1.9 -> 0.8 ms at 256
 // tokens, 1.8 -> 1.03 ms at 512, 1.65 -> 1.45 ms at 1024); their qualities are those of the direct-to-LDS loop. 256 x 192:
 // dX of 14336 inputs, 4096 outputs at 540 / 1300 tokens 106 / 169 -> 68 / 142 us, of 4096, 6144 at 2300 tokens 108 -> 95.
+//
+// The `four` column is that of the four-wave forms of the native shapes (det_gemm_solo.h, 0: none), which whole K tiles and bf16
+// results have. Waves of half a tile by half read every row of a K tile from LDS twice, where eight of a quarter by half read token
+// rows four times; those reads and what arrives are 1856 cycles of LDS a K tile beside 1536 of MFMAs in 192 x 256, 1344 with four
+// waves, 1536 / 1152 beside 1152 in 192 x 192. With them a round that fills part of the chip costs less, the more so behind others
+// (kPartialFirst, kPartialLast). 170 shapes of 14 layers, 300 to 7000 tokens, weights in turn: 0.957 of the time before on the 91 that
+// are not the deep tiles', 0.2 % above the best shape of each (worst 4 %). Before -> with them, us: 4096 outputs, K = 4096 at 1400 /
+// 2047 / 3000 tokens 53.9 / 62.8 / 79.1 -> 49.7 / 57.8 / 73.8, 6144 at 1024 / 2048 / 3072 56.9 / 83.6 / 124.8 -> 51.7 / 78.4 /
+// 117.9, K = 12288 at 2047 176 -> 164, 24576 outputs at 700 / 1024 129.9 / 167.4 -> 120.2 / 156.6. (256 x 128 and 128 x 128 on four
+// waves were never the best shape by more than the noise.)
 struct TileCandidate {
   int config, bn, bm;
   double native, ragged192, w_kmajor;
   bool x_kmajor;
+  double four;
 };
 static const TileCandidate kTileCandidates[] = {
-    {RLK_GEMM_CFG_256x256, 256, 256, 1.00, 0.00, 1.00, true},  {RLK_GEMM_CFG_192x256, 192, 256, 0.89, 0.85, 0.00, false},
-    {RLK_GEMM_CFG_256x192, 256, 192, 0.87, 0.00, 0.87, false}, {RLK_GEMM_CFG_192x192, 192, 192, 0.75, 0.68, 0.00, false},
-    {RLK_GEMM_CFG_256x128, 256, 128, 0.65, 0.00, 0.70, true},  {RLK_GEMM_CFG_192x128, 192, 128, 0.56, 0.53, 0.00, false},
-    {RLK_GEMM_CFG_256x64, 256, 64, 0.50, 0.00, 0.56, false},   {RLK_GEMM_CFG_128x128, 128, 128, 0.65, 0.00, 0.62, false},
-    {RLK_GEMM_CFG_128x64, 128, 64, 0.45, 0.00, 0.40, false},   {RLK_GEMM_CFG_64x64, 64, 64, 0.42, 0.00, 0.25, false},
+    {RLK_GEMM_CFG_256x256, 256, 256, 1.00, 0.00, 1.00, true, 1.00},  {RLK_GEMM_CFG_192x256, 192, 256, 0.89, 0.85, 0.00, false, 0.95},
+    {RLK_GEMM_CFG_256x192, 256, 192, 0.87, 0.00, 0.87, false, 0.94}, {RLK_GEMM_CFG_192x192, 192, 192, 0.75, 0.68, 0.00, false, 0.93},
+    {RLK_GEMM_CFG_256x128, 256, 128, 0.65, 0.00, 0.70, true, 0.00},  {RLK_GEMM_CFG_192x128, 192, 128, 0.56, 0.53, 0.00, false, 0.80},
+    {RLK_GEMM_CFG_256x64, 256, 64, 0.50, 0.00, 0.56, false, 0.00},   {RLK_GEMM_CFG_128x128, 128, 128, 0.65, 0.00, 0.62, false, 0.40},
+    {RLK_GEMM_CFG_128x64, 128, 64, 0.45, 0.00, 0.40, false, 0.25},   {RLK_GEMM_CFG_64x64, 64, 64, 0.42, 0.00, 0.25, false, 0.00},
 };
+constexpr double kPartialFirst = 0.82, kPartialLast = 0.6, kFourRagged192 = 0.92;
+
+// The cheapest shape for native operands whose K tiles are whole, bf16 results: four waves where the shape has them.
+static int pick_four_wave_shape(int M, int N) {
+  const int cus = device_cu_count();
+  int best = RLK_GEMM_CFG_256x256;
+  double best_time = 1e300;
+  for (const TileCandidate& c : kTileCandidates) {
+    if (c.four == 0.0) continue;
+    const double quality = c.four * (c.bn == 192 && N % 192 != 0 ? kFourRagged192 : 1.0);
+    const int64_t tiles = tile_count(M, N, c.bm, c.bn);
+    const double t = rounds_of_workgroups(tiles, cus, tiles <= cus ? kPartialFirst : kPartialLast) * (double)(c.bn * c.bm) / quality;
+    if (t < best_time * 0.999) {
+      best_time = t;
+      best = c.config;
+    }
+  }
+  return best;
+}
 
 // The cheapest candidate by the estimate above. `w_kmajor` / `x_kmajor`: the operand layouts of the call.
 static const TileCandidate& best_tile_candidate(int M, int N, int K, bool w_kmajor, bool x_kmajor, double partial_floor,
@@ -306,7 +342,7 @@ double det_gemm_kmajor_us(int M, int N, int K, bool w_kmajor, bool x_kmajor, dou
   return (11.0 + 21.0 * K / 1024.0) * outputs / 65536.0;
 }
 
-int pick_det_gemm_config(int M, int N, int K) {
+int pick_det_gemm_config(int M, int N, int K, bool out_f32) {
   const int cus = device_cu_count();
   // Decode (weights fitted while they rotate through 1.3 GB, i.e. come from HBM as in a model with
   // many layers, not from the 256 MB memory-side cache): up to 16 tokens the streaming kernel with
@@ -350,7 +386,7 @@ int pick_det_gemm_config(int M, int N, int K) {
     if (tile_count(M, N, 160, 64) <= cus) return RLK_GEMM_CFG_64x160_DEEP;
     if (tile_count(M, N, 128, 128) <= cus) return RLK_GEMM_CFG_128x128_DEEP;
   }
-  return pick_tile_candidate(M, N, K, false, false);
+  return K % kTileK == 0 && !out_f32 ? pick_four_wave_shape(M, N) : pick_tile_candidate(M, N, K, false, false);
 }
 
 // A K-major view (element [row, k] at ptr[k * k_stride + row], rows contiguous: B[K,N] as the
@@ -429,7 +465,8 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
   const bool w_native = view_is_vectorizable(W), x_native = view_is_vectorizable(X);
   const bool vec = w_native && x_native && (K % kChunkElems) == 0;
   const bool allow_pingpong = (config & RLK_GEMM_CFG_FORCE_STAGED) == 0;
-  config &= ~RLK_GEMM_CFG_FORCE_STAGED;
+  bool four_waves = (config & RLK_GEMM_CFG_FOUR_WAVES) != 0;
+  config &= ~(RLK_GEMM_CFG_FORCE_STAGED | RLK_GEMM_CFG_FOUR_WAVES);
   const bool w_kmajor = !w_native && view_is_kmajor_fast(W), x_kmajor = !x_native && view_is_kmajor_fast(X);
   if (allow_pingpong && det_gemm_takes_kmajor(W, X, K)) {
     const int loop = w_kmajor ? (x_kmajor ? kLoopPingPongBothKMajor : kLoopPingPongKMajor) : kLoopPingPongXKMajor;
@@ -439,6 +476,10 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     // K = 151936) a smaller token tile doubles the workgroups, every one of which still streams its whole weight panel.
     if (config == RLK_GEMM_CFG_AUTO) {
       config = pick_tile_candidate(M, N, K, w_kmajor, x_kmajor);
+      // 256 x 192 always; 256 x 128 where the weight can still be in the memory-side cache: from HBM the eight waves are faster (12288
+      // outputs, K = 4096 at 324 / 483 tokens 58.9 / 61.1 us, four 65.4 / 68.7). Eight -> four: 4096 outputs at 1400 / 2047 tokens
+      // 59.5 / 66.7 -> 54.3 / 59.1, 256 x 192: 2300 tokens, K = 6144 104 -> 98, K = 14336 at 5969 495 -> 467.
+      four_waves = config == RLK_GEMM_CFG_256x192 || (int64_t)N * K * 2 < ((int64_t)96 << 20);
       if (config == RLK_GEMM_CFG_256x256 && solo_kmajor_pays(tile_count(M, N, 256, 256), device_cu_count(), w_kmajor && x_kmajor))
         config = RLK_GEMM_CFG_256x256_SOLO;
     }
@@ -453,9 +494,13 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
       case RLK_GEMM_CFG_256x256:
         return launch_kmajor<Shape256x256>(W, X, C, ldc, M, N, K, loop, out_f32, stream);
       case RLK_GEMM_CFG_256x192:
+        if (four_waves && w_kmajor && !out_f32 && solo_kmajor_fits(W) && solo_kmajor_fits(X))
+          return launch_solo<SoloLayout<true, false, TileShape<256, 192, 2, 2>>>(W, X, C, ldc, M, N, K, stream);
         if (!x_kmajor) return launch_kmajor<Shape256x192>(W, X, C, ldc, M, N, K, loop, out_f32, stream);
         break;
       case RLK_GEMM_CFG_256x128:
+        if (four_waves && w_kmajor && !x_kmajor && !out_f32 && solo_kmajor_fits(W) && solo_kmajor_fits(X))
+          return launch_solo<SoloLayout<true, false, TileShape<256, 128, 2, 2>>>(W, X, C, ldc, M, N, K, stream);
         return launch_kmajor<Shape256x128>(W, X, C, ldc, M, N, K, loop, out_f32, stream);
       case RLK_GEMM_CFG_256x64:
         if (!x_kmajor) return launch_kmajor<Shape256x64>(W, X, C, ldc, M, N, K, loop, out_f32, stream);
@@ -474,7 +519,8 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     }
   }
   if (config == RLK_GEMM_CFG_AUTO) {
-    config = pick_det_gemm_config(M, N, K);
+    config = pick_det_gemm_config(M, N, K, out_f32);
+    four_waves = true;  // where the shape has them and the operands are theirs
     // the picked shape with one wave per SIMD (which a call can ask for, and which is 256 x 256 again for what it does not take)
     if (config == RLK_GEMM_CFG_256x256 && solo_tiles_pay(tile_count(M, N, 256, 256), device_cu_count()))
       config = RLK_GEMM_CFG_256x256_SOLO;
@@ -485,7 +531,7 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     const int max_m = config == RLK_GEMM_CFG_STREAM64 ? 64 : 16;
     if (M <= max_m && vec && allow_pingpong && K % kTileK == 0)
       return det_gemm_stream_launch(W, X, C, ldc, M, N, K, out_f32, config == RLK_GEMM_CFG_STREAM16, stream);
-    config = M <= 16 ? RLK_GEMM_CFG_16x16 : M <= 64 ? RLK_GEMM_CFG_64x64 : pick_det_gemm_config(M, N, K);
+    config = M <= 16 ? RLK_GEMM_CFG_16x16 : M <= 64 ? RLK_GEMM_CFG_64x64 : pick_det_gemm_config(M, N, K, out_f32);
     if (config == RLK_GEMM_CFG_STREAM64) config = RLK_GEMM_CFG_64x64;
   }
   // Deep-stage variants need the fast layout and whole stages; otherwise the plain shape
@@ -523,6 +569,21 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     if (vec && allow_pingpong && K % kTileK == 0 && !out_f32 && solo_offsets_fit(W) && solo_offsets_fit(X))
       return launch_solo<SoloLayout<false, false>>(W, X, C, ldc, M, N, K, stream);
     config = RLK_GEMM_CFG_256x256;
+  }
+  if (four_waves && vec && allow_pingpong && K % kTileK == 0 && !out_f32 && solo_offsets_fit(W) && solo_offsets_fit(X)) {
+    switch (config) {  // (weights read past the caches are the eight waves')
+      case RLK_GEMM_CFG_256x192:
+        return launch_solo_shape<256, 192>(W, X, C, ldc, M, N, K, stream);
+      case RLK_GEMM_CFG_192x256:
+        return launch_solo_shape<192, 256>(W, X, C, ldc, M, N, K, stream);
+      case RLK_GEMM_CFG_192x192:
+        return launch_solo_shape<192, 192>(W, X, C, ldc, M, N, K, stream);
+      case RLK_GEMM_CFG_192x128:
+        if (!streamed_weight(N, K, M, 128)) return launch_solo_shape<192, 128>(W, X, C, ldc, M, N, K, stream);
+        break;
+      default:
+        break;
+    }
   }
   // The element-wise loader keeps eight values per chunk in flight, and a picked 256-feature tile gives way to 128 x 128, which
   // holds them without spilling. The 192-feature and 192-token tiles, which have no such loader, become 256-feature tiles

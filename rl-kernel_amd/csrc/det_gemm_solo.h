@@ -29,6 +29,10 @@
 // 3689; a K-major weight, 4096 x 12288 with K = 4096 297 -> 291, 4096 x 4096 98.5 -> 96.7. Where a launch leaves the last round
 // half empty, or holds two products (det_gemm_pair.hip), more.
 //
+// Smaller shapes (192 x 256, 256 x 192 in five parts; 192 x 192, 256 x 128, 192 x 128 in a ring of three or four stages of a K tile,
+// token rows a step behind weight rows) have the same wave layout, half a tile by half. What bounds them is LDS and, in one
+// round with a weight from HBM, the loads; kTileCandidates has what they measured beside eight waves.
+//
 // Same MFMA chain per output element as every other loop. Needs 16-byte aligned rows and rows whose byte offsets inside a tile stay
 // below 4 GiB (solo_offsets_fit(); 2 GiB beside a K-major operand, solo_kmajor_fits()); K % 64 == 0 with two native operands.
 #pragma once
@@ -41,7 +45,6 @@ using SoloShape = TileShape<256, 256, 2, 2>;
 constexpr int kSoloPartBytes = 256 * kRowBytes;
 constexpr int kSoloParts = 5;
 constexpr int kSoloLdsBytes = kSoloParts * kSoloPartBytes;
-constexpr int kSoloLoads = 8;  // load instructions of a wave per part
 
 // `rows`: from the first row of a tile to its last.
 inline bool solo_offsets_fit(const MatView& v, int64_t rows = SoloShape::BN) {
@@ -54,8 +57,15 @@ inline bool solo_offsets_fit(const MatView& v, int64_t rows = SoloShape::BN) {
 //   acc[4 h + jn][jm][q] is feature 128 wave_n + 64 h + 16 (lane >> 4) + 4 jn + q of token 128 wave_m + 16 jm + (lane & 15).
 // Gated: 128 features of both halves of a packed gate/up weight [2 I, K],
 //   acc[jn][jm][q] the gate and acc[4 + jn][jm][q] the up projection of feature 64 wave_n + 16 (lane >> 4) + 4 jn + q.
+// (Of a wave's 96 features the last 32 are a span of two MFMA tiles, a lane's eight features.)
+template <class S>
 struct SoloPlainRows {
-  static __device__ __forceinline__ int feature(int r) { return (r & ~63) + ((r & 15) >> 2) * 16 + ((r >> 4) & 3) * 4 + (r & 3); }
+  static __device__ __forceinline__ int feature(int r) {
+    constexpr int kWaveRows = 16 * S::TN;
+    const int in_wave = r % kWaveRows, span = in_wave & ~63;
+    const bool half = kWaveRows % 64 != 0 && span + 64 > kWaveRows;
+    return r - in_wave + span + ((r & 15) >> 2) * (half ? 8 : 16) + (((in_wave - span) >> 4) & 3) * 4 + (r & 3);
+  }
   static __device__ __forceinline__ int64_t row(int r, int last, int) { return min(feature(r), last); }
   static __device__ __forceinline__ int features(const MatView& W) { return W.rows; }
 };
@@ -74,9 +84,15 @@ struct SoloGatedRows {
 // zeros, in either operand: a K-major buffer ends behind the last K row (a block's scalar offset never exceeds its size, or the
 // check, offset >= size - scalar offset, would wrap), and chunks of a native one get an offset beyond it (whole chunks are read:
 // K % 8 == 0 or MatView::k_padded).
-template <bool W_KMAJOR, bool X_KMAJOR>
+template <bool W_KMAJOR, bool X_KMAJOR, class SHAPE = SoloShape>
 struct SoloLayout {
+  using Shape = SHAPE;
   static constexpr bool kW = W_KMAJOR, kX = X_KMAJOR, kTail = W_KMAJOR || X_KMAJOR;
+  static_assert((!W_KMAJOR || SHAPE::BN == 256) && (!X_KMAJOR || SHAPE::BM == 256), "a column for each wave");
+  // Stages of a whole K tile where three or more of them fit, else five parts.
+  static constexpr int kStages = kSoloLdsBytes / SHAPE::kStageBytes;
+  static constexpr bool kRing = kStages >= 3;
+  static constexpr int kLds = kRing ? kStages * SHAPE::kStageBytes : kSoloLdsBytes;
 };
 constexpr uint32_t kSoloRange = 0x7fff0000, kSoloOutside = 0x80000000;  // of a native buffer, bytes; what takes an offset out of it
 
@@ -152,7 +168,9 @@ __device__ __forceinline__ float solo_result(float accumulator) {
   return value;
 }
 
-typedef f32x4_t SoloAcc[SoloShape::TN][SoloShape::TM];
+template <class S>
+using SoloAccOf = f32x4_t[S::TN][S::TM];
+typedef SoloAccOf<SoloShape> SoloAcc;
 
 // Runs the tiles first, first + step, ... < total (at least one). tile_at(i, n0, m0) says where tile i lies; done(i, acc, scratch)
 // takes its results, may use the spare part of the LDS if it ends on a barrier then, and returns whether this wave has issued STORES
@@ -165,20 +183,23 @@ struct SoloKeepsNothing {
 template <class Rows, int STORES, bool LONG = false, class Layout = SoloLayout<false, false>, class TileAt, class Done, class Keep = SoloKeepsNothing>
 __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, int K, int first, int step, int total, char* lds,
                                            TileAt tile_at, Done done, Keep keep = Keep()) {
-  using S = SoloShape;
-  constexpr int kBehind = STORES + kSoloLoads < 63 ? STORES + kSoloLoads : 63;
+  using S = typename Layout::Shape;
+  constexpr int kLoadsW = S::BN / 32, kLoadsX = S::BM / 32;  // load instructions of a wave per part
+  // Loads of K tiles behind the next one that may be in flight when that one is waited for.
+  constexpr int kAhead = Layout::kRing ? (Layout::kStages - 2) * (kLoadsW + kLoadsX) : kLoadsW;
+  constexpr int kBehind = STORES + kAhead < 63 ? STORES + kAhead : 63;
   const int lane = solo_lane();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15;
   const int grp = lane >> 4;
   const int nk = Layout::kTail ? (K + kTileK - 1) / kTileK : K / kTileK;
 
-  // The load stream: the next K tile of its output tile, at w_at and x_at. A wave loads LDS rows [64 wave, + 64) of either part in eight
+  // The load stream: the next K tile of its output tile, at w_at and x_at. A wave loads a quarter of the rows of either part in
   // blocks of eight rows; block j adds (j & 3) KiB as the instruction's offset, which counts for the LDS address and the global one.
   constexpr int kBlockBytes = 1024, kBlocksPerBase = 4;
   // A K-major operand's column is the wave's, block j K rows [8 j, + 8): a lane has one offset for either chunk position that the
   // swizzle gives it, and the block's K rows are the instruction's scalar offset.
-  uint32_t off_w[Layout::kW ? 2 : kSoloLoads], off_x[Layout::kX ? 2 : kSoloLoads];
+  uint32_t off_w[Layout::kW ? 2 : kLoadsW], off_x[Layout::kX ? 2 : kLoadsX];
   const uint32_t block_w = (uint32_t)W.k_stride * 16, block_x = (uint32_t)X.k_stride * 16;  // bytes of eight K rows
   const char *w_at, *x_at;
   uint32_t range_w = Layout::kTail ? kSoloRange : 0xffffffff, range_x = range_w;  // of the K tile's buffers, which begin below it
@@ -203,20 +224,24 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
     else x_at = reinterpret_cast<const char*>(X.ptr + (int64_t)m0 * X.row_stride) - kBlocksPerBase * kBlockBytes;
     const int lane = solo_lane();
 #pragma unroll
-    for (int j = 0; j < kSoloLoads; ++j) {
-      const int r = wave * 64 + j * 8 + (lane >> 3);
+    for (int j = 0; j < 8; ++j) {
+      const int r = j * 8 + (lane >> 3);
       // rows past the edge: computed, never stored
       const uint32_t in_row = ((lane & 7) ^ (lane >> 3)) * 16 + (kBlocksPerBase - j % kBlocksPerBase) * kBlockBytes;
       // (32 bits each: as halves of 64-bit products they took two registers)
       if constexpr (!Layout::kW) {
-        const uint32_t row_w = (uint32_t)Rows::row(r, Rows::features(W) - n0 - 1, W.rows / 2);
-        off_w[j] = row_w * (uint32_t)W.row_stride * 2 + in_row;
-        asm volatile("" : "+v"(off_w[j]));
+        if (j < kLoadsW) {
+          const uint32_t row_w = (uint32_t)Rows::row(wave * (8 * kLoadsW) + r, Rows::features(W) - n0 - 1, W.rows / 2);
+          off_w[j] = row_w * (uint32_t)W.row_stride * 2 + in_row;
+          asm volatile("" : "+v"(off_w[j]));
+        }
       }
       if constexpr (!Layout::kX) {
-        const uint32_t row_x = min(r, X.rows - m0 - 1);
-        off_x[j] = row_x * (uint32_t)X.row_stride * 2 + in_row;
-        asm volatile("" : "+v"(off_x[j]));
+        if (j < kLoadsX) {
+          const uint32_t row_x = min(wave * (8 * kLoadsX) + r, X.rows - m0 - 1);
+          off_x[j] = row_x * (uint32_t)X.row_stride * 2 + in_row;
+          asm volatile("" : "+v"(off_x[j]));
+        }
       }
     }
   };
@@ -232,7 +257,7 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
         const int lane = solo_lane();
         const uint32_t out = ((lane & 7) ^ (lane >> 3)) * kChunkElems < k_rest ? 0 : kSoloOutside;
 #pragma unroll
-        for (int j = 0; j < kSoloLoads; ++j) {
+        for (int j = 0; j < (Layout::kW ? kLoadsX : kLoadsW); ++j) {
           if constexpr (!Layout::kW) off_w[j] |= out;
           if constexpr (!Layout::kX) off_x[j] |= out;
         }
@@ -256,7 +281,7 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
     constexpr bool kWeight = decltype(weight)::value != 0, kKMajor = kWeight ? Layout::kW : Layout::kX;
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<char*>(kWeight ? w_at : x_at), 0, kWeight ? range_w : range_x, 0x00027000);
-    lds_ptr_t to = (lds_ptr_t)(part + (wave * kSoloLoads + j / kBlocksPerBase * kBlocksPerBase) * kBlockBytes);
+    lds_ptr_t to = (lds_ptr_t)(part + (wave * (kWeight ? kLoadsW : kLoadsX) + j / kBlocksPerBase * kBlocksPerBase) * kBlockBytes);
     constexpr int kOffset = j % kBlocksPerBase * kBlockBytes;
     if constexpr (kKMajor) {
       const uint32_t rows_at = (kWeight ? block_w : block_x) * j + (kBlocksPerBase * kBlockBytes - kOffset);
@@ -270,7 +295,13 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
     f(IntTag<0>{}), f(IntTag<1>{}), f(IntTag<2>{}), f(IntTag<3>{}), f(IntTag<4>{}), f(IntTag<5>{}), f(IntTag<6>{}), f(IntTag<7>{});
   };
 
-  SoloAcc acc;
+  auto load_part = [&](auto weight, char* part) __attribute__((always_inline)) {
+    for_blocks([&](auto j) __attribute__((always_inline)) {
+      if constexpr (decltype(j)::value < (decltype(weight)::value ? kLoadsW : kLoadsX)) load(weight, j, part);
+    });
+  };
+
+  SoloAccOf<S> acc;
   struct Frags {
     u32x4_t w[S::TN], x[S::TM];
   };
@@ -279,8 +310,8 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
   constexpr int kColumnBytes = kTileK * kRowBytes;  // 64 rows of a K-major part
   const int tr_row = grp * 8 + (l16 >> 2);          // K row of a transposing read, and its place in a column
   const int tr_at = tr_row * kRowBytes + ((((l16 & 3) >> 1) ^ kmajor_swizzle(tr_row)) << 4) + (l16 & 1) * 8;
-  const lds_bytes_t w_rows = (lds_bytes_t)lds + (Layout::kW ? wave % S::WN * 2 * kColumnBytes + tr_at : ((wave % S::WN) * 128 + l16) * kRowBytes);
-  const lds_bytes_t x_rows = (lds_bytes_t)lds + (Layout::kX ? wave / S::WN * 2 * kColumnBytes + tr_at : ((wave / S::WN) * 128 + l16) * kRowBytes);
+  const lds_bytes_t w_rows = (lds_bytes_t)lds + (Layout::kW ? wave % S::WN * 2 * kColumnBytes + tr_at : (wave % S::WN * 16 * S::TN + l16) * kRowBytes);
+  const lds_bytes_t x_rows = (lds_bytes_t)lds + (Layout::kX ? wave / S::WN * 2 * kColumnBytes + tr_at : (wave / S::WN * 16 * S::TM + l16) * kRowBytes);
   // Reads of a K step, in the order of the fragments' use: w[0], x[0] to x[7], w[1] to w[7], a K-major one in two halves.
   constexpr int kWReads = Layout::kW ? 2 : 1, kXReads = Layout::kX ? 2 : 1;
   constexpr int kReads = S::TN * kWReads + S::TM * kXReads;
@@ -308,14 +339,19 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
   };
 
   auto next_part = [](int at) { return at + kSoloPartBytes < kSoloLdsBytes ? at + kSoloPartBytes : 0; };
-  int w_part = 0, x_part = kSoloPartBytes, spare = 4 * kSoloPartBytes;  // of the K tile at hand
+  // of the K tile at hand; the spare part, in a ring the stage of the K tile before
+  constexpr int kWBytes = S::BN * kRowBytes;
+  int w_part = 0, x_part = Layout::kRing ? kWBytes : kSoloPartBytes;
+  int spare = Layout::kRing ? (Layout::kStages - 1) * S::kStageBytes : 4 * kSoloPartBytes;
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    for_blocks([&](auto j) __attribute__((always_inline)) { load(IntTag<1>{}, j, lds + 2 * t * kSoloPartBytes); });
-    for_blocks([&](auto j) __attribute__((always_inline)) { load(IntTag<0>{}, j, lds + (2 * t + 1) * kSoloPartBytes); });
+  for (int t = 0; t < (Layout::kRing ? Layout::kStages - 1 : 2); ++t) {
+    load_part(IntTag<1>{}, lds + t * (Layout::kRing ? S::kStageBytes : 2 * kSoloPartBytes));
+    load_part(IntTag<0>{}, lds + t * (Layout::kRing ? S::kStageBytes : 2 * kSoloPartBytes) + x_part);
     advance();
   }
-  __builtin_amdgcn_s_waitcnt(wait_vmcnt(2 * kSoloLoads));  // my part of the first K tile has landed
+  if constexpr (Layout::kRing) load_part(IntTag<1>{}, lds + spare);
+  // my part of the first K tile has landed
+  __builtin_amdgcn_s_waitcnt(wait_vmcnt(Layout::kRing ? kAhead + kLoadsW : kLoadsW + kLoadsX));
   wg_barrier();
   Frags a, b;
 #pragma unroll
@@ -331,19 +367,28 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
       if (kFirst && STORES > 0 && behind)
         __builtin_amdgcn_s_waitcnt(wait_vmcnt(kBehind) & kWaitLgkm0);
       else
-        __builtin_amdgcn_s_waitcnt(wait_vmcnt(kSoloLoads) & kWaitLgkm0);
+        __builtin_amdgcn_s_waitcnt(wait_vmcnt(kAhead) & kWaitLgkm0);
       wg_barrier();
       to = lds + w_part;
-      spare = x_part;
-      w_part = next_part(x_part);
-      x_part = next_part(w_part);
+      if constexpr (Layout::kRing) {
+        spare = w_part;
+        w_part = w_part + S::kStageBytes < Layout::kLds ? w_part + S::kStageBytes : 0;
+        x_part = w_part + kWBytes;
+      } else {
+        spare = x_part;
+        w_part = next_part(x_part);
+        x_part = next_part(w_part);
+      }
     } else {
       __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
-      to = lds + spare;
+      to = lds + spare + (Layout::kRing ? kWBytes : 0);
     }
     const lds_bytes_t w = step_at(w_rows, w_part, Layout::kW, !kSecond), x = step_at(x_rows, x_part, Layout::kX, !kSecond);
     __builtin_amdgcn_sched_barrier(0);
-    for_blocks([&](auto row) __attribute__((always_inline)) {
+    // the part that is loaded: weight rows under the first K step, token rows under the second, in a ring the other way round
+    constexpr bool kLoadsWeight = kSecond == Layout::kRing;
+    constexpr int kLoads = kLoadsWeight ? kLoadsW : kLoadsX;
+    if constexpr (S::TN * S::TM == 64) for_blocks([&](auto row) __attribute__((always_inline)) {
       constexpr int jn = decltype(row)::value;
 #pragma unroll
       for (int jm = 0; jm < S::TM; ++jm) {
@@ -353,11 +398,31 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
           asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[jn][jm]) : "v"(now.w[jn]), "v"(now.x[jm]));
         constexpr int kPerRow = kReads / 8, kApart = kPerRow == 2 ? 4 : kPerRow == 3 ? 3 : 2;
         if (jn < 7 ? jm % kApart == 0 : jm < kPerRow) read(w, x, kPerRow * jn + (jn < 7 ? jm / kApart : jm), next);
-        if (jm == (kPerRow == 4 ? 3 : 2)) load(IntTag<kSecond ? 0 : 1>{}, row, to);
+        if (jm == (kPerRow == 4 ? 3 : 2)) load(IntTag<kLoadsWeight>{}, row, to);
         __builtin_amdgcn_sched_barrier(0);
       }
     });
-    if constexpr (kSecond) advance();
+    else for_blocks([&](auto share) __attribute__((always_inline)) {
+      // eight shares of the MFMAs, the reads evenly between all but the last few, the loads in the shares from the first on
+      constexpr int kMfmas = S::TN * S::TM, q = decltype(share)::value;
+#pragma unroll
+      for (int i = q * kMfmas / 8; i < (q + 1) * kMfmas / 8; ++i) {
+        const int jn = i / S::TM, jm = i % S::TM;
+        if constexpr (kFirst && !kSecond)
+          asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc[jn][jm]) : "v"(now.w[jn]), "v"(now.x[jm]));
+        else
+          asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[jn][jm]) : "v"(now.w[jn]), "v"(now.x[jm]));
+        constexpr int kSpan = kMfmas - 4;
+#pragma unroll
+        for (int r = 0; r < kReads; ++r)
+          if (r * kSpan / kReads == i) read(w, x, r, next);
+        if (i == q * kMfmas / 8 + 1) {
+          if constexpr (q < kLoads) load(IntTag<kLoadsWeight>{}, share, to);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+    if constexpr (kSecond != Layout::kRing) advance();
   };
   bool behind = false;
   for (int tile = first; tile < total; tile += step) {
@@ -369,8 +434,10 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
       k_step(b, a, IntTag<1>{}, IntTag<0>{}, false);
     }
     // the compiler does not know these for MFMAs, whose results take a while
+    constexpr int kTN = S::TN, kTM = S::TM, kBefore = kTM == 4 ? kTN - 2 : kTN - 1;  // the last five
     asm volatile("s_nop 15\n s_nop 15"
-                 : "+a"(acc[7][3]), "+a"(acc[7][4]), "+a"(acc[7][5]), "+a"(acc[7][6]), "+a"(acc[7][7])
+                 : "+a"(acc[kBefore][kTM == 4 ? 3 : kTM - 5]), "+a"(acc[kTN - 1][kTM - 4]), "+a"(acc[kTN - 1][kTM - 3]),
+                   "+a"(acc[kTN - 1][kTM - 2]), "+a"(acc[kTN - 1][kTM - 1])
                  :
                  : "memory");
     behind = done(tile, acc, lds + spare);

@@ -369,7 +369,7 @@ __global__ __launch_bounds__(SoloShape::kThreads) void linear_logp_solo_kernel(L
     for (int jm = 0; jm < S::TM; ++jm)
       asm volatile("" : "+v"(run_m[0][jm]), "+v"(run_m[1][jm]), "+v"(run_s[0][jm]), "+v"(run_s[1][jm]));
   };
-  solo_tiles<SoloPlainRows, LOGITS ? 55 : 0, true>(a.W, a.H, a.D, 0, 1, tiles, lds, tile_at, done, keep);
+  solo_tiles<SoloPlainRows<SoloShape>, LOGITS ? 55 : 0, true>(a.W, a.H, a.D, 0, 1, tiles, lds, tile_at, done, keep);
 }
 
 // Few token tiles: a split of 1024 columns gives the chip only tiles_m * ceil(V / 1024)

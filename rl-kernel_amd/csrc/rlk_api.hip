@@ -88,7 +88,10 @@ int rlk_det_gemm_bf16(const void* a, int64_t a_row_stride, int64_t a_k_stride, c
     set_last_error("rlk_det_gemm_bf16: operands must not use negative strides");
     return RLK_ERR_INVALID_ARGUMENT;
   }
-  if (config < 0 || (config & ~RLK_GEMM_CFG_FORCE_STAGED) >= RLK_GEMM_CFG_COUNT) {
+  const int shape = config & ~RLK_GEMM_CFG_FOUR_WAVES;
+  const bool four_waves = shape == RLK_GEMM_CFG_256x128 || shape == RLK_GEMM_CFG_192x256 || shape == RLK_GEMM_CFG_192x128 ||
+                          shape == RLK_GEMM_CFG_256x192 || shape == RLK_GEMM_CFG_192x192;
+  if (config < 0 || ((four_waves ? shape : config) & ~RLK_GEMM_CFG_FORCE_STAGED) >= RLK_GEMM_CFG_COUNT) {
     set_last_error("rlk_det_gemm_bf16: unknown config %d", config);
     return RLK_ERR_INVALID_ARGUMENT;
   }

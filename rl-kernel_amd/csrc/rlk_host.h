@@ -83,7 +83,7 @@ inline bool streamed_weight(int64_t rows, int64_t k, int M, int bm) {
   return (M <= bm && bytes >= ((int64_t)96 << 20)) || (M == 2 * bm && bytes >= ((int64_t)128 << 20));
 }
 
-int pick_det_gemm_config(int M, int N, int K);
+int pick_det_gemm_config(int M, int N, int K, bool out_f32 = false);
 
 // W[N,K] is the operand whose rows are output features, X[M,K] the one whose
 // rows are tokens; C[m*ldc + n].

@@ -52,6 +52,8 @@ GEMM_CONFIGS = {
 }
 # OR-ed into a GEMM or LogP configuration: register-staged main loop (bit-neutral).
 FORCE_STAGED = 0x100
+# OR-ed into GEMM configurations of 192 or 256 features: one wave per SIMD (bit-neutral).
+FOUR_WAVES = 0x200
 # rlk_linear_bwd_config: the automatic choice for one of many weights
 LINEAR_BWD_MANY_WEIGHTS = 0x400
 # both products in 256 x 256 tiles with one wave per SIMD

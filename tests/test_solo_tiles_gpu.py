@@ -65,6 +65,33 @@ def test_gated_projection(tokens, inter, k):
     assert torch.equal(y.view(torch.int16), _C.swiglu_packed_forward(gate_up).view(torch.int16))
 
 
+# one K tile, as many as stages and one more or less, edges of tiles of either side, tails of a few rows, more tiles than CUs
+@pytest.mark.parametrize("shape", [(1, 8, 64), (192, 192, 128), (129, 200, 192), (400, 392, 256), (257, 777, 320), (300, 500, 1024), (3100, 3200, 448)])
+@pytest.mark.parametrize("name", ["256x192", "192x256", "192x192", "256x128", "192x128"])
+def test_smaller_shapes_on_four_waves(shape, name):
+    """The bits of the small tiles; whole 16-byte stores and element stores, nothing written beside the result."""
+    from rl_engine import _C, _lib
+
+    m, n, _ = shape
+    x, w = _operands(shape, m * n)
+    want = torch.empty((m, n), device=DEV, dtype=torch.bfloat16)
+    _C.gemm_strided(x, w.t(), want, config=_lib.GEMM_CONFIGS["64x64"])
+    for pitch in (8, 3):
+        pad = torch.full((m + 1, n + pitch), 7.0, device=DEV, dtype=torch.bfloat16)
+        _C.gemm_strided(x, w.t(), pad[:m, :n], config=_lib.GEMM_CONFIGS[name] | _lib.FOUR_WAVES)
+        assert torch.equal(pad[:m, :n].contiguous().view(torch.int16), want.view(torch.int16))
+        assert bool((pad[m] == 7.0).all()) and bool((pad[:, n:] == 7.0).all())
+    if name in ("256x192", "256x128"):  # a K-major weight, whose rows come in eights
+        n8 = (n + 7) // 8 * 8
+        wt = torch.zeros((w.size(1), n8), device=DEV, dtype=torch.bfloat16)
+        wt[:, :n] = w.t()
+        for k in (w.size(1), w.size(1) - 8, w.size(1) - 56):
+            _C.gemm_strided(x[:, :k].contiguous(), w[:, :k].contiguous().t(), want, config=_lib.GEMM_CONFIGS["64x64"])
+            got = torch.empty((m, n8), device=DEV, dtype=torch.bfloat16)
+            _C.gemm_strided(x[:, :k].contiguous(), wt[:k], got, config=_lib.GEMM_CONFIGS[name] | _lib.FOUR_WAVES)
+            assert torch.equal(got[:, :n].contiguous().view(torch.int16), want.view(torch.int16)), k
+
+
 # (tokens, outputs, K): one K tile and less, a few values more than whole K tiles, odd ones, edges of tiles of either side, more
 # tiles than CUs
 KMAJOR_SHAPES = [(8, 8, 8), (256, 256, 24), (264, 520, 64), (248, 776, 72), (1000, 264, 200), (512, 512, 2056), (4360, 4360, 136)]
