@@ -125,9 +125,11 @@ typedef enum rlk_linear_bwd_config {
   /* The automatic choice for one of several weights that are together more than the memory-side cache holds from their forward
    * to their backward (a gated FFN's). */
   RLK_LINEAR_BWD_CFG_MANY_WEIGHTS = 0x400,
-  /* One launch: 256 x 256 tiles of both products on four waves (one per SIMD), one workgroup per CU. The automatic choices run it
-   * instead of what they resolve to where that is faster. */
-  RLK_LINEAR_BWD_CFG_SOLO = 0x800
+  /* One launch on four waves (one per SIMD), one workgroup per CU: tiles of 256 inputs x 256, 192 or 128 tokens of dx, 256 x 256 of dw.
+   * The automatic choices run it instead of what they resolve to where that is faster. */
+  RLK_LINEAR_BWD_CFG_SOLO = 0x800,
+  RLK_LINEAR_BWD_CFG_SOLO_192 = 0x801,
+  RLK_LINEAR_BWD_CFG_SOLO_128 = 0x802
 } rlk_linear_bwd_config;
 
 /* The configuration that the automatic choice resolves to for contiguous operands of a shape: RLK_LINEAR_BWD_CFG_AUTO's,

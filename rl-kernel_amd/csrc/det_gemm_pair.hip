@@ -41,8 +41,8 @@ __global__ __launch_bounds__(SX::kThreads) void det_gemm_pair_kernel(PairProblem
   }
 }
 
-// The same in 256 x 256 tiles with one wave per SIMD (det_gemm_solo.h), one workgroup per CU with a share of both products fixed by the
-// host: the tiles of `first` in turn, then those of the other product, of which workgroups [0, late), which have one tile of the
+// The same with one wave per SIMD (det_gemm_solo.h), 256 x BM tiles of dX and 256 x 256 of dW, one workgroup per CU with a share of both
+// products fixed by the host: the tiles of `first` in turn, then those of the other product, of which workgroups [0, late), which have one tile of the
 // first more, take late_tiles each and the others the rest.
 struct SoloShares {
   bool dx_first;
@@ -52,18 +52,27 @@ struct SoloPair {
   SoloProblem dx, dw;
   SoloShares shares;
 };
+// Read from the arguments when its turn comes: as values of the kernel, the two products are in scalar registers at once, and spill a
+// hundred.
+__device__ __forceinline__ SoloProblem solo_argument(bool is_dx) {
+  const __attribute__((address_space(4))) SoloPair* args =
+      (const __attribute__((address_space(4))) SoloPair*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args));
+  SoloProblem p;
+  __builtin_memcpy(&p, is_dx ? &args->dx : &args->dw, sizeof(p));
+  return p;
+}
+template <int BM>
+using SoloDx = SoloLayout<true, false, TileShape<256, BM, 2, 2>>;
+using SoloDw = SoloLayout<true, true>;
+template <int BM>
 __global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_pair_solo_kernel(SoloPair pair) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const SoloShares shares = pair.shares;
   const int group = blockIdx.x, groups = gridDim.x;
   for (int product = 0; product < 2; ++product) {
     const bool is_dx = (product == 0) == shares.dx_first;
-    // Read from the arguments when its turn comes: as values of the kernel, the two products are in scalar registers at once, and
-    // spill a hundred.
-    const __attribute__((address_space(4))) SoloPair* args = (const __attribute__((address_space(4))) SoloPair*)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(args));
-    SoloProblem p;
-    __builtin_memcpy(&p, is_dx ? &args->dx : &args->dw, sizeof(p));
+    const SoloProblem p = solo_argument(is_dx);
     const int tiles = p.tiles_m * p.tiles_n;
     int at = group, step = groups, total = tiles;
     if (product == 1) {
@@ -74,8 +83,8 @@ __global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_pair_solo_kernel
       total = late ? of_late : tiles;
     }
     if (at >= total) continue;
-    if (is_dx) solo_product<SoloLayout<true, false>>(p, at, step, total, lds);
-    else solo_product<SoloLayout<true, true>>(p, at, step, total, lds);
+    if (is_dx) solo_product<SoloDx<BM>>(p, at, step, total, lds);
+    else solo_product<SoloDw>(p, at, step, total, lds);
     wg_barrier();  // the next product's loads overwrite what the last reads are of
   }
 }
@@ -130,62 +139,77 @@ static hipError_t launch_pair(const GemmProblem& dx, const GemmProblem& dw, bool
 
 static int64_t tile_count(const GemmProblem& p, int bn, int bm) { return (int64_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); }
 
-constexpr int64_t kSoloTileCost = 6;  // of a tile beside its K tiles, in K tiles
-static int64_t solo_length(const GemmProblem& p) { return ((int64_t)p.K + kTileK - 1) / kTileK + kSoloTileCost; }
+// The length of a tile in K tiles of 256 x 256: beside its K tiles each has a cost, and a K tile of fewer tokens takes its part of the
+// time. (What it takes of the power, solo_pair_us(), is another part.)
+constexpr double kSoloTileCost = 7.0;
+static double solo_tile_length(const GemmProblem& p, int bm = 256) {
+  return (((int64_t)p.K + kTileK - 1) / kTileK + kSoloTileCost) * (bm == 256 ? 1.0 : bm == 192 ? 0.83 : 0.55);
+}
 
-// The shares of the one-wave-per-SIMD launch, and what the workgroup with the most to do has, in K tiles. The product with the longer
-// tiles comes first; `late` workgroups have one of its tiles more than the others, and late_tiles is what evens that out.
-static SoloShares solo_shares(const GemmProblem& dx, const GemmProblem& dw, int groups, int64_t* k_tiles) {
-  SoloShares s{solo_length(dx) >= solo_length(dw), 0, 0};
-  const GemmProblem &a = s.dx_first ? dx : dw, &b = s.dx_first ? dw : dx;
-  const int64_t na = tile_count(a, 256, 256), nb = tile_count(b, 256, 256), la = solo_length(a), lb = solo_length(b);
+// The shares of the one-wave-per-SIMD launch, and what the workgroup with the most to do has. The product with the longer tiles comes
+// first; `late` workgroups have one of its tiles more than the others, and late_tiles is what evens that out.
+static SoloShares solo_shares(const GemmProblem& dx, const GemmProblem& dw, int bm, int groups, double* longest) {
+  const double length_dx = solo_tile_length(dx, bm), length_dw = solo_tile_length(dw);
+  const int64_t tiles_dx = tile_count(dx, 256, bm), tiles_dw = tile_count(dw, 256, 256);
+  SoloShares s{length_dx >= length_dw, 0, 0};
+  const int64_t na = s.dx_first ? tiles_dx : tiles_dw, nb = s.dx_first ? tiles_dw : tiles_dx;
+  const double la = s.dx_first ? length_dx : length_dw, lb = s.dx_first ? length_dw : length_dx;
   const int64_t rounds = na / groups, late = na % groups;
   s.late = (int)late;
-  *k_tiles = 0;
-  const int64_t even = ((na * la + nb * lb) / groups - (rounds + 1) * la) / lb;  // late_tiles, if all had the same
-  for (int64_t t = even < 0 ? 0 : even; t <= (even < 0 ? 0 : even + 1); ++t) {
+  *longest = 1e300;
+  const double even = ((na * la + nb * lb) / groups - (rounds + 1) * la) / lb;  // late_tiles, if all had the same
+  const int64_t least = even > 0.0 ? (int64_t)even : 0;
+  for (int64_t t = least; t <= (even > 0.0 ? least + 1 : least); ++t) {
     const int64_t of_late = late * t < nb ? late * t : nb;
     const int64_t others = (nb - of_late + groups - late - 1) / (groups - late);
-    int64_t span = rounds * la + others * lb;
+    double span = rounds * la + others * lb;
     if (late > 0 && (rounds + 1) * la + t * lb > span) span = (rounds + 1) * la + t * lb;
-    if (*k_tiles == 0 || span < *k_tiles) {
-      *k_tiles = span;
+    if (span < *longest) {
+      *longest = span;
       s.late_tiles = (int)t;
     }
   }
   return s;
 }
-static int solo_groups(const GemmProblem& dx, const GemmProblem& dw) {
-  const int64_t tiles = tile_count(dx, 256, 256) + tile_count(dw, 256, 256);
+static int solo_groups(const GemmProblem& dx, const GemmProblem& dw, int bm) {
+  const int64_t tiles = tile_count(dx, 256, bm) + tile_count(dw, 256, 256);
   const int cus = device_cu_count();
   return (int)(tiles < cus ? tiles : cus);
 }
-// What that launch takes, on the scale of pair_us() (whose figures are 8 to 10 % below what a chip at its power cap takes): the longest
-// share at a rate, and all the work at a rate that the package's power gives. Fitted to 62 shapes of 200 to 8000 tokens within
-// 4 %. The best other configuration -> this, us, where the rule takes it (tokens, inputs, outputs):
-//   2047, 4096, 4096: 110.8 -> 102.6    601, 14336, 4096: 165.8 -> 138.9    855, 12288, 4096: 182 -> 159     1882, 14336, 4096: 372 -> 339
-//   2325, 4096, 3072: 118.6 -> 104.3    2048, 4096, 12288: 327 -> 305       5872, 4096, 14336: 1023 -> 965   7438, 4096, 1536: 179.6 -> 162.0
-//   4120, 4096, 151936: 7524 -> 7230    4120, 1024, 4096: 80.4 -> 75.6      2064, 6144, 2048: 94.5 -> 95.4   1472, 4096, 14336: 291 -> 294
-// where it does not: 1024, 4096, 4096: 64.9 / 80.1    8192, 1024, 1024: 98 / 146    1407, 4096, 24576: 474 / 489   1478, 6144, 4096: 136 / 130.5
-static double solo_pair_us(const GemmProblem& dx, const GemmProblem& dw, int cus) {
-  int64_t k_tiles;
-  solo_shares(dx, dw, solo_groups(dx, dw), &k_tiles);
-  const double work = (double)(tile_count(dx, 256, 256) * solo_length(dx) + tile_count(dw, 256, 256) * solo_length(dw)) / cus;
-  return 0.805 * k_tiles + 0.435 * work;
+// What that launch takes: the longest share at a rate, and all the work at a rate that the package's power gives, fitted to the three
+// tiles of dX on 94 shapes of 500 to 8000 tokens (4.4 %; the cheapest of the three is 0.2 % above the best). On the scale of pair_us(),
+// whose figures are 7 % below what a chip at its power cap takes. Where the rule takes it, best other configuration -> this, us
+// (tokens, inputs, outputs, tokens per tile of dX):
+//   2047, 4096, 4096, 256: 112.2 -> 102.7    601, 14336, 4096, 256: 166 -> 139     2910, 4096, 12288, 256: 465 -> 416   4120, 4096, 151936: 7524 -> 7230
+//   1508, 4096, 4096, 192: 87.9 -> 81.1      842, 6144, 2048, 192: 53.5 -> 48.1    2095, 4096, 6144, 192: 175 -> 165    1506, 4096, 24576: 500 -> 475
+//   1024, 4096, 4096, 128: 64.0 -> 60.3      1519, 2048, 6144, 128: 80.2 -> 73.0   908, 4096, 24576, 128: 370 -> 349    1030, 4096, 151936: 2590 -> 2373
+//   8094, 4096, 14336, 256: 1339 -> 1335     528, 6144, 4096, 128: 69.9 -> 72.7
+// where it does not: 8192, 1024, 1024: 98 / 146    603, 3072, 4096: 42.5 / 45.7    663, 2048, 6144: 46.8 / 61.9. Small tiles of dX (few
+// tokens: 64 or 128 outputs by as many tokens) are not compared: with a weight from HBM a tile of 128 tokens takes 0.9 us a K tile
+// instead of 0.6 (608, 4096, 6144: 80 / 92; 631, 4096, 3072: 42 / 38).
+constexpr double kPairScale = 0.935, kPairScaleFew = 1.0;  // few tokens: up to 640 (593, 6144, 4096: 71 / 75; 591, 4096, 4096: 53 / 49)
+static double solo_pair_us(const GemmProblem& dx, const GemmProblem& dw, int bm, int cus) {
+  double longest;
+  solo_shares(dx, dw, bm, solo_groups(dx, dw, bm), &longest);
+  const double work_dx = tile_count(dx, 256, bm) * solo_tile_length(dx) * (bm == 256 ? 1.0 : bm == 192 ? 0.70 : 0.73);
+  const double work_dw = tile_count(dw, 256, 256) * solo_tile_length(dw);
+  return (dw.K <= 640 ? kPairScaleFew : kPairScale) * (0.89 * longest + 0.455 * (work_dx + work_dw) / cus);
 }
 static bool solo_pair_serves(const GemmProblem& dx, const GemmProblem& dw) {
   return solo_kmajor_fits(dx.W) && solo_kmajor_fits(dx.X) && solo_kmajor_fits(dw.W) && solo_kmajor_fits(dw.X);
 }
+template <int BM>
 static hipError_t launch_pair_solo(const GemmProblem& dx, const GemmProblem& dw, hipStream_t stream) {
+  auto kernel = det_gemm_pair_solo_kernel<BM>;
+  constexpr int kLds = SoloDx<BM>::kLds > SoloDw::kLds ? SoloDx<BM>::kLds : SoloDw::kLds;
   static PerDeviceOnce once;
-  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(det_gemm_pair_solo_kernel), kSoloLdsBytes, once);
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds, once);
   if (err != hipSuccess) return err;
-  auto problem = [](const GemmProblem& p) { return solo_problem(p.W, p.X, p.C, p.ldc, p.M, p.N, p.K); };
-  const int groups = solo_groups(dx, dw);
-  int64_t k_tiles;
-  const SoloShares shares = solo_shares(dx, dw, groups, &k_tiles);
-  hipLaunchKernelGGL(det_gemm_pair_solo_kernel, dim3(groups), dim3(SoloShape::kThreads), kSoloLdsBytes, stream,
-                     SoloPair{problem(dx), problem(dw), shares});
+  const int groups = solo_groups(dx, dw, BM);
+  double longest;
+  const SoloPair pair{solo_problem<typename SoloDx<BM>::Shape>(dx.W, dx.X, dx.C, dx.ldc, dx.M, dx.N, dx.K),
+                      solo_problem(dw.W, dw.X, dw.C, dw.ldc, dw.M, dw.N, dw.K), solo_shares(dx, dw, BM, groups, &longest)};
+  hipLaunchKernelGGL(kernel, dim3(groups), dim3(SoloShape::kThreads), kLds, stream, pair);
   return hipGetLastError();
 }
 
@@ -347,14 +371,25 @@ LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem
       plan = {config, whole};
     }
   }
-  const double solo = solo_pair_us(dx, dw, cus);
-  plan.solo = solo < best && solo_pair_serves(dx, dw);
+  const bool small_dx = plan.config != RLK_LINEAR_BWD_CFG_SEPARATE && kPairTiles[plan.config].dx_bn < 256 && plan.head_rows == 0;
+  if (!small_dx && solo_pair_serves(dx, dw)) {
+    for (const int bm : {256, 192, 128}) {
+      const double us = solo_pair_us(dx, dw, bm, cus);
+      if (us < best) {
+        best = us;
+        plan.solo_tokens = bm;
+      }
+    }
+  }
   return plan;
 }
 
 hipError_t linear_backward_launch(GemmProblem dx, const GemmProblem& dw, LinearBackwardPlan plan, hipStream_t stream) {
   if (!one_launch_serves(dx, dw)) plan = {RLK_LINEAR_BWD_CFG_SEPARATE, 0};
-  if (plan.solo && solo_pair_serves(dx, dw)) return launch_pair_solo(dx, dw, stream);
+  if (plan.solo_tokens != 0 && solo_pair_serves(dx, dw))
+    return plan.solo_tokens == 256   ? launch_pair_solo<256>(dx, dw, stream)
+           : plan.solo_tokens == 192 ? launch_pair_solo<192>(dx, dw, stream)
+                                     : launch_pair_solo<128>(dx, dw, stream);
   if (plan.head_rows > 0) {
     const GemmProblem head = head_of(dx, plan.head_rows);
     const hipError_t err = det_gemm_launch(head.W, head.X, head.C, head.ldc, head.M, head.N, head.K, false, RLK_GEMM_CFG_AUTO, stream);

@@ -483,7 +483,7 @@ hipError_t linear_logp_bwd_launch(const MatView& H, const MatView& W, const int6
   const LinearBackwardPlan plan = grad_hidden && grad_weight && !force_staged
                                       ? linear_backward_plan(to_hidden, to_weight, BackwardOf::kLogp)
                                       : LinearBackwardPlan{RLK_LINEAR_BWD_CFG_SEPARATE, 0};
-  if (plan.config != RLK_LINEAR_BWD_CFG_SEPARATE || plan.solo) {
+  if (plan.config != RLK_LINEAR_BWD_CFG_SEPARATE || plan.solo_tokens != 0) {
     err = linear_backward_launch(to_hidden, to_weight, plan, stream);
     if (err != hipSuccess) return err;
     grad_hidden = grad_weight = nullptr;  // done

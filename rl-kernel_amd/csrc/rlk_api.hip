@@ -156,7 +156,7 @@ int rlk_linear_bwd_bf16(const void* dy, int64_t dy_row_stride, const void* x, in
     return RLK_ERR_INVALID_ARGUMENT;
   }
   const int rest_beside = config & RLK_LINEAR_BWD_CFG_REST_BESIDE;
-  if (config != RLK_LINEAR_BWD_CFG_MANY_WEIGHTS && config != RLK_LINEAR_BWD_CFG_SOLO &&
+  if (config != RLK_LINEAR_BWD_CFG_MANY_WEIGHTS && (config < RLK_LINEAR_BWD_CFG_SOLO || config > RLK_LINEAR_BWD_CFG_SOLO_128) &&
       (config < 0 || (config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE) >= RLK_LINEAR_BWD_CFG_COUNT ||
        (rest_beside && (config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE) <= RLK_LINEAR_BWD_CFG_SEPARATE))) {
     set_last_error("rlk_linear_bwd_bf16: unknown config %d", config);
@@ -178,8 +178,8 @@ int rlk_linear_bwd_bf16(const void* dy, int64_t dy_row_stride, const void* x, in
       config == RLK_LINEAR_BWD_CFG_AUTO ? linear_backward_plan(to_dx, to_dw, BackwardOf::kLinear)
       : config == RLK_LINEAR_BWD_CFG_MANY_WEIGHTS
           ? linear_backward_plan(to_dx, to_dw, BackwardOf::kManyWeights)
-      : config == RLK_LINEAR_BWD_CFG_SOLO
-          ? LinearBackwardPlan{RLK_LINEAR_BWD_CFG_256x256_256x256, 0, true}
+      : config >= RLK_LINEAR_BWD_CFG_SOLO
+          ? LinearBackwardPlan{RLK_LINEAR_BWD_CFG_256x256_256x256, 0, 256 - 64 * (config - RLK_LINEAR_BWD_CFG_SOLO)}
           : LinearBackwardPlan{config & ~RLK_LINEAR_BWD_CFG_REST_BESIDE, head};
   hipError_t err = linear_backward_launch(to_dx, to_dw, plan, reinterpret_cast<hipStream_t>(stream));
   return err == hipSuccess ? RLK_OK : device_error("rlk_linear_bwd_bf16", err);

@@ -106,7 +106,7 @@ struct GemmProblem {
 struct LinearBackwardPlan {
   int config;     // rlk_linear_bwd_config, not AUTO
   int head_rows;  // rows of dx that a launch of their own computes first
-  bool solo = false;  // instead, all of both products in 256 x 256 tiles with one wave per SIMD
+  int solo_tokens = 0;  // 256, 192 or 128: instead, all of both products with one wave per SIMD, dx in tiles of so many tokens
 };
 // Whose backward it is: a linear layer's right behind its forward; the LogP's, whose own two launches are what the one competes
 // with; or that of a layer with more weights than the memory-side cache holds from the forward to the backward.

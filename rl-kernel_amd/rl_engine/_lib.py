@@ -56,8 +56,8 @@ FORCE_STAGED = 0x100
 FOUR_WAVES = 0x200
 # rlk_linear_bwd_config: the automatic choice for one of many weights
 LINEAR_BWD_MANY_WEIGHTS = 0x400
-# both products in 256 x 256 tiles with one wave per SIMD
-LINEAR_BWD_SOLO = 0x800
+# both products with one wave per SIMD, dx in tiles of 256, 192 or 128 tokens
+LINEAR_BWD_SOLO, LINEAR_BWD_SOLO_192, LINEAR_BWD_SOLO_128 = 0x800, 0x801, 0x802
 TREE_LEAF_SPACE = 0x100  # RLK_TREE_CFG_LEAF_SPACE: OR-ed into rlk_tree_config 0 (auto) or 2 (matrix pipe)
 NOALLOC_SCRATCH_BYTES = 32 << 20  # RLK_NOALLOC_SCRATCH_BYTES
 # rlk_dtype (element types of materialised logits)

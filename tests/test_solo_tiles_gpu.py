@@ -165,7 +165,7 @@ def test_both_gradients_of_a_linear_layer(tokens, inputs, outputs):
         return dx.view(torch.int16), dw.view(torch.int16)
 
     want = backward(1)
-    for config in (_lib.LINEAR_BWD_SOLO, 0):
+    for config in (_lib.LINEAR_BWD_SOLO, _lib.LINEAR_BWD_SOLO_192, _lib.LINEAR_BWD_SOLO_128, 0):
         got = backward(config)
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
