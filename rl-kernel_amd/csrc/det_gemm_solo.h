@@ -55,8 +55,8 @@ inline bool solo_offsets_fit(const MatView& v, int64_t rows = SoloShape::BN) {
 // Plain: a wave's 128 features are two spans of 64, and in each of them a lane owns 16 consecutive ones, as with the four MFMA
 // tiles of a 64-feature wave column (weight_row_of_lds_row):
 //   acc[4 h + jn][jm][q] is feature 128 wave_n + 64 h + 16 (lane >> 4) + 4 jn + q of token 128 wave_m + 16 jm + (lane & 15).
-// Gated: 128 features of both halves of a packed gate/up weight [2 I, K],
-//   acc[jn][jm][q] the gate and acc[4 + jn][jm][q] the up projection of feature 64 wave_n + 16 (lane >> 4) + 4 jn + q.
+// Gated: half as many features of both halves of a packed gate/up weight [2 I, K], with T = TN / 2,
+//   acc[jn][jm][q] the gate and acc[T + jn][jm][q] the up projection of feature 16 T wave_n + 4 T (lane >> 4) + 4 jn + q.
 // (Of a wave's 96 features the last 32 are a span of two MFMA tiles, a lane's eight features.)
 template <class S>
 struct SoloPlainRows {
@@ -69,10 +69,13 @@ struct SoloPlainRows {
   static __device__ __forceinline__ int64_t row(int r, int last, int) { return min(feature(r), last); }
   static __device__ __forceinline__ int features(const MatView& W) { return W.rows; }
 };
+template <class S>
 struct SoloGatedRows {
   static __device__ __forceinline__ int64_t row(int r, int last, int half_rows) {
-    const int f = (r >> 7) * 64 + ((r & 15) >> 2) * 16 + ((r >> 4) & 3) * 4 + (r & 3);
-    return min(f, last) + ((r >> 6) & 1) * half_rows;
+    constexpr int kWaveRows = 16 * S::TN, kTiles = S::TN / 2;
+    const int wave = r / kWaveRows, tile = r % kWaveRows / 16;
+    const int f = wave * (kWaveRows / 2) + ((r & 15) >> 2) * (4 * kTiles) + tile % kTiles * 4 + (r & 3);
+    return min(f, last) + tile / kTiles * half_rows;
   }
   static __device__ __forceinline__ int features(const MatView& W) { return W.rows / 2; }
 };
@@ -416,7 +419,7 @@ __device__ __forceinline__ void solo_tiles(const MatView& W, const MatView& X, i
 #pragma unroll
         for (int r = 0; r < kReads; ++r)
           if (r * kSpan / kReads == i) read(w, x, r, next);
-        if (i == q * kMfmas / 8 + 1) {
+        if (i == q * kMfmas / 8 + (kMfmas >= 16 ? 1 : 0)) {
           if constexpr (q < kLoads) load(IntTag<kLoadsWeight>{}, share, to);
         }
         __builtin_amdgcn_sched_barrier(0);

@@ -231,12 +231,14 @@ __global__ __launch_bounds__(S::kThreads) void det_gemm_swiglu_kernel(MatView W,
   }
 }
 
-// The same on 256 weight rows x 256 tokens with one wave per SIMD, a workgroup per CU (det_gemm_solo.h).
+// The same with one wave per SIMD, a workgroup per CU (det_gemm_solo.h).
+template <class Layout>
 __global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_swiglu_solo_kernel(MatView W, MatView X,
                                                                                    bf16_bits* __restrict__ Y, int64_t ldy,
                                                                                    int M, int I, int K, int tiles_m,
                                                                                    int tiles_n, int group_m) {
-  using S = SoloShape;
+  using S = typename Layout::Shape;
+  constexpr int kTiles = S::TN / 2;  // MFMA tiles of a wave that hold gate features, and that hold up features
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   auto tile_at = [&](int block, int& f0, int& m0) __attribute__((always_inline)) {
@@ -244,35 +246,46 @@ __global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_swiglu_solo_kern
     f0 = at.tile_n * (S::BN / 2);
     m0 = at.tile_m * S::BM;
   };
-  auto done = [&](int block, SoloAcc& acc, char*) __attribute__((always_inline)) -> bool {
+  auto done = [&](int block, SoloAccOf<S>& acc, char*) __attribute__((always_inline)) -> bool {
     int f0, m0;
     tile_at(block, f0, m0);
     const int lane = solo_lane(), grp = lane >> 4;
-    const int f_wave = f0 + wave % S::WN * 64, m_wave = m0 + wave / S::WN * 128;
+    const int f_wave = f0 + wave % S::WN * (16 * kTiles), m_wave = m0 + wave / S::WN * (16 * S::TM);
     const int m_lane = m_wave + (lane & 15);
-    const bool whole = f_wave + 64 <= I && (reinterpret_cast<uintptr_t>(Y) & 15) == 0 && (ldy & 7) == 0;
+    const bool whole = f_wave + 16 * kTiles <= I && (reinterpret_cast<uintptr_t>(Y) & 15) == 0 && (ldy & 7) == 0;
 #pragma unroll
     for (int jm = 0; jm < S::TM; ++jm) {
-      f32x4_t y[4];
+      f32x4_t y[kTiles];
 #pragma unroll
-      for (int jn = 0; jn < 4; ++jn)
+      for (int jn = 0; jn < kTiles; ++jn)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          y[jn][q] = swiglu_f32(round_through_bf16(acc[jn][jm][q]), round_through_bf16(acc[jn + 4][jm][q]));
+          y[jn][q] = swiglu_f32(round_through_bf16(acc[jn][jm][q]), round_through_bf16(acc[jn + kTiles][jm][q]));
       const int m = m_lane + jm * 16;
       bf16_bits* const row = Y + (int64_t)m * ldy;
+      const int f = f_wave + grp * (4 * kTiles);
       if (whole) {
-        solo_store_span(row + f_wave, grp, m < M, y[0], y[1], y[2], y[3]);
-      } else if (m < M) {
-        const int f = f_wave + grp * 16;
+        if constexpr (kTiles == 4) {
+          solo_store_span(row + f_wave, grp, m < M, y[0], y[1], y[2], y[3]);
+        } else if (kTiles == 2) {
+          if (m < M)
+            *reinterpret_cast<u32x4_t*>(row + f) = u32x4_t{pack_bf16x2(y[0][0], y[0][1]), pack_bf16x2(y[0][2], y[0][3]),
+                                                           pack_bf16x2(y[kTiles - 1][0], y[kTiles - 1][1]), pack_bf16x2(y[kTiles - 1][2], y[kTiles - 1][3])};
+        } else if (m < M) {  // twelve features of a lane, 24 bytes, or four
 #pragma unroll
-        for (int e = 0; e < 16; ++e)
+          for (int jn = 0; jn < kTiles; ++jn)
+            *reinterpret_cast<u32x2_t*>(row + f + jn * 4) = u32x2_t{pack_bf16x2(y[jn][0], y[jn][1]), pack_bf16x2(y[jn][2], y[jn][3])};
+        }
+      } else if (m < M) {
+#pragma unroll
+        for (int e = 0; e < 4 * kTiles; ++e)
           if (f + e < I) row[f + e] = to_bf16_bits(y[e >> 2][e & 3]);
       }
     }
-    return whole && m_wave + 128 <= M;
+    return whole && m_wave + 16 * S::TM <= M;
   };
-  solo_tiles<SoloGatedRows, 2 * S::TM>(W, X, K, blockIdx.x, gridDim.x, tiles_m * tiles_n, lds, tile_at, done);
+  // (the three pieces of twelve features may leave as two stores)
+  solo_tiles<SoloGatedRows<S>, (kTiles > 2 ? 2 : 1) * S::TM, false, Layout>(W, X, K, blockIdx.x, gridDim.x, tiles_m * tiles_n, lds, tile_at, done);
 }
 
 // The same for few tokens: four waves over one wave column of BN / 2 gate rows and the up rows of the same features, all of
@@ -335,24 +348,24 @@ static hipError_t launch_gated_few(const MatView& W, const MatView& X, void* Y, 
   return hipGetLastError();
 }
 
+template <int BN, int BM>
 static hipError_t launch_gated_solo(const MatView& W, const MatView& X, void* Y, int64_t ldy, int M, int I, int K,
                                     hipStream_t stream) {
+  using Layout = SoloLayout<false, false, TileShape<BN, BM, 2, 2>>;
+  auto kernel = det_gemm_swiglu_solo_kernel<Layout>;
   static PerDeviceOnce once;
-  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(det_gemm_swiglu_solo_kernel), kSoloLdsBytes, once);
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), Layout::kLds, once);
   if (err != hipSuccess) return err;
-  const int tiles_m = (M + SoloShape::BM - 1) / SoloShape::BM;
-  const int tiles_n = (I + SoloShape::BN / 2 - 1) / (SoloShape::BN / 2);
+  const int tiles_m = (M + BM - 1) / BM;
+  const int tiles_n = (I + BN / 2 - 1) / (BN / 2);
   const int cus = device_cu_count();
   const int grid = tiles_m * tiles_n < cus ? tiles_m * tiles_n : cus;
-  hipLaunchKernelGGL(det_gemm_swiglu_solo_kernel, dim3(grid), dim3(SoloShape::kThreads), kSoloLdsBytes, stream, W, X,
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(SoloShape::kThreads), Layout::kLds, stream, W, X,
                      reinterpret_cast<bf16_bits*>(Y), ldy, M, I, K, tiles_m, tiles_n, tiles_m < 8 ? tiles_m : 8);
   return hipGetLastError();
 }
 
 using GatedShape256 = TileShape<256, 256, 4, 2>;
-using GatedShape192 = TileShape<256, 192, 4, 2>;
-using GatedShape128 = TileShape<256, 128, 4, 2>;
-using GatedShape64 = TileShape<256, 64, 4, 2>;
 
 template <class S, bool WSTREAM = false>
 static hipError_t launch_gated(const MatView& W, const MatView& X, void* Y, int64_t ldy, int M, int I, int K,
@@ -370,6 +383,41 @@ static hipError_t launch_gated(const MatView& W, const MatView& X, void* Y, int6
   hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n), dim3(S::kThreads), S::kLdsBytes, stream, W, X,
                      reinterpret_cast<bf16_bits*>(Y), ldy, M, I, K, tiles_m, tiles_n, group_m);
   return hipGetLastError();
+}
+
+// The tiles of the fused gate/up above 128 tokens, weight rows (gate and up) x tokens on four waves, and what a round of them takes
+// relative to 256 x 256 (us at K = 4096); a round that fills part of the chip takes its share of that, and no less than
+// kGatedPartial. Fitted to 140 shapes (I = 3072, 6144, 12288 with K = 4096, 6144 with 2048; 130 to 8200 tokens), 0.6 % above the
+// best tile of each. What takes the time of the small ones is the loads of one round, so a tile no larger than gives every CU one.
+// Eight waves in 256 rows x 256 / 192 / 128 / 64 tokens -> these, us, weights in turn: I = 3072 at 146 / 228 / 411 / 605 / 947 / 1214 tokens
+// 58.7 / 58.0 / 57.5 / 57.9 / 56.9 / 59.5 -> 27.2 / 27.1 / 36.0 / 37.7 / 48.2 / 54.6, 6144 at 150 / 250 / 349 / 725 / 1319 59.7 / 59.7 / 56.7
+// / 68.5 / 132 -> 35.1 / 41.4 / 49.2 / 59.7 / 111, 12288 at 231 / 310 / 474 / 987 66.2 / 73.8 / 87.1 / 171 -> 60.9 / 66.3 / 77.6 / 149, K = 2048
+// at 163 / 448 / 1929 32.7 / 32.1 / 93.5 -> 20.3 / 27.3 / 77.3. (The projection and the activation as two launches: 27.1 at I = 3072
+// and 146 tokens, 39 to 42 at 6144 up to 254, elsewhere slower.)
+struct GatedTile {
+  int bn, bm;
+  double us;
+  hipError_t (*launch)(const MatView&, const MatView&, void*, int64_t, int, int, int, hipStream_t);
+};
+static const GatedTile kGatedTiles[] = {
+    {256, 256, 97.0, launch_gated_solo<256, 256>}, {192, 256, 78.4, launch_gated_solo<192, 256>}, {256, 192, 79.0, launch_gated_solo<256, 192>},
+    {192, 192, 60.0, launch_gated_solo<192, 192>}, {256, 128, 59.0, launch_gated_solo<256, 128>}, {192, 128, 46.6, launch_gated_solo<192, 128>},
+    {128, 192, 47.7, launch_gated_solo<128, 192>}, {128, 128, 36.1, launch_gated_solo<128, 128>}, {64, 192, 24.5, launch_gated_solo<64, 192>},
+    {64, 128, 20.0, launch_gated_solo<64, 128>},
+};
+constexpr double kGatedPartial = 0.82;
+static const GatedTile& pick_gated_tile(int M, int I, int cus) {
+  const GatedTile* best = kGatedTiles;
+  double best_us = 1e300;
+  for (const GatedTile& t : kGatedTiles) {
+    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((I + t.bn / 2 - 1) / (t.bn / 2));
+    const double us = rounds_of_workgroups(tiles, cus, kGatedPartial) * t.us;
+    if (us < best_us * 0.999) {
+      best_us = us;
+      best = &t;
+    }
+  }
+  return *best;
 }
 
 // Up to 16 tokens the streaming kernel serves the packed projection (the same panels of 16 weight
@@ -412,27 +460,14 @@ hipError_t det_gemm_swiglu_launch(const MatView& W, const MatView& X, void* Y, i
       if (I <= 48 * cus) return launch_gated_few<96, 2, 1, 5>(W, X, Y, ldy, M, I, K, stream);
       return launch_gated_few<128, 2, 1, 4>(W, X, Y, ldy, M, I, K, stream);
     }
-    const int64_t t256 = (int64_t)((M + 255) / 256) * ((I + 127) / 128);
-    const int64_t t192 = (int64_t)((M + 191) / 192) * ((I + 127) / 128);
-    const int64_t t128 = (int64_t)((M + 127) / 128) * ((I + 127) / 128);
-    // Rounds of workgroups x tokens per tile / relative throughput, as in pick_det_gemm_config:
-    // a partly filled last round costs little more than its share, so the large tile wins early. 192-token tiles, K = 4096,
-    // before -> with them: I = 12288 at 308 / 778 / 1492 tokens 85.8 / 163 / 249 -> 72.0 / 144 / 220 us, 6144 at 722 tokens 78.6
-    // -> 68.2, 3072 at 1908 tokens 76.8 -> 69.6.
     const int cus = device_cu_count();
-    auto cost = [cus](int64_t tiles, double tokens, double quality) {
-      return rounds_of_workgroups(tiles, cus) * tokens / quality;
-    };
-    const double c256 = cost(t256, 256.0, 1.0), c192 = cost(t192, 192.0, 0.87), c128 = cost(t128, 128.0, 0.65);
-    if (M > 128 && c192 < c256 && c192 < c128) return launch_gated<GatedShape192>(W, X, Y, ldy, M, I, K, stream);
-    if (M > 128 && c256 <= c128) {
-      // (a weight that is read past the caches has the ping-pong loop only)
-      if (solo_tiles_pay(t256, cus) && !streamed_weight(2 * (int64_t)I, K, M, 256) && solo_offsets_fit(W, (int64_t)I + 128) && solo_offsets_fit(X))
-        return launch_gated_solo(W, X, Y, ldy, M, I, K, stream);
+    const bool fits = solo_offsets_fit(W, (int64_t)I + 128) && solo_offsets_fit(X);
+    const int64_t t256 = (int64_t)((M + 255) / 256) * ((I + 127) / 128);
+    const GatedTile& tile = fits ? pick_gated_tile(M, I, cus) : kGatedTiles[0];
+    // (256 x 256 on eight waves: few tiles, a weight that is read past the caches, operands of 4 GiB)
+    if (tile.launch == kGatedTiles[0].launch && !(fits && solo_tiles_pay(t256, cus) && !streamed_weight(2 * (int64_t)I, K, M, 256)))
       return launch_gated<GatedShape256>(W, X, Y, ldy, M, I, K, stream);
-    }
-    if (M > 64 && t128 >= 128) return launch_gated<GatedShape128>(W, X, Y, ldy, M, I, K, stream);
-    return launch_gated<GatedShape64>(W, X, Y, ldy, M, I, K, stream);
+    return tile.launch(W, X, Y, ldy, M, I, K, stream);
   }
   if (workspace == nullptr) return hipErrorInvalidValue;
   hipError_t err = det_gemm_launch(W, X, workspace, 2 * (int64_t)I, M, 2 * I, K, false, RLK_GEMM_CFG_AUTO, stream);

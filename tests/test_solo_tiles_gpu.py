@@ -65,6 +65,25 @@ def test_gated_projection(tokens, inter, k):
     assert torch.equal(y.view(torch.int16), _C.swiglu_packed_forward(gate_up).view(torch.int16))
 
 
+# sizes that the choice gives each of the gated tiles, on 256 CUs: 64 x 128, 64 x 192, 128 x 128, 192 x 128, 128 x 192, 256 x 128, 192 x
+# 192, 192 x 256, 256 x 192; rows of the result whole 16 bytes (whole stores and element stores of the last tile) and not
+@pytest.mark.parametrize("tokens,inter", [(129, 3064), (300, 2049), (150, 6136), (411, 3064), (390, 6136), (390, 6141), (947, 3064), (947, 3066),
+                                          (640, 6136), (310, 12280), (310, 12281), (474, 12280), (1800, 3064)])  # fmt: skip
+@pytest.mark.parametrize("k", [64, 128, 512])
+def test_gated_tiles_of_few_tokens(tokens, inter, k):
+    """The projection followed by the activation, bit for bit; from one K tile to more than the stages of a ring."""
+    from rl_engine import _C
+
+    gen = torch.Generator(device=DEV).manual_seed(tokens + k)
+    x = torch.randn((tokens, k), generator=gen, device=DEV, dtype=torch.bfloat16)
+    w = torch.randn((2 * inter, k), generator=gen, device=DEV, dtype=torch.bfloat16).mul_(0.1)
+    gate_up = torch.empty((tokens, 2 * inter), device=DEV, dtype=torch.bfloat16)
+    _C.gemm_strided(x, w.t(), gate_up, config=5)  # 64 x 64
+    want = _C.swiglu_packed_forward(gate_up)
+    for _ in range(2):
+        assert torch.equal(_C.det_gemm_swiglu(x, w).view(torch.int16), want.view(torch.int16))
+
+
 # one K tile, as many as stages and one more or less, edges of tiles of either side, tails of a few rows, more tiles than CUs
 @pytest.mark.parametrize("shape", [(1, 8, 64), (192, 192, 128), (129, 200, 192), (400, 392, 256), (257, 777, 320), (300, 500, 1024), (3100, 3200, 448)])
 @pytest.mark.parametrize("name", ["256x192", "192x256", "192x192", "256x128", "192x128"])
