@@ -526,6 +526,13 @@ int rlk_det_gemm_swiglu_bf16(const void* a, int64_t a_row_stride, const void* w_
                              void* y, int64_t ldy, void* workspace, size_t workspace_bytes, int M, int I, int K,
                              void* stream);
 
+/*
+ * The forward of a gated FFN's training step: gate[M, I] = a @ w_gate^T, up[M, I] = a @ w_up^T and y = swiglu(gate, up), the bits of
+ * two calls of rlk_det_gemm_bf16 and one of rlk_swiglu_fwd; weights [I, K] of one row stride, results of one row stride.
+ */
+int rlk_det_gemm_swiglu_training_bf16(const void* a, int64_t a_row_stride, const void* w_gate, const void* w_up, int64_t w_row_stride,
+                                      void* gate, void* up, void* y, int64_t ld, int M, int I, int K, void* stream);
+
 /* Bytes of workspace rlk_grpo_ratio_kl_loss needs. */
 size_t rlk_grpo_workspace_bytes(int rollouts);
 

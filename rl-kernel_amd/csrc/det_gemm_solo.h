@@ -69,15 +69,16 @@ struct SoloPlainRows {
   static __device__ __forceinline__ int64_t row(int r, int last, int) { return min(feature(r), last); }
   static __device__ __forceinline__ int features(const MatView& W) { return W.rows; }
 };
-template <class S>
+// SPLIT: of two weights [I, K]. Odd waves load the up rows, even ones the gate rows: W.ptr is the one or the other.
+template <class S, bool SPLIT = false>
 struct SoloGatedRows {
   static __device__ __forceinline__ int64_t row(int r, int last, int half_rows) {
     constexpr int kWaveRows = 16 * S::TN, kTiles = S::TN / 2;
     const int wave = r / kWaveRows, tile = r % kWaveRows / 16;
     const int f = wave * (kWaveRows / 2) + ((r & 15) >> 2) * (4 * kTiles) + tile % kTiles * 4 + (r & 3);
-    return min(f, last) + tile / kTiles * half_rows;
+    return min(f, last) + (SPLIT ? 0 : tile / kTiles * half_rows);
   }
-  static __device__ __forceinline__ int features(const MatView& W) { return W.rows / 2; }
+  static __device__ __forceinline__ int features(const MatView& W) { return SPLIT ? W.rows : W.rows / 2; }
 };
 
 // How the operands lie in memory. A K-major part holds four columns of 64 rows (features, tokens), each 64 K rows of 128 bytes, in the

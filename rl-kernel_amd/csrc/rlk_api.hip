@@ -672,6 +672,24 @@ int rlk_det_gemm_swiglu_bf16(const void* a, int64_t a_row_stride, const void* w_
   return err == hipSuccess ? RLK_OK : device_error("rlk_det_gemm_swiglu_bf16", err);
 }
 
+int rlk_det_gemm_swiglu_training_bf16(const void* a, int64_t a_row_stride, const void* w_gate, const void* w_up, int64_t w_row_stride,
+                                      void* gate, void* up, void* y, int64_t ld, int M, int I, int K, void* stream) {
+  if (M < 1 || I < 1 || K < 1) {
+    set_last_error("rlk_det_gemm_swiglu_training_bf16: M=%d I=%d K=%d must be positive", M, I, K);
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  if (a == nullptr || w_gate == nullptr || w_up == nullptr || gate == nullptr || up == nullptr || y == nullptr || a_row_stride < K ||
+      w_row_stride < K || ld < I) {
+    set_last_error("rlk_det_gemm_swiglu_training_bf16: null pointer, or a row stride below the columns");
+    return RLK_ERR_INVALID_ARGUMENT;
+  }
+  const MatView X{reinterpret_cast<const bf16_bits*>(a), a_row_stride, 1, M};
+  const MatView W_gate{reinterpret_cast<const bf16_bits*>(w_gate), w_row_stride, 1, I};
+  const MatView W_up{reinterpret_cast<const bf16_bits*>(w_up), w_row_stride, 1, I};
+  const hipError_t err = det_gemm_swiglu_training_launch(W_gate, W_up, X, gate, up, y, ld, M, I, K, reinterpret_cast<hipStream_t>(stream));
+  return err == hipSuccess ? RLK_OK : device_error("rlk_det_gemm_swiglu_training_bf16", err);
+}
+
 size_t rlk_grpo_workspace_bytes(int rollouts) { return rollouts > 0 ? (size_t)3 * rollouts * sizeof(float) : 0; }
 
 int rlk_grpo_ratio_kl_loss(const float* logp, const float* old_logp, const float* ref_logp,

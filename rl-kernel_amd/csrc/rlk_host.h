@@ -214,6 +214,8 @@ hipError_t swiglu_launch(const void* gate, int64_t ld_g, const void* up, int64_t
 // Packed gate/up projection W[2 I, K] with the SwiGLU epilogue; workspace ([M, 2 I] bf16) is
 // only touched when det_gemm_swiglu_fused_supported() is false.
 bool det_gemm_swiglu_fused_supported(const MatView& W, const MatView& X, int M, int K);
+hipError_t det_gemm_swiglu_training_launch(const MatView& W_gate, const MatView& W_up, const MatView& X, void* gate, void* up, void* Y,
+                                           int64_t ldy, int M, int I, int K, hipStream_t stream);
 hipError_t det_gemm_swiglu_launch(const MatView& W, const MatView& X, void* Y, int64_t ldy, void* workspace, int M,
                                   int I, int K, hipStream_t stream);
 

@@ -231,16 +231,40 @@ __global__ __launch_bounds__(S::kThreads) void det_gemm_swiglu_kernel(MatView W,
   }
 }
 
-// The same with one wave per SIMD, a workgroup per CU (det_gemm_solo.h).
-template <class Layout>
+// The same with one wave per SIMD, a workgroup per CU (det_gemm_solo.h). Training: gate and up weights apart, and both projections
+// are stored beside the activation, for the backward.
+struct GatedTraining {
+  const bf16_bits* up_weight;
+  bf16_bits *gate, *up;
+};
+
+// KT MFMA tiles of 16 features each, a lane's 4 KT of them consecutive, at `row`, the wave's first feature of a token.
+template <int KT>
+__device__ __forceinline__ void store_gated_span(bf16_bits* row, int grp, bool live, const f32x4_t (&y)[KT]) {
+  bf16_bits* const mine = row + grp * (4 * KT);
+  if constexpr (KT == 4) {
+    solo_store_span(row, grp, live, y[0], y[1], y[2], y[3]);
+  } else if constexpr (KT == 2) {
+    if (live)
+      *reinterpret_cast<u32x4_t*>(mine) = u32x4_t{pack_bf16x2(y[0][0], y[0][1]), pack_bf16x2(y[0][2], y[0][3]),
+                                                  pack_bf16x2(y[1][0], y[1][1]), pack_bf16x2(y[1][2], y[1][3])};
+  } else if (live) {  // 24 bytes, or 8
+#pragma unroll
+    for (int jn = 0; jn < KT; ++jn)
+      *reinterpret_cast<u32x2_t*>(mine + jn * 4) = u32x2_t{pack_bf16x2(y[jn][0], y[jn][1]), pack_bf16x2(y[jn][2], y[jn][3])};
+  }
+}
+
+template <class Layout, bool TRAINING>
 __global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_swiglu_solo_kernel(MatView W, MatView X,
                                                                                    bf16_bits* __restrict__ Y, int64_t ldy,
                                                                                    int M, int I, int K, int tiles_m,
-                                                                                   int tiles_n, int group_m) {
+                                                                                   int tiles_n, int group_m, GatedTraining training) {
   using S = typename Layout::Shape;
   constexpr int kTiles = S::TN / 2;  // MFMA tiles of a wave that hold gate features, and that hold up features
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (TRAINING && (wave & 1)) W.ptr = training.up_weight;
   auto tile_at = [&](int block, int& f0, int& m0) __attribute__((always_inline)) {
     const TileOrder at = tile_order(block, tiles_m, tiles_n, group_m);
     f0 = at.tile_n * (S::BN / 2);
@@ -255,37 +279,41 @@ __global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_swiglu_solo_kern
     const bool whole = f_wave + 16 * kTiles <= I && (reinterpret_cast<uintptr_t>(Y) & 15) == 0 && (ldy & 7) == 0;
 #pragma unroll
     for (int jm = 0; jm < S::TM; ++jm) {
-      f32x4_t y[kTiles];
+      f32x4_t y[kTiles], g[kTiles], u[kTiles];
 #pragma unroll
       for (int jn = 0; jn < kTiles; ++jn)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          y[jn][q] = swiglu_f32(round_through_bf16(acc[jn][jm][q]), round_through_bf16(acc[jn + kTiles][jm][q]));
+        for (int q = 0; q < 4; ++q) {
+          g[jn][q] = round_through_bf16(acc[jn][jm][q]);
+          u[jn][q] = round_through_bf16(acc[jn + kTiles][jm][q]);
+          y[jn][q] = swiglu_f32(g[jn][q], u[jn][q]);
+        }
       const int m = m_lane + jm * 16;
-      bf16_bits* const row = Y + (int64_t)m * ldy;
-      const int f = f_wave + grp * (4 * kTiles);
+      const int64_t at = (int64_t)m * ldy;
       if (whole) {
-        if constexpr (kTiles == 4) {
-          solo_store_span(row + f_wave, grp, m < M, y[0], y[1], y[2], y[3]);
-        } else if (kTiles == 2) {
-          if (m < M)
-            *reinterpret_cast<u32x4_t*>(row + f) = u32x4_t{pack_bf16x2(y[0][0], y[0][1]), pack_bf16x2(y[0][2], y[0][3]),
-                                                           pack_bf16x2(y[kTiles - 1][0], y[kTiles - 1][1]), pack_bf16x2(y[kTiles - 1][2], y[kTiles - 1][3])};
-        } else if (m < M) {  // twelve features of a lane, 24 bytes, or four
-#pragma unroll
-          for (int jn = 0; jn < kTiles; ++jn)
-            *reinterpret_cast<u32x2_t*>(row + f + jn * 4) = u32x2_t{pack_bf16x2(y[jn][0], y[jn][1]), pack_bf16x2(y[jn][2], y[jn][3])};
+        store_gated_span<kTiles>(Y + at + f_wave, grp, m < M, y);
+        if constexpr (TRAINING) {
+          store_gated_span<kTiles>(training.gate + at + f_wave, grp, m < M, g);
+          store_gated_span<kTiles>(training.up + at + f_wave, grp, m < M, u);
         }
       } else if (m < M) {
+        const int f = f_wave + grp * (4 * kTiles);
 #pragma unroll
         for (int e = 0; e < 4 * kTiles; ++e)
-          if (f + e < I) row[f + e] = to_bf16_bits(y[e >> 2][e & 3]);
+          if (f + e < I) {
+            Y[at + f + e] = to_bf16_bits(y[e >> 2][e & 3]);
+            if constexpr (TRAINING) {
+              training.gate[at + f + e] = to_bf16_bits(g[e >> 2][e & 3]);
+              training.up[at + f + e] = to_bf16_bits(u[e >> 2][e & 3]);
+            }
+          }
       }
     }
     return whole && m_wave + 16 * S::TM <= M;
   };
   // (the three pieces of twelve features may leave as two stores)
-  solo_tiles<SoloGatedRows<S>, (kTiles > 2 ? 2 : 1) * S::TM, false, Layout>(W, X, K, blockIdx.x, gridDim.x, tiles_m * tiles_n, lds, tile_at, done);
+  constexpr int kStores = (kTiles > 2 ? 2 : 1) * S::TM * (TRAINING ? 3 : 1);
+  solo_tiles<SoloGatedRows<S, TRAINING>, kStores, false, Layout>(W, X, K, blockIdx.x, gridDim.x, tiles_m * tiles_n, lds, tile_at, done);
 }
 
 // The same for few tokens: four waves over one wave column of BN / 2 gate rows and the up rows of the same features, all of
@@ -348,11 +376,11 @@ static hipError_t launch_gated_few(const MatView& W, const MatView& X, void* Y, 
   return hipGetLastError();
 }
 
-template <int BN, int BM>
+template <int BN, int BM, bool TRAINING>
 static hipError_t launch_gated_solo(const MatView& W, const MatView& X, void* Y, int64_t ldy, int M, int I, int K,
-                                    hipStream_t stream) {
+                                    const GatedTraining& training, hipStream_t stream) {
   using Layout = SoloLayout<false, false, TileShape<BN, BM, 2, 2>>;
-  auto kernel = det_gemm_swiglu_solo_kernel<Layout>;
+  auto kernel = det_gemm_swiglu_solo_kernel<Layout, TRAINING>;
   static PerDeviceOnce once;
   hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), Layout::kLds, once);
   if (err != hipSuccess) return err;
@@ -361,7 +389,7 @@ static hipError_t launch_gated_solo(const MatView& W, const MatView& X, void* Y,
   const int cus = device_cu_count();
   const int grid = tiles_m * tiles_n < cus ? tiles_m * tiles_n : cus;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(SoloShape::kThreads), Layout::kLds, stream, W, X,
-                     reinterpret_cast<bf16_bits*>(Y), ldy, M, I, K, tiles_m, tiles_n, tiles_m < 8 ? tiles_m : 8);
+                     reinterpret_cast<bf16_bits*>(Y), ldy, M, I, K, tiles_m, tiles_n, tiles_m < 8 ? tiles_m : 8, training);
   return hipGetLastError();
 }
 
@@ -394,16 +422,27 @@ static hipError_t launch_gated(const MatView& W, const MatView& X, void* Y, int6
 // / 68.5 / 132 -> 35.1 / 41.4 / 49.2 / 59.7 / 111, 12288 at 231 / 310 / 474 / 987 66.2 / 73.8 / 87.1 / 171 -> 60.9 / 66.3 / 77.6 / 149, K = 2048
 // at 163 / 448 / 1929 32.7 / 32.1 / 93.5 -> 20.3 / 27.3 / 77.3. (The projection and the activation as two launches: 27.1 at I = 3072
 // and 146 tokens, 39 to 42 at 6144 up to 254, elsewhere slower.)
+typedef hipError_t (*GatedLaunch)(const MatView&, const MatView&, void*, int64_t, int, int, int, const GatedTraining&, hipStream_t);
 struct GatedTile {
   int bn, bm;
   double us;
-  hipError_t (*launch)(const MatView&, const MatView&, void*, int64_t, int, int, int, hipStream_t);
+  GatedLaunch launch, launch_training;
 };
+template <int BN, int BM>
+constexpr GatedTile gated_tile(double us) {
+  return {BN, BM, us, launch_gated_solo<BN, BM, false>, launch_gated_solo<BN, BM, true>};
+}
 static const GatedTile kGatedTiles[] = {
-    {256, 256, 97.0, launch_gated_solo<256, 256>}, {192, 256, 78.4, launch_gated_solo<192, 256>}, {256, 192, 79.0, launch_gated_solo<256, 192>},
-    {192, 192, 60.0, launch_gated_solo<192, 192>}, {256, 128, 59.0, launch_gated_solo<256, 128>}, {192, 128, 46.6, launch_gated_solo<192, 128>},
-    {128, 192, 47.7, launch_gated_solo<128, 192>}, {128, 128, 36.1, launch_gated_solo<128, 128>}, {64, 192, 24.5, launch_gated_solo<64, 192>},
-    {64, 128, 20.0, launch_gated_solo<64, 128>},
+    gated_tile<256, 256>(97.0),
+    gated_tile<192, 256>(78.4),
+    gated_tile<256, 192>(79.0),
+    gated_tile<192, 192>(60.0),
+    gated_tile<256, 128>(59.0),
+    gated_tile<192, 128>(46.6),
+    gated_tile<128, 192>(47.7),
+    gated_tile<128, 128>(36.1),
+    gated_tile<64, 192>(24.5),
+    gated_tile<64, 128>(20.0),
 };
 constexpr double kGatedPartial = 0.82;
 static const GatedTile& pick_gated_tile(int M, int I, int cus) {
@@ -467,7 +506,7 @@ hipError_t det_gemm_swiglu_launch(const MatView& W, const MatView& X, void* Y, i
     // (256 x 256 on eight waves: few tiles, a weight that is read past the caches, operands of 4 GiB)
     if (tile.launch == kGatedTiles[0].launch && !(fits && solo_tiles_pay(t256, cus) && !streamed_weight(2 * (int64_t)I, K, M, 256)))
       return launch_gated<GatedShape256>(W, X, Y, ldy, M, I, K, stream);
-    return tile.launch(W, X, Y, ldy, M, I, K, stream);
+    return tile.launch(W, X, Y, ldy, M, I, K, GatedTraining{}, stream);
   }
   if (workspace == nullptr) return hipErrorInvalidValue;
   hipError_t err = det_gemm_launch(W, X, workspace, 2 * (int64_t)I, M, 2 * I, K, false, RLK_GEMM_CFG_AUTO, stream);
@@ -475,6 +514,27 @@ hipError_t det_gemm_swiglu_launch(const MatView& W, const MatView& X, void* Y, i
   const bf16_bits* gu = reinterpret_cast<const bf16_bits*>(workspace);
   return swiglu_launch(gu, 2 * (int64_t)I, gu + I, 2 * (int64_t)I, nullptr, 0, Y, ldy, nullptr, 0, M, I, false,
                        RLK_DTYPE_BF16, stream);
+}
+
+// gate[M, I], up[M, I] and Y[M, I] = swiglu(gate, up) of two weights, in one launch above 128 tokens: the activation's launch read both
+// projections again, and tiles of both together fill the chip better than those of each. Three launches -> one, us (tokens, I, K):
+// 4096, 12288, 4096 629 -> 601; 2026, 12288, 4096 337 -> 296; 359, 12288, 4096 109 -> 75; 803, 6144, 4096 98 -> 80; 923, 3072, 4096 73 -> 51; 215, 3072,
+// 4096 37 -> 26; 736, 6144, 2048 62 -> 41; of 46 shapes none slower (2110, 12288, 4096: 371 both).
+hipError_t det_gemm_swiglu_training_launch(const MatView& W_gate, const MatView& W_up, const MatView& X, void* gate, void* up, void* Y,
+                                           int64_t ldy, int M, int I, int K, hipStream_t stream) {
+  // (what holds of the gate weight's rows holds of the up weight's: the same pitch, and the alignment is looked at)
+  const bool fused = M > 128 && det_gemm_swiglu_fused_supported(W_gate, X, M, K) && (reinterpret_cast<uintptr_t>(W_up.ptr) & 15) == 0 &&
+                     ((reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up)) & 15) == 0 && solo_offsets_fit(W_gate) &&
+                     solo_offsets_fit(X);
+  if (fused) {
+    const GatedTraining training{W_up.ptr, reinterpret_cast<bf16_bits*>(gate), reinterpret_cast<bf16_bits*>(up)};
+    return pick_gated_tile(M, I, device_cu_count()).launch_training(W_gate, X, Y, ldy, M, I, K, training, stream);
+  }
+  hipError_t err = det_gemm_launch(W_gate, X, gate, ldy, M, I, K, false, RLK_GEMM_CFG_AUTO, stream);
+  if (err != hipSuccess) return err;
+  err = det_gemm_launch(W_up, X, up, ldy, M, I, K, false, RLK_GEMM_CFG_AUTO, stream);
+  if (err != hipSuccess) return err;
+  return swiglu_launch(gate, ldy, up, ldy, nullptr, 0, Y, ldy, nullptr, 0, M, I, false, RLK_DTYPE_BF16, stream);
 }
 
 }  // namespace rlk

@@ -41,7 +41,7 @@ decltype(&rlk_det_gemm_bf16) gemm_entry = nullptr;
 decltype(&rlk_linear_bwd_bf16) linear_bwd_entry = nullptr;
 decltype(&rlk_det_gemm_swiglu_workspace_bytes) swiglu_workspace_entry = nullptr;
 decltype(&rlk_det_gemm_swiglu_bf16) swiglu_entry = nullptr;
-decltype(&rlk_swiglu_fwd) swiglu_fwd_entry = nullptr;
+decltype(&rlk_det_gemm_swiglu_training_bf16) swiglu_training_entry = nullptr;
 decltype(&rlk_swiglu_bwd) swiglu_bwd_entry = nullptr;
 decltype(&rlk_grpo_workspace_bytes) grpo_workspace_entry = nullptr;
 decltype(&rlk_grpo_ratio_kl_loss) grpo_entry = nullptr;
@@ -213,12 +213,11 @@ struct FfnFn : torch::autograd::Function<FfnFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& input, const Tensor& gate_weight, const Tensor& up_weight,
                         const Tensor& down_weight) {
     const Tensor x = input.dim() == 2 ? input : input.view({-1, input.size(-1)});
-    const Tensor gate = project(x, gate_weight), up = project(x, up_weight);
-    const int64_t m = x.size(0), inter = gate.size(1);
-    const Tensor activated = empty({m, inter}, kBf16, x);
-    check_status(swiglu_fwd_entry(gate.data_ptr(), inter, up.data_ptr(), inter, activated.data_ptr(), inter, (int)m, (int)inter,
-                                  RLK_DTYPE_BF16, stream_of(x)),
-                 "rlk_swiglu_fwd failed");
+    const int64_t m = x.size(0), k = x.size(1), inter = gate_weight.size(0);
+    const Tensor gate = empty({m, inter}, kBf16, x), up = empty({m, inter}, kBf16, x), activated = empty({m, inter}, kBf16, x);
+    check_status(swiglu_training_entry(x.data_ptr(), k, gate_weight.data_ptr(), up_weight.data_ptr(), k, gate.data_ptr(), up.data_ptr(),
+                                       activated.data_ptr(), inter, (int)m, (int)inter, (int)k, stream_of(x)),
+                 "rlk_det_gemm_swiglu_training_bf16 failed");
     ctx->save_for_backward({x, gate, up, activated, gate_weight, up_weight, down_weight});
     ctx->saved_data["shape"] = input.sizes().vec();
     const Tensor out = project(activated, down_weight);
@@ -454,7 +453,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
   entry("rlk_linear_bwd_bf16", linear_bwd_entry);
   entry("rlk_det_gemm_swiglu_workspace_bytes", swiglu_workspace_entry);
   entry("rlk_det_gemm_swiglu_bf16", swiglu_entry);
-  entry("rlk_swiglu_fwd", swiglu_fwd_entry);
+  entry("rlk_det_gemm_swiglu_training_bf16", swiglu_training_entry);
   entry("rlk_swiglu_bwd", swiglu_bwd_entry);
   entry("rlk_grpo_workspace_bytes", grpo_workspace_entry);
   entry("rlk_grpo_ratio_kl_loss", grpo_entry);

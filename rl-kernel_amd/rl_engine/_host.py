@@ -8,7 +8,7 @@ from rl_engine import _lib
 
 _ENTRIES = (
     "rlk_last_error", "rlk_det_gemm_bf16", "rlk_linear_bwd_bf16", "rlk_det_gemm_swiglu_workspace_bytes", "rlk_det_gemm_swiglu_bf16",
-    "rlk_swiglu_fwd", "rlk_swiglu_bwd", "rlk_grpo_workspace_bytes", "rlk_grpo_ratio_kl_loss", "rlk_grpo_ratio_kl_loss_bwd",
+    "rlk_det_gemm_swiglu_training_bf16", "rlk_swiglu_bwd", "rlk_grpo_workspace_bytes", "rlk_grpo_ratio_kl_loss", "rlk_grpo_ratio_kl_loss_bwd",
 )  # fmt: skip
 _native = None
 

@@ -101,6 +101,7 @@ EXPORTED_SYMBOLS = (
     "rlk_swiglu_bwd",
     "rlk_det_gemm_swiglu_workspace_bytes",
     "rlk_det_gemm_swiglu_bf16",
+    "rlk_det_gemm_swiglu_training_bf16",
     "rlk_grpo_workspace_bytes",
     "rlk_grpo_ratio_kl_loss",
     "rlk_grpo_ratio_kl_loss_bwd",
@@ -210,6 +211,8 @@ def load() -> ctypes.CDLL:
     lib.rlk_swiglu_bwd.argtypes = [vp, i64, vp, i64, vp, i64, vp, i64, vp, i64, i32, i32, i32, vp]
     lib.rlk_det_gemm_swiglu_workspace_bytes.restype = sz
     lib.rlk_det_gemm_swiglu_workspace_bytes.argtypes = [vp, i64, vp, i64, i32, i32, i32]
+    lib.rlk_det_gemm_swiglu_training_bf16.restype = i32
+    lib.rlk_det_gemm_swiglu_training_bf16.argtypes = [vp, i64, vp, vp, i64, vp, vp, vp, i64, i32, i32, i32, vp]
     lib.rlk_det_gemm_swiglu_bf16.restype = i32
     lib.rlk_det_gemm_swiglu_bf16.argtypes = [vp, i64, vp, i64, vp, i64, vp, sz, i32, i32, i32, vp]
 

@@ -84,6 +84,29 @@ def test_gated_tiles_of_few_tokens(tokens, inter, k):
         assert torch.equal(_C.det_gemm_swiglu(x, w).view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("tokens,inter,k", [(1, 8, 64), (128, 264, 128), (129, 3064, 64), (300, 2049, 192), (150, 6136, 128), (411, 3064, 512), (390, 6141, 128),
+                                            (947, 3064, 64), (640, 6136, 128), (310, 12280, 64), (474, 12280, 128), (1800, 3064, 128),
+                                            (4096, 4100, 128), (200, 264, 72)])  # fmt: skip
+def test_gate_and_up_of_a_training_step(tokens, inter, k):
+    """Two weights, both projections kept: the bits of three launches; what the one launch does not take among the sizes."""
+    from rl_engine import _C, _lib
+
+    gen = torch.Generator(device=DEV).manual_seed(tokens + k)
+    x = torch.randn((tokens, k), generator=gen, device=DEV, dtype=torch.bfloat16)
+    up_w, gate_w = (torch.randn((inter, k), generator=gen, device=DEV, dtype=torch.bfloat16).mul_(0.1) for _ in range(2))
+    want = []
+    for w in (gate_w, up_w):
+        want.append(torch.empty((tokens, inter), device=DEV, dtype=torch.bfloat16))
+        _C.gemm_strided(x, w.t(), want[-1], config=5)  # 64 x 64
+    want.append(_C.swiglu_forward(*want))
+    got = [torch.full((tokens, inter), 7.0, device=DEV, dtype=torch.bfloat16) for _ in range(3)]
+    status = _lib.load().rlk_det_gemm_swiglu_training_bf16(
+        x.data_ptr(), k, gate_w.data_ptr(), up_w.data_ptr(), k, *(t.data_ptr() for t in got), inter, tokens, inter, k,
+        torch.cuda.current_stream().cuda_stream)  # fmt: skip
+    assert status == 0
+    assert all(torch.equal(g.view(torch.int16), w.view(torch.int16)) for g, w in zip(got, want))
+
+
 # one K tile, as many as stages and one more or less, edges of tiles of either side, tails of a few rows, more tiles than CUs
 @pytest.mark.parametrize("shape", [(1, 8, 64), (192, 192, 128), (129, 200, 192), (400, 392, 256), (257, 777, 320), (300, 500, 1024), (3100, 3200, 448)])
 @pytest.mark.parametrize("name", ["256x192", "192x256", "192x192", "256x128", "192x128"])
