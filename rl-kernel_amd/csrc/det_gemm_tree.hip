@@ -965,16 +965,22 @@ __device__ __forceinline__ float round_bf16(float zero, float x) {
   return __builtin_bit_cast(float, __builtin_convertvector((f32x2_t{zero, x}), bf16x2_t));
 }
 
-template <int R, int CHUNKS, int SLOTS>
+// Leaves of 20 and 28 (K = 5120, 14336) do not start on 16 bytes: their loads move four bytes a lane, into the places that the
+// chunks of a 32-wide leaf have (what lies past the leaf is read again from its end and not used). 16 + 4 R loads a leaf instead of
+// 4 + R are still few beside its matrix instructions. Such trees ran the tiled kernel with loads of single elements: 4096 outputs, K =
+// 14336 at 2 / 406 rows 2774 / 2799 us, here 108 / 636.
+template <int R, int CHUNKS, int SLOTS, int LEN = 8 * CHUNKS>
 __global__ __launch_bounds__(64 << tree_rows_split<R>(), (R == 1 ? 4 : 2)) void det_gemm_tree_rows_kernel(
     MatView A, MatView B, bf16_bits* __restrict__ C, int64_t ldc, int M, int N, int K, int depth, int row_groups) {
   using L = TreeRowsLds<R, CHUNKS>;
-  static_assert(CHUNKS == 3 || CHUNKS == 4, "leaves of 24 or 32");
+  constexpr bool kDwords = LEN % 8 != 0;
+  static_assert(kDwords ? CHUNKS == 4 && LEN % 4 == 0 : LEN == 8 * CHUNKS && (CHUNKS == 3 || CHUNKS == 4), "leaves of 20, 24, 28 or 32");
   constexpr int kRows = 16 * R;
   constexpr int kSets = 4 / R;                              // k steps that a widened register of A serves
-  constexpr int kAReads = (CHUNKS + kSets - 1) / kSets;     // of 16 bytes, per lane and leaf
-  constexpr int kLoadsPerLeaf = CHUNKS + R;
-  constexpr int len = 8 * CHUNKS;  // leaf length
+  constexpr int kUsed = (LEN + 7) / 8;                      // chunks that hold k of the leaf
+  constexpr int kAReads = (kUsed + kSets - 1) / kSets;      // of 16 bytes, per lane and leaf
+  constexpr int kLoadsPerLeaf = kDwords ? 16 + 4 * R : CHUNKS + R;
+  constexpr int len = LEN;
   extern __shared__ __attribute__((aligned(16))) char tree_lds[];
 
   float zero = 0.f;
@@ -1003,6 +1009,21 @@ __global__ __launch_bounds__(64 << tree_rows_split<R>(), (R == 1 ? 4 : 2)) void 
     const int row_in = m0 + row < M ? row : M - 1 - m0;
     a_off[j] = 2u * (uint32_t)(row_in * (int)A.row_stride + 8 * ((g % CHUNKS) ^ swizzle(row)));
   }
+  // Loads of four bytes: load j brings columns (rows) 4 j + lane / 16, the sixteen lanes of each its 64 bytes; which of the leaf's
+  // 32-bit words a lane fetches depends on the swizzle of those four columns, j % 4. A buffer ends with its last row: what lies past
+  // it reads zeros, and no load needs a vector instruction (the scalar offset stays within the size, or the check would wrap).
+  uint32_t w_word[4], a_word[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int w = 4 * (((lane & 15) >> 2) ^ s) + (lane & 3), word = w < len / 2 ? w : len / 2 - 1;
+    w_word[s] = 2u * (uint32_t)((lane >> 4) * (int)B.row_stride) + 4 * word;
+    a_word[s] = 2u * (uint32_t)((lane >> 4) * (int)A.row_stride) + 4 * word;
+  }
+  const uint32_t w_pitch = 8u * (uint32_t)B.row_stride, a_pitch = 8u * (uint32_t)A.row_stride;  // bytes of four rows
+  auto extent = [&](const MatView& v, int last, int most) __attribute__((always_inline)) {
+    return (uint32_t)(last < most ? last : most) * 2u * (uint32_t)v.row_stride + 2u * (uint32_t)(K - wave_k);
+  };
+  const uint32_t w_bytes = extent(B, N - 1 - n0, 63), a_bytes = extent(A, M - 1 - m0, kRows - 1);
   char* const mine = tree_lds + wave * L::kWaveBytes;
   // Lane l reads column l, and row l % kRows: chunk kSets i + l / kRows of it in read i (past the leaf: its last chunk,
   // not used).
@@ -1026,6 +1047,19 @@ __global__ __launch_bounds__(64 << tree_rows_split<R>(), (R == 1 ? 4 : 2)) void 
     const char* a_leaf = a_base + lo;
     asm volatile("" : "+s"(w_leaf));
     asm volatile("" : "+s"(a_leaf));
+    if constexpr (kDwords) {
+      const __amdgpu_buffer_rsrc_t w_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(w_base), 0, w_bytes, 0x00027000);
+      const __amdgpu_buffer_rsrc_t a_rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a_base), 0, a_bytes, 0x00027000);
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rows, (lds_ptr_t)(stage + L::kABytes + 256 * j), 4, w_word[j & 3],
+                                                 min((uint32_t)lo + j * w_pitch, w_bytes), 0, 0);
+#pragma unroll
+      for (int j = 0; j < 4 * R; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rows, (lds_ptr_t)(stage + 256 * j), 4, a_word[j & 3],
+                                                 min((uint32_t)lo + j * a_pitch, a_bytes), 0, 0);
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < CHUNKS; ++j) {
       uint32_t off = w_off[j];
@@ -1044,7 +1078,7 @@ __global__ __launch_bounds__(64 << tree_rows_split<R>(), (R == 1 ? 4 : 2)) void 
 #pragma unroll
     for (int i = 0; i < kAReads; ++i) aq[i] = *reinterpret_cast<const u32x4_t*>(a_at[i] + stage_index * L::kLeafBytes);
 #pragma unroll
-    for (int c = 0; c < CHUNKS; ++c) wq[c] = *reinterpret_cast<const u32x4_t*>(w_at[c] + stage_index * L::kLeafBytes);
+    for (int c = 0; c < kUsed; ++c) wq[c] = *reinterpret_cast<const u32x4_t*>(w_at[c] + stage_index * L::kLeafBytes);
   };
   auto widen = [](const u32x4_t& v, int e) __attribute__((always_inline)) {
     return __uint_as_float((e & 1) ? (v[e >> 1] & 0xffff0000u) : (v[e >> 1] << 16));
@@ -1066,9 +1100,10 @@ __global__ __launch_bounds__(64 << tree_rows_split<R>(), (R == 1 ? 4 : 2)) void 
 #pragma unroll
       for (int set = 0; set < kSets; ++set) {
         const int c = kSets * i2 + set;
-        if (c >= CHUNKS) continue;
+        if (c >= kUsed) continue;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
+          if (8 * c + e >= len) continue;
           const float b = widen(wq[c], e);
           // the broadcast block is an immediate: block set * R + r holds row group r of this k
           if constexpr (R == 1) {
@@ -1167,12 +1202,12 @@ __global__ __launch_bounds__(64 << tree_rows_split<R>(), (R == 1 ? 4 : 2)) void 
   }
 }
 
-template <int R, int CHUNKS, int SLOTS>
+template <int R, int CHUNKS, int SLOTS, int LEN = 8 * CHUNKS>
 static hipError_t launch_rows_kernel(const MatView& A, const MatView& B, bf16_bits* out, int64_t ldc, int M, int N, int K,
                                      int depth, hipStream_t stream) {
   using L = TreeRowsLds<R, CHUNKS>;
   static PerDeviceOnce once;
-  auto kernel = det_gemm_tree_rows_kernel<R, CHUNKS, SLOTS>;
+  auto kernel = det_gemm_tree_rows_kernel<R, CHUNKS, SLOTS, LEN>;
   hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), L::kBytes, once);
   if (err != hipSuccess) return err;
   const int row_groups = (M + 16 * R - 1) / (16 * R);
@@ -1188,6 +1223,12 @@ template <int R>
 static hipError_t launch_rows(const MatView& A, const MatView& B, bf16_bits* out, int64_t ldc, int M, int N, int K,
                               int depth, hipStream_t stream) {
   constexpr int kFew = 7 - tree_rows_split<R>() - 2, kMany = 10 - tree_rows_split<R>() - 2;
+  if ((K >> depth) == 20)
+    return depth <= 7 ? launch_rows_kernel<R, 4, kFew, 20>(A, B, out, ldc, M, N, K, depth, stream)
+                      : launch_rows_kernel<R, 4, kMany, 20>(A, B, out, ldc, M, N, K, depth, stream);
+  if ((K >> depth) == 28)
+    return depth <= 7 ? launch_rows_kernel<R, 4, kFew, 28>(A, B, out, ldc, M, N, K, depth, stream)
+                      : launch_rows_kernel<R, 4, kMany, 28>(A, B, out, ldc, M, N, K, depth, stream);
   if ((K >> depth) == 24)
     return depth <= 7 ? launch_rows_kernel<R, 3, kFew>(A, B, out, ldc, M, N, K, depth, stream)
                       : launch_rows_kernel<R, 3, kMany>(A, B, out, ldc, M, N, K, depth, stream);
@@ -1285,7 +1326,13 @@ hipError_t det_gemm_tree_launch(const MatView& A, const MatView& B, void* C, int
   // conversion pass. Up to 8 rows they are ahead of the vector-ALU kernel below as well, with weights that come from HBM
   // (gate_up at one token 57 against 84 us, the lm_head 287 against 403 us, down 33 against 75 us).
   if (config == RLK_TREE_CFG_AUTO && nodes_ok) config = RLK_TREE_CFG_NODES;
-  if (config == RLK_TREE_CFG_NODES) {
+  // Leaves of 20 and 28: those kernels as well, but not the one that splits a node over the blocks of its instruction.
+  auto words = [&](const MatView& v) {
+    return v.k_stride == 1 && v.row_stride % 8 == 0 && v.row_stride >= 0 && v.row_stride < (1 << 23) && (reinterpret_cast<uintptr_t>(v.ptr) & 15) == 0;
+  };
+  const bool rows_of_words = config == RLK_TREE_CFG_AUTO && uniform && depth > 4 && depth <= kTreeNodeMaxDepth &&
+                             ((K >> depth) == 20 || (K >> depth) == 28) && words(A) && words(B);
+  if (config == RLK_TREE_CFG_NODES || rows_of_words) {
     // Which of them. Workgroups of 16 x 64 / 32 x 64 outputs that the busiest CU runs one after the other (pairs of them
     // side by side), K = 4096: one 26 / 48 us, two 46 / 84, every further one 21 / 41. So 32 rows from two on where that
     // is at least 4 % less than 16 rows (o_proj at 256 rows 88 / 85 us, qkv at 509 263 / 246, but qkv at 384, five against
@@ -1295,7 +1342,7 @@ hipError_t det_gemm_tree_launch(const MatView& A, const MatView& B, void* C, int
     const int64_t cus = device_cu_count();
     const int64_t groups16 = (int64_t)((N + 63) / 64) * ((M + 15) / 16), groups32 = (int64_t)((N + 63) / 64) * ((M + 31) / 32);
     const int64_t turns16 = (groups16 + cus - 1) / cus, turns32 = (groups32 + cus - 1) / cus;
-    if (2 * groups16 <= cus && depth > kTreeNodeSplit + 2) return launch_nodes(A, B, out, ldc, M, N, K, depth, stream);
+    if (!rows_of_words && 2 * groups16 <= cus && depth > kTreeNodeSplit + 2) return launch_nodes(A, B, out, ldc, M, N, K, depth, stream);
     if (depth == 4 || (turns32 >= 2 && 48 * turns32 < 25 * turns16))
       return launch_rows<2>(A, B, out, ldc, M, N, K, depth, stream);
     return launch_rows<1>(A, B, out, ldc, M, N, K, depth, stream);

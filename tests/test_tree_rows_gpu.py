@@ -57,3 +57,28 @@ def test_rows_per_wave_keep_the_bits(oracle, shape, special):
         columns = torch.tensor(sorted({0, 15, 16, 63, 64, n // 2, n - 1} & set(range(n))), device="cuda")
         want = oracle.k_tree_gemm(inputs.bits(a.cpu()), inputs.bits(w[columns].cpu()))
         assert np.array_equal(inputs.bits(out[:, columns].contiguous().cpu()), want)
+
+
+# leaves of 20 and 28, five levels to ten; one row and column, edges of tiles, 16 and 32 rows per wave
+@pytest.mark.parametrize("shape", [(1, 1, 640), (2, 4096, 14336), (17, 130, 896), (33, 8200, 1792), (16, 9000, 5120), (300, 4100, 14336),
+                                   (70, 16390, 2560), (5, 70, 20480), (40, 16384, 28672)])  # fmt: skip
+@pytest.mark.parametrize("special", [False, True])
+def test_leaves_that_do_not_start_on_sixteen_bytes(oracle, shape, special):
+    test_rows_per_wave_keep_the_bits(oracle, shape, special)
+
+
+def test_operands_of_other_pitches_and_places(oracle):
+    """Rows inside longer ones and repeated rows, whose ends the loads must not pass; a place that is not aligned goes the other way."""
+    from rl_engine import _C
+
+    m, n, k = 21, 70, 1792
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    store = torch.randn(n * (k + 24) + 8, generator=gen, device="cuda", dtype=torch.bfloat16)
+    a = torch.randn(m, k, generator=gen, device="cuda", dtype=torch.bfloat16)
+    for first, pitch in ((0, k + 24), (0, k), (8, k), (0, 0), (3, k)):
+        w = store.as_strided((n, k), (pitch, 1), first)
+        for rows in (a, a[:1].expand(m, k)):
+            got, want = (torch.empty(m, n, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+            _C.gemm_tree_strided(rows, w.t(), got)
+            _C.gemm_tree_strided(rows, w.t(), want, 1)
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (first, pitch)
