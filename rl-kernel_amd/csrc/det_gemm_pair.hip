@@ -193,7 +193,14 @@ static double solo_pair_us(const GemmProblem& dx, const GemmProblem& dw, int bm,
   solo_shares(dx, dw, bm, solo_groups(dx, dw, bm), &longest);
   const double work_dx = tile_count(dx, 256, bm) * solo_tile_length(dx) * (bm == 256 ? 1.0 : bm == 192 ? 0.70 : 0.73);
   const double work_dw = tile_count(dw, 256, 256) * solo_tile_length(dw);
-  return (dw.K <= 640 ? kPairScaleFew : kPairScale) * (0.89 * longest + 0.455 * (work_dx + work_dw) / cus);
+  // One tile's K tiles, one after the other: what its loads take where few tiles share them. A long reduction against few tiles stays with
+  // the smaller ones for it (lm_head backwards, us, this / theirs: 353, 4096, 151936 2550 / 1980; 729, 2048, 50257 813 / 607; 978, 2048,
+  // 32768 486 / 431; 298, 4096, 18992 269 / 248).
+  const bool cached = (int64_t)dx.N * dx.K * 2 < ((int64_t)40 << 20);
+  const double k_tile_us = bm == 256 ? 1.15 : bm == 192 ? 0.97 : cached ? 0.70 : 0.85;
+  const double chain_dx = k_tile_us * dx.K / kTileK, chain_dw = 1.15 * dw.K / kTileK;
+  const double chain = chain_dx > chain_dw ? chain_dx : chain_dw, us = 0.89 * longest + 0.455 * (work_dx + work_dw) / cus;
+  return (dw.K <= 640 ? kPairScaleFew : kPairScale) * (chain > us ? chain : us);
 }
 static bool solo_pair_serves(const GemmProblem& dx, const GemmProblem& dw) {
   return solo_kmajor_fits(dx.W) && solo_kmajor_fits(dx.X) && solo_kmajor_fits(dw.W) && solo_kmajor_fits(dw.X);
