@@ -467,6 +467,106 @@ __global__ __launch_bounds__(S::kThreads) void linear_logp_streamgroup_kernel(Lo
   }
 }
 
+// The same with one wave per SIMD (det_gemm_solo.h), a workgroup per CU: a wave has two of the four tiles' slices, and the state goes
+// through LDS once, from the waves of tiles 0 and 1 to those of 2 and 3. The next GEMM tile's loads run under the folds.
+struct SoloStreamRows {
+  static __device__ __forceinline__ int64_t row(int r, int last, int) {
+    return min((r >> 6) * kLogpTileCols + SoloPlainRows<SoloShape>::feature(r & 63), last);
+  }
+  static __device__ __forceinline__ int features(const MatView& W) { return W.rows; }
+};
+template <int BM>
+struct LogpStreamsSolo {
+  using Layout = SoloLayout<false, false, TileShape<256, BM, 2, 2>>;
+  static constexpr int kStateBytes = 3 * (kLogpStreams / 4) * BM * 4;
+  static constexpr int kLds = Layout::kLds + (Layout::kRing ? kStateBytes : 0);  // (else in the spare part)
+  static_assert(kLds <= 160 * 1024, "a ring and the states");
+};
+template <bool LOGITS, int BM>
+__global__ __launch_bounds__(SoloShape::kThreads) void linear_logp_streamgroup_solo_kernel(LogpArgs a, float* __restrict__ spart) {
+  using L = LogpStreamsSolo<BM>;
+  using S = typename L::Layout::Shape;
+  constexpr int kGroups = kLogpStreams / 4;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_n = wave % S::WN, wave_m = wave / S::WN;
+  const int total = a.tiles_m * a.n_split * kGroups;
+  auto unit_at = [&](int i, int& split, int& sg, int& m0) __attribute__((always_inline)) {
+    const int id = xcd_compact_id(i, total), unit = id / a.tiles_m;
+    m0 = id % a.tiles_m * BM;
+    split = unit / kGroups;
+    sg = unit % kGroups;
+  };
+  auto tile_at = [&](int i, int& n0, int& m0) __attribute__((always_inline)) {
+    int split, sg;
+    unit_at(i, split, sg, m0);
+    n0 = min(split * kLogpSplitCols + sg * 64, a.V - 1);  // (columns past the vocabulary are masked)
+  };
+  auto done = [&](int i, SoloAccOf<S>& acc, char* spare) __attribute__((always_inline)) -> bool {
+    int split, sg, m0;
+    unit_at(i, split, sg, m0);
+    const int lane = solo_lane(), grp = lane >> 4;
+    const int tok_local = wave_m * (BM / 2) + (lane & 15);
+    float* const sm = reinterpret_cast<float*>(L::Layout::kRing ? lds + L::Layout::kLds : spare);
+    float *const ss = sm + kGroups * BM, *const sz = ss + kGroups * BM;
+    const int span = split * kLogpSplitCols + wave_n * 2 * kLogpTileCols + sg * 64;  // of the wave's first tile
+    const int64_t plane = (int64_t)a.n_split * kLogpStreams * a.T;
+    const int64_t at = ((int64_t)split * kLogpStreams + sg * 4 + grp) * a.T + m0 + tok_local;
+#pragma unroll 1
+    for (int turn = 0; turn < 2; ++turn) {
+      if (wave_n == turn) {
+#pragma unroll
+        for (int jm = 0; jm < S::TM; ++jm) {
+          const int slot = grp * BM + tok_local + jm * 16, m = m0 + tok_local + jm * 16;
+          const int tgt = logp_target(a, m);
+          const float inv_t = logp_inverse_temperature(a, m);
+          float run_m = kNegInf, run_s = 0.f, run_zt = 0.f;
+          if (turn == 1) {
+            run_m = sm[slot];
+            run_s = ss[slot];
+            run_zt = sz[slot];
+          }
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int span0 = span + h * kLogpTileCols, col0 = span0 + grp * 16;
+            __builtin_amdgcn_sched_barrier(0);
+            float y[16];
+#pragma unroll
+            for (int c = 0; c < 16; ++c) y[c] = solo_result(acc[4 * h + (c >> 2)][jm][c & 3]);
+            if (span0 + 64 > a.vocab_limit) {  // uniform: the last columns
+#pragma unroll
+              for (int c = 0; c < 16; ++c) y[c] = col0 + c < a.vocab_limit ? y[c] : kNegInf;
+            }
+            if constexpr (LOGITS) {
+              float* row = a.logits + (int64_t)(m < a.T ? m : 0) * a.logits_ld;
+              if (span0 + 64 <= a.V) store_logit_span(row, span0, grp, m < a.T, y);
+              else if (m < a.T) store_logit_run(row, col0, a.V, y);
+            }
+#pragma unroll
+            for (int c = 0; c < 16; ++c) y[c] = y[c] * inv_t;  // (by one without a temperature, see logp_fold_tile)
+            logp_fold_run(y, tgt - col0, run_m, run_s, run_zt);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (turn == 0) {
+            sm[slot] = run_m;
+            ss[slot] = run_s;
+            sz[slot] = run_zt;
+          } else if (m < a.T) {
+            spart[at + jm * 16] = run_m;
+            spart[plane + at + jm * 16] = run_s;
+            spart[2 * plane + at + jm * 16] = run_zt;
+          }
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+      wg_barrier();
+    }
+    return LOGITS && span + kLogpTileCols + 64 <= a.V && m0 + BM <= a.T;
+  };
+  constexpr int kStores = LOGITS ? (8 * S::TM < 55 ? 8 * S::TM : 55) : 0;
+  solo_tiles<SoloStreamRows, kStores, true, typename L::Layout>(a.W, a.H, a.D, blockIdx.x, gridDim.x, total, lds, tile_at, done);
+}
+
 // Per-(split, stream) states [3][n_split * 16][T] -> per-split partials [3][n_split][T], streams
 // ascending: the arithmetic of the stream merge at the end of linear_logp_partial_kernel.
 __global__ __launch_bounds__(256) void linear_logp_stream_merge_kernel(const float* __restrict__ spart,
@@ -662,7 +762,8 @@ static bool logp_solo_pays(const LogpArgs& a) {
   if (!spans || a.bias != nullptr || !solo_offsets_fit(a.W) || !solo_offsets_fit(a.H)) return false;
   const int cus = device_cu_count();
   const int64_t units = (int64_t)((a.T + 127) / SoloShape::BM) * a.n_split;
-  return solo_tiles_pay(units, cus) || (a.logits != nullptr && units >= cus);
+  if (units < cus) return 10 * units >= 7 * cus;  // (160 units, V = 32768, D = 2048 at 1356 tokens with logits, 206 / 213; 190, V = 37984 at 1193, 346 / 333)
+  return solo_tiles_pay(units, cus) || a.logits != nullptr;
 }
 
 // 256-token tiles; a last one with few tokens runs as a tile of its size. With the groups above, us: V = 151936, D = 4096 at
@@ -714,6 +815,26 @@ static int balanced_tail_splits(int T, int n_split, int cus) {
 // 256 tokens and V = 151936, 596 workgroups are 2.33 rounds of 256; 512 of them plus 168
 // half-height ones are two rounds and a short one (350 -> 290 us). Same bits: the tile height
 // is not part of the contract.
+template <int BM>
+static hipError_t launch_streams_solo_tile(LogpArgs a, float* spart, hipStream_t stream) {
+  auto kernel = a.logits != nullptr ? linear_logp_streamgroup_solo_kernel<true, BM> : linear_logp_streamgroup_solo_kernel<false, BM>;
+  static PerDeviceOnce once[2];
+  hipError_t err = allow_dynamic_lds(reinterpret_cast<const void*>(kernel), LogpStreamsSolo<BM>::kLds, once[a.logits != nullptr]);
+  if (err != hipSuccess) return err;
+  a.tiles_m = (a.T + BM - 1) / BM;
+  const int64_t tiles = (int64_t)a.tiles_m * a.n_split * (kLogpStreams / 4);
+  const int cus = device_cu_count();
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles < cus ? tiles : cus)), dim3(SoloShape::kThreads), LogpStreamsSolo<BM>::kLds, stream, a,
+                     spart);
+  return hipGetLastError();
+}
+
+static hipError_t launch_stream_merge(const LogpArgs& a, const float* spart, hipStream_t stream) {
+  const int threads = a.T * a.n_split;
+  hipLaunchKernelGGL(linear_logp_stream_merge_kernel, dim3((threads + 255) / 256), dim3(256), 0, stream, spart, a.part, a.T, a.n_split);
+  return hipGetLastError();
+}
+
 template <class S>
 static hipError_t launch_streamgroup(LogpArgs a, bool balance, hipStream_t stream) {
   float* spart = a.part + (size_t)3 * a.n_split * a.T;  // behind the per-split partials
@@ -725,10 +846,65 @@ static hipError_t launch_streamgroup(LogpArgs a, bool balance, hipStream_t strea
     err = launch_streamgroup_range<LogpShape128>(a, spart, main_splits, a.n_split - main_splits, stream);
     if (err != hipSuccess) return err;
   }
-  const int threads = a.T * a.n_split;
-  hipLaunchKernelGGL(linear_logp_stream_merge_kernel, dim3((threads + 255) / 256), dim3(256), 0, stream, spart,
-                     a.part, a.T, a.n_split);
-  return hipGetLastError();
+  return launch_stream_merge(a, spart, stream);
+}
+
+// Whether the one-wave-per-SIMD form takes the operands.
+static bool streams_solo_fits(const LogpArgs& a) {
+  const bool spans = a.logits == nullptr || ((a.logits_ld & 3) == 0 && (reinterpret_cast<uintptr_t>(a.logits) & 15) == 0);
+  return spans && a.bias == nullptr && solo_offsets_fit(a.W, 3 * kLogpTileCols + 64) && solo_offsets_fit(a.H);
+}
+static hipError_t launch_streams_solo(const LogpArgs& a, int bm, hipStream_t stream) {
+  float* spart = a.part + (size_t)3 * a.n_split * a.T;
+  const hipError_t err = bm == 256   ? launch_streams_solo_tile<256>(a, spart, stream)
+                         : bm == 192 ? launch_streams_solo_tile<192>(a, spart, stream)
+                                     : launch_streams_solo_tile<128>(a, spart, stream);
+  return err == hipSuccess ? launch_stream_merge(a, spart, stream) : err;
+}
+
+// What the eight-wave stream groups take: rounds of workgroups x tokens per tile / relative throughput, of the tile for T tokens.
+static double streams_cost(int T, int n_split, int bm, double quality, double partial_floor = 0.9) {
+  return rounds_of_workgroups((int64_t)((T + bm - 1) / bm) * n_split * (kLogpStreams / 4), device_cu_count(), partial_floor) * bm / quality;
+}
+struct StreamsChoice {
+  int config;
+  double cost;
+};
+static StreamsChoice best_streams(int T, int n_split) {
+  // 128 / 256 / 192 tokens, us: V = 151936, D = 4096 at 300 tokens 482 / 523 / 432, 540: 779 / 737 / 608, 700: 914 / 746 / 811; V = 37984
+  // at 300: 137 / 199 / 161, 450: 193 / 203 / 166, 800: 307 / 303 / 256; V = 32768, D = 2048 at 300: 84 / 74 / 62, 700: 122 / 128 / 109.
+  const int tail = balanced_tail_splits(T, n_split, device_cu_count());
+  const double c256 = tail ? streams_cost(T, n_split - tail, 256, 1.0) + streams_cost(T, tail, 128, 0.76) : streams_cost(T, n_split, 256, 1.0);
+  const double c192 = streams_cost(T, n_split, 192, 0.945), c128 = streams_cost(T, n_split, 128, 0.76);
+  if (T <= 128) return {RLK_LOGP_CFG_128_STREAMS, c128};
+  if (T <= 256) return {RLK_LOGP_CFG_256_STREAMS, c256};
+  if (c192 < c256 && c192 < c128) return {RLK_LOGP_CFG_192_STREAMS, c192};
+  return c128 < c256 ? StreamsChoice{RLK_LOGP_CFG_128_STREAMS, c128} : StreamsChoice{RLK_LOGP_CFG_256_STREAMS, c256};
+}
+
+// The tokens of a tile of the one-wave-per-SIMD form, 0 for the eight-wave one. 256 tokens with stored logits do not fit its registers. Costs
+// fitted to 64 shapes of six heads and 100 to 1024 tokens, on the eight-wave form's scale. It runs where it has the same tile in no more
+// rounds (0.63 and 0.82 of the cost, 2 to 8 % of the time) or a better one; what lies above is faster on one machine and slower on
+// another (no logits, 203 tokens, V = 151936, D = 4096: 344 / 336 and 325 / 341; 226, 37984, 4096: 109 / 101 and 109 / 116; logits, 484, 151936, 4096
+// 589 / 621). Eight waves -> this, us (tokens, V, D): 168, 18992, 4096 85 -> 52; 237, 32768, 2048 59 -> 42; 121, 50257, 2048 55 -> 46; 266, 37984, 4096
+// 138 -> 122; 595, 131072, 2048 394 -> 348; 891, 151936, 4096 1013 -> 964; with stored logits 127, 32768, 2048 54 -> 42; 548, 151936, 4096 678 -> 640;
+// 753, 131072, 2048 502 -> 451; it stays with eight at 698, 37984, 4096 (230 / 248) and 995, 32768, 2048 (154 / 160).
+static int pick_streams_solo(const LogpArgs& a) {
+  // One token tile of a weight that HBM alone sets the pace of: read past the caches (V = 151936, D = 4096 at 76 / 99 tokens 253 / 257, 258 /
+  // 260; V = 131072, D = 2048 at 83 tokens 147 / 145).
+  if (a.T <= 128 && 2 * (int64_t)a.V * a.D >= ((int64_t)1 << 30)) return 0;
+  constexpr double kPartial = 0.965;
+  const double eight = best_streams(a.T, a.n_split).cost;
+  if (a.logits != nullptr) {
+    const double c128 = streams_cost(a.T, a.n_split, 128, 1.012, kPartial), c192 = streams_cost(a.T, a.n_split, 192, 1.157, kPartial);
+    const double best = c192 < c128 ? c192 : c128;
+    return best > 0.83 * eight ? 0 : c192 < c128 ? 192 : 128;
+  }
+  const double c128 = streams_cost(a.T, a.n_split, 128, 1.437, kPartial), c192 = streams_cost(a.T, a.n_split, 192, 1.574, kPartial);
+  const double c256 = streams_cost(a.T, a.n_split, 256, 1.585, kPartial);
+  const int tokens = c256 <= c192 && c256 <= c128 ? 256 : c192 < c128 ? 192 : 128;
+  const double best = tokens == 256 ? c256 : tokens == 192 ? c192 : c128;
+  return best > 0.64 * eight ? 0 : tokens;
 }
 
 int pick_linear_logp_config(int T, int V) {
@@ -736,22 +912,8 @@ int pick_linear_logp_config(int T, int V) {
   // loop) is the fastest from decode sizes up to 64 tokens, the 256-token tile from 1024 tokens on
   // even where it leaves the last round of workgroups part empty.
   if (T <= 64) return RLK_LOGP_CFG_64_STREAMS;
-  if (T <= 128) return RLK_LOGP_CFG_128_STREAMS;
-  if (T <= 256) return RLK_LOGP_CFG_256_STREAMS;
   if (T > kStreamGroupMaxTokens) return RLK_LOGP_CFG_256;
-  // Between them by rounds of workgroups x tokens per tile / relative throughput. 128 / 256 / 192 tokens, us: V = 151936, D =
-  // 4096 at 300 tokens 482 / 523 / 432, 540: 779 / 737 / 608, 700: 914 / 746 / 811; V = 37984 at 300: 137 / 199 / 161, 450: 193
-  // / 203 / 166, 800: 307 / 303 / 256; V = 32768, D = 2048 at 300: 84 / 74 / 62, 700: 122 / 128 / 109.
-  const int cus = device_cu_count();
-  const int n_split = linear_logp_split_count(V);
-  auto cost = [&](int splits, int bm, double quality) {
-    return rounds_of_workgroups((int64_t)((T + bm - 1) / bm) * splits * (kLogpStreams / 4), cus) * bm / quality;
-  };
-  const int tail = balanced_tail_splits(T, n_split, cus);
-  const double c256 = tail ? cost(n_split - tail, 256, 1.0) + cost(tail, 128, 0.76) : cost(n_split, 256, 1.0);
-  const double c192 = cost(n_split, 192, 0.945), c128 = cost(n_split, 128, 0.76);
-  if (c192 < c256 && c192 < c128) return RLK_LOGP_CFG_192_STREAMS;
-  return c128 < c256 ? RLK_LOGP_CFG_128_STREAMS : RLK_LOGP_CFG_256_STREAMS;
+  return best_streams(T, linear_logp_split_count(V)).config;
 }
 
 hipError_t linear_logp_launch(const MatView& H, const MatView& W, const int64_t* target, const float* bias,
@@ -792,7 +954,11 @@ hipError_t linear_logp_launch(const MatView& H, const MatView& W, const int64_t*
   }
   if (!vec && config == RLK_LOGP_CFG_256) config = RLK_LOGP_CFG_128;  // which has the element-wise loader
   hipError_t err;
-  switch (config) {
+  const bool streams = config == RLK_LOGP_CFG_128_STREAMS || config == RLK_LOGP_CFG_192_STREAMS || config == RLK_LOGP_CFG_256_STREAMS;
+  const int solo_tokens = requested == RLK_LOGP_CFG_AUTO && streams && streams_solo_fits(a) ? pick_streams_solo(a) : 0;
+  if (solo_tokens != 0) {
+    err = launch_streams_solo(a, solo_tokens, stream);
+  } else switch (config) {
     case RLK_LOGP_CFG_64_STREAMS:
       err = launch_streamgroup<LogpShape64>(a, false, stream);
       break;

@@ -228,3 +228,32 @@ def test_gradients_of_the_logp_at_a_ragged_vocabulary(tokens, vocab):
     weight = _C.fused_linear_logp_bwd(h, w, ids, lse, grad, None, need_grad_hidden=False)
     assert torch.equal(both[0].view(torch.int16), hidden[0].view(torch.int16))
     assert torch.equal(both[1].view(torch.int16), weight[1].view(torch.int16))
+
+
+# (tokens, vocabulary, hidden): one more token than 64, tiles of 128, 192 and 256 tokens at their edges, a vocabulary that ends inside a
+# split's first slice, inside its second tile, on a tile; more tiles than compute units
+STREAM_SHAPES = [(65, 1030, 64), (128, 2304, 192), (129, 2100, 128), (192, 50257, 64), (193, 9000, 256), (257, 8192, 64), (300, 18992, 128),
+                 (640, 37984, 64), (1000, 20001, 128), (1024, 33000, 64)]  # fmt: skip
+
+
+@pytest.mark.parametrize("shape", STREAM_SHAPES)
+@pytest.mark.parametrize("temperature", [False, True])
+@pytest.mark.parametrize("padded", [0, 7])  # columns of the vocabulary that are not real
+def test_stream_groups_of_the_logp(shape, temperature, padded):
+    """Up to 1024 tokens: the bits of the eight-wave kernel that keeps a split to one workgroup, with and without the logits."""
+    from rl_engine import _C
+
+    t, v, d = shape
+    gen = torch.Generator(device=DEV).manual_seed(t + v)
+    h = torch.randn((t, d), generator=gen, device=DEV, dtype=torch.bfloat16)
+    w = torch.randn((v, d), generator=gen, device=DEV, dtype=torch.bfloat16).mul_(0.1)
+    ids = torch.randint(0, v - padded, (t,), generator=gen, device=DEV)
+    ids[:2] = torch.tensor([0, v - padded - 1], device=DEV)
+    temp = torch.rand(t, generator=gen, device=DEV) + 0.5 if temperature else None
+    want = _C.fused_linear_logp(h, w, ids, None, temp, True, v - padded, config=1)  # 256 tokens, a split to a workgroup
+    plain = _C.fused_linear_logp(h, w, ids, None, temp, False, v - padded)
+    logits = torch.empty(t, _C.linear_logp_logits_row_stride(v), device=DEV)
+    kept = _C.fused_linear_logp_into(h, w, ids, None, temp, v - padded, logits)
+    for got in (plain, kept):
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert torch.equal(logits[:, :v], want[2])
