@@ -392,7 +392,7 @@ def main() -> int:
     achieved = flops_gu / ms_gu * 1e-9
     traffic = _measured_traffic()
     roofline = {
-        "kernel": "det_gemm_kernel<256x256 tile, 8 waves> on gate_up [4096x4096]x[24576x4096]^T",
+        "kernel": "det_gemm_solo_kernel<256x256 tile, 4 waves> on gate_up [4096x4096]x[24576x4096]^T",
         "bound": "mfma",
         "achieved": round(achieved, 1),
         "peak": PEAK_BF16_TFLOPS,
