@@ -494,7 +494,7 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
       case RLK_GEMM_CFG_256x256:
         return launch_kmajor<Shape256x256>(W, X, C, ldc, M, N, K, loop, out_f32, stream);
       case RLK_GEMM_CFG_256x192:
-        if (four_waves && w_kmajor && !out_f32 && solo_kmajor_fits(W) && solo_kmajor_fits(X))
+        if (four_waves && w_kmajor && !x_kmajor && !out_f32 && solo_kmajor_fits(W) && solo_kmajor_fits(X))
           return launch_solo<SoloLayout<true, false, TileShape<256, 192, 2, 2>>>(W, X, C, ldc, M, N, K, stream);
         if (!x_kmajor) return launch_kmajor<Shape256x192>(W, X, C, ldc, M, N, K, loop, out_f32, stream);
         break;

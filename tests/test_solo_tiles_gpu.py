@@ -134,6 +134,26 @@ def test_smaller_shapes_on_four_waves(shape, name):
             assert torch.equal(got[:, :n].contiguous().view(torch.int16), want.view(torch.int16)), k
 
 
+# K-major tokens, which the four-wave forms of these shapes do not take: whole K tiles (read as rows of 64 values they would
+# be there) and a ragged reduction
+@pytest.mark.parametrize("shape", [(264, 520, 64), (520, 392, 200), (256, 384, 256)])
+@pytest.mark.parametrize("w_kmajor", [False, True])
+@pytest.mark.parametrize("name", ["256x192", "256x128", "192x256", "192x192", "192x128"])
+def test_four_waves_asked_for_with_kmajor_tokens_run_the_plain_shape(shape, w_kmajor, name):
+    from rl_engine import _C, _lib
+
+    m, n, k = shape
+    x, w = _operands(shape, m + n + k)
+    want = torch.empty((m, n), device=DEV, dtype=torch.bfloat16)
+    _C.gemm_strided(x, w.t(), want, config=_lib.GEMM_CONFIGS["64x64"])
+    xt = x.t().contiguous().t()
+    b = w.t().contiguous() if w_kmajor else w.t()
+    for config in (_lib.GEMM_CONFIGS[name], _lib.GEMM_CONFIGS[name] | _lib.FOUR_WAVES):
+        got = torch.full((m, n), 7.0, device=DEV, dtype=torch.bfloat16)
+        _C.gemm_strided(xt, b, got, config=config)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), config
+
+
 # (tokens, outputs, K): one K tile and less, a few values more than whole K tiles, odd ones, edges of tiles of either side, more
 # tiles than CUs
 KMAJOR_SHAPES = [(8, 8, 8), (256, 256, 24), (264, 520, 64), (248, 776, 72), (1000, 264, 200), (512, 512, 2056), (4360, 4360, 136)]
