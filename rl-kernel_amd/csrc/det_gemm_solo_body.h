@@ -57,18 +57,29 @@ __device__ __forceinline__ void solo_product(const SoloProblem& p, int first, in
       }
       return m_wave + kWaveM <= p.M;
     }
+    const int alignment = solo_row_alignment(p.C, p.ldc);
 #pragma unroll
     for (int jm = 0; jm < S::TM; ++jm) {
       const int m = m_lane + jm * 16;
       if (m >= p.M) continue;
       bf16_bits* const row = p.C + (int64_t)m * p.ldc;
+      auto run = [&](auto tiles, int jn, int n) __attribute__((always_inline)) {  // a lane's consecutive features: four of each MFMA tile
+        constexpr int kTiles = decltype(tiles)::value;
+        uint32_t packed[2 * kTiles];
 #pragma unroll
-      for (int jn = 0; jn < S::TN; ++jn) {
-        const int run = jn / 4 * 4 + 4 <= S::TN ? 16 : 8;  // consecutive features of a lane
-        const int n = n_wave + (Layout::kW ? jn * 16 + grp * 4 : jn / 4 * 64 + grp * run + jn % 4 * 4);
+        for (int t = 0; t < kTiles; ++t) {
+          packed[2 * t] = pack_bf16x2(acc[jn + t][jm][0], acc[jn + t][jm][1]);
+          packed[2 * t + 1] = pack_bf16x2(acc[jn + t][jm][2], acc[jn + t][jm][3]);
+        }
+        solo_store_run<4 * kTiles>(row + n, p.N - n, alignment, packed);
+      };
+      if constexpr (Layout::kW) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (n + q < p.N) row[n + q] = to_bf16_bits(acc[jn][jm][q]);
+        for (int jn = 0; jn < S::TN; ++jn) run(IntTag<1>{}, jn, n_wave + jn * 16 + grp * 4);
+      } else {
+#pragma unroll
+        for (int h = 0; h < S::TN / 4; ++h) run(IntTag<4>{}, 4 * h, n_wave + h * 64 + grp * 16);
+        if constexpr (S::TN % 4 != 0) run(IntTag<2>{}, S::TN - 2, n_wave + S::TN / 4 * 64 + grp * 8);
       }
     }
     return false;

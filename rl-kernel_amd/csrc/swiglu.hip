@@ -255,6 +255,17 @@ __device__ __forceinline__ void store_gated_span(bf16_bits* row, int grp, bool l
   }
 }
 
+template <int KT>
+__device__ __forceinline__ void store_gated_run(bf16_bits* to, int inside, int alignment, const f32x4_t (&y)[KT]) {
+  uint32_t packed[2 * KT];
+#pragma unroll
+  for (int jn = 0; jn < KT; ++jn) {
+    packed[2 * jn] = pack_bf16x2(y[jn][0], y[jn][1]);
+    packed[2 * jn + 1] = pack_bf16x2(y[jn][2], y[jn][3]);
+  }
+  solo_store_run<4 * KT>(to, inside, alignment, packed);
+}
+
 template <class Layout, bool TRAINING>
 __global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_swiglu_solo_kernel(MatView W, MatView X,
                                                                                    bf16_bits* __restrict__ Y, int64_t ldy,
@@ -277,9 +288,7 @@ __global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_swiglu_solo_kern
     const int f_wave = f0 + wave % S::WN * (16 * kTiles), m_wave = m0 + wave / S::WN * (16 * S::TM);
     const int m_lane = m_wave + (lane & 15);
     const bool whole = f_wave + 16 * kTiles <= I && (reinterpret_cast<uintptr_t>(Y) & 15) == 0 && (ldy & 7) == 0;
-#pragma unroll
-    for (int jm = 0; jm < S::TM; ++jm) {
-      f32x4_t y[kTiles], g[kTiles], u[kTiles];
+    auto activate = [&](int jm, f32x4_t (&y)[kTiles], f32x4_t (&g)[kTiles], f32x4_t (&u)[kTiles]) __attribute__((always_inline)) {
 #pragma unroll
       for (int jn = 0; jn < kTiles; ++jn)
 #pragma unroll
@@ -288,28 +297,36 @@ __global__ __launch_bounds__(SoloShape::kThreads) void det_gemm_swiglu_solo_kern
           u[jn][q] = round_through_bf16(acc[jn + kTiles][jm][q]);
           y[jn][q] = swiglu_f32(g[jn][q], u[jn][q]);
         }
-      const int m = m_lane + jm * 16;
-      const int64_t at = (int64_t)m * ldy;
-      if (whole) {
-        store_gated_span<kTiles>(Y + at + f_wave, grp, m < M, y);
-        if constexpr (TRAINING) {
-          store_gated_span<kTiles>(training.gate + at + f_wave, grp, m < M, g);
-          store_gated_span<kTiles>(training.up + at + f_wave, grp, m < M, u);
-        }
-      } else if (m < M) {
-        const int f = f_wave + grp * (4 * kTiles);
+    };
+    if (whole) {
 #pragma unroll
-        for (int e = 0; e < 4 * kTiles; ++e)
-          if (f + e < I) {
-            Y[at + f + e] = to_bf16_bits(y[e >> 2][e & 3]);
-            if constexpr (TRAINING) {
-              training.gate[at + f + e] = to_bf16_bits(g[e >> 2][e & 3]);
-              training.up[at + f + e] = to_bf16_bits(u[e >> 2][e & 3]);
-            }
-          }
+      for (int jm = 0; jm < S::TM; ++jm) {
+        f32x4_t y[kTiles], g[kTiles], u[kTiles];
+        activate(jm, y, g, u);
+        const int m = m_lane + jm * 16;
+        const int64_t at = (int64_t)m * ldy + f_wave;
+        store_gated_span<kTiles>(Y + at, grp, m < M, y);
+        if constexpr (TRAINING) {
+          store_gated_span<kTiles>(training.gate + at, grp, m < M, g);
+          store_gated_span<kTiles>(training.up + at, grp, m < M, u);
+        }
+      }
+      return m_wave + 16 * S::TM <= M;
+    }
+#pragma unroll
+    for (int jm = 0; jm < S::TM; ++jm) {
+      f32x4_t y[kTiles], g[kTiles], u[kTiles];
+      activate(jm, y, g, u);
+      const int m = m_lane + jm * 16, f = f_wave + grp * (4 * kTiles);
+      if (m >= M) continue;
+      const int64_t at = (int64_t)m * ldy + f;
+      store_gated_run<kTiles>(Y + at, I - f, solo_row_alignment(Y, ldy), y);
+      if constexpr (TRAINING) {
+        store_gated_run<kTiles>(training.gate + at, I - f, solo_row_alignment(training.gate, ldy), g);
+        store_gated_run<kTiles>(training.up + at, I - f, solo_row_alignment(training.up, ldy), u);
       }
     }
-    return whole && m_wave + 16 * S::TM <= M;
+    return false;
   };
   // (the three pieces of twelve features may leave as two stores)
   constexpr int kStores = (kTiles > 2 ? 2 : 1) * S::TM * (TRAINING ? 3 : 1);

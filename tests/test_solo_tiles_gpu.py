@@ -134,6 +134,64 @@ def test_smaller_shapes_on_four_waves(shape, name):
             assert torch.equal(got[:, :n].contiguous().view(torch.int16), want.view(torch.int16)), k
 
 
+# rows of the result that start on 16, 8, 4 and 2 bytes, by their pitch and by where the first one starts; columns that end inside a
+# lane's run, on it and on a span of 64
+@pytest.mark.parametrize("outputs", [320, 328, 517, 382])
+@pytest.mark.parametrize("pitch,first", [(0, 0), (4, 4), (2, 8), (2, 2), (1, 0), (3, 1), (8, 1)])
+@pytest.mark.parametrize("name", ["256x256_solo", "192x256", "192x192", "192x128", "256x192 K-major"])
+def test_rows_of_every_alignment(outputs, pitch, first, name):
+    """The bits of the small tiles, nothing written before, between and behind the rows."""
+    from rl_engine import _C, _lib
+
+    m, n, k = 300, outputs, 128
+    x, w = _operands((m, n, k), outputs + pitch)
+    want = torch.empty((m, n), device=DEV, dtype=torch.bfloat16)
+    _C.gemm_strided(x, w.t(), want, config=_lib.GEMM_CONFIGS["64x64"])
+    ld = (n + 7) // 8 * 8 + pitch
+    flat = torch.full((first + m * ld + 8,), 7.0, device=DEV, dtype=torch.bfloat16)
+    got = flat.as_strided((m, n), (ld, 1), first)
+    shape, _, kmajor = name.partition(" ")
+    b = w.t()
+    if kmajor:
+        n8 = (n + 7) // 8 * 8
+        wt = torch.zeros((k, n8), device=DEV, dtype=torch.bfloat16)
+        wt[:, :n] = w.t()
+        if n8 != n:  # a K-major weight has whole eights of outputs
+            got = flat.as_strided((m, n8), (ld, 1), first)
+            b = wt
+            want = torch.cat([want, torch.zeros((m, n8 - n), device=DEV, dtype=torch.bfloat16)], 1)
+        else:
+            b = w.t().contiguous()
+    config = _lib.GEMM_CONFIGS[shape] | (_lib.FOUR_WAVES if "solo" not in shape else 0)
+    _C.gemm_strided(x, b, got, config=config)
+    assert torch.equal(got.contiguous().view(torch.int16), want.view(torch.int16))
+    got.fill_(7.0)
+    assert bool((flat == 7.0).all())
+
+
+# the same of the fused gate/up: whole tiles and ragged ones, rows on 8, 4 and 2 bytes
+@pytest.mark.parametrize("inter", [3068, 3070, 3071, 516, 514, 515])
+@pytest.mark.parametrize("tokens", [129, 411, 1029, 4100])
+def test_gated_rows_of_every_alignment(tokens, inter):
+    from rl_engine import _C, _lib
+
+    k = 64
+    gen = torch.Generator(device=DEV).manual_seed(tokens + inter)
+    x = torch.randn((tokens, k), generator=gen, device=DEV, dtype=torch.bfloat16)
+    w = torch.randn((2 * inter, k), generator=gen, device=DEV, dtype=torch.bfloat16).mul_(0.1)
+    gate_up = torch.empty((tokens, 2 * inter), device=DEV, dtype=torch.bfloat16)
+    _C.gemm_strided(x, w.t(), gate_up, config=5)  # 64 x 64
+    want = _C.swiglu_packed_forward(gate_up)
+    assert torch.equal(_C.det_gemm_swiglu(x, w).view(torch.int16), want.view(torch.int16))
+    got = [torch.full((tokens, inter), 7.0, device=DEV, dtype=torch.bfloat16) for _ in range(3)]
+    gate_w, up_w = w[:inter].contiguous(), w[inter:].contiguous()
+    assert 0 == _lib.load().rlk_det_gemm_swiglu_training_bf16(
+        x.data_ptr(), k, gate_w.data_ptr(), up_w.data_ptr(), k, *(t.data_ptr() for t in got), inter, tokens, inter, k,
+        torch.cuda.current_stream().cuda_stream)  # fmt: skip
+    for g, part in zip(got, (gate_up[:, :inter], gate_up[:, inter:], want)):
+        assert torch.equal(g.view(torch.int16), part.contiguous().view(torch.int16))
+
+
 # K-major tokens, which the four-wave forms of these shapes do not take: whole K tiles (read as rows of 64 values they would
 # be there) and a ragged reduction
 @pytest.mark.parametrize("shape", [(264, 520, 64), (520, 392, 200), (256, 384, 256)])
