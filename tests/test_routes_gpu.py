@@ -1,0 +1,49 @@
+"""Which kernels the automatic choices launch, by the names that a trace of the call shows: the rules at the sizes where they turn."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+def launched(call) -> list[str]:
+    """The kernels of ``call``, in order."""
+    call()  # the first call's allocations and attributes are not of interest
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU, torch.profiler.ProfilerActivity.CUDA]) as trace:
+        call()
+        torch.cuda.synchronize()
+    events = [e for e in trace.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+    names = [e.name for e in sorted(events, key=lambda e: e.time_range.start)]
+    assert names, "the trace holds no kernel"
+    return names
+
+
+def _rand(*shape):
+    return torch.randn(shape, device=DEV, dtype=torch.bfloat16)
+
+
+# one token tile: (tokens, vocabulary, hidden, stored logits, four waves); 76, 128, 132, 152, 260 and 512 tiles, a vocabulary of half a split
+@pytest.mark.parametrize(
+    "tokens,vocab,hidden,logits,four",
+    [(96, 18992, 64, False, True), (96, 18992, 64, True, True), (96, 32768, 64, False, True), (128, 33000, 64, True, False),
+     (128, 33000, 64, False, True), (96, 37984, 64, True, False), (96, 37984, 64, False, False), (65, 66000, 64, True, False),
+     (65, 66000, 64, False, True), (96, 131072, 64, True, True), (96, 131072, 64, False, True), (100, 512, 64, False, False),
+     (100, 500, 64, True, False), (100, 513, 64, True, True), (300, 512, 64, False, True)],
+)  # fmt: skip
+def test_stream_groups_of_one_token_tile(tokens, vocab, hidden, logits, four):
+    from rl_engine import _C
+
+    h, w = _rand(tokens, hidden), _rand(vocab, hidden)
+    ids = torch.zeros(tokens, dtype=torch.int64, device=DEV)
+    out = torch.empty(tokens, _C.linear_logp_logits_row_stride(vocab), device=DEV)
+    if logits:
+        names = launched(lambda: _C.fused_linear_logp_into(h, w, ids, None, None, vocab, out))
+    else:
+        names = launched(lambda: _C.fused_linear_logp(h, w, ids, None, None, False, vocab))
+    assert any("linear_logp_streamgroup_solo_kernel" in n for n in names) == four
+    assert any("linear_logp_streamgroup_kernel" in n for n in names) != four
