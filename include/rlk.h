@@ -212,7 +212,8 @@ int rlk_det_gemm_tree_bf16_config(const void* a, int64_t a_row_stride, int64_t a
  * "rlkernel.det_gemm.triton_tree_rocm.v1", rl_engine/backends/rocm/gemm/det_gemm.py:101-104). */
 const char* rlk_det_gemm_tree_contract_id(void);
 
-/* The configuration RLK_GEMM_CFG_AUTO resolves to for a shape (host only, no GPU call).
+/* The configuration RLK_GEMM_CFG_AUTO resolves to for a shape, native operands with rows of whole 16 bytes and bf16 results: the
+ * tiles, not the waves that they run on, which the launch adds (RLK_GEMM_CFG_256x256, RLK_GEMM_CFG_FOUR_WAVES). Host only, no GPU call.
  * Stands in for select_config, rl_engine/backends/rocm/gemm/mfma_gemm.py:76-92. */
 int rlk_det_gemm_pick_config(int M, int N, int K);
 

@@ -261,15 +261,18 @@ int device_cu_count() {
 // tokens, 1.8 -> 1.03 ms at 512, 1.65 -> 1.45 ms at 1024); their qualities are those of the direct-to-LDS loop. 256 x 192:
 // dX of 14336 inputs, 4096 outputs at 540 / 1300 tokens 106 / 169 -> 68 / 142 us, of 4096, 6144 at 2300 tokens 108 -> 95.
 //
-// The `four` column is that of the four-wave forms of the native shapes (det_gemm_solo.h, 0: none), which whole K tiles and bf16
-// results have. Waves of half a tile by half read every row of a K tile from LDS twice, where eight of a quarter by half read token
-// rows four times; those reads and what arrives are 1856 cycles of LDS a K tile beside 1536 of MFMAs in 192 x 256, 1344 with four
-// waves, 1536 / 1152 beside 1152 in 192 x 192. With them a round that fills part of the chip costs less, the more so behind others
-// (kPartialFirst, kPartialLast). 170 shapes of 14 layers, 300 to 7000 tokens, weights in turn: 0.957 of the time before on the 91 that
-// are not the deep tiles', 0.2 % above the best shape of each (worst 4 %). Before -> with them, us: 4096 outputs, K = 4096 at 1400 /
-// 2047 / 3000 tokens 53.9 / 62.8 / 79.1 -> 49.7 / 57.8 / 73.8, 6144 at 1024 / 2048 / 3072 56.9 / 83.6 / 124.8 -> 51.7 / 78.4 /
-// 117.9, K = 12288 at 2047 176 -> 164, 24576 outputs at 700 / 1024 129.9 / 167.4 -> 120.2 / 156.6. (256 x 128 and 128 x 128 on four
-// waves were never the best shape by more than the noise.)
+// The `four` column is the relative throughput of a shape's four-wave form (det_gemm_solo.h, 0: none), which native operands with
+// whole K tiles and bf16 results have. Waves of half a tile by half read every row of a K tile from LDS twice, where eight of a
+// quarter by half read token rows four times; those reads and what arrives are 1856 cycles of LDS a K tile beside 1536 of MFMAs in 192
+// x 256, 1344 with four waves, 1536 / 1152 beside 1152 in 192 x 192. With them a round that fills part of the chip costs less, the more
+// so behind others (kPartialFirst, kPartialLast). Shapes without such a form are weighed beside them at their `native` quality, 256 x
+// 128 in one round at a better one. 560 shapes of 33 to 16000 tokens, 128 to 24576 outputs, K = 64 to 14336, weights in turn: where 128 does
+// not divide K, which shuts out the deep tiles of few tokens, 0.983 of the eight waves' time, 0.6 % above the best shape of each, where
+// it does 0.935 and 1.2 %. Eight waves -> these, us: 4096 outputs, K = 4096 at 1400 / 2047 / 3000 tokens 53.9 / 62.8 / 79.1 -> 49.7 /
+// 57.8 / 73.8, 6144 at 1024 / 2048 / 3072 56.9 / 83.6 / 124.8 -> 51.7 / 78.4 / 117.9, K = 12288 at 2047 176 -> 164, 24576 outputs at 700 /
+// 1024 129.9 / 167.4 -> 120.2 / 156.6. What the small shapes and 256 x 128 are there for (the best without them / with): K = 2880, 2880
+// outputs at 65 / 200 tokens 31.9 / 32.9 -> 22.6 / 22.5, 5760 at 100 34.6 -> 23.1, K = 1600, 1536 outputs at 300 16.6 -> 11.2; K = 12288,
+// 8192 outputs at 1009 191 -> 169. (256 x 128 and 128 x 128 on four waves were never the best shape by more than the noise.)
 struct TileCandidate {
   int config, bn, bm;
   double native, ragged192, w_kmajor;
@@ -280,21 +283,27 @@ static const TileCandidate kTileCandidates[] = {
     {RLK_GEMM_CFG_256x256, 256, 256, 1.00, 0.00, 1.00, true, 1.00},  {RLK_GEMM_CFG_192x256, 192, 256, 0.89, 0.85, 0.00, false, 0.95},
     {RLK_GEMM_CFG_256x192, 256, 192, 0.87, 0.00, 0.87, false, 0.94}, {RLK_GEMM_CFG_192x192, 192, 192, 0.75, 0.68, 0.00, false, 0.93},
     {RLK_GEMM_CFG_256x128, 256, 128, 0.65, 0.00, 0.70, true, 0.00},  {RLK_GEMM_CFG_192x128, 192, 128, 0.56, 0.53, 0.00, false, 0.80},
-    {RLK_GEMM_CFG_256x64, 256, 64, 0.50, 0.00, 0.56, false, 0.00},   {RLK_GEMM_CFG_128x128, 128, 128, 0.65, 0.00, 0.62, false, 0.40},
-    {RLK_GEMM_CFG_128x64, 128, 64, 0.45, 0.00, 0.40, false, 0.25},   {RLK_GEMM_CFG_64x64, 64, 64, 0.42, 0.00, 0.25, false, 0.00},
+    {RLK_GEMM_CFG_256x64, 256, 64, 0.50, 0.00, 0.56, false, 0.00},   {RLK_GEMM_CFG_128x128, 128, 128, 0.65, 0.00, 0.62, false, 0.00},
+    {RLK_GEMM_CFG_128x64, 128, 64, 0.45, 0.00, 0.40, false, 0.00},   {RLK_GEMM_CFG_64x64, 64, 64, 0.42, 0.00, 0.25, false, 0.00},
 };
-constexpr double kPartialFirst = 0.82, kPartialLast = 0.6, kFourRagged192 = 0.92;
+constexpr double kPartialFirst = 0.82, kPartialLast = 0.6, kFourRagged192 = 0.92, kPartialEight = 0.9, kOneRound256x128 = 0.80;
 
-// The cheapest shape for native operands whose K tiles are whole, bf16 results: four waves where the shape has them.
+// The cheapest shape for operands that the four-wave forms take.
 static int pick_four_wave_shape(int M, int N) {
   const int cus = device_cu_count();
   int best = RLK_GEMM_CFG_256x256;
   double best_time = 1e300;
   for (const TileCandidate& c : kTileCandidates) {
-    if (c.four == 0.0) continue;
-    const double quality = c.four * (c.bn == 192 && N % 192 != 0 ? kFourRagged192 : 1.0);
     const int64_t tiles = tile_count(M, N, c.bm, c.bn);
-    const double t = rounds_of_workgroups(tiles, cus, tiles <= cus ? kPartialFirst : kPartialLast) * (double)(c.bn * c.bm) / quality;
+    const bool one_round = tiles <= cus;
+    double quality = c.four, partial = one_round ? kPartialFirst : kPartialLast;
+    if (c.four == 0.0) {
+      quality = one_round && c.config == RLK_GEMM_CFG_256x128 ? kOneRound256x128 : c.native;
+      partial = kPartialEight;
+    } else if (c.bn == 192 && N % 192 != 0) {
+      quality *= kFourRagged192;
+    }
+    const double t = rounds_of_workgroups(tiles, cus, partial) * (double)(c.bn * c.bm) / quality;
     if (t < best_time * 0.999) {
       best_time = t;
       best = c.config;
@@ -332,7 +341,7 @@ static const TileCandidate& best_tile_candidate(int M, int N, int K, bool w_kmaj
 
 static int pick_tile_candidate(int M, int N, int K, bool w_kmajor, bool x_kmajor) {
   double estimate;
-  return best_tile_candidate(M, N, K, w_kmajor, x_kmajor, 0.9, &estimate).config;
+  return best_tile_candidate(M, N, K, w_kmajor, x_kmajor, kPartialEight, &estimate).config;
 }
 
 double det_gemm_kmajor_us(int M, int N, int K, bool w_kmajor, bool x_kmajor, double partial_floor, int* tile_outputs) {

@@ -85,6 +85,20 @@ def test_the_pick_names_the_few_token_tile_that_runs(rlk_lib, m, n, k, name):
     assert rlk_lib.rlk_det_gemm_pick_config(m, n, k) == _lib.GEMM_CONFIGS[name]
 
 
+# A reduction that 64 divides and 128 does not has no deep tiles: small tiles where larger ones would leave most CUs without one, the
+# shapes with four waves where they fill the chip
+@pytest.mark.parametrize(
+    "m,n,k,name",
+    [(65, 2880, 2880, "64x64"), (65, 1536, 2880, "64x64"), (65, 5760, 2880, "64x64"), (100, 640, 1600, "64x64"), (300, 2880, 2880, "64x64"),
+     (47, 14400, 64, "64x64"), (129, 5760, 2880, "128x64"), (600, 2880, 2880, "128x64"), (441, 5000, 64, "128x128"),
+     (2047, 4096, 2880, "192x192"), (3000, 2880, 2880, "192x192"), (8192, 8192, 2880, "256x256"), (1009, 8192, 12288, "256x128")],
+)  # fmt: skip
+def test_the_pick_of_reductions_without_deep_tiles(rlk_lib, m, n, k, name):
+    from rl_engine import _lib
+
+    assert rlk_lib.rlk_det_gemm_pick_config(m, n, k) == _lib.GEMM_CONFIGS[name]
+
+
 # (tokens, hidden size, vocabulary): two launches where they are faster (whole token tiles and whole K tiles of a weight from
 # HBM), one launch in the tiles that are the faster ones, the rest behind whole tiles beside the weight gradient
 @pytest.mark.parametrize(
