@@ -351,7 +351,7 @@ double det_gemm_kmajor_us(int M, int N, int K, bool w_kmajor, bool x_kmajor, dou
   return (11.0 + 21.0 * K / 1024.0) * outputs / 65536.0;
 }
 
-int pick_det_gemm_config(int M, int N, int K, bool out_f32) {
+int pick_det_gemm_config(int M, int N, int K, bool four_waves) {
   const int cus = device_cu_count();
   // Decode (weights fitted while they rotate through 1.3 GB, i.e. come from HBM as in a model with
   // many layers, not from the 256 MB memory-side cache): up to 16 tokens the streaming kernel with
@@ -395,7 +395,7 @@ int pick_det_gemm_config(int M, int N, int K, bool out_f32) {
     if (tile_count(M, N, 160, 64) <= cus) return RLK_GEMM_CFG_64x160_DEEP;
     if (tile_count(M, N, 128, 128) <= cus) return RLK_GEMM_CFG_128x128_DEEP;
   }
-  return K % kTileK == 0 && !out_f32 ? pick_four_wave_shape(M, N) : pick_tile_candidate(M, N, K, false, false);
+  return four_waves ? pick_four_wave_shape(M, N) : pick_tile_candidate(M, N, K, false, false);
 }
 
 // A K-major view (element [row, k] at ptr[k * k_stride + row], rows contiguous: B[K,N] as the
@@ -441,6 +441,11 @@ static bool remainder_launch_pays(int M, int N, int K, int rest, bool fast_few_t
     return false;
   }
   return rest_us < 0.8 * round_us;
+}
+
+// Native operands (16-byte rows) that the four-wave forms take.
+static bool four_waves_take(const MatView& W, const MatView& X, int K, bool out_f32) {
+  return K % kTileK == 0 && !out_f32 && solo_offsets_fit(W) && solo_offsets_fit(X);
 }
 
 hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
@@ -528,10 +533,11 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     }
   }
   if (config == RLK_GEMM_CFG_AUTO) {
-    config = pick_det_gemm_config(M, N, K, out_f32);
-    four_waves = true;  // where the shape has them and the operands are theirs
+    const bool takes = vec && allow_pingpong && four_waves_take(W, X, K, out_f32);
+    config = pick_det_gemm_config(M, N, K, takes);
+    four_waves = takes;
     // the picked shape with one wave per SIMD (which a call can ask for, and which is 256 x 256 again for what it does not take)
-    if (config == RLK_GEMM_CFG_256x256 && solo_tiles_pay(tile_count(M, N, 256, 256), device_cu_count()))
+    if (config == RLK_GEMM_CFG_256x256 && four_waves && solo_tiles_pay(tile_count(M, N, 256, 256), device_cu_count()))
       config = RLK_GEMM_CFG_256x256_SOLO;
   }
   if (config == RLK_GEMM_CFG_STREAM16_DEEP || config == RLK_GEMM_CFG_STREAM16 || config == RLK_GEMM_CFG_STREAM64) {
@@ -540,7 +546,7 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     const int max_m = config == RLK_GEMM_CFG_STREAM64 ? 64 : 16;
     if (M <= max_m && vec && allow_pingpong && K % kTileK == 0)
       return det_gemm_stream_launch(W, X, C, ldc, M, N, K, out_f32, config == RLK_GEMM_CFG_STREAM16, stream);
-    config = M <= 16 ? RLK_GEMM_CFG_16x16 : M <= 64 ? RLK_GEMM_CFG_64x64 : pick_det_gemm_config(M, N, K, out_f32);
+    config = M <= 16 ? RLK_GEMM_CFG_16x16 : M <= 64 ? RLK_GEMM_CFG_64x64 : pick_det_gemm_config(M, N, K, false);
     if (config == RLK_GEMM_CFG_STREAM64) config = RLK_GEMM_CFG_64x64;
   }
   // Deep-stage variants need the fast layout and whole stages; otherwise the plain shape
@@ -575,11 +581,11 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
                                                                                        : RLK_GEMM_CFG_64x64;
   }
   if (config == RLK_GEMM_CFG_256x256_SOLO) {
-    if (vec && allow_pingpong && K % kTileK == 0 && !out_f32 && solo_offsets_fit(W) && solo_offsets_fit(X))
+    if (vec && allow_pingpong && four_waves_take(W, X, K, out_f32))
       return launch_solo<SoloLayout<false, false>>(W, X, C, ldc, M, N, K, stream);
     config = RLK_GEMM_CFG_256x256;
   }
-  if (four_waves && vec && allow_pingpong && K % kTileK == 0 && !out_f32 && solo_offsets_fit(W) && solo_offsets_fit(X)) {
+  if (four_waves && vec && allow_pingpong && four_waves_take(W, X, K, out_f32)) {
     switch (config) {  // (weights read past the caches are the eight waves')
       case RLK_GEMM_CFG_256x192:
         return launch_solo_shape<256, 192>(W, X, C, ldc, M, N, K, stream);

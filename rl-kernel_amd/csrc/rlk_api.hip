@@ -75,7 +75,7 @@ const char* rlk_version(void) { return "0.1.0"; }
 
 const char* rlk_last_error(void) { return g_last_error; }
 
-int rlk_det_gemm_pick_config(int M, int N, int K) { return pick_det_gemm_config(M, N, K); }
+int rlk_det_gemm_pick_config(int M, int N, int K) { return pick_det_gemm_config(M, N, K, K % 64 == 0); }
 
 int rlk_det_gemm_bf16(const void* a, int64_t a_row_stride, int64_t a_k_stride, const void* b,
                       int64_t b_k_stride, int64_t b_n_stride, void* c, int64_t ldc, int M, int N, int K,

@@ -83,7 +83,8 @@ inline bool streamed_weight(int64_t rows, int64_t k, int M, int bm) {
   return (M <= bm && bytes >= ((int64_t)96 << 20)) || (M == 2 * bm && bytes >= ((int64_t)128 << 20));
 }
 
-int pick_det_gemm_config(int M, int N, int K, bool out_f32 = false);
+// `four_waves`: the operands are ones that the four-wave forms of the shapes take.
+int pick_det_gemm_config(int M, int N, int K, bool four_waves);
 
 // W[N,K] is the operand whose rows are output features, X[M,K] the one whose
 // rows are tokens; C[m*ldc + n].

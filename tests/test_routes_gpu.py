@@ -47,3 +47,26 @@ def test_stream_groups_of_one_token_tile(tokens, vocab, hidden, logits, four):
         names = launched(lambda: _C.fused_linear_logp(h, w, ids, None, None, False, vocab))
     assert any("linear_logp_streamgroup_solo_kernel" in n for n in names) == four
     assert any("linear_logp_streamgroup_kernel" in n for n in names) != four
+
+
+# (tokens, outputs, K, operand, configuration): reductions that 64 divides and 128 does not, as small tiles; what the four-wave forms
+# do not take - rows off 16 bytes, fp32 results, the staged loop - as the shapes of eight waves
+@pytest.mark.parametrize(
+    "tokens,outputs,k,operand,config",
+    [(65, 2880, 2880, "native", "64x64"), (300, 2880, 1600, "native", "64x64"), (441, 5000, 64, "native", "128x128"),
+     (104, 1536, 1600, "pitch", "64x64"), (189, 6144, 2880, "pitch", "128x64"), (241, 12288, 1600, "pitch", "128x128"),
+     (65, 2880, 2880, "fp32", "64x64"), (600, 1536, 1600, "staged", "64x64"),
+     (2047, 4096, 2880, "native", "192x192 four"), (1822, 5760, 128, "native", "256x192 four")],
+)  # fmt: skip
+def test_tiles_of_a_projection(tokens, outputs, k, operand, config):
+    from rl_engine import _C, _lib
+
+    pad = 1 if operand == "pitch" else 0
+    x, w = _rand(tokens, k + pad)[:, :k], _rand(outputs, k + pad)[:, :k]
+    out = torch.empty((tokens, outputs), device=DEV, dtype=torch.float32 if operand == "fp32" else torch.bfloat16)
+    name, _, four = config.partition(" ")
+    asked = _lib.GEMM_CONFIGS[name] | (_lib.FOUR_WAVES if four else 0)
+    staged = _lib.FORCE_STAGED if operand == "staged" else 0
+    auto = launched(lambda: _C.gemm_strided(x, w.t(), out, config=staged))
+    assert auto == launched(lambda: _C.gemm_strided(x, w.t(), out, config=asked | staged))
+    assert len(auto) == 1 and ("det_gemm_solo_kernel" in auto[0]) == bool(four)
