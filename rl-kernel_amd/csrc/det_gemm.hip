@@ -344,6 +344,15 @@ static int pick_tile_candidate(int M, int N, int K, bool w_kmajor, bool x_kmajor
   return best_tile_candidate(M, N, K, w_kmajor, x_kmajor, kPartialEight, &estimate).config;
 }
 
+// Not where a single K tile is one round of the shape that eight waves would have: four have nothing in front of its loads (eight /
+// four waves, us, K = 64: 1822 x 5760 10.6 / 12.3, 1590 x 4096 8.6 / 11.6; of more rounds 6000 x 5760 28.6 / 20.9).
+static bool four_waves_pay(int M, int N, int K) {
+  if (K > kTileK) return true;
+  double estimate;
+  const TileCandidate& c = best_tile_candidate(M, N, K, false, false, kPartialEight, &estimate);
+  return tile_count(M, N, c.bm, c.bn) > device_cu_count();
+}
+
 double det_gemm_kmajor_us(int M, int N, int K, bool w_kmajor, bool x_kmajor, double partial_floor, int* tile_outputs) {
   double outputs;  // of 256 x 256 tiles at the native rate, 11 + 21 K / 1024 us each (see remainder_launch_pays)
   const TileCandidate& tile = best_tile_candidate(M, N, K, w_kmajor, x_kmajor, partial_floor, &outputs);
@@ -395,7 +404,7 @@ int pick_det_gemm_config(int M, int N, int K, bool four_waves) {
     if (tile_count(M, N, 160, 64) <= cus) return RLK_GEMM_CFG_64x160_DEEP;
     if (tile_count(M, N, 128, 128) <= cus) return RLK_GEMM_CFG_128x128_DEEP;
   }
-  return four_waves ? pick_four_wave_shape(M, N) : pick_tile_candidate(M, N, K, false, false);
+  return four_waves && four_waves_pay(M, N, K) ? pick_four_wave_shape(M, N) : pick_tile_candidate(M, N, K, false, false);
 }
 
 // A K-major view (element [row, k] at ptr[k * k_stride + row], rows contiguous: B[K,N] as the
@@ -533,9 +542,8 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     }
   }
   if (config == RLK_GEMM_CFG_AUTO) {
-    const bool takes = vec && allow_pingpong && four_waves_take(W, X, K, out_f32);
-    config = pick_det_gemm_config(M, N, K, takes);
-    four_waves = takes;
+    four_waves = vec && allow_pingpong && four_waves_take(W, X, K, out_f32) && four_waves_pay(M, N, K);
+    config = pick_det_gemm_config(M, N, K, four_waves);
     // the picked shape with one wave per SIMD (which a call can ask for, and which is 256 x 256 again for what it does not take)
     if (config == RLK_GEMM_CFG_256x256 && four_waves && solo_tiles_pay(tile_count(M, N, 256, 256), device_cu_count()))
       config = RLK_GEMM_CFG_256x256_SOLO;
