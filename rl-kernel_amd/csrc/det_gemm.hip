@@ -457,6 +457,16 @@ static bool four_waves_take(const MatView& W, const MatView& X, int K, bool out_
   return K % kTileK == 0 && !out_f32 && solo_offsets_fit(W) && solo_offsets_fit(X);
 }
 
+// K rows of a K-major weight a multiple of 4 KiB apart that is no power of two: the columns that four waves load each for itself take
+// longer there than the rows that eight load side by side. Eight / four, us, 256 x 128, K = 2880 at 200 tokens, by outputs: 4096 40.2 /
+// 38.4, 5120 45.1 / 41.7, 6144 42.1 / 43.9, 7680 44.1 / 41.9, 8192 40.4 / 38.2, 10240 44.4 / 45.7, 11264 43.1 / 43.6, 12288 43.1 / 47.4, 13312
+// 43.6 / 43.6, 14336 43.0 / 45.3, 16384 42.2 / 40.4, 18432 44.3 / 46.8, 20480 45.5 / 56.5; 256 x 192, K = 4096 at 700, 12288 69.7 / 77.5,
+// 14336 77.2 / 78.2, in two rounds, 2047 tokens, 214.6 / 199.8, 217.6 / 208.4. (256 x 256: four at every pitch.)
+static bool kmajor_rows_clash(const MatView& v) {
+  const int64_t pitch = v.k_stride * 2;
+  return pitch % 4096 == 0 && (pitch & (pitch - 1)) != 0;
+}
+
 hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t ldc, int M, int N, int K,
                            bool out_f32, int config, hipStream_t stream) {
   if (config == RLK_GEMM_CFG_AUTO && M > 256 && M % 256 >= 1 && M % 256 <= 64) {
@@ -499,10 +509,12 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
     // K = 151936) a smaller token tile doubles the workgroups, every one of which still streams its whole weight panel.
     if (config == RLK_GEMM_CFG_AUTO) {
       config = pick_tile_candidate(M, N, K, w_kmajor, x_kmajor);
-      // 256 x 192 always; 256 x 128 where the weight can still be in the memory-side cache: from HBM the eight waves are faster (12288
-      // outputs, K = 4096 at 324 / 483 tokens 58.9 / 61.1 us, four 65.4 / 68.7). Eight -> four: 4096 outputs at 1400 / 2047 tokens
-      // 59.5 / 66.7 -> 54.3 / 59.1, 256 x 192: 2300 tokens, K = 6144 104 -> 98, K = 14336 at 5969 495 -> 467.
-      four_waves = config == RLK_GEMM_CFG_256x192 || (int64_t)N * K * 2 < ((int64_t)96 << 20);
+      // 256 x 128 where the weight can still be in the memory-side cache, from HBM the eight waves are faster (12288 outputs, K = 4096 at
+      // 324 / 483 tokens 58.9 / 61.1 us, four 65.4 / 68.7), 256 x 192 wherever its rows do not clash in one round. Eight -> four: 4096
+      // outputs at 1400 / 2047 tokens 59.5 / 66.7 -> 54.3 / 59.1, 256 x 192: 2300 tokens, K = 6144 104 -> 98, K = 14336 at 5969 495 -> 467.
+      const bool clash = kmajor_rows_clash(W);
+      four_waves = config == RLK_GEMM_CFG_256x192 ? !clash || tile_count(M, N, 192, 256) > device_cu_count()
+                                                  : !clash && (int64_t)N * K * 2 < ((int64_t)96 << 20);
       if (config == RLK_GEMM_CFG_256x256 && solo_kmajor_pays(tile_count(M, N, 256, 256), device_cu_count(), w_kmajor && x_kmajor))
         config = RLK_GEMM_CFG_256x256_SOLO;
     }

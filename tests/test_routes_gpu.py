@@ -71,3 +71,22 @@ def test_tiles_of_a_projection(tokens, outputs, k, operand, config):
     auto = launched(lambda: _C.gemm_strided(x, w.t(), out, config=staged))
     assert auto == launched(lambda: _C.gemm_strided(x, w.t(), out, config=asked | staged))
     assert len(auto) == 1 and ("det_gemm_solo_kernel" in auto[0]) == bool(four)
+
+
+# K-major weights (rows of a multiple of 4 KiB that is no power of two: 6144, 12288 outputs): 256 x 128 and 256 x 192 with four waves or
+# with eight
+@pytest.mark.parametrize(
+    "tokens,outputs,config",
+    [(1024, 8192, "256x128 four"), (1000, 5128, "256x128 four"), (640, 12288, "256x128"), (1100, 6144, "256x128"),
+     (700, 12288, "256x192"), (1500, 6144, "256x192"), (700, 13312, "256x192 four"), (3400, 6144, "256x192 four")],
+)  # fmt: skip
+def test_tiles_of_a_kmajor_weight(tokens, outputs, config):
+    from rl_engine import _C, _lib
+
+    k = 256
+    x, w = _rand(tokens, k), _rand(k, outputs)
+    out = torch.empty((tokens, outputs), device=DEV, dtype=torch.bfloat16)
+    name, _, four = config.partition(" ")
+    auto = launched(lambda: _C.gemm_strided(x, w, out))
+    assert auto == launched(lambda: _C.gemm_strided(x, w, out, config=_lib.GEMM_CONFIGS[name] | (_lib.FOUR_WAVES if four else 0)))
+    assert len(auto) == 1 and ("det_gemm_solo_kernel" in auto[0]) == bool(four)
