@@ -132,10 +132,12 @@ typedef enum rlk_linear_bwd_config {
   RLK_LINEAR_BWD_CFG_SOLO_128 = 0x802
 } rlk_linear_bwd_config;
 
-/* The configuration that the automatic choice resolves to for contiguous operands of a shape: RLK_LINEAR_BWD_CFG_AUTO's,
- * the one that the fused linear-LogP backward runs both its gradients in (tokens x hidden size x vocabulary), or
- * RLK_LINEAR_BWD_CFG_MANY_WEIGHTS's; host only, no GPU call. */
+/* The configuration on eight waves that the automatic choice resolves to for contiguous operands of a shape:
+ * RLK_LINEAR_BWD_CFG_AUTO's, the one that the fused linear-LogP backward runs both its gradients in (tokens x hidden size x
+ * vocabulary), or RLK_LINEAR_BWD_CFG_MANY_WEIGHTS's. It runs unless rlk_linear_bwd_pick_solo() names the four-wave launch
+ * (RLK_LINEAR_BWD_CFG_SOLO, _192 or _128, else 0) that runs instead. Host only, no GPU call. */
 enum { RLK_LINEAR_BWD_OF_LINEAR = 0, RLK_LINEAR_BWD_OF_LOGP = 1, RLK_LINEAR_BWD_OF_MANY_WEIGHTS = 2 };
+int rlk_linear_bwd_pick_solo(int tokens, int inputs, int outputs, int of);
 int rlk_linear_bwd_pick_config(int tokens, int inputs, int outputs, int of);
 
 /*

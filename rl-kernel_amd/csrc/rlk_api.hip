@@ -127,25 +127,37 @@ static GemmProblem linear_dw(const void* dy, int64_t dy_ld, const void* x, int64
           dw, dw_ld, outputs, inputs, tokens};
 }
 
-int rlk_linear_bwd_pick_config(int tokens, int inputs, int outputs, int of) {
+// The plan of contiguous operands of a shape; `what` names the entry point in errors.
+static int linear_bwd_pick_plan(const char* what, int tokens, int inputs, int outputs, int of, LinearBackwardPlan* plan) {
   if (tokens < 1 || inputs < 1 || outputs < 1) {
-    set_last_error("rlk_linear_bwd_pick_config: tokens=%d inputs=%d outputs=%d must be positive", tokens, inputs, outputs);
+    set_last_error("%s: tokens=%d inputs=%d outputs=%d must be positive", what, tokens, inputs, outputs);
     return RLK_ERR_INVALID_ARGUMENT;
   }
   if (of < RLK_LINEAR_BWD_OF_LINEAR || of > RLK_LINEAR_BWD_OF_MANY_WEIGHTS) {
-    set_last_error("rlk_linear_bwd_pick_config: unknown backward %d", of);
+    set_last_error("%s: unknown backward %d", what, of);
     return RLK_ERR_INVALID_ARGUMENT;
   }
-  LinearBackwardPlan plan;
   if (of == RLK_LINEAR_BWD_OF_LOGP) {
-    plan = linear_logp_bwd_plan(tokens, inputs, outputs);
+    *plan = linear_logp_bwd_plan(tokens, inputs, outputs);
   } else {
     const void* any = reinterpret_cast<const void*>(uintptr_t{256});  // its alignment is all that is looked at
-    plan = linear_backward_plan(linear_dx(any, outputs, any, inputs, nullptr, inputs, tokens, inputs, outputs),
-                                linear_dw(any, outputs, any, inputs, nullptr, inputs, tokens, inputs, outputs),
-                                of == RLK_LINEAR_BWD_OF_LINEAR ? BackwardOf::kLinear : BackwardOf::kManyWeights);
+    *plan = linear_backward_plan(linear_dx(any, outputs, any, inputs, nullptr, inputs, tokens, inputs, outputs),
+                                 linear_dw(any, outputs, any, inputs, nullptr, inputs, tokens, inputs, outputs),
+                                 of == RLK_LINEAR_BWD_OF_LINEAR ? BackwardOf::kLinear : BackwardOf::kManyWeights);
   }
-  return plan.config | (plan.head_rows > 0 ? RLK_LINEAR_BWD_CFG_REST_BESIDE : 0);
+  return RLK_OK;
+}
+
+int rlk_linear_bwd_pick_config(int tokens, int inputs, int outputs, int of) {
+  LinearBackwardPlan plan;
+  const int status = linear_bwd_pick_plan("rlk_linear_bwd_pick_config", tokens, inputs, outputs, of, &plan);
+  return status != RLK_OK ? status : plan.config | (plan.head_rows > 0 ? RLK_LINEAR_BWD_CFG_REST_BESIDE : 0);
+}
+
+int rlk_linear_bwd_pick_solo(int tokens, int inputs, int outputs, int of) {
+  LinearBackwardPlan plan;
+  const int status = linear_bwd_pick_plan("rlk_linear_bwd_pick_solo", tokens, inputs, outputs, of, &plan);
+  return status != RLK_OK ? status : plan.solo_tokens == 0 ? 0 : RLK_LINEAR_BWD_CFG_SOLO + (256 - plan.solo_tokens) / 64;
 }
 
 int rlk_linear_bwd_bf16(const void* dy, int64_t dy_row_stride, const void* x, int64_t x_row_stride, const void* w,

@@ -74,6 +74,7 @@ EXPORTED_SYMBOLS = (
     "rlk_det_gemm_bf16",
     "rlk_linear_bwd_bf16",
     "rlk_linear_bwd_pick_config",
+    "rlk_linear_bwd_pick_solo",
     "rlk_det_gemm_pick_config",
     "rlk_det_gemm_tree_bf16",
     "rlk_det_gemm_tree_bf16_config",
@@ -148,6 +149,8 @@ def load() -> ctypes.CDLL:
     lib.rlk_linear_bwd_bf16.argtypes = [vp, i64, vp, i64, vp, i64, vp, i64, vp, i64, i32, i32, i32, i32, vp]
     lib.rlk_linear_bwd_pick_config.restype = i32
     lib.rlk_linear_bwd_pick_config.argtypes = [i32, i32, i32, i32]
+    lib.rlk_linear_bwd_pick_solo.restype = i32
+    lib.rlk_linear_bwd_pick_solo.argtypes = [i32, i32, i32, i32]
     lib.rlk_det_gemm_tree_bf16.restype = i32
     lib.rlk_det_gemm_tree_bf16.argtypes = [vp, i64, i64, vp, i64, i64, vp, i64, i32, i32, i32, vp]
     lib.rlk_det_gemm_tree_bf16_config.restype = i32

@@ -124,7 +124,19 @@ def test_the_launches_of_a_linear_backward(rlk_lib, of, m, k, n, config):
     assert rlk_lib.rlk_linear_bwd_pick_config(m, k, n, of) == config
 
 
+# (whose backward, tokens, inputs, outputs): the four-wave launch, its tiles of dX in 256, 192 and 128 tokens, or none
+@pytest.mark.parametrize(
+    "of,m,k,n,config",
+    [(0, 2047, 4096, 4096, 0x800), (0, 1508, 4096, 4096, 0x801), (0, 1024, 4096, 4096, 0x802), (0, 8192, 1024, 1024, 0),
+     (0, 603, 3072, 4096, 0), (0, 128, 4096, 4096, 0), (0, 2910, 4096, 12288, 0x800), (1, 4120, 4096, 151936, 0x800),
+     (1, 353, 4096, 151936, 0), (2, 4096, 4096, 12288, 0x800), (2, 300, 4096, 6144, 0)],
+)  # fmt: skip
+def test_the_four_wave_launch_of_a_linear_backward(rlk_lib, of, m, k, n, config):
+    assert rlk_lib.rlk_linear_bwd_pick_solo(m, k, n, of) == config
+
+
 def test_unknown_backwards_have_no_choice(rlk_lib):
+    assert rlk_lib.rlk_linear_bwd_pick_solo(64, 64, 64, 3) < 0 and rlk_lib.rlk_linear_bwd_pick_solo(0, 64, 64, 0) < 0
     assert rlk_lib.rlk_linear_bwd_pick_config(64, 64, 64, -1) < 0 and rlk_lib.rlk_linear_bwd_pick_config(64, 64, 64, 3) < 0
 
 

@@ -90,3 +90,22 @@ def test_tiles_of_a_kmajor_weight(tokens, outputs, config):
     auto = launched(lambda: _C.gemm_strided(x, w, out))
     assert auto == launched(lambda: _C.gemm_strided(x, w, out, config=_lib.GEMM_CONFIGS[name] | (_lib.FOUR_WAVES if four else 0)))
     assert len(auto) == 1 and ("det_gemm_solo_kernel" in auto[0]) == bool(four)
+
+
+# what rlk_linear_bwd_pick_solo() names is what runs, four waves and eight
+@pytest.mark.parametrize("tokens,inputs,outputs", [(2047, 4096, 4096), (1508, 4096, 4096), (1024, 4096, 4096), (8192, 1024, 1024), (128, 4096, 4096)])
+def test_launches_of_a_linear_backward(tokens, inputs, outputs):
+    from rl_engine import _lib
+
+    lib = _lib.load()
+    g, x, w = _rand(tokens, outputs), _rand(tokens, inputs), _rand(outputs, inputs)
+    dx, dw = torch.empty_like(x), torch.empty_like(w)
+
+    def backward(config):
+        assert 0 == lib.rlk_linear_bwd_bf16(g.data_ptr(), outputs, x.data_ptr(), inputs, w.data_ptr(), inputs, dx.data_ptr(), inputs,
+                                            dw.data_ptr(), inputs, tokens, inputs, outputs, config, torch.cuda.current_stream().cuda_stream)  # fmt: skip
+
+    solo = lib.rlk_linear_bwd_pick_solo(tokens, inputs, outputs, 0)
+    auto = launched(lambda: backward(0))
+    assert auto == launched(lambda: backward(solo or lib.rlk_linear_bwd_pick_config(tokens, inputs, outputs, 0)))
+    assert any("det_gemm_pair_solo_kernel" in n for n in auto) == (solo != 0)
