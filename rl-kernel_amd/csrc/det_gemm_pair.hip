@@ -379,11 +379,15 @@ LinearBackwardPlan linear_backward_plan(const GemmProblem& dx, const GemmProblem
     }
   }
   const bool small_dx = plan.config != RLK_LINEAR_BWD_CFG_SEPARATE && kPairTiles[plan.config].dx_bn < 256 && plan.head_rows == 0;
+  // Nor are those of 256 x 128 of dW, which are chosen where its few tiles of 256 x 256 would leave compute units idle (theirs / 192
+  // tokens on four waves, us: 1614, 2048, 2048 33.1 / 39.7; 3358, 1024, 4096 55.0 / 64.5; 803, 4096, 1024 21.1 / 25.0; 2960, 4096, 1024 51.3 /
+  // 59.8; 6069, 2880, 1440 107.1 / 118.1).
+  const bool half_dw = plan.config != RLK_LINEAR_BWD_CFG_SEPARATE && kPairTiles[plan.config].dw_bm < 256;
   // Below its fit solo_pair_us() took what eight waves do faster. Their launch / the one that it chose, us: behind the forward up to 256
   // tokens, 157, 12288, 4096 122.5 / 126.6, 163, 14336, 4096 141.4 / 144.3; with weights of which the forward left nothing in the caches up to
   // 448, the backward alone at 129, 12288, 4096 72.8 / 76.7, 264: 84.2 / 88.6, 440, 6144, 4096 67.6 / 70.9, 380, 14336, 4096 108.4 / 111.6.
   const int least_tokens = of == BackwardOf::kManyWeights ? 449 : 257;
-  if (!small_dx && dw.K >= least_tokens && solo_pair_serves(dx, dw)) {
+  if (!small_dx && !half_dw && dw.K >= least_tokens && solo_pair_serves(dx, dw)) {
     for (const int bm : {256, 192, 128}) {
       const double us = solo_pair_us(dx, dw, bm, cus);
       if (us < best) {

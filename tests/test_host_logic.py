@@ -131,7 +131,7 @@ def test_the_launches_of_a_linear_backward(rlk_lib, of, m, k, n, config):
      (0, 603, 3072, 4096, 0), (0, 128, 4096, 4096, 0), (0, 2910, 4096, 12288, 0x800), (1, 4120, 4096, 151936, 0x800),
      (1, 353, 4096, 151936, 0), (2, 4096, 4096, 12288, 0x800), (2, 300, 4096, 6144, 0),
      (0, 157, 12288, 4096, 0), (0, 256, 14336, 4096, 0), (0, 257, 14336, 4096, 0x801), (2, 129, 12288, 4096, 0), (2, 264, 12288, 4096, 0),
-     (2, 448, 6144, 4096, 0), (2, 449, 6144, 4096, 0x802)],
+     (2, 448, 6144, 4096, 0), (2, 449, 6144, 4096, 0x802), (0, 1614, 2048, 2048, 0), (0, 3358, 1024, 4096, 0), (0, 2960, 4096, 1024, 0)],
 )  # fmt: skip
 def test_the_four_wave_launch_of_a_linear_backward(rlk_lib, of, m, k, n, config):
     assert rlk_lib.rlk_linear_bwd_pick_solo(m, k, n, of) == config
