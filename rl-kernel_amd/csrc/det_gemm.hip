@@ -266,13 +266,13 @@ int device_cu_count() {
 // quarter by half read token rows four times; those reads and what arrives are 1856 cycles of LDS a K tile beside 1536 of MFMAs in 192
 // x 256, 1344 with four waves, 1536 / 1152 beside 1152 in 192 x 192. With them a round that fills part of the chip costs less, the more
 // so behind others (kPartialFirst, kPartialLast). Shapes without such a form are weighed beside them at their `native` quality, 256 x
-// 128 in one round at a better one. 560 shapes of 33 to 16000 tokens, 128 to 24576 outputs, K = 64 to 14336, weights in turn: where 128 does
+// 128 in one full round at a better one. 560 shapes of 33 to 16000 tokens, 128 to 24576 outputs, K = 64 to 14336, weights in turn: where 128 does
 // not divide K, which shuts out the deep tiles of few tokens, 0.983 of the eight waves' time, 0.6 % above the best shape of each, where
 // it does 0.935 and 1.2 %. Eight waves -> these, us: 4096 outputs, K = 4096 at 1400 / 2047 / 3000 tokens 53.9 / 62.8 / 79.1 -> 49.7 /
 // 57.8 / 73.8, 6144 at 1024 / 2048 / 3072 56.9 / 83.6 / 124.8 -> 51.7 / 78.4 / 117.9, K = 12288 at 2047 176 -> 164, 24576 outputs at 700 /
 // 1024 129.9 / 167.4 -> 120.2 / 156.6. What the small shapes and 256 x 128 are there for (the best without them / with): K = 2880, 2880
 // outputs at 65 / 200 tokens 31.9 / 32.9 -> 22.6 / 22.5, 5760 at 100 34.6 -> 23.1, K = 1600, 1536 outputs at 300 16.6 -> 11.2; K = 12288,
-// 8192 outputs at 1009 191 -> 169. (256 x 128 and 128 x 128 on four waves were never the best shape by more than the noise.)
+// 8192 outputs at 1009 191 -> 169 (but K = 4096, 14336 outputs at 487, 7 / 8 of a round, 58.9 / 62.7). (256 x 128 and 128 x 128 on four waves were never the best shape by more than the noise.)
 struct TileCandidate {
   int config, bn, bm;
   double native, ragged192, w_kmajor;
@@ -286,7 +286,7 @@ static const TileCandidate kTileCandidates[] = {
     {RLK_GEMM_CFG_256x64, 256, 64, 0.50, 0.00, 0.56, false, 0.00},   {RLK_GEMM_CFG_128x128, 128, 128, 0.65, 0.00, 0.62, false, 0.00},
     {RLK_GEMM_CFG_128x64, 128, 64, 0.45, 0.00, 0.40, false, 0.00},   {RLK_GEMM_CFG_64x64, 64, 64, 0.42, 0.00, 0.25, false, 0.00},
 };
-constexpr double kPartialFirst = 0.82, kPartialLast = 0.6, kFourRagged192 = 0.92, kPartialEight = 0.9, kOneRound256x128 = 0.80;
+constexpr double kPartialFirst = 0.82, kPartialLast = 0.6, kFourRagged192 = 0.92, kPartialEight = 0.9, kFullRound256x128 = 0.80;
 
 // The cheapest shape for operands that the four-wave forms take.
 static int pick_four_wave_shape(int M, int N) {
@@ -298,7 +298,7 @@ static int pick_four_wave_shape(int M, int N) {
     const bool one_round = tiles <= cus;
     double quality = c.four, partial = one_round ? kPartialFirst : kPartialLast;
     if (c.four == 0.0) {
-      quality = one_round && c.config == RLK_GEMM_CFG_256x128 ? kOneRound256x128 : c.native;
+      quality = one_round && 16 * tiles >= 15 * cus && c.config == RLK_GEMM_CFG_256x128 ? kFullRound256x128 : c.native;
       partial = kPartialEight;
     } else if (c.bn == 192 && N % 192 != 0) {
       quality *= kFourRagged192;
