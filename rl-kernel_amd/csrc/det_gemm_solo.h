@@ -172,39 +172,45 @@ __device__ __forceinline__ int solo_row_alignment(const void* C, int64_t ld) {
 
 // E results of a lane in a row (`packed` in pairs) at `to`, E elements into which the row's alignment goes on; `inside` of them are
 // columns of the result. For the waves whose features are not whole 16-byte spans inside the result: the last columns, and rows of
-// any pitch. Bound by the addresses that the stores of scattered rows take, so whole runs leave in the widest stores there are, from
-// odd addresses on in pairs behind one element. Eight waves a tile / four, element by element / this, us: 4000 tokens, K = 512,
-// 4100 outputs 27.1 / 61.2 / 24.3, 4098: 45.9 / 62.6 / 28.7, 4097: 57.8 / 61.9 / 31.0, K = 1024, 8274 tokens, 1000 outputs 24.4 / 29.5 /
-// 23.7; a K-major weight, 5152 tokens, 2808 outputs, K = 296 21.0 / 26.8 / 19.0; gated, 3000 tokens, K = 512, I = 5004 48.4 / 70.4 /
-// 37.0, 5001: 59.4 / 69.5 / 39.8. (A branch of its own for rows on 4 bytes: up to 10 % less there, and accumulators spilled.)
+// any pitch. Bound by the addresses that the stores of scattered rows take and by code that is fetched for the first time, so whole
+// runs leave in the widest stores there are, from odd addresses on in pairs behind one element, and the last columns in fours. Eight
+// waves a tile / four, element by element / this, us: 4000 tokens, K = 512, 4100 outputs 29.7 / 61.0 / 24.7, 4098: 46.3 / 63.3 / 28.9,
+// 4097: 56.0 / 62.5 / 30.5, K = 1024, 8274 tokens, 1000 outputs 23.4 / 27.4 / 21.5; a K-major weight, 5152 tokens, 2808 outputs, K =
+// 296 20.7 / 25.6 / 18.1; gated, 3000 tokens, K = 512, I = 5004 49.9 / 71.1 / 37.8, 5001: 58.9 / 71.1 / 39.6. (A branch of its own
+// for rows on 4 bytes: up to 10 % less there, and accumulators spilled.)
 template <int E>
 __device__ __forceinline__ void solo_store_run(bf16_bits* to, int inside, int alignment, const uint32_t (&packed)[E / 2]) {
   constexpr int kPairs = E / 2;
-  if (inside < E) {
+  if (inside >= E) {
+    if (E % 8 == 0 && alignment == 16) {
 #pragma unroll
-    for (int i = 0; i < kPairs; ++i) {
-      if (2 * i < inside) to[2 * i] = (bf16_bits)(packed[i] & 0xffffu);
-      if (2 * i + 1 < inside) to[2 * i + 1] = (bf16_bits)(packed[i] >> 16);
-    }
-  } else if (E % 8 == 0 && alignment == 16) {
+      for (int i = 0; i + 4 <= kPairs; i += 4)
+        *reinterpret_cast<u32x4_t*>(to + 2 * i) = u32x4_t{packed[i], packed[i + 1], packed[i + 2], packed[i + 3]};
+    } else if (alignment >= 8) {
 #pragma unroll
-    for (int i = 0; i + 4 <= kPairs; i += 4)
-      *reinterpret_cast<u32x4_t*>(to + 2 * i) = u32x4_t{packed[i], packed[i + 1], packed[i + 2], packed[i + 3]};
-  } else if (alignment >= 8) {
-#pragma unroll
-    for (int i = 0; i < kPairs; i += 2) *reinterpret_cast<u32x2_t*>(to + 2 * i) = u32x2_t{packed[i], packed[i + 1]};
-  } else {
-    const bool odd = (reinterpret_cast<uintptr_t>(to) & 2) != 0;
-    uint32_t* const words = reinterpret_cast<uint32_t*>(to + (odd ? 1 : 0));
-#pragma unroll
-    for (int i = 0; i + 1 < kPairs; ++i)
-      words[i] = odd ? __builtin_amdgcn_alignbit(packed[i + 1], packed[i], 16) : packed[i];
-    if (odd) {
-      to[0] = (bf16_bits)(packed[0] & 0xffffu);
-      to[E - 1] = (bf16_bits)(packed[kPairs - 1] >> 16);
+      for (int i = 0; i < kPairs; i += 2) *reinterpret_cast<u32x2_t*>(to + 2 * i) = u32x2_t{packed[i], packed[i + 1]};
     } else {
-      words[kPairs - 1] = packed[kPairs - 1];
+      const bool odd = (reinterpret_cast<uintptr_t>(to) & 2) != 0;
+      uint32_t* const words = reinterpret_cast<uint32_t*>(to + (odd ? 1 : 0));
+#pragma unroll
+      for (int i = 0; i + 1 < kPairs; ++i)
+        words[i] = odd ? __builtin_amdgcn_alignbit(packed[i + 1], packed[i], 16) : packed[i];
+      if (odd) {
+        to[0] = (bf16_bits)(packed[0] & 0xffffu);
+        to[E - 1] = (bf16_bits)(packed[kPairs - 1] >> 16);
+      } else {
+        words[kPairs - 1] = packed[kPairs - 1];
+      }
     }
+  } else if (inside > 0) {  // the last columns: fours, and element by element behind them
+    const int fours = alignment >= 8 ? inside & ~3 : 0;
+#pragma unroll
+    for (int i = 0; i < kPairs; i += 2)
+      if (2 * i < fours) *reinterpret_cast<u32x2_t*>(to + 2 * i) = u32x2_t{packed[i], packed[i + 1]};
+    if (fours == inside) return;
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (e >= fours && e < inside) to[e] = (bf16_bits)((packed[e >> 1] >> ((e & 1) * 16)) & 0xffffu);
   }
 }
 
