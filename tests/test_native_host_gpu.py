@@ -269,3 +269,30 @@ def test_captured_calls_replay():
             graph.replay()
             torch.cuda.synchronize()
             _same(out, call())
+
+
+def test_gradients_under_create_graph(general):
+    """Of a linear layer and of the FFN: values without a graph, as in the general way; of the loss: differentiable in both."""
+    from rl_engine.ops.ffn import qwen3_ffn
+    from rl_engine.ops.gemm import DetGemmOp
+    from rl_engine.ops.loss import grpo_ratio_kl_loss
+
+    op = DetGemmOp()
+    x, w, down = (t.requires_grad_() for t in (_normal(16, 64, seed=1), _normal(128, 64, seed=2, scale=0.1), _normal(64, 128, seed=3, scale=0.1)))
+    up = _normal(128, 64, seed=4, scale=0.1).requires_grad_()
+    logp = torch.randn(4, 32, device=DEV).mul_(0.1).requires_grad_()
+    fixed = [torch.randn(4, 32, device=DEV).mul_(0.1), torch.randn(4, 32, device=DEV).mul_(0.1), torch.randn(4, device=DEV)]
+
+    def gradients():
+        y, f = op.linear(x, w), qwen3_ffn(x, w, up, down)
+        loss = grpo_ratio_kl_loss(logp, *fixed, beta=0.1).loss
+        return [
+            *torch.autograd.grad(y, (x, w), torch.ones_like(y), create_graph=True),
+            *torch.autograd.grad(f, (x, w, up, down), torch.ones_like(f), create_graph=True),
+            *torch.autograd.grad(loss, logp, create_graph=True),
+        ]
+
+    got, want = gradients(), general(gradients)
+    assert [g.requires_grad for g in got] == [g.requires_grad for g in want] == [False] * 6 + [True]
+    _same(got[:6], want[:6])
+    torch.testing.assert_close(got[6], want[6], rtol=0, atol=0)

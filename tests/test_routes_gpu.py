@@ -110,3 +110,56 @@ def test_launches_of_a_linear_backward(tokens, inputs, outputs):
     auto = launched(lambda: backward(0))
     assert auto == launched(lambda: backward(solo or lib.rlk_linear_bwd_pick_config(tokens, inputs, outputs, 0)))
     assert any("det_gemm_pair_solo_kernel" in n for n in auto) == (solo != 0)
+
+
+# the kernels that the large shapes run by the automatic choices: on four waves, and on eight with few tiles
+def test_kernels_of_the_large_shapes():
+    from rl_engine import _C, _lib
+
+    lib = _lib.load()
+
+    def one(call, kernel):
+        names = [n for n in launched(call) if "merge" not in n]
+        assert any(kernel in n for n in names), names
+
+    x, w = _rand(4096, 256), _rand(4096, 256)
+    out = torch.empty((4096, 4096), device=DEV, dtype=torch.bfloat16)
+    one(lambda: _C.gemm_strided(x, w.t(), out), "det_gemm_solo_kernel")
+    one(lambda: _C.gemm_strided(x, w.t().contiguous(), out), "det_gemm_solo_kernel")
+    few = torch.empty((1024, 2048), device=DEV, dtype=torch.bfloat16)  # 32 tiles
+    one(lambda: _C.gemm_strided(x[:1024], w[:2048].t(), few, config=1), "det_gemm_kernel")
+    one(lambda: _C.det_gemm_swiglu(x, w), "det_gemm_swiglu_solo_kernel")
+    y = [torch.empty((4096, 4096), device=DEV, dtype=torch.bfloat16) for _ in range(3)]
+    stream = torch.cuda.current_stream().cuda_stream
+    one(lambda: lib.rlk_det_gemm_swiglu_training_bf16(x.data_ptr(), 256, w.data_ptr(), w.data_ptr(), 256, *(t.data_ptr() for t in y), 4096,
+                                                      4096, 4096, 256, stream), "det_gemm_swiglu_solo_kernel")  # fmt: skip
+
+
+# LogP above 1024 tokens: whole units on four waves, with a bias or few units on eight; both gradients in one launch of them
+@pytest.mark.parametrize("tokens,vocab,bias,logits,four", [(2048, 50257, False, False, True), (4000, 18992, False, True, True),
+                                                           (2048, 50257, True, False, False), (2048, 37984, False, False, False)])  # fmt: skip
+def test_units_of_the_logp(tokens, vocab, bias, logits, four):
+    from rl_engine import _C
+
+    h, w = _rand(tokens, 64), _rand(vocab, 64)
+    ids = torch.zeros(tokens, dtype=torch.int64, device=DEV)
+    b = torch.zeros(vocab, device=DEV) if bias else None
+    out = torch.empty(tokens, _C.linear_logp_logits_row_stride(vocab), device=DEV)
+    if logits:
+        names = launched(lambda: _C.fused_linear_logp_into(h, w, ids, b, None, vocab, out))
+    else:
+        names = launched(lambda: _C.fused_linear_logp(h, w, ids, b, None, False, vocab))
+    assert any("linear_logp_solo_kernel" in n for n in names) == four
+    assert any("linear_logp_partial_kernel" in n for n in names) != four
+
+
+@pytest.mark.parametrize("tokens,vocab", [(2050, 12337), (4120, 9000), (300, 9000)])
+def test_launches_of_the_logp_backward(tokens, vocab):
+    from rl_engine import _C, _lib
+
+    h, w = _rand(tokens, 2048), _rand(vocab, 2048).mul_(0.02)
+    ids = torch.zeros(tokens, dtype=torch.int64, device=DEV)
+    _, lse = _C.fused_linear_logp(h, w, ids)
+    grad = torch.ones(tokens, device=DEV)
+    names = launched(lambda: _C.fused_linear_logp_bwd(h, w, ids, lse, grad, None))
+    assert any("det_gemm_pair_solo_kernel" in n for n in names) == (_lib.load().rlk_linear_bwd_pick_solo(tokens, 2048, vocab, 1) != 0)
