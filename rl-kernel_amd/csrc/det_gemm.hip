@@ -354,7 +354,10 @@ static bool four_waves_pay(int M, int N, int K) {
 }
 
 double det_gemm_kmajor_us(int M, int N, int K, bool w_kmajor, bool x_kmajor, double partial_floor, int* tile_outputs) {
-  double outputs;  // of 256 x 256 tiles at the native rate, 11 + 21 K / 1024 us each (see remainder_launch_pays)
+  // Of 256 x 256 tiles at the native rate, 11 + 21 K / 1024 us each (see remainder_launch_pays): the eight-wave loops. On the four waves
+  // that det_gemm_launch() gives most of them the products take 2 to 10 % less, which the estimates of linear_backward_plan(), fitted
+  // beside this one, do not have.
+  double outputs;
   const TileCandidate& tile = best_tile_candidate(M, N, K, w_kmajor, x_kmajor, partial_floor, &outputs);
   if (tile_outputs) *tile_outputs = tile.bn * tile.bm;
   return (11.0 + 21.0 * K / 1024.0) * outputs / 65536.0;

@@ -171,8 +171,9 @@ __global__ __launch_bounds__(S::kThreads) void linear_logp_partial_kernel(LogpAr
 
 // One wave per SIMD (det_gemm_solo.h): the loads of a unit's vocabulary tile run ahead under the tile before and its fold, and
 // stored logits leave under the next tile's products. A lane holds two runs of 16 columns, i.e. two streams, of eight tokens.
-// Bound by the package's power cap, with stored logits also by HBM. Ping-pong -> this, us, V = 151936, D = 4096: 2048 tokens 1848 ->
-// 1808 (1410 TFLOP/s), 4200 3800 -> 3700, 8192 7027 -> 6870 (1484); with stored logits at 4120 tokens 4306 -> 4167. (A workgroup per CU
+// Bound by the package's power cap, with stored logits also by HBM. Ping-pong -> this, us, V = 151936, D = 4096, the same weights in one
+// process: 2048 tokens 1873 -> 1854, 4200 3816 -> 3712, 8192 7064 -> 7038 (one part in 300, 1449 TFLOP/s; 7027 -> 6870 on another
+// machine), 8200 7654 -> 7077; with stored logits at 2048 tokens 2152 -> 2085, 4120 4330 -> 4175. (A workgroup per CU
 // that goes through many units, as in the GEMM, measures the same up to 10 rounds of them; behind 18 the workgroups that share
 // panels have drifted apart: 1 % slower. The two runs of a token folded side by side: 4 % slower.)
 // ST: the tile of a last row of token tiles that has at most ST::BM tokens left, a four-wave loop over 256 columns x ST::BM tokens.
@@ -810,11 +811,6 @@ static int balanced_tail_splits(int T, int n_split, int cus) {
   return tail * per_split * 2 <= cus && n_split > tail ? tail : 0;
 }
 
-// `balance`: with the 256-token tile, a last round that would fill at most half of the chip
-// runs as 128-token tiles instead (twice the workgroups, each about 0.57 of the time): for
-// 256 tokens and V = 151936, 596 workgroups are 2.33 rounds of 256; 512 of them plus 168
-// half-height ones are two rounds and a short one (350 -> 290 us). Same bits: the tile height
-// is not part of the contract.
 template <int BM>
 static hipError_t launch_streams_solo_tile(LogpArgs a, float* spart, hipStream_t stream) {
   auto kernel = a.logits != nullptr ? linear_logp_streamgroup_solo_kernel<true, BM> : linear_logp_streamgroup_solo_kernel<false, BM>;
@@ -835,6 +831,11 @@ static hipError_t launch_stream_merge(const LogpArgs& a, const float* spart, hip
   return hipGetLastError();
 }
 
+// `balance`: with the 256-token tile, a last round that would fill at most half of the chip
+// runs as 128-token tiles instead (twice the workgroups, each about 0.57 of the time): for
+// 256 tokens and V = 151936, 596 workgroups are 2.33 rounds of 256; 512 of them plus 168
+// half-height ones are two rounds and a short one (350 -> 290 us). Same bits: the tile height
+// is not part of the contract.
 template <class S>
 static hipError_t launch_streamgroup(LogpArgs a, bool balance, hipStream_t stream) {
   float* spart = a.part + (size_t)3 * a.n_split * a.T;  // behind the per-split partials

@@ -7,9 +7,11 @@
 // in the stretches in which autograd's device thread has to be woken for every backward.
 //
 // Every function takes everyday arguments only and answers None to anything else - other types, layouts and devices, subclasses,
-// batched and functorch tensors, tangents, dispatch and function modes, tracing, profilers -, for which the caller goes the way it
-// went before. The autograd functions hand what is not everyday in a backward (create_graph, gradients or saved tensors that are
-// more than their values) to the Python functions that bind() was given. Nothing is kept from one call for the next.
+// batched and functorch tensors, tangents, dispatch and function modes (torch.set_default_device() is one), tracing, profilers -, for
+// which the caller goes the way it went before. The autograd functions hand what is not everyday in a backward (an operand that wants
+// no gradient, gradients or saved tensors that are more than their values) to the Python functions that bind() was given. Under
+// create_graph the loss does so too, whose gradient is differentiable; those of the linear layer and the FFN have no graph either way.
+// Nothing is kept from one call for the next.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
