@@ -502,6 +502,7 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
   const bool vec = w_native && x_native && (K % kChunkElems) == 0;
   const bool allow_pingpong = (config & RLK_GEMM_CFG_FORCE_STAGED) == 0;
   bool four_waves = (config & RLK_GEMM_CFG_FOUR_WAVES) != 0;
+  const bool automatic = (config & ~RLK_GEMM_CFG_FORCE_STAGED) == RLK_GEMM_CFG_AUTO;
   config &= ~(RLK_GEMM_CFG_FORCE_STAGED | RLK_GEMM_CFG_FOUR_WAVES);
   const bool w_kmajor = !w_native && view_is_kmajor_fast(W), x_kmajor = !x_native && view_is_kmajor_fast(X);
   if (allow_pingpong && det_gemm_takes_kmajor(W, X, K)) {
@@ -630,6 +631,15 @@ hipError_t det_gemm_launch(const MatView& W, const MatView& X, void* C, int64_t 
   // 565 / 779, 6144 at 768 (192 x 128) 295 / 567; K = 128: 36.5 / 35.4, 64: 26.5 / 25.2.
   if (!vec && (config == RLK_GEMM_CFG_256x256 || config == RLK_GEMM_CFG_256x128 || config == RLK_GEMM_CFG_256x64))
     config = RLK_GEMM_CFG_128x128;
+  // A round of 256 x 128 takes 5.5 us a K tile, one of 128 x 128 4.8, full or not, so the first where it saves a round: odd pitch, as
+  // 128 x 128 / 256 x 128, K = 4992, 4096 outputs at 1452 tokens (384 / 192 tiles) 775 / 429, K = 2048, 8695 outputs at 1830 (1020 / 510) 661 /
+  // 393, but K = 2880, 4096 at 830 (224 / 112) 215 / 244. Not of short reductions, whose tiles are their stores: K = 200, 6141 outputs, K-major
+  // tokens at 1733 62 / 73 (K = 320, a K-major weight, 2875 at 2206 60.0 / 47.6).
+  if (!vec && automatic && config == RLK_GEMM_CFG_128x128 && K >= 256) {
+    const int64_t cus = device_cu_count();
+    const int64_t rounds128 = (tile_count(M, N, 128, 128) + cus - 1) / cus, rounds256 = (tile_count(M, N, 128, 256) + cus - 1) / cus;
+    if (25 * rounds128 > 28 * rounds256) config = RLK_GEMM_CFG_256x128;
+  }
   if (config == RLK_GEMM_CFG_192x128) {
     if (vec && allow_pingpong && K % kTileK == 0)
       return launch_loop<Shape192x128, kLoopPingPong, pingpong_stages<Shape192x128>()>(W, X, C, ldc, M, N, K, out_f32, stream);

@@ -55,7 +55,7 @@ def test_stream_groups_of_the_logp(tokens, vocab, hidden, logits, four):
 @pytest.mark.parametrize(
     "tokens,outputs,k,operand,config",
     [(65, 2880, 2880, "native", "64x64"), (300, 2880, 1600, "native", "64x64"), (441, 5000, 64, "native", "128x128"),
-     (104, 1536, 1600, "pitch", "64x64"), (189, 6144, 2880, "pitch", "128x64"), (241, 12288, 1600, "pitch", "128x128"),
+     (104, 1536, 1600, "pitch", "64x64"), (1452, 4096, 320, "pitch", "192x128"), (830, 4096, 64, "pitch", "128x128"), (189, 6144, 2880, "pitch", "128x64"), (241, 12288, 1600, "pitch", "128x128"),
      (65, 2880, 2880, "fp32", "64x64"), (600, 1536, 1600, "staged", "64x64"), (1822, 5760, 64, "native", "256x192"),
      (1590, 4096, 64, "native", "256x128"), (6000, 5760, 64, "native", "192x256 four"),
      (2047, 4096, 2880, "native", "192x192 four"), (1822, 5760, 128, "native", "256x192 four")],
