@@ -891,22 +891,24 @@ static StreamsChoice best_streams(int T, int n_split) {
 // 138 -> 122; 595, 131072, 2048 394 -> 348; 891, 151936, 4096 1013 -> 964; with stored logits 127, 32768, 2048 54 -> 42; 548, 151936, 4096 678 -> 640;
 // 753, 131072, 2048 502 -> 451; it stays with eight at 698, 37984, 4096 (230 / 248) and 995, 32768, 2048 (154 / 160).
 static int pick_streams_solo(const LogpArgs& a) {
-  // One token tile of 128. A weight that HBM alone sets the pace of is read past the caches (V = 151936, D = 4096 at 76 / 99 tokens 253 / 257, 258 /
-  // 260; V = 131072, D = 2048 at 83 tokens 147 / 145). Where most CUs have one tile, its fold and the stores of its logits run behind
-  // the loads of nothing else, and four waves take longer for them (eight / four, us): with stored logits from 100 tiles on until every CU
-  // has two, 96, 24576, 4096 (96 tiles) 83.5 / 83.2; 96, 37984, 4096 (152) 96.2 / 102.6; 96, 50257, 4096 (200) 112.4 / 122.1; 120, 80000, 4096
-  // (316) 203.8 / 212.2; 96, 131072, 2048 (512) 172 / 168; without them from 144 on, 96, 32768, 4096 (128) 90.2 / 89.5; 120, 40960, 4096 (160)
-  // 96.6 / 98.5; 120, 60000, 4096 (236) 119.9 / 123.6; 120, 66000, 2048 (260) 117.6 / 114.6; 96, 32000, 8192 146.7 / 148.1. A vocabulary that
-  // ends in the first half of a split has two of its four tiles empty, which eight waves leave out: 79, 500, 256 18.2 / 20.3, with logits
-  // 18.7 / 23.6; 100, 512, 1024 25.5 / 26.2, 26.3 / 28.6; 289, 500, 576 with logits 22.8 / 26.4, but D = 2048 34.9 / 33.9, 35.4 / 36.3, and at
-  // 129 to 256 tokens, for which the eight waves' tile is one of 256 tokens, 165, 500, 576 30.7 / 24.8.
+  // One token tile of 128. A weight that HBM alone sets the pace of is read past the caches (V = 151936, D = 4096 at 76 / 99 tokens 253 / 257,
+  // 258 / 260; V = 131072, D = 2048 at 83 tokens 147 / 145). Where most CUs have one tile, its fold and the stores of its logits run
+  // behind the loads of nothing else, and four waves lose what they are ahead with weights that come from HBM (eight / four, us):
+  //   with stored logits from 100 tiles on until every CU has two: 96, 24576, 4096 (96 tiles) 83.5 / 83.2; 96, 37984, 4096 (152) 96.2 / 102.6; 96,
+  //   50257, 4096 (200) 112.4 / 122.1; 120, 80000, 4096 (316) 203.8 / 212.2; 96, 131072, 2048 (512) 172 / 168; 1.08 and 1.04 times at 62000 rows of
+  //   181 MiB, 1.00 and 0.98 at 37984 of 185, 0.95 at 31014 of 113;
+  //   without them from 144 tiles to a round: 96, 32768, 4096 (128) 90.2 / 89.5; 120, 40960, 4096 (160) 96.6 / 98.5; 120, 60000, 4096 (236) 119.9 /
+  //   123.6; 120, 66000, 2048 (260) 117.6 / 114.6; 96, 32000, 8192 146.7 / 148.1; 1.05 times at 50257 rows of 294 MiB, 1.01 of 245, 0.97 of 184.
+  // A vocabulary that ends in the first half of a split has two of its four tiles empty, which eight waves leave out: 79, 500, 256 18.2 /
+  // 20.3, with logits 18.7 / 23.6; 100, 512, 1024 25.5 / 26.2, 26.3 / 28.6; 289, 500, 576 with logits 22.8 / 26.4, but D = 2048 34.9 / 33.9, 35.4 /
+  // 36.3, and at 129 to 256 tokens, for which the eight waves' tile is one of 256 tokens, 165, 500, 576 30.7 / 24.8.
   if (a.V <= 2 * kLogpTileCols && a.D < 2048 && (a.T <= 128 || a.T > 256)) return 0;
   if (a.T <= 128) {
-    const int64_t bytes = 2 * (int64_t)a.V * a.D, tiles = (int64_t)a.n_split * (kLogpStreams / 4);
+    const int64_t mib = ((int64_t)a.V * a.D) >> 19, tiles = (int64_t)a.n_split * (kLogpStreams / 4);
     const int cus = device_cu_count();
-    if (bytes >= ((int64_t)1 << 30)) return 0;
-    if (a.logits != nullptr ? 64 * tiles > 25 * cus && tiles < 2 * cus
-                            : tiles <= cus && (16 * tiles > 9 * cus || bytes >= ((int64_t)500 << 20)))
+    if (mib >= 1024) return 0;
+    if (a.logits != nullptr ? 64 * tiles > 25 * cus && tiles < 2 * cus && mib >= 192
+                            : tiles <= cus && mib >= (16 * tiles > 9 * cus ? 224 : 480))
       return 0;
   }
   constexpr double kPartial = 0.965;

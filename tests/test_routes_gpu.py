@@ -27,14 +27,15 @@ def _rand(*shape):
     return torch.randn(shape, device=DEV, dtype=torch.bfloat16)
 
 
-# (tokens, vocabulary, hidden, stored logits, four waves); 76, 128, 132, 152, 260 and 512 tiles, a vocabulary of half a split and one more
+# (tokens, vocabulary, hidden, stored logits, four waves); 76, 128, 132, 152, 260 and 512 tiles of weights below and from 192 MiB (with
+# stored logits) and 224 MiB, a vocabulary of half a split and one more
 @pytest.mark.parametrize(
     "tokens,vocab,hidden,logits,four",
-    [(96, 18992, 64, False, True), (96, 18992, 64, True, True), (96, 32768, 64, False, True), (128, 33000, 64, True, False),
-     (128, 33000, 64, False, True), (96, 37984, 64, True, False), (96, 37984, 64, False, False), (65, 66000, 64, True, False),
-     (65, 66000, 64, False, True), (96, 131072, 64, True, True), (96, 131072, 64, False, True), (100, 512, 64, False, False),
-     (100, 500, 64, True, False), (100, 513, 64, True, True), (300, 512, 64, False, False), (300, 513, 64, True, True),
-     (200, 512, 64, True, True)],
+    [(96, 18992, 64, False, True), (96, 18992, 64, True, True), (96, 32768, 64, False, True), (128, 33000, 64, True, True),
+     (128, 33000, 3072, True, False), (128, 33000, 3072, False, True), (96, 37984, 3072, False, True),
+     (96, 37984, 3136, False, False), (65, 66000, 1024, True, True), (65, 66000, 1600, True, False), (65, 66000, 1600, False, True),
+     (96, 131072, 64, True, True), (96, 131072, 64, False, True), (100, 512, 64, False, False), (100, 500, 64, True, False),
+     (100, 513, 64, True, True), (300, 512, 64, False, False), (300, 513, 64, True, True), (200, 512, 64, True, True)],
 )  # fmt: skip
 def test_stream_groups_of_the_logp(tokens, vocab, hidden, logits, four):
     from rl_engine import _C
