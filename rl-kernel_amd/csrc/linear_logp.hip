@@ -762,6 +762,20 @@ static bool logp_solo_pays(const LogpArgs& a) {
   const bool spans = a.logits == nullptr || ((a.logits_ld & 3) == 0 && (reinterpret_cast<uintptr_t>(a.logits) & 15) == 0);
   if (!spans || a.bias != nullptr || !solo_offsets_fit(a.W) || !solo_offsets_fit(a.H)) return false;
   const int cus = device_cu_count();
+  const int whole = a.T / SoloShape::BM, rest = a.T % SoloShape::BM;
+  // Units of a last tile of up to 128 tokens that come behind the others. Eight waves are ahead, four / eight in us,
+  //   where they open a round behind one or two of few token tiles: V = 32768, D = 2880 at 2158 tokens (256 + 32 units) 500 / 423; V = 24576,
+  //   D = 1024 at 2635 (240 + 24) 209 / 182; V = 49152, D = 2048 at 2646 (480 + 48) 549 / 492; V = 37984, D = 1024 at 1658 (228 + 38) 208 / 190, but
+  //   with stored logits, where the rounds before are not nearly full, 261 / 274 at 1624; from 12 token tiles on V = 37984, D = 2048 at 3436
+  //   652 / 680, V = 24576, D = 4096 at 5478 1112 / 1167;
+  //   with stored logits just above one round: V = 32768, D = 2048 at 2311 (288 + 32) 445 / 415; V = 37984, D = 4096 at 1820 (266 + 38) 730 / 733;
+  //   but V = 50257, D = 4096 at 1564 (300 + 50) 752 / 771, V = 37984, D = 2880 at 2108 (304 + 38) 563 / 574.
+  if (rest >= 1 && rest <= 128 && logp_rest_behind(whole, a.n_split, cus)) {
+    const int64_t ahead = (int64_t)whole * a.n_split, all = ahead + a.n_split;
+    const bool opens = ahead <= 2 * cus && (all - 1) / cus > (ahead - 1) / cus;
+    if (rest > 64 && whole < 12 && opens && (a.logits == nullptr || ((ahead - 1) % cus + 1) * 16 >= 15 * cus)) return false;
+    if (a.logits != nullptr && ahead > cus && 8 * ahead <= 9 * cus) return false;
+  }
   const int64_t units = (int64_t)((a.T + 127) / SoloShape::BM) * a.n_split;
   if (units < cus) return 10 * units >= 7 * cus;  // (160 units, V = 32768, D = 2048 at 1356 tokens with logits, 206 / 213; 190, V = 37984 at 1193, 346 / 333)
   return solo_tiles_pay(units, cus) || a.logits != nullptr;

@@ -16,11 +16,12 @@ def _same(a, b):
     return torch.equal(a.contiguous().view(torch.int32), b.contiguous().view(torch.int32))
 
 
-# (tokens, vocabulary, hidden, real vocabulary): units of 192 to 300 (whole round and more of 256 CUs), 1 ... 4 tiles in the last split
+# (tokens, vocabulary, hidden, real vocabulary): units of 192 to 320 (whole round and more of 256 CUs), 1 ... 4 tiles in the last split
 @pytest.mark.parametrize(
     "tokens,vocab,hidden,real",
     [(1024 + 1, 50000, 64, 50000), (1280 + 64, 45001, 64, 44900), (1536 + 65, 40704, 128, 40704), (2048 + 128, 32769, 64, 32769),
-     (2048 + 129, 33024, 64, 32000), (2303, 28672, 192, 28672), (4096, 17000, 64, 16999), (4096 + 30, 16641, 64, 16641)],
+     (2048 + 129, 33024, 64, 32000), (2303, 28672, 192, 28672), (4096, 17000, 64, 16999), (4096 + 30, 16641, 64, 16641),
+     (3072 + 100, 25000, 64, 25000), (3072 + 1, 25473, 128, 25400), (2048 + 64, 40001, 64, 40001)],
 )  # fmt: skip
 @pytest.mark.parametrize("temperature", [False, True])
 def test_same_bits_as_the_small_token_tiles(tokens, vocab, hidden, real, temperature):
@@ -56,7 +57,7 @@ def test_targets_of_another_shard_and_strided_logits():
     assert bool(torch.isnan(out[0][0][outside]).all()) and not bool(torch.isnan(out[0][0][~outside]).any())
 
 
-@pytest.mark.parametrize("vocab", [33001, 33088])
+@pytest.mark.parametrize("vocab", [33001, 33088, 40001, 40064])
 def test_kept_logits_are_the_returned_ones_and_end_at_the_vocabulary(vocab):
     from rl_engine import _C
 

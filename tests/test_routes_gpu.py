@@ -136,9 +136,14 @@ def test_kernels_of_the_large_shapes():
                                                       4096, 4096, 256, stream), "det_gemm_swiglu_solo_kernel")  # fmt: skip
 
 
-# LogP above 1024 tokens: whole units on four waves, with a bias or few units on eight; both gradients in one launch of them
+# LogP above 1024 tokens: units on four waves, with a bias or few units on eight; both gradients in one launch of them
 @pytest.mark.parametrize("tokens,vocab,bias,logits,four", [(2048, 50257, False, False, True), (4000, 18992, False, True, True),
-                                                           (2048, 50257, True, False, False), (2048, 37984, False, False, False)])  # fmt: skip
+                                                           (2048, 50257, True, False, False), (2048, 37984, False, False, False),
+                                                           # a rest of up to 128 tokens: whose units open a round behind one or two, or with
+                                                           # stored logits just above one round; and the nearest that don't
+                                                           (2126, 32768, False, False, False), (2110, 32768, False, True, True), (2060, 32768, False, False, True),
+                                                           (3430, 37984, False, True, True), (1640, 37984, False, True, True), (1640, 37984, False, False, False),
+                                                           (2311, 32768, False, True, False), (2320, 37984, False, True, True)])  # fmt: skip
 def test_units_of_the_logp(tokens, vocab, bias, logits, four):
     from rl_engine import _C
 
