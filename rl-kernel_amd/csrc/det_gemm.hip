@@ -272,7 +272,8 @@ int device_cu_count() {
 // 57.8 / 73.8, 6144 at 1024 / 2048 / 3072 56.9 / 83.6 / 124.8 -> 51.7 / 78.4 / 117.9, K = 12288 at 2047 176 -> 164, 24576 outputs at 700 /
 // 1024 129.9 / 167.4 -> 120.2 / 156.6. What the small shapes and 256 x 128 are there for (the best without them / with): K = 2880, 2880
 // outputs at 65 / 200 tokens 31.9 / 32.9 -> 22.6 / 22.5, 5760 at 100 34.6 -> 23.1, K = 1600, 1536 outputs at 300 16.6 -> 11.2; K = 12288,
-// 8192 outputs at 1009 191 -> 169 (but K = 4096, 14336 outputs at 487, 7 / 8 of a round, 58.9 / 62.7). (256 x 128 and 128 x 128 on four waves were never the best shape by more than the noise.)
+// 8192 outputs at 1009 191 -> 169 (but K = 4096, 14336 outputs at 487, 7 / 8 of a round, 58.9 / 62.7). (256 x 128 and 128 x 128 on four
+// waves were never the best shape by more than the noise.)
 struct TileCandidate {
   int config, bn, bm;
   double native, ragged192, w_kmajor;
